@@ -118,8 +118,8 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     __shared__ float decayed[12][2][256];
     // clip factor left on the device by the gradient-norm pass (1.0 when there is none)
     const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
-    for (uint32_t i = threadIdx.x; i < kLdsImageBytes / 16; i += blockDim.x) lds_raw[i] = lds_image[i];
-    __syncthreads();
+    stage_begin<kLdsImageBytes>(lds_raw, lds_image);
+    stage_end();
     const char *base = reinterpret_cast<const char *>(lds_raw);
     Lds L;
     L.map_s = reinterpret_cast<const float *>(base + kOffMapS);

@@ -32,8 +32,8 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
     // the binary search needs the maps and midpoints only (4 KB); the slot tables are the other 96 KB
     constexpr uint32_t staged = KEYTAB ? kLdsImageBytes : kOffKeyU;
-    for (uint32_t i = threadIdx.x; i < staged / 16; i += blockDim.x) lds_raw[i] = lds_image[i];
-    __syncthreads();
+    stage_begin<staged>(lds_raw, lds_image);
+    stage_end();
     const char *base = reinterpret_cast<const char *>(lds_raw);
     Lds L;
     L.map_s = reinterpret_cast<const float *>(base + kOffMapS);

@@ -33,8 +33,8 @@ __global__ __launch_bounds__(1024) void adam8_step_split_kernel(const DevTensor 
     const uint32_t quarter = wave_in_wg & 3; // which 512 elements of the team's block
     const uint32_t o = quarter * 512 + lane * 8;
 
-    // One quarter block as it comes from memory.  The first one is requested before the table image is
-    // staged, so that its trip to HBM overlaps the staging.
+    // One quarter block as it comes from memory.  The first one is requested while the table image is on its way.
+    stage_begin<kLdsImageBytes>(lds_raw, lds_image);
     struct Quarter {
         DevTensor t;
         uint32_t lb;
@@ -63,8 +63,7 @@ __global__ __launch_bounds__(1024) void adam8_step_split_kernel(const DevTensor 
     };
     request(blockIdx.x * teams);
 
-    for (uint32_t i = threadIdx.x; i < kLdsImageBytes / 16; i += blockDim.x) lds_raw[i] = lds_image[i];
-    __syncthreads();
+    stage_end();
     const char *base = reinterpret_cast<const char *>(lds_raw);
     Lds L;
     L.map_s = reinterpret_cast<const float *>(base + kOffMapS);
