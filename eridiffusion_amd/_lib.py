@@ -114,6 +114,8 @@ EXPORTS = {
     "eri_adam8_step_multi": (C.c_int, [C.POINTER(TensorRow), C.c_uint32, C.POINTER(Hyper), C.c_void_p]),
     "eri_adam8_dequantize": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_uint64, C.c_void_p, C.c_void_p]),
     "eri_adam8_quantize": (C.c_int, [C.c_void_p, C.c_int, C.c_uint64, C.c_void_p, C.c_void_p, C.c_void_p]),
+    "eri_adam8_dequantize_state": (C.c_int, [C.c_void_p] * 4 + [C.c_uint64] + [C.c_void_p] * 3),
+    "eri_adam8_quantize_state": (C.c_int, [C.c_void_p] * 2 + [C.c_uint64] + [C.c_void_p] * 5),
     "eri_adamw32_step_multi": (C.c_int, [C.POINTER(AdamW32Row), C.c_uint32, C.POINTER(AdamW32Hyper), C.c_void_p]),
     "eri_adamw32_step_multi_scaled": (C.c_int, [C.POINTER(AdamW32Row), C.c_uint32, C.POINTER(AdamW32Hyper), C.c_float,
                                               C.c_void_p, C.c_void_p]),

@@ -74,6 +74,20 @@ constexpr uint32_t kLdsImageBytes = kOffKeyS + kSKeyCount * kSKeyStride;
 static_assert(kOffKeyS < 65536 && kOffKeyU < 65536, "slot table offsets must fit a ds_read immediate");
 static_assert(kLdsImageBytes % 16 == 0, "the image is staged in 16-byte words");
 
+/* The same lookup in 12 KB, for kernels that cannot afford to stage 100 KB per workgroup: a slot keeps only its `lo`,
+ * one byte.  Its midpoint need not be stored, because the one midpoint a slot can contain is midpoint number `lo`,
+ * and where it contains none, no quotient of the slot lies above midpoint `lo` either:
+ *     code(x) = lo[slot] + (x * kKeyScale > scaled_mid[lo[slot]])
+ * Two dependent LDS reads instead of one. */
+constexpr uint32_t kSmallMapS = 0;                        /* 256 floats: code -> value */
+constexpr uint32_t kSmallMapU = kSmallMapS + 1024;
+constexpr uint32_t kSmallMidS = kSmallMapU + 1024;        /* 255 midpoints times kKeyScale + one +inf */
+constexpr uint32_t kSmallMidU = kSmallMidS + 1024;
+constexpr uint32_t kSmallLoS = kSmallMidU + 1024;         /* kSKeyCount bytes */
+constexpr uint32_t kSmallLoU = kSmallLoS + kSKeyCount;    /* kUKeyCount bytes */
+constexpr uint32_t kSmallImageBytes = kSmallLoU + kUKeyCount;
+static_assert(kSmallImageBytes % 1024 == 0, "the image is staged in pieces of 1 KB");
+
 /* Launchers implemented in eri_adam8_kernels.hip; `stream` is a hipStream_t.  All return a
  * hipError_t as int.  `lds_image` is the device copy of the kLdsImageBytes table image. */
 int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, int layout,
@@ -133,10 +147,16 @@ int launch_traffic_probe(const DevTensor *rows, uint32_t n_rows, uint32_t total_
 /* Clears `bytes` bytes at `p`; both multiples of 16. */
 int launch_fill_zero(void *p, size_t bytes, void *stream);
 int launch_state_init(uint8_t *m, uint8_t *v, float *absmax_m, float *absmax_v, uint64_t numel, void *stream);
-int launch_dequantize(const uint8_t *codes, const float *absmax, int signed_map, uint64_t numel, float *out,
-                      const void *lds_image, void *stream);
-int launch_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax,
-                    const void *lds_image, void *stream);
+/* fp32 moments <-> codes and absmax, one or two moments of `numel` elements in one launch; `small_image` is the device
+ * copy of the kSmallImageBytes image. */
+struct MomentArgs {
+    float *x[2];       /* fp32 values: read by quantize, written by dequantize */
+    uint8_t *codes[2];
+    float *absmax[2];
+    int32_t is_signed[2];
+};
+int launch_dequantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream);
+int launch_quantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream);
 
 /* Row of the plain element-wise sweeps (32-bit AdamW, EMA): up to five streams of one tensor. */
 struct ElemRow {

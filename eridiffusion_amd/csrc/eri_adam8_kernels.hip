@@ -180,59 +180,165 @@ int launch_state_init(uint8_t *m, uint8_t *v, float *absmax_m, float *absmax_v, 
     return (int)hipGetLastError();
 }
 
-__global__ void dequantize_kernel(const uint8_t *codes, const float *absmax, uint64_t numel, float *out,
-                                  const float *map) {
-    __shared__ float lmap[256];
-    lmap[threadIdx.x] = map[threadIdx.x];
-    __syncthreads();
-    const uint64_t n = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < numel; i += n)
-        out[i] = lmap[codes[i]] * absmax[i / kBlock];
+/* Checkpoint traffic: fp32 moments to codes and absmax and back.  HBM is the bound, 5 bytes per element (4 of fp32, 1 of
+ * code) each way; blockIdx.y is the moment, so that both moments of a tensor are one launch.  One wave takes a
+ * 2048-element block: lane l of pass c holds elements c*256 + 4l .. +3, which is one 128-bit access of fp32 and one
+ * 32-bit access of codes per lane, both contiguous over the wave.
+ * Measured on both moments of 24 tensors, 340 M parameters: quantise 2.84 -> 0.69 ms in all, dequantise 1.51 -> 0.68 ms,
+ * 5.0 TB/s each (before: one element per access, IEEE division, an eight-step search, a launch per moment). */
+constexpr uint32_t kMomentThreads = 256;
+
+/* Pass c of a block of n elements: whole = this lane's four elements exist, else the ones below n - o do. */
+template <bool VEC>
+__device__ __forceinline__ f32x4 moment_load(const float *x, uint32_t o, uint32_t n) {
+    f32x4 r = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (VEC && o + 4 <= n) return __builtin_nontemporal_load(as_global(reinterpret_cast<const f32x4 *>(x + o)));
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (o + k < n) r[k] = as_global(x)[o + k];
+    return r;
 }
 
-int launch_dequantize(const uint8_t *codes, const float *absmax, int signed_map, uint64_t numel, float *out,
-                      const void *lds_image, void *stream) {
-    const float *map = reinterpret_cast<const float *>(static_cast<const char *>(lds_image) +
-                                                       (signed_map ? kOffMapS : kOffMapU));
-    uint64_t grid = (numel + 255) / 256;
-    if (grid > 16384) grid = 16384;
-    hipLaunchKernelGGL(dequantize_kernel, dim3((uint32_t)grid), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       codes, absmax, numel, out, map);
-    return (int)hipGetLastError();
+template <bool SIGNED>
+__device__ __forceinline__ uint32_t small_code(float xs, uint32_t half, const unsigned char *lo, const float *mid) {
+    const uint32_t base = lo[SIGNED ? half >> kSKeyDrop : (half & 0x7fffu) >> kUKeyDrop];
+    return base + (xs > mid[base] ? 1u : 0u);
 }
 
-/* One wavefront per block: absmax by DPP, then the nearest code by binary search. */
-__global__ void quantize_kernel(const float *x, uint64_t numel, uint64_t nblocks, uint8_t *codes, float *absmax,
-                                const float *mid) {
-    __shared__ float lmid[256];
-    lmid[threadIdx.x] = mid[threadIdx.x];
+template <bool VEC, bool SIGNED>
+__device__ __forceinline__ void quantize_block(const float *x, uint8_t *codes, float *absmax, uint32_t n, uint32_t lane,
+                                               const unsigned char *lo, const float *mid) {
+    f32x4 v[8];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) v[c] = moment_load<VEC>(x, c * 256 + lane * 4, n);
+    float a = 0.0f;
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) a = fmaxf(a, __builtin_fabsf(v[c][k]));
+    a = wave_max(a);
+    const BlockDiv d(a, kKeyScale, kKeyScaleInv);
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+        const uint32_t o = c * 256 + lane * 4;
+        float q[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            q[k] = d.fast ? d.div_fast(v[c][k]) : d.div_slow(v[c][k]);
+            if (!SIGNED) q[k] = fmaxf(q[k], 0.0f); // the unsigned map answers code 0 below zero and for NaN
+        }
+        const uint32_t h01 = half_key2(q[0], q[1]), h23 = half_key2(q[2], q[3]);
+        const uint32_t c0 = small_code<SIGNED>(q[0], h01 & 0xffffu, lo, mid), c1 = small_code<SIGNED>(q[1], h01 >> 16, lo, mid);
+        const uint32_t c2 = small_code<SIGNED>(q[2], h23 & 0xffffu, lo, mid), c3 = small_code<SIGNED>(q[3], h23 >> 16, lo, mid);
+        const uint32_t w = c0 | (c1 << 8) | (c2 << 16) | (c3 << 24);
+        if (VEC && o + 4 <= n) {
+            __builtin_nontemporal_store(w, as_global(reinterpret_cast<uint32_t *>(codes + o)));
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if (o + k < n) as_global(codes)[o + k] = (uint8_t)(w >> (8 * k));
+        }
+    }
+    if (lane == 0) *as_global(absmax) = a;
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(kMomentThreads) void quantize_kernel(MomentArgs args, uint64_t numel, uint64_t nblocks,
+                                                                  const unsigned char *__restrict__ image) {
+    __shared__ float mid[256];
+    __shared__ unsigned char lo[kSKeyCount];
+    static_assert(kSKeyCount == kUKeyCount && kSKeyCount == 16 * kMomentThreads, "one 16-byte word per thread");
+    const uint32_t which = blockIdx.y;
+    const bool is_signed = args.is_signed[which] != 0;
+    mid[threadIdx.x] = reinterpret_cast<const float *>(image + (is_signed ? kSmallMidS : kSmallMidU))[threadIdx.x];
+    reinterpret_cast<uint4 *>(lo)[threadIdx.x] = reinterpret_cast<const uint4 *>(image + (is_signed ? kSmallLoS : kSmallLoU))[threadIdx.x];
     __syncthreads();
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    const uint64_t nw = (uint64_t)gridDim.x * (blockDim.x / kWave);
-    for (uint64_t b = wave; b < nblocks; b += nw) {
+    const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kMomentThreads / kWave) + threadIdx.x / kWave);
+    const uint64_t stride = (uint64_t)gridDim.x * (kMomentThreads / kWave);
+    for (uint64_t b = wave; b < nblocks; b += stride) {
         const uint64_t e0 = b * kBlock;
         const uint32_t n = (uint32_t)((numel - e0) < kBlock ? (numel - e0) : kBlock);
-        float a = 0.0f;
-        for (uint32_t i = lane; i < n; i += kWave) a = fmaxf(a, __builtin_fabsf(x[e0 + i]));
-        a = wave_max(a);
-        for (uint32_t i = lane; i < n; i += kWave) {
-            const float q = a == 0.0f ? 0.0f : x[e0 + i] / a;
-            codes[e0 + i] = (uint8_t)code_bsearch(q, lmid);
-        }
-        if (lane == 0) absmax[b] = a;
+        if (is_signed) quantize_block<VEC, true>(args.x[which] + e0, args.codes[which] + e0, args.absmax[which] + b, n, lane, lo, mid);
+        else quantize_block<VEC, false>(args.x[which] + e0, args.codes[which] + e0, args.absmax[which] + b, n, lane, lo, mid);
     }
 }
 
-int launch_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax,
-                    const void *lds_image, void *stream) {
-    const float *mid = reinterpret_cast<const float *>(static_cast<const char *>(lds_image) +
-                                                       (signed_map ? kOffMidS : kOffMidU));
-    const uint64_t nblocks = (numel + kBlock - 1) / kBlock;
+template <bool VEC>
+__global__ __launch_bounds__(kMomentThreads) void dequantize_kernel(MomentArgs args, uint64_t numel, uint64_t nblocks,
+                                                                    const unsigned char *__restrict__ image) {
+    __shared__ float map[256];
+    const uint32_t which = blockIdx.y;
+    map[threadIdx.x] = reinterpret_cast<const float *>(image + (args.is_signed[which] ? kSmallMapS : kSmallMapU))[threadIdx.x];
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kMomentThreads / kWave) + threadIdx.x / kWave);
+    const uint64_t stride = (uint64_t)gridDim.x * (kMomentThreads / kWave);
+    for (uint64_t b = wave; b < nblocks; b += stride) {
+        const uint64_t e0 = b * kBlock;
+        const uint32_t n = (uint32_t)((numel - e0) < kBlock ? (numel - e0) : kBlock);
+        const uint8_t *codes = args.codes[which] + e0;
+        float *out = args.x[which] + e0;
+        const float a = as_global(args.absmax[which])[b];
+        uint32_t w[8];
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) {
+            const uint32_t o = c * 256 + lane * 4;
+            if (VEC && o + 4 <= n) {
+                w[c] = __builtin_nontemporal_load(as_global(reinterpret_cast<const uint32_t *>(codes + o)));
+            } else {
+                w[c] = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+                    if (o + k < n) w[c] |= (uint32_t)as_global(codes)[o + k] << (8 * k);
+            }
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) {
+            const uint32_t o = c * 256 + lane * 4;
+            const f32x4 r = {map[w[c] & 0xffu] * a, map[(w[c] >> 8) & 0xffu] * a, map[(w[c] >> 16) & 0xffu] * a, map[w[c] >> 24] * a};
+            if (VEC && o + 4 <= n) {
+                __builtin_nontemporal_store(r, as_global(reinterpret_cast<f32x4 *>(out + o)));
+            } else {
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+                    if (o + k < n) as_global(out)[o + k] = r[k];
+            }
+        }
+    }
+}
+
+/* Whole words need fp32 pointers on 16 bytes and code pointers on 4 (the optimizers' states and every allocator's
+ * buffers are); other addresses take the same kernels element by element. */
+static bool moments_aligned(const MomentArgs &a, uint32_t moments) {
+    uintptr_t wide = 0, codes = 0;
+    for (uint32_t i = 0; i < moments; ++i) {
+        wide |= (uintptr_t)a.x[i];
+        codes |= (uintptr_t)a.codes[i];
+    }
+    return (wide & 15u) == 0 && (codes & 3u) == 0;
+}
+
+/* Workgroups of four waves, up to eight per compute unit over both moments: 32 waves fill its wave slots. */
+static dim3 moments_grid(uint64_t nblocks, uint32_t moments, uint32_t compute_units) {
     uint64_t grid = (nblocks + 3) / 4;
-    if (grid > 8192) grid = 8192;
-    hipLaunchKernelGGL(quantize_kernel, dim3((uint32_t)grid), dim3(256), 0, static_cast<hipStream_t>(stream), x,
-                       numel, nblocks, codes, absmax, mid);
+    const uint64_t cap = (uint64_t)compute_units * 8 / moments;
+    return dim3((uint32_t)(grid < cap ? grid : cap), moments);
+}
+
+int launch_dequantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream) {
+    const uint64_t nblocks = (numel + kBlock - 1) / kBlock;
+    const auto k = moments_aligned(a, moments) ? dequantize_kernel<true> : dequantize_kernel<false>;
+    hipLaunchKernelGGL(k, moments_grid(nblocks, moments, compute_units), dim3(kMomentThreads), 0, static_cast<hipStream_t>(stream), a, numel,
+                       nblocks, static_cast<const unsigned char *>(small_image));
+    return (int)hipGetLastError();
+}
+
+int launch_quantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream) {
+    const uint64_t nblocks = (numel + kBlock - 1) / kBlock;
+    const auto k = moments_aligned(a, moments) ? quantize_kernel<true> : quantize_kernel<false>;
+    hipLaunchKernelGGL(k, moments_grid(nblocks, moments, compute_units), dim3(kMomentThreads), 0, static_cast<hipStream_t>(stream), a, numel,
+                       nblocks, static_cast<const unsigned char *>(small_image));
     return (int)hipGetLastError();
 }
 

@@ -1614,9 +1614,7 @@ int eri_adam8bit_fn_get_state_fp32(EriAdam8bitFn *o, const char *name, float *m_
     auto it = o->states.find(std::string_view(name));
     if (it == o->states.end()) return fail(ERI_ERR_ARG, std::string("no optimizer state named '") + name + "'");
     State8 &s = *it->second;
-    rc = eri_adam8_dequantize(s.m, s.absmax_m, 1, s.numel, m_out, o->stream);
-    if (rc) return rc;
-    return eri_adam8_dequantize(s.v, s.absmax_v, 0, s.numel, v_out, o->stream);
+    return eri_adam8_dequantize_state(s.m, s.v, s.absmax_m, s.absmax_v, s.numel, m_out, v_out, o->stream);
 }
 
 int eri_adam8bit_fn_load_state_fp32(EriAdam8bitFn *o, const char *name, const float *m, const float *v,
@@ -1629,9 +1627,7 @@ int eri_adam8bit_fn_load_state_fp32(EriAdam8bitFn *o, const char *name, const fl
     std::unique_ptr<FnState> s(new FnState());
     rc = s->allocate(numel, o->stream, o->state_pool, o->state_lane);
     if (rc) return rc;
-    rc = eri_adam8_quantize(m, 1, numel, s->m, s->absmax_m, o->stream);
-    if (rc) return rc;
-    rc = eri_adam8_quantize(v, 0, numel, s->v, s->absmax_v, o->stream);
+    rc = eri_adam8_quantize_state(m, v, numel, s->m, s->v, s->absmax_m, s->absmax_v, o->stream);
     if (rc) return rc;
     o->states[name] = std::move(s);
     return 0;

@@ -51,7 +51,7 @@ inline float bits_to_float(uint32_t u) {
 struct Tables {
     float map_s[256], map_u[256];
     float mid_s[256], mid_u[256]; // 255 midpoints + inf
-    std::vector<unsigned char> image;
+    std::vector<unsigned char> image, small_image;
     bool ok = false;
     std::string why;
 };
@@ -138,6 +138,20 @@ bool build_slots(const float *mid, uint32_t drop, uint32_t mask, uint32_t stride
     return true;
 }
 
+/* The one-byte slots of the small image out of the slots of the large one: `lo` must name the midpoint of its slot. */
+bool build_small_slots(const unsigned char *slots, uint32_t stride, uint32_t count, const float *mid, unsigned char *lo, std::string &why) {
+    for (uint32_t k = 0; k < count; ++k) {
+        eri::KeySlot s;
+        std::memcpy(&s, slots + (size_t)k * stride, sizeof s);
+        if (s.lo > 255 || (!std::isinf(s.mid) && s.mid != mid[s.lo] * eri::kKeyScale)) {
+            why = "a lookup slot's midpoint is not the one its base code names";
+            return false;
+        }
+        lo[k] = (unsigned char)s.lo;
+    }
+    return true;
+}
+
 const Tables &tables() {
     static Tables t;
     static std::once_flag once;
@@ -170,6 +184,16 @@ const Tables &tables() {
         std::memcpy(&t.image[eri::kOffMidU], t.mid_u, 1024);
         if (!build_slots(t.mid_s, eri::kSKeyDrop, 0xffffu, eri::kSKeyStride, eri::kSKeyCount, &t.image[eri::kOffKeyS], t.why)) return;
         if (!build_slots(t.mid_u, eri::kUKeyDrop, 0x7fffu, eri::kUKeyStride, eri::kUKeyCount, &t.image[eri::kOffKeyU], t.why)) return;
+        t.small_image.assign(eri::kSmallImageBytes, 0);
+        std::memcpy(&t.small_image[eri::kSmallMapS], t.map_s, 1024);
+        std::memcpy(&t.small_image[eri::kSmallMapU], t.map_u, 1024);
+        float scaled[256];
+        for (int j = 0; j < 256; ++j) scaled[j] = t.mid_s[j] * eri::kKeyScale;
+        std::memcpy(&t.small_image[eri::kSmallMidS], scaled, 1024);
+        for (int j = 0; j < 256; ++j) scaled[j] = t.mid_u[j] * eri::kKeyScale;
+        std::memcpy(&t.small_image[eri::kSmallMidU], scaled, 1024);
+        if (!build_small_slots(&t.image[eri::kOffKeyS], eri::kSKeyStride, eri::kSKeyCount, t.mid_s, &t.small_image[eri::kSmallLoS], t.why)) return;
+        if (!build_small_slots(&t.image[eri::kOffKeyU], eri::kUKeyStride, eri::kUKeyCount, t.mid_u, &t.small_image[eri::kSmallLoU], t.why)) return;
         t.ok = true;
     });
     return t;
@@ -190,6 +214,7 @@ static __device__ __align__(256) double scratch[2 * kNormScratchPairs];
 
 struct DeviceCtx {
     void *image = nullptr; // device copy of the LDS image
+    void *small_image = nullptr; // device copy of the small one, behind it in the same allocation
     double *scratch_ptr = nullptr; // address of this device's copy of the static array `scratch`
     uint32_t cus = 0;
     uint32_t wg = 1024;      // threads per workgroup: the table image (~100 KB of LDS) allows one per CU
@@ -213,8 +238,10 @@ int get_ctx(DeviceCtx **out) {
         ERI_HIP(hipGetDeviceProperties(&prop, dev));
         c.cus = (uint32_t)prop.multiProcessorCount;
         void *image = nullptr;
-        ERI_HIP(hipMalloc(&image, eri::kLdsImageBytes));
-        const hipError_t e = hipMemcpy(image, t.image.data(), eri::kLdsImageBytes, hipMemcpyHostToDevice);
+        ERI_HIP(hipMalloc(&image, eri::kLdsImageBytes + eri::kSmallImageBytes));
+        void *small_image = static_cast<char *>(image) + eri::kLdsImageBytes;
+        hipError_t e = hipMemcpy(image, t.image.data(), eri::kLdsImageBytes, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(small_image, t.small_image.data(), eri::kSmallImageBytes, hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             (void)hipFree(image);
             return hip_fail(e, "upload of the quantisation tables");
@@ -227,6 +254,7 @@ int get_ctx(DeviceCtx **out) {
         }
         c.scratch_ptr = ptr;
         c.image = image;
+        c.small_image = small_image;
         c.ready = true;
     }
     *out = &c;
@@ -1255,33 +1283,62 @@ int eri_adam8_step_multi(const EriAdam8Tensor *rows, uint32_t n, const EriAdam8H
     return eri_adam8_step_table(cache.table, h, stream);
 }
 
-int eri_adam8_dequantize(const uint8_t *codes, const float *absmax, int signed_map, uint64_t numel, float *out,
-                         void *stream) {
-    if (!codes || !absmax || !out) return fail(ERI_ERR_NULL, "dequantize with NULL pointer");
+static int dequantize(const eri::MomentArgs &a, uint32_t moments, uint64_t numel, void *stream) {
+    for (uint32_t i = 0; i < moments; ++i)
+        if (!a.codes[i] || !a.absmax[i] || !a.x[i]) return fail(ERI_ERR_NULL, "dequantize with NULL pointer");
     if (numel == 0) return fail(ERI_ERR_EMPTY, "Empty quantized data");
     DeviceCtx *ctx = nullptr;
     int rc = get_ctx(&ctx);
+    for (uint32_t i = 0; i < moments && rc == 0; ++i) {
+        rc = require_kernel_visible(a.codes[i], "dequantize: codes");
+        if (rc == 0) rc = require_kernel_visible(a.absmax[i], "dequantize: absmax");
+        if (rc == 0) rc = require_kernel_visible(a.x[i], "dequantize: out");
+    }
     if (rc) return rc;
-    if ((rc = require_kernel_visible(codes, "dequantize: codes")) != 0) return rc;
-    if ((rc = require_kernel_visible(absmax, "dequantize: absmax")) != 0) return rc;
-    if ((rc = require_kernel_visible(out, "dequantize: out")) != 0) return rc;
-    rc = eri::launch_dequantize(codes, absmax, signed_map, numel, out, ctx->image, stream);
+    rc = eri::launch_dequantize(a, moments, numel, ctx->small_image, ctx->cus, stream);
     if (rc) return hip_fail((hipError_t)rc, "dequantize launch");
     return 0;
 }
 
-int eri_adam8_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax, void *stream) {
-    if (!x || !codes || !absmax) return fail(ERI_ERR_NULL, "quantize with NULL pointer");
+static int quantize(const eri::MomentArgs &a, uint32_t moments, uint64_t numel, void *stream) {
+    for (uint32_t i = 0; i < moments; ++i)
+        if (!a.x[i] || !a.codes[i] || !a.absmax[i]) return fail(ERI_ERR_NULL, "quantize with NULL pointer");
     if (numel == 0) return fail(ERI_ERR_EMPTY, "Empty tensor for quantization");
     DeviceCtx *ctx = nullptr;
     int rc = get_ctx(&ctx);
+    for (uint32_t i = 0; i < moments && rc == 0; ++i) {
+        rc = require_kernel_visible(a.x[i], "quantize: x");
+        if (rc == 0) rc = require_kernel_visible(a.codes[i], "quantize: codes");
+        if (rc == 0) rc = require_kernel_visible(a.absmax[i], "quantize: absmax");
+    }
     if (rc) return rc;
-    if ((rc = require_kernel_visible(x, "quantize: x")) != 0) return rc;
-    if ((rc = require_kernel_visible(codes, "quantize: codes")) != 0) return rc;
-    if ((rc = require_kernel_visible(absmax, "quantize: absmax")) != 0) return rc;
-    rc = eri::launch_quantize(x, signed_map, numel, codes, absmax, ctx->image, stream);
+    rc = eri::launch_quantize(a, moments, numel, ctx->small_image, ctx->cus, stream);
     if (rc) return hip_fail((hipError_t)rc, "quantize launch");
     return 0;
+}
+
+int eri_adam8_dequantize(const uint8_t *codes, const float *absmax, int signed_map, uint64_t numel, float *out,
+                         void *stream) {
+    const eri::MomentArgs a = {{out, nullptr}, {const_cast<uint8_t *>(codes), nullptr}, {const_cast<float *>(absmax), nullptr}, {signed_map != 0, 0}};
+    return dequantize(a, 1, numel, stream);
+}
+
+int eri_adam8_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax, void *stream) {
+    const eri::MomentArgs a = {{const_cast<float *>(x), nullptr}, {codes, nullptr}, {absmax, nullptr}, {signed_map != 0, 0}};
+    return quantize(a, 1, numel, stream);
+}
+
+int eri_adam8_dequantize_state(const uint8_t *m, const uint8_t *v, const float *absmax_m, const float *absmax_v, uint64_t numel,
+                               float *m_out, float *v_out, void *stream) {
+    const eri::MomentArgs a = {{m_out, v_out}, {const_cast<uint8_t *>(m), const_cast<uint8_t *>(v)},
+                               {const_cast<float *>(absmax_m), const_cast<float *>(absmax_v)}, {1, 0}};
+    return dequantize(a, 2, numel, stream);
+}
+
+int eri_adam8_quantize_state(const float *m_in, const float *v_in, uint64_t numel, uint8_t *m, uint8_t *v, float *absmax_m,
+                             float *absmax_v, void *stream) {
+    const eri::MomentArgs a = {{const_cast<float *>(m_in), const_cast<float *>(v_in)}, {m, v}, {absmax_m, absmax_v}, {1, 0}};
+    return quantize(a, 2, numel, stream);
 }
 
 } // extern "C"

@@ -119,6 +119,8 @@ extern "C" {
     pub fn eri_adam8_step_multi(rows: *const EriAdam8Tensor, n: u32, hyper: *const EriAdam8Hyper, stream: *mut c_void) -> c_int;
     pub fn eri_adam8_dequantize(codes: *const u8, absmax: *const f32, signed_map: c_int, numel: u64, out: *mut f32, stream: *mut c_void) -> c_int;
     pub fn eri_adam8_quantize(x: *const f32, signed_map: c_int, numel: u64, codes: *mut u8, absmax: *mut f32, stream: *mut c_void) -> c_int;
+    pub fn eri_adam8_dequantize_state(m: *const u8, v: *const u8, absmax_m: *const f32, absmax_v: *const f32, numel: u64, m_out: *mut f32, v_out: *mut f32, stream: *mut c_void) -> c_int;
+    pub fn eri_adam8_quantize_state(m_in: *const f32, v_in: *const f32, numel: u64, m: *mut u8, v: *mut u8, absmax_m: *mut f32, absmax_v: *mut f32, stream: *mut c_void) -> c_int;
     // 32-bit sibling and EMA sweep
     pub fn eri_adamw32_step_multi(rows: *const EriAdamW32Tensor, n: u32, hyper: *const EriAdamW32Hyper, stream: *mut c_void) -> c_int;
     pub fn eri_adamw32_step_multi_scaled(rows: *const EriAdamW32Tensor, n: u32, hyper: *const EriAdamW32Hyper, grad_scale: f32, dev_scale: *const f32, stream: *mut c_void) -> c_int;

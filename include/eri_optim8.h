@@ -328,6 +328,11 @@ int eri_adam8_dequantize(const uint8_t *codes, const float *absmax, int signed_m
                          float *out, void *stream);
 int eri_adam8_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax,
                        void *stream);
+/* Both moments of one tensor in one launch.  Nothing is launched if any pointer is refused. */
+int eri_adam8_dequantize_state(const uint8_t *m, const uint8_t *v, const float *absmax_m, const float *absmax_v,
+                               uint64_t numel, float *m_out, float *v_out, void *stream);
+int eri_adam8_quantize_state(const float *m_in, const float *v_in, uint64_t numel, uint8_t *m, uint8_t *v,
+                             float *absmax_m, float *absmax_v, void *stream);
 
 /* ---------------------------------------------------------------------------------------------
  * 32-bit sibling: fused multi-tensor AdamW with fp32 moments, for tensors kept out of the 8-bit

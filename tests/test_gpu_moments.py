@@ -1,0 +1,73 @@
+"""The kernels between fp32 moments and codes + absmax at the sizes and addresses where they can go wrong: remainders of
+the four elements a lane holds, of a 256-element pass and of a block, whole words and single elements, negative
+values under the unsigned map.  The format is specified bit for bit: every comparison is exact."""
+import numpy as np
+import pytest
+
+import harness as hs
+import oracle_c as oc
+
+pytestmark = pytest.mark.gpu
+
+
+def _moments(n, signed, rng):
+    x = (rng.standard_normal(n) * 10.0 ** rng.uniform(-6, 0, n)).astype(np.float32)
+    x[rng.random(n) < 0.05] = 0.0  # negative values stay in for the unsigned map too: they take code 0
+    return x
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 255, 257, 2047, 2048, 2049, 4099, 3 * 2048 + 1022, 2048 * 4100 + 7])
+@pytest.mark.parametrize("x_off,code_off", [(0, 0), (1, 0), (0, 1), (4, 4)])
+def test_quantise_and_dequantise_equal_the_oracle(n, x_off, code_off):
+    import torch
+    from eridiffusion_amd import _lib as L
+    rng = np.random.default_rng(n + 7 * x_off + code_off)
+    nb = (n + 2047) // 2048
+    dev, stream = torch.device("cuda:0"), torch.cuda.current_stream().cuda_stream
+    guard = 64
+    xs, want = [], []
+    for signed in (1, 0):
+        x = _moments(n, signed, rng)
+        wc, wa, wb = np.empty(n, np.uint8), np.empty(nb, np.float32), np.empty(n, np.float32)
+        oc.lib().eri_oracle_quantize(oc.ptr(x), oc.ptr(hs.MAPS[1 - signed]), n, oc.ptr(wc), oc.ptr(wa))
+        oc.lib().eri_oracle_dequantize(oc.ptr(wc), oc.ptr(wa), oc.ptr(hs.MAPS[1 - signed]), n, oc.ptr(wb))
+        xs.append(x)
+        want.append((wc, wa, wb))
+
+    def buffers():
+        xd = [torch.full((n + x_off + guard,), 7.0, device=dev) for _ in xs]
+        for d, x in zip(xd, xs):
+            d[x_off:x_off + n] = torch.from_numpy(x).to(dev)
+        codes = [torch.full((n + code_off + guard,), 99, dtype=torch.uint8, device=dev) for _ in xs]
+        absmax = [torch.full((nb + guard,), 5.0, device=dev) for _ in xs]
+        back = [torch.full((n + x_off + guard,), 7.0, device=dev) for _ in xs]
+        return xd, codes, absmax, back
+
+    def check(codes, absmax, back):
+        torch.cuda.synchronize()
+        for i in (0, 1):
+            c, a, b = codes[i].cpu().numpy(), absmax[i].cpu().numpy(), back[i].cpu().numpy()
+            wc, wa, wb = want[i]
+            assert np.array_equal(c[code_off:code_off + n], wc), i
+            assert np.array_equal(a[:nb].view(np.uint32), wa.view(np.uint32)), i
+            assert np.array_equal(b[x_off:x_off + n].view(np.uint32), wb.view(np.uint32)), i
+            assert (c[:code_off] == 99).all() and (c[code_off + n:] == 99).all(), i  # nothing outside the tensor is written
+            assert (a[nb:] == 5.0).all() and (b[:x_off] == 7.0).all() and (b[x_off + n:] == 7.0).all(), i
+
+    xd, codes, absmax, back = buffers()
+    x_ptr = [d.data_ptr() + 4 * x_off for d in xd]
+    c_ptr = [c.data_ptr() + code_off for c in codes]
+    b_ptr = [b.data_ptr() + 4 * x_off for b in back]
+    for i, signed in enumerate((1, 0)):
+        L.check(L.lib().eri_adam8_quantize(x_ptr[i], signed, n, c_ptr[i], absmax[i].data_ptr(), stream), "quantize")
+        L.check(L.lib().eri_adam8_dequantize(c_ptr[i], absmax[i].data_ptr(), signed, n, b_ptr[i], stream), "dequantize")
+    check(codes, absmax, back)
+
+    xd, codes, absmax, back = buffers()  # both moments in one launch
+    x_ptr = [d.data_ptr() + 4 * x_off for d in xd]
+    c_ptr = [c.data_ptr() + code_off for c in codes]
+    b_ptr = [b.data_ptr() + 4 * x_off for b in back]
+    am, av = absmax[0].data_ptr(), absmax[1].data_ptr()
+    L.check(L.lib().eri_adam8_quantize_state(x_ptr[0], x_ptr[1], n, c_ptr[0], c_ptr[1], am, av, stream), "quantize_state")
+    L.check(L.lib().eri_adam8_dequantize_state(c_ptr[0], c_ptr[1], am, av, n, b_ptr[0], b_ptr[1], stream), "dequantize_state")
+    check(codes, absmax, back)
