@@ -71,3 +71,26 @@ def test_quantise_and_dequantise_equal_the_oracle(n, x_off, code_off):
     L.check(L.lib().eri_adam8_quantize_state(x_ptr[0], x_ptr[1], n, c_ptr[0], c_ptr[1], am, av, stream), "quantize_state")
     L.check(L.lib().eri_adam8_dequantize_state(c_ptr[0], c_ptr[1], am, av, n, b_ptr[0], b_ptr[1], stream), "dequantize_state")
     check(codes, absmax, back)
+
+
+def test_loading_moments_of_the_same_size_keeps_the_state_where_it_is():
+    """update, load, update: the second update starts from the loaded moments, and a load that is refused (the second
+    moment is ordinary host memory) leaves the state as it was."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    n = 2048 * 3 + 130
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(11)
+    p, g = torch.randn(n, device=dev, generator=gen), torch.randn(n, device=dev, generator=gen) * 1e-3
+    m, v = torch.randn(n, device=dev, generator=gen) * 1e-3, torch.rand(n, device=dev, generator=gen) * 1e-6
+    used, new = Adam8bitFunctional(), Adam8bitFunctional()
+    used.update("w", p, g)
+    used.load_state_from_tensors({"w": (m, v)})
+    new.load_state_from_tensors({"w": (m, v)})
+    assert torch.equal(used.update("w", p, g), new.update("w", p, g))
+    before = used.get_state_as_tensors()["w"]
+    host = np.zeros(n, np.float32)
+    assert L.lib().eri_adam8bit_fn_load_state_fp32(used._opt, b"w", p.data_ptr(), host.ctypes.data, n) == -6
+    after = used.get_state_as_tensors()["w"]
+    assert torch.equal(before[0], after[0]) and torch.equal(before[1], after[1])
