@@ -90,7 +90,7 @@ static_assert(kSmallImageBytes % 1024 == 0, "the image is staged in pieces of 1 
 
 /* Launchers implemented in eri_adam8_kernels.hip; `stream` is a hipStream_t.  All return a
  * hipError_t as int.  `lds_image` is the device copy of the kLdsImageBytes table image. */
-int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, int layout,
+int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, uint32_t n_tails, int layout,
                 const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg,
                 uint32_t compute_units, void *stream);
 
@@ -110,26 +110,26 @@ inline uint32_t chunks_for(uint32_t grid) { return grid % kChunks == 0 ? kChunks
  * picks one.  wd / gs / keytab / exact select template instances: decay present, gradient scale present,
  * slot-table (rather than binary-search) requantisation, IEEE square root and division on bf16. */
 int launch_step_plain_f32(int mode, bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows,
-                          uint32_t total_blocks, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
+                          uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream);
 int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, bool grad_f32, const DevTensor *rows, uint32_t n_rows,
-                           uint32_t total_blocks, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
+                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                            uint32_t grid, uint32_t wg, void *stream);
 /* Four waves per block, for tables of few blocks; `grid` workgroups of 1024 threads. */
 int launch_step_split(int layout, int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows,
-                      uint32_t total_blocks, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
+                      uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                       uint32_t grid, uint32_t teams, void *stream);
 /* Whether launch_step would run this group on the prefetching kernel with the EMA update inside it. */
 bool step_fuses_ema(uint32_t total_full_blocks, int layout, const EriAdam8Hyper &h, uint32_t compute_units);
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
-                          uint32_t total_blocks, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
+                          uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream);
 /* The same kernel for bf16 parameters whose gradients are fp32. */
 int launch_step_pipelined_grad_f32(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
-                                   uint32_t total_blocks, const EriAdam8Hyper &h, const void *lds_image,
+                                   uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image,
                                    const float *dev_scale, uint32_t grid, uint32_t wg, void *stream);
 /* The same kernel for fp32 parameters (IEEE chain throughout, no EMA inside it). */
-int launch_step_pipelined_f32(int mode, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks,
+int launch_step_pipelined_f32(int mode, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                               const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid,
                               uint32_t wg, void *stream);
 /* Sum of |moment - dequantised moment| of the coming step, per row: err[2r] first moment, err[2r+1] second. */

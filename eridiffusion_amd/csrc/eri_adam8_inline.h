@@ -435,6 +435,15 @@ struct Raw8<true> {
         // every byte these kernels stream is touched once per launch: non-temporal throughout
         w = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(base) + elem)));
     }
+    /* The first `count` (< 8) elements, zeros for the rest; nothing past them is read. */
+    __device__ __forceinline__ void load_some(const void *base, uint32_t elem, uint32_t count) {
+        ERI_GLOBAL const uint16_t *q = as_global(static_cast<const uint16_t *>(base) + elem);
+        uint32_t x[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t k = 0; k < 7; ++k)
+            if (k < count) x[k] = q[k];
+        w = u32x4{x[0] | x[1] << 16, x[2] | x[3] << 16, x[4] | x[5] << 16, x[6]};
+    }
     __device__ __forceinline__ void unpack(float (&out)[8]) const {
         out[0] = bf16_lo(w.x); out[1] = bf16_hi(w.x); out[2] = bf16_lo(w.y); out[3] = bf16_hi(w.y);
         out[4] = bf16_lo(w.z); out[5] = bf16_hi(w.z); out[6] = bf16_lo(w.w); out[7] = bf16_hi(w.w);
@@ -449,6 +458,13 @@ struct Raw8<false> {
         // stay ordinary loads: streamed, the second instruction would fetch every line again
         a = q[0];
         b = q[1];
+    }
+    __device__ __forceinline__ void load_some(const void *base, uint32_t elem, uint32_t count) {
+        ERI_GLOBAL const float *q = as_global(static_cast<const float *>(base) + elem);
+        a = b = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (uint32_t k = 0; k < 7; ++k)
+            if (k < count) (k < 4 ? a : b)[k & 3] = q[k];
     }
     __device__ __forceinline__ void unpack(float (&out)[8]) const {
         out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
@@ -470,6 +486,37 @@ __device__ __forceinline__ void store8(void *base, uint32_t elem, const float (&
         q[0] = f32x4{v[0], v[1], v[2], v[3]}; // half a line per instruction: left to the cache to merge
         q[1] = f32x4{v[4], v[5], v[6], v[7]};
     }
+}
+
+/* A partial block of n elements: how many of a lane's eight elements o .. o + 7 exist. */
+__device__ __forceinline__ uint32_t lane_count(uint32_t o, uint32_t n) { return o + 8 <= n ? 8u : o < n ? n - o : 0u; }
+
+/* store8 of the first `count` (< 8) elements. */
+template <bool BF16>
+__device__ __forceinline__ void store_some(void *base, uint32_t elem, const float (&v)[8], uint32_t count) {
+#pragma unroll
+    for (uint32_t k = 0; k < 7; ++k) {
+        if (k >= count) continue;
+        if (BF16) as_global(static_cast<uint16_t *>(base))[elem + k] = (uint16_t)bf16_bits(v[k]);
+        else as_global(static_cast<float *>(base))[elem + k] = v[k];
+    }
+}
+
+/* Eight codes of a lane, the first `count` (< 8) of them from memory and the others those of a zero moment. */
+constexpr uint32_t kZeroCodesS = 0x7f7f7f7fu, kZeroCodesU = 0u;
+__device__ __forceinline__ u32x2 load_codes_some(const uint8_t *codes, uint32_t count, uint32_t zero_codes) {
+    uint32_t x[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) x[k] = zero_codes & 0xffu;
+#pragma unroll
+    for (uint32_t k = 0; k < 7; ++k)
+        if (k < count) x[k] = as_global(codes)[k];
+    return u32x2{x[0] | x[1] << 8 | x[2] << 16 | x[3] << 24, x[4] | x[5] << 8 | x[6] << 16 | x[7] << 24};
+}
+__device__ __forceinline__ void store_codes_some(uint8_t *codes, const u32x2 w, uint32_t count) {
+#pragma unroll
+    for (uint32_t k = 0; k < 7; ++k)
+        if (k < count) as_global(codes)[k] = (uint8_t)((k < 4 ? w.x : w.y) >> (8 * (k & 3)));
 }
 
 __device__ __forceinline__ uint32_t byte_of(const u32x2 w, int k) {
@@ -694,8 +741,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
 }
 
 // ------------------------------------------------------------------------------------------
-// the last, partial block of a tensor: element-wise, bounds-checked, moments recomputed in the
-// second sweep instead of being held (n < 2048 elements, once per tensor at most)
+// the last, partial block of a tensor (n < 2048 elements, once per tensor at most)
 // ------------------------------------------------------------------------------------------
 
 template <bool BF16>
@@ -704,115 +750,103 @@ __device__ __forceinline__ float load1(const void *base, size_t i) {
     return as_global(static_cast<const float *>(base))[i];
 }
 
+/* One wave, the 8-elements-per-lane accesses of a full block with the lanes past the end switched off; the one
+ * lane the end falls into moves its up to seven elements one by one.  What is filled in for missing elements
+ * are zero moments and zero gradients, which make zero or NaN moments whatever the scalars are: neither moves a
+ * maximum, and nothing of them is stored.  What bounds it is latency, one trip to memory per 512 elements and
+ * sweep: two sweeps, the second recomputing the moments, so that nothing but one pass of values is held -- this
+ * code is inlined into kernels whose register budget belongs to their main loop. */
 template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16>
 __device__ __forceinline__ void tail_block(const DevTensor &t, uint32_t lb, uint32_t n, uint32_t lane,
                                         const StepHyper &h, float gscale, const BlockDiv &dbc1,
                                         const BlockDiv &dbc2, const Lds &L) {
     const size_t e0 = (size_t)lb * kBlock;
-    ERI_GLOBAL uint8_t *mc = as_global(t.m);
-    ERI_GLOBAL uint8_t *vc = as_global(t.v);
     const float a_m = as_global(t.absmax_m)[lb];
     const float a_v = as_global(t.absmax_v)[lb];
     float lm = 0.0f, lv = 0.0f;
     constexpr float ks = KEYTAB ? kKeyScale : 1.0f, ksi = KEYTAB ? kKeyScaleInv : 1.0f;
-    if ((n & 7u) == 0) {
-        // The usual case (tensor sizes are multiples of eight): the same 8-elements-per-lane accesses as a
-        // full block, lanes past the end switched off.  Two sweeps, the second recomputing the moments,
-        // so that nothing but one pass of values is held -- this code is inlined into kernels whose
-        // register budget belongs to their main loop.
-        const size_t esz = BF16 ? 2 : 4;
-        char *p = static_cast<char *>(t.p) + e0 * esz;
-        const char *p_in = static_cast<const char *>(t.p_in) + e0 * esz;
-        const char *g = static_cast<const char *>(t.g) + e0 * (GBF16 ? 2 : 4);
-        const uint32_t passes = (n + 511) / 512;
-        for (uint32_t c = 0; c < passes; ++c) {
-            const uint32_t o = c * 512 + lane * 8;
-            if (o < n) {
-                Raw8<BF16> pr;
-                Raw8<GBF16> gr;
+    const size_t esz = BF16 ? 2 : 4;
+    char *p = static_cast<char *>(t.p) + e0 * esz;
+    const char *p_in = static_cast<const char *>(t.p_in) + e0 * esz;
+    const char *g = static_cast<const char *>(t.g) + e0 * (GBF16 ? 2 : 4);
+    const uint32_t passes = (n + 511) / 512;
+    for (uint32_t c = 0; c < passes; ++c) {
+        const uint32_t o = c * 512 + lane * 8;
+        const uint32_t count = lane_count(o, n);
+        if (count != 0) {
+            Raw8<BF16> pr;
+            Raw8<GBF16> gr;
+            u32x2 mr, vr;
+            if (count == 8) {
                 pr.load(p_in, o);
                 gr.load(g, o);
-                const u32x2 mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
-                const u32x2 vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
-                float pv[8], gv[8];
-                pr.unpack(pv);
-                gr.unpack(gv);
+                mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
+                vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
+            } else {
+                pr.load_some(p_in, o, count);
+                gr.load_some(g, o, count);
+                mr = load_codes_some(t.m + e0 + o, count, kZeroCodesS);
+                vr = load_codes_some(t.v + e0 + o, count, kZeroCodesU);
+            }
+            float pv[8], gv[8];
+            pr.unpack(pv);
+            gr.unpack(gv);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    float m, v, pn;
-                    uint64_t unused = 0;
-                    adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
-                                                         L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m, v, pn, unused);
-                    lm = fmaxf(lm, __builtin_fabsf(m));
-                    lv = fmaxf(lv, __builtin_fabsf(v));
-                }
+            for (int k = 0; k < 8; ++k) {
+                float m, v, pn;
+                uint64_t unused = 0;
+                adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
+                                                     L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m, v, pn, unused);
+                lm = fmaxf(lm, __builtin_fabsf(m));
+                lv = fmaxf(lv, __builtin_fabsf(v));
             }
         }
-        float nam = lm, nav = lv;
-        wave_max2(nam, nav);
-        const BlockDiv dm(nam, ks, ksi), dv(nav, ks, ksi);
-        for (uint32_t c = 0; c < passes; ++c) {
-            const uint32_t o = c * 512 + lane * 8;
-            if (o < n) {
-                Raw8<BF16> pr;
-                Raw8<GBF16> gr;
-                pr.load(p_in, o);
-                gr.load(g, o);
-                const u32x2 mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
-                const u32x2 vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
-                float pv[8], gv[8], pn[8], m[8], v[8];
-                pr.unpack(pv);
-                gr.unpack(gv);
-                uint64_t cancel = (BF16 && MODE == ERI_ADAM8_MODE_L2 && h.l2_all_exact) ? ~0ull : 0ull;
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
-                                                         L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m[k], v[k], pn[k], cancel);
-                if (BF16 && __builtin_amdgcn_inverse_ballot_w64(cancel)) { // a lane with a flagged element redoes its eight
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) pn[k] = param_exact<MODE, WD, BF16>(pv[k], m[k], v[k], h, dbc1, dbc2);
-                }
-                u32x2 mw, vw;
-                requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(m, v, dm, dv, L, mw, vw);
-                *as_global(reinterpret_cast<u32x2 *>(t.m + e0 + o)) = mw;
-                *as_global(reinterpret_cast<u32x2 *>(t.v + e0 + o)) = vw;
-                store8<BF16>(p, o, pn);
-            }
-        }
-        if (lane == 0) {
-            as_global(t.absmax_m)[lb] = nam;
-            as_global(t.absmax_v)[lb] = nav;
-        }
-        return;
-    }
-    for (uint32_t i = lane; i < n; i += kWave) {
-        const size_t e = e0 + i;
-        float m, v, pn;
-        uint64_t unused = 0;
-        adam_elem<MODE, EXACT, BF16, WD, GS>(load1<BF16>(t.p_in, e), load1<GBF16>(t.g, e), L.map_s[mc[e]] * a_m,
-                                             L.map_u[vc[e]] * a_v, h, gscale, dbc1, dbc2, m, v, pn, unused);
-        lm = fmaxf(lm, __builtin_fabsf(m));
-        lv = fmaxf(lv, __builtin_fabsf(v));
     }
     float nam = lm, nav = lv;
     wave_max2(nam, nav);
     const BlockDiv dm(nam, ks, ksi), dv(nav, ks, ksi);
-    for (uint32_t i = lane; i < n; i += kWave) {
-        const size_t e = e0 + i;
-        float m, v, pn;
-        uint64_t cancel = (BF16 && MODE == ERI_ADAM8_MODE_L2 && h.l2_all_exact) ? ~0ull : 0ull;
-        const float p_old = load1<BF16>(t.p_in, e);
-        adam_elem<MODE, EXACT, BF16, WD, GS>(p_old, load1<GBF16>(t.g, e), L.map_s[mc[e]] * a_m,
-                                             L.map_u[vc[e]] * a_v, h, gscale, dbc1, dbc2, m, v, pn, cancel);
-        if (BF16 && __builtin_amdgcn_inverse_ballot_w64(cancel)) pn = param_exact<MODE, WD, BF16>(p_old, m, v, h, dbc1, dbc2);
-        const float xm = dm.div_slow(m);
-        const float xv = dv.div_slow(v);
-        uint32_t cm = KEYTAB ? code_signed_key(xm, L.key_s) : code_bsearch(xm, L.mid_s);
-        if (MODE == ERI_ADAM8_MODE_BNB) cm = keep_sign(cm, m, nam);
-        mc[e] = (uint8_t)cm;
-        vc[e] = (uint8_t)(KEYTAB ? code_unsigned_key(xv, L.key_u) : code_bsearch(xv, L.mid_u));
-        if (BF16) as_global(static_cast<uint16_t *>(t.p))[e] = (uint16_t)bf16_bits(pn);
-        else as_global(static_cast<float *>(t.p))[e] = pn;
+    for (uint32_t c = 0; c < passes; ++c) {
+        const uint32_t o = c * 512 + lane * 8;
+        const uint32_t count = lane_count(o, n);
+        if (count != 0) {
+            Raw8<BF16> pr;
+            Raw8<GBF16> gr;
+            u32x2 mr, vr;
+            if (count == 8) {
+                pr.load(p_in, o);
+                gr.load(g, o);
+                mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
+                vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
+            } else {
+                pr.load_some(p_in, o, count);
+                gr.load_some(g, o, count);
+                mr = load_codes_some(t.m + e0 + o, count, kZeroCodesS);
+                vr = load_codes_some(t.v + e0 + o, count, kZeroCodesU);
+            }
+            float pv[8], gv[8], pn[8], m[8], v[8];
+            pr.unpack(pv);
+            gr.unpack(gv);
+            uint64_t cancel = (BF16 && MODE == ERI_ADAM8_MODE_L2 && h.l2_all_exact) ? ~0ull : 0ull;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
+                                                     L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m[k], v[k], pn[k], cancel);
+            if (BF16 && __builtin_amdgcn_inverse_ballot_w64(cancel)) { // a lane with a flagged element redoes its eight
+#pragma unroll
+                for (int k = 0; k < 8; ++k) pn[k] = param_exact<MODE, WD, BF16>(pv[k], m[k], v[k], h, dbc1, dbc2);
+            }
+            u32x2 mw, vw;
+            requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(m, v, dm, dv, L, mw, vw);
+            if (count == 8) {
+                *as_global(reinterpret_cast<u32x2 *>(t.m + e0 + o)) = mw;
+                *as_global(reinterpret_cast<u32x2 *>(t.v + e0 + o)) = vw;
+                store8<BF16>(p, o, pn);
+            } else {
+                store_codes_some(t.m + e0 + o, mw, count);
+                store_codes_some(t.v + e0 + o, vw, count);
+                store_some<BF16>(p, o, pn, count);
+            }
+        }
     }
     if (lane == 0) {
         as_global(t.absmax_m)[lb] = nam;
@@ -890,6 +924,8 @@ struct BlockRowMap {
             t_end = t.full_start + (uint32_t)(t.numel / kBlock);
         }
     }
+    /* Row of partial block i: behind the map stands the list of the rows that have one. */
+    __device__ __forceinline__ uint32_t tail_row(uint32_t total_blocks, uint32_t i) const { return row_of[total_blocks + i]; }
 };
 
 /* The full blocks one wave walks.  Workgroup i of a launch runs on accelerator die (XCD) i mod 8.  The

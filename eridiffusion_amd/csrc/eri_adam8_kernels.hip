@@ -23,7 +23,7 @@ static bool prefetch_pays(uint32_t total_blocks, const EriAdam8Hyper &h, uint32_
     return (uint64_t)total_blocks > (uint64_t)compute_units * (uint64_t)kPrefetchBlocksPerCu;
 }
 
-int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, int layout,
+int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, int layout,
                 const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg,
                 uint32_t compute_units, void *stream) {
     const bool bf16 = layout_param_bf16(layout);
@@ -41,14 +41,13 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, i
         const bool exact_s = !bf16 || (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
         // Up to four blocks per workgroup at a time (a team of four waves each), but no more than it takes to
         // give every compute unit a workgroup: 512 blocks on 256 units run as 256 workgroups of two teams.
-        uint32_t teams = (total_blocks + compute_units - 1) / compute_units;
+        const uint32_t units = total_blocks + n_tails; // a partial block counts like a full one here
+        uint32_t teams = (units + compute_units - 1) / compute_units;
         teams = teams < 1 ? 1 : teams > 4 ? 4 : teams;
-        uint32_t need = (total_blocks + teams - 1) / teams;
-        const uint32_t for_tails = (n_rows + 15) / 16;
-        if (need < for_tails) need = for_tails;
+        uint32_t need = (units + teams - 1) / teams;
         if (need > compute_units) need = compute_units;
         if (need == 0) need = 1;
-        return launch_step_split(layout, h.mode, exact_s, wd_s, gs, rows, n_rows, total_blocks, h, lds_image, dev_scale, need,
+        return launch_step_split(layout, h.mode, exact_s, wd_s, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, need,
                                  teams, stream);
     }
     if (mixed) {
@@ -56,30 +55,30 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, i
         if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
             return launch_step_pipelined_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs,
                                                   step_fuses_ema(total_blocks, layout, h, compute_units), rows, n_rows,
-                                                  total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+                                                  total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_bf16(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs, true, true, rows, n_rows,
-                                      total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     }
     if (h.mode == ERI_ADAM8_MODE_BNB) { // slot table only; the decay is a factor
         const bool wd = h.weight_decay != 1.0f;
         const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
         if (bf16 && !kernel_named && prefetch_pays(total_blocks, h, compute_units))
-            return launch_step_pipelined(h.mode, exact, wd, gs, false, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
-        if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, false, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+            return launch_step_pipelined(h.mode, exact, wd, gs, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+        if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         if (!kernel_named && prefetch_pays(total_blocks, h, compute_units))
-            return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
-        return launch_step_plain_f32(h.mode, wd, gs, true, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+            return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+        return launch_step_plain_f32(h.mode, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     }
     const bool wd = h.weight_decay > 0.0f;
     const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
     const bool keytab = (h.flags & ERI_ADAM8_FLAG_BSEARCH) == 0;
     if (!bf16 && !kernel_named && prefetch_pays(total_blocks, h, compute_units))
-        return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
-    if (!bf16) return launch_step_plain_f32(h.mode, wd, gs, keytab, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+        return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+    if (!bf16) return launch_step_plain_f32(h.mode, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
         return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(total_blocks, layout, h, compute_units), rows, n_rows,
-                                     total_blocks, h, lds_image, dev_scale, grid, wg, stream);
-    return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, false, rows, n_rows, total_blocks, h, lds_image, dev_scale, grid, wg, stream);
+                                     total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+    return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
 }
 
 // ------------------------------------------------------------------------------------------

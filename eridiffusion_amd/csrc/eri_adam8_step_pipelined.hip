@@ -98,7 +98,7 @@ struct RawBlock {
  * p' being the parameter as it is stored (rounded to bf16). */
 template <int MODE, bool EXACT, bool WD, bool GS, bool EMA>
 __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor *__restrict__ rows,
-                                                                   uint32_t n_rows, uint32_t total_blocks,
+                                                                   uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                                                                    EriAdam8Hyper h_in,
                                                                    const uint4 *__restrict__ lds_image,
                                                                    const float *__restrict__ dev_scale,
@@ -134,37 +134,35 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     const uint32_t stride = gridDim.x * waves_per_wg;
     const BlockDiv dbc1(h.bc1), dbc2(h.bc2);
     float(*const mine)[256] = decayed[threadIdx.x / kWave];
-    const f32x4 base_s = reinterpret_cast<const f32x4 *>(L.map_s)[lane]; // codes 4*lane .. 4*lane + 3
-    const f32x4 base_u = reinterpret_cast<const f32x4 *>(L.map_u)[lane];
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
-    // partial last blocks first: one per row at most, handed out from the last wave backwards -- the
-    // waves at the end of each range are the ones that get one full block fewer when the blocks do not
-    // divide evenly, so the slower element-wise tail lands where there is slack
-    for (uint32_t r = stride - 1 - wave; r < n_rows; r += stride) {
-        const DevTensor t = rows[r];
+    // partial last blocks first, handed out from the last wave backwards -- the waves at the end of each range
+    // are the ones that get one full block fewer when the blocks do not divide evenly, so the slower two-sweep
+    // tail lands where there is slack
+    const BlockRowMap map(rows, n_rows);
+    for (uint32_t i = stride - 1 - wave; i < n_tails; i += stride) {
+        const DevTensor t = rows[map.tail_row(total_blocks, i)];
         const uint32_t n = (uint32_t)(t.numel % kBlock);
-        if (n != 0) {
-            const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
-            tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
-            if (EMA && t.shadow != nullptr) { // the partial block's shadow, element by element, from the parameters just stored
-                const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-                const float omd = 1.0f - h.ema_decay;
-                for (uint32_t i = lane; i < n; i += kWave) {
-                    const float a = load1<true>(t.shadow, e0 + i) * h.ema_decay;
-                    const float b = load1<true>(t.p, e0 + i) * omd;
-                    as_global(static_cast<uint16_t *>(t.shadow))[e0 + i] = (uint16_t)bf16_bits(a + b);
-                }
+        const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
+        tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
+        if (EMA && t.shadow != nullptr) { // the partial block's shadow, element by element, from the parameters just stored
+            const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
+            const float omd = 1.0f - h.ema_decay;
+            for (uint32_t j = lane; j < n; j += kWave) {
+                const float a = load1<true>(t.shadow, e0 + j) * h.ema_decay;
+                const float b = load1<true>(t.p, e0 + j) * omd;
+                as_global(static_cast<uint16_t *>(t.shadow))[e0 + j] = (uint16_t)bf16_bits(a + b);
             }
         }
     }
     const BlockWalk walk(total_blocks, chunks);
     uint32_t blk = walk.first;
     if (blk >= walk.end) return;
+    const f32x4 base_s = reinterpret_cast<const f32x4 *>(L.map_s)[lane]; // codes 4*lane .. 4*lane + 3
+    const f32x4 base_u = reinterpret_cast<const f32x4 *>(L.map_u)[lane];
 
     uint32_t ti = 0, t_end = 0;
     DevTensor t;
-    const BlockRowMap map(rows, n_rows);
     map.seek(rows, blk, ti, t, t_end);
     uint32_t nti = ti, nt_end = t_end;
     DevTensor nt = t;
@@ -305,33 +303,33 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
 namespace {
 
 template <int MODE, bool EXACT, bool WD, bool GS, bool EMA = false>
-int launch_pipelined(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, const EriAdam8Hyper &h,
+int launch_pipelined(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h,
                      const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
     if (wg > kPipeThreads) wg = kPipeThreads;
-    hipLaunchKernelGGL((ERI_PIPE_KERNEL<MODE, EXACT, WD, GS, EMA>), dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, h,
+    hipLaunchKernelGGL((ERI_PIPE_KERNEL<MODE, EXACT, WD, GS, EMA>), dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, n_tails, h,
                        static_cast<const uint4 *>(lds_image), dev_scale, chunks_for(grid));
     return (int)hipGetLastError();
 }
 
 template <int MODE, bool EXACT>
-int launch_flags(bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, const EriAdam8Hyper &h,
+int launch_flags(bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h,
                  const void *img, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
     if constexpr (MODE == ERI_ADAM8_MODE_ERI && kParamBf16) { // the EMA is built into the reference's own update, on bf16 parameters
         if (ema) {
             if (wd) {
-                if (gs) return launch_pipelined<MODE, EXACT, true, true, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
-                return launch_pipelined<MODE, EXACT, true, false, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
+                if (gs) return launch_pipelined<MODE, EXACT, true, true, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
+                return launch_pipelined<MODE, EXACT, true, false, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
             }
-            if (gs) return launch_pipelined<MODE, EXACT, false, true, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
-            return launch_pipelined<MODE, EXACT, false, false, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
+            if (gs) return launch_pipelined<MODE, EXACT, false, true, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
+            return launch_pipelined<MODE, EXACT, false, false, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
         }
     }
     if (wd) {
-        if (gs) return launch_pipelined<MODE, EXACT, true, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
-        return launch_pipelined<MODE, EXACT, true, false>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
+        if (gs) return launch_pipelined<MODE, EXACT, true, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
+        return launch_pipelined<MODE, EXACT, true, false>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
     }
-    if (gs) return launch_pipelined<MODE, EXACT, false, true>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
-    return launch_pipelined<MODE, EXACT, false, false>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s);
+    if (gs) return launch_pipelined<MODE, EXACT, false, true>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
+    return launch_pipelined<MODE, EXACT, false, false>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s);
 }
 
 } // namespace
@@ -340,21 +338,21 @@ int launch_flags(bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_r
  * products in the fast chain: 168 registers, no scratch; with the two divisions it spilled 80-232 B per lane.) */
 #if ERI_PIPE_LAYOUT == 1
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
-                          uint32_t total_blocks, const EriAdam8Hyper &h, const void *img, const float *dev_scale,
+                          uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream) {
 #elif ERI_PIPE_LAYOUT == 2
 int launch_step_pipelined_grad_f32(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
-                                   uint32_t total_blocks, const EriAdam8Hyper &h, const void *img,
+                                   uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img,
                                    const float *dev_scale, uint32_t grid, uint32_t wg, void *stream) {
 #else
-int launch_step_pipelined_f32(int mode, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks,
+int launch_step_pipelined_f32(int mode, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                               const EriAdam8Hyper &h, const void *img, const float *dev_scale, uint32_t grid,
                               uint32_t wg, void *stream) {
     const bool ema = false;   // fp32 rows get their EMA from the sweep
     constexpr bool exact = true; // fp32 parameters always take the IEEE square root and division
 #endif
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_ARGS wd, gs, ema, rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s
+#define ERI_ARGS wd, gs, ema, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s
 #if ERI_PIPE_LAYOUT == 0
     if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, exact>(ERI_ARGS);
     if (mode == ERI_ADAM8_MODE_BNB) return launch_flags<ERI_ADAM8_MODE_BNB, exact>(ERI_ARGS);

@@ -22,7 +22,7 @@ constexpr uint32_t plain_threads(int mode, bool gs, bool keytab, bool gbf16) {
 
 template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16>
 __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_step_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,
-                                                          uint32_t total_blocks, EriAdam8Hyper h_in,
+                                                          uint32_t total_blocks, uint32_t n_tails, EriAdam8Hyper h_in,
                                                           const uint4 *__restrict__ lds_image,
                                                           const float *__restrict__ dev_scale) {
     ERI_LDS_IMAGE;
@@ -59,20 +59,17 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     const uint32_t left_mine = wave_in_wg * gridDim.x + blockIdx.x;
     const bool has_left = left_first + left_mine < total_blocks;
 
-    // partial last blocks first: one per row at most, one to each workgroup in turn, from a workgroup's last
-    // wave backwards: those are the waves without a left-over block, so the slower element-wise tail lands
-    // where there is slack
-    for (uint32_t r = blockIdx.x + (waves_per_wg - 1 - wave_in_wg) * gridDim.x; r < n_rows; r += stride) {
-        const DevTensor t = rows[r];
-        const uint32_t n = (uint32_t)(t.numel % kBlock);
-        if (n != 0) {
-            const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
-            tail_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
-        }
+    // partial last blocks first, one to each workgroup in turn, from a workgroup's last wave backwards: those are
+    // the waves without a left-over block, so the slower two-sweep tail lands where there is slack
+    const BlockRowMap map(rows, n_rows);
+    for (uint32_t i = blockIdx.x + (waves_per_wg - 1 - wave_in_wg) * gridDim.x; i < n_tails; i += stride) {
+        const DevTensor t = rows[map.tail_row(total_blocks, i)];
+        const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
+        tail_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, (uint32_t)(t.numel / kBlock), (uint32_t)(t.numel % kBlock), lane,
+                                                             h, gscale, dbc1, dbc2, L);
     }
     uint32_t ti = 0, t_end = 0;
     DevTensor t;
-    const BlockRowMap map(rows, n_rows);
     const uint32_t trips = rounds + (has_left ? 1u : 0u);
     for (uint32_t k = 0; k < trips; ++k) {
         const uint32_t blk = k < rounds ? k * stride + wave : left_first + left_mine;
@@ -88,23 +85,23 @@ namespace {
 constexpr bool kBf16 = ERI_PLAIN_BF16 != 0;
 
 template <int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16>
-int launch_one(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, const EriAdam8Hyper &h,
+int launch_one(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h,
                const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
     auto k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, GBF16>;
     if (wg > plain_threads(MODE, GS, KEYTAB, GBF16)) wg = plain_threads(MODE, GS, KEYTAB, GBF16);
     // One common window for all dies (a grid-stride walk): on the tables this kernel takes, up to 1,024
     // blocks per compute unit, it measured 2 % ahead of one range per die with the arrays far apart in device
     // memory and 5 % with them adjacent; the tables of the prefetching kernel want the ranges.
-    hipLaunchKernelGGL(k, dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, h,
+    hipLaunchKernelGGL(k, dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, n_tails, h,
                        static_cast<const uint4 *>(lds_image), dev_scale);
     return (int)hipGetLastError();
 }
 
 /* BSEARCH selects the cross-check variants (binary search of the midpoint table); mode BNB has none. */
 template <int MODE, bool EXACT, bool BSEARCH, bool GBF16 = kBf16>
-int launch_flags(bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks,
+int launch_flags(bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                  const EriAdam8Hyper &h, const void *img, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
-#define ERI_GO(W, G, K) return launch_one<MODE, EXACT, W, G, K, GBF16>(rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s)
+#define ERI_GO(W, G, K) return launch_one<MODE, EXACT, W, G, K, GBF16>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s)
     if (BSEARCH && !keytab) {
         if (wd) { if (gs) ERI_GO(true, true, !BSEARCH); ERI_GO(true, false, !BSEARCH); }
         if (gs) ERI_GO(false, true, !BSEARCH);
@@ -120,10 +117,10 @@ int launch_flags(bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t 
 
 #if ERI_PLAIN_BF16
 int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, bool grad_f32, const DevTensor *rows,
-                           uint32_t n_rows, uint32_t total_blocks, const EriAdam8Hyper &h, const void *img,
+                           uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img,
                            const float *dev_scale, uint32_t grid, uint32_t wg, void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s
+#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s
     if (grad_f32) { // fp32 gradients for bf16 parameters: slot-table variants only
         if (!keytab) return (int)hipErrorInvalidValue;
         if (mode == ERI_ADAM8_MODE_BNB)
@@ -142,10 +139,10 @@ int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, 
 #else
 /* fp32 parameters always take the IEEE square root and division. */
 int launch_step_plain_f32(int mode, bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows,
-                          uint32_t total_blocks, const EriAdam8Hyper &h, const void *img, const float *dev_scale,
+                          uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, h, img, dev_scale, grid, wg, s
+#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s
     if (mode == ERI_ADAM8_MODE_BNB) return launch_flags<ERI_ADAM8_MODE_BNB, true, false>(ERI_ARGS);
     if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, true, true>(ERI_ARGS);
     return launch_flags<ERI_ADAM8_MODE_ERI, true, true>(ERI_ARGS);

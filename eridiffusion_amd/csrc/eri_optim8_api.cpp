@@ -299,7 +299,8 @@ struct EriAdam8Table {
         int dtype = 0;
         uint32_t n = 0;
         uint32_t total_blocks = 0; // full blocks only; a row's partial last block is handled per row
-        eri::DevTensor *dev = nullptr;    // n rows, then one uint32 row index per full block (BlockRowMap)
+        uint32_t n_tails = 0;      // rows with a partial last block
+        eri::DevTensor *dev = nullptr;    // n rows, then one uint32 row index per full block and one per partial block (BlockRowMap)
         eri::DevTensor *pinned = nullptr; // the rows only
         std::vector<uint32_t> src; // index into the caller's rows
         bool unit_scales = true;   // every row's grad_scale is exactly 1
@@ -939,16 +940,21 @@ static int table_create(const EriAdam8Tensor *rows, uint32_t n, bool grads_only,
         g.n = (uint32_t)g.src.size();
         if (g.n == 0 || e != hipSuccess) continue;
         uint64_t full = 0;
-        for (uint32_t j = 0; j < g.n; ++j) full += rows[g.src[j]].numel / eri::kBlock;
-        e = hipMalloc((void **)&g.dev, sizeof(eri::DevTensor) * g.n + sizeof(uint32_t) * (full ? full : 1));
+        for (uint32_t j = 0; j < g.n; ++j) {
+            full += rows[g.src[j]].numel / eri::kBlock;
+            if (rows[g.src[j]].numel % eri::kBlock) ++g.n_tails;
+        }
+        e = hipMalloc((void **)&g.dev, sizeof(eri::DevTensor) * g.n + sizeof(uint32_t) * (size_t)(full + g.n_tails));
         if (e == hipSuccess) e = hipHostMalloc((void **)&g.pinned, sizeof(eri::DevTensor) * g.n, hipHostMallocDefault);
         if (e == hipSuccess) fill_group(g, rows);
-        if (e == hipSuccess && full) { // which row owns which full block: fixed for the table's life
-            std::vector<uint32_t> row_of((size_t)full);
+        if (e == hipSuccess) { // which row owns which full block, and which rows have a partial one: fixed for the table's life
+            std::vector<uint32_t> row_of((size_t)(full + g.n_tails));
             size_t at = 0;
             for (uint32_t j = 0; j < g.n; ++j)
                 for (uint64_t k = rows[g.src[j]].numel / eri::kBlock; k > 0; --k) row_of[at++] = j;
-            e = hipMemcpy(g.dev + g.n, row_of.data(), sizeof(uint32_t) * (size_t)full, hipMemcpyHostToDevice);
+            for (uint32_t j = 0; j < g.n; ++j)
+                if (rows[g.src[j]].numel % eri::kBlock) row_of[at++] = j;
+            e = hipMemcpy(g.dev + g.n, row_of.data(), sizeof(uint32_t) * row_of.size(), hipMemcpyHostToDevice);
         }
     }
     if (e != hipSuccess) {
@@ -1044,7 +1050,7 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
                 hh.grad_scale = 1.0f;
             }
         }
-        rc = eri::launch_step(g.dev, g.n, g.total_blocks, g.dtype, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
+        rc = eri::launch_step(g.dev, g.n, g.total_blocks, g.n_tails, g.dtype, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
         if (rc) return hip_fail((hipError_t)rc, "adam8 step launch");
         if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(g.total_blocks, g.dtype, hh, ctx->cus)) {
             // not the kernel that carries the EMA: this group's shadows join the plain sweep that follows the step

@@ -551,3 +551,19 @@ def test_five_thousand_small_tensors_in_one_launch():
     sizes = [int(x) for x in rng.integers(1, 6000, 5000)]
     run_case(sizes, True, 5001, steps=2, flags=2, label="5000-tensors")
     run_case(sizes[:1500], False, 5002, steps=2, use_multi=True, label="1500-tensors-multi")
+
+
+@pytest.mark.parametrize("bf16", [True, False], ids=["bf16", "f32"])
+@pytest.mark.parametrize("mode", [0, 1, 2], ids=["eri", "l2", "bnb"])
+def test_partial_blocks_of_every_shape(mode, bf16):
+    """Last blocks that end inside a lane's eight elements, on a lane's edge, on a quarter's edge and one element
+    short of a whole block, as the only block of a tensor and behind full ones."""
+    ends = [1, 7, 8, 9, 505, 511, 512, 513, 520, 1023, 1025, 1536, 1543, 2041, 2047]
+    sizes = ends + [2048 + e for e in ends] + [2048, 2 * 2048 + 3]
+    run_case(sizes, bf16, 4100 + 10 * mode + bf16, steps=2, mode=mode, flags=2, prior=1, label="partial blocks")
+
+
+def test_more_partial_blocks_than_waves():
+    # 4,500 tensors of which every other one is a partial block and nothing else: more of them than four per workgroup
+    sizes = [(5 * i) % 61 + 1 if i % 2 else 2048 for i in range(4500)]
+    run_case(sizes, True, 4200, steps=1, flags=2, prior=1, label="many partial blocks")
