@@ -6,7 +6,8 @@ set_learning_rate / quantized_memory_usage / save_state / load_state), `Adam8bit
 configuration (:372-395), and `Adam8bitFunctional` the per-tensor flavour
 (src/trainers/adam8bit.rs:49-345: with_params / update / step / set_lr / get_step / memory_stats /
 get_state_as_tensors / load_state_from_tensors).  Every method forwards to the C functions of the
-same name; torch supplies device memory and the current stream, nothing else.
+same name; torch supplies device memory and the current stream, nothing else.  The loops over plain tensors run in
+_torch_face (csrc/eri_torch_face.cpp); what it leaves to the Python code below is anything out of the ordinary.
 """
 import ctypes as C
 from dataclasses import dataclass
@@ -14,6 +15,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
+from . import _torch_face
 from ._lib import DTYPE_BF16, DTYPE_F32, Adam8bitConfigC, check, lib
 
 
@@ -111,8 +113,10 @@ class Adam8bit:
 
     def step(self) -> int:
         """One optimizer step; returns how many parameters were skipped for lack of a gradient."""
-        live = []
-        for i, p in enumerate(self.params):
+        held, rest = _torch_face.bind(self.params, C.addressof(self._handles))
+        live = [held]
+        for i in rest:
+            p = self.params[i]
             g = p.grad
             if g is not None:
                 g = _usable_grad(g, p)
@@ -228,7 +232,7 @@ class Adam8bitFunctional:
         self._opt = C.c_void_p()
         check(lib().eri_adam8bit_fn_with_params(learning_rate, beta1, beta2, eps, weight_decay, _stream_ptr(),
                                                 C.byref(self._opt)), "eri_adam8bit_fn_with_params")
-        self._names: List[str] = []
+        self._names: Dict[str, None] = {}  # in the order the names came up
         self._live: List[torch.Tensor] = []
         self._launched = False
         self._batched = bool(batched)
@@ -276,12 +280,19 @@ class Adam8bitFunctional:
         self._keep([p, g, out])
         if not self._batched:
             self._launched = True  # ran at once; released when the next update arrives
-        if name not in self._names:
-            self._names.append(name)
+        self._names[name] = None
         return out
 
     def update_many(self, params: Dict[str, torch.Tensor], grads: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
         """Every named parameter that has a gradient, in one launch; returns the new tensors by name."""
+        done = _torch_face.update_many(self._opt.value, params, grads) if type(params) is dict and type(grads) is dict else None
+        if done is not None:
+            code, outs, held = done
+            check(code, "eri_adam8bit_fn_update_many")
+            self._keep([held])
+            self._launched = True
+            self._names.update(dict.fromkeys(outs))
+            return outs
         names = [n for n in params if n in grads]
         k = len(names)
         ps = [params[n].detach().contiguous() for n in names]
@@ -296,9 +307,7 @@ class Adam8bitFunctional:
               "eri_adam8bit_fn_update_many")
         self._keep(ps + gs + outs)
         self._launched = True
-        for n in names:
-            if n not in self._names:
-                self._names.append(n)
+        self._names.update(dict.fromkeys(names))
         return dict(zip(names, outs))
 
     def memory_stats(self) -> Tuple[int, int]:
@@ -324,8 +333,7 @@ class Adam8bitFunctional:
             v = v.detach().to(torch.float32).contiguous().view(-1)
             check(lib().eri_adam8bit_fn_load_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr(),
                                                         m.numel()), "eri_adam8bit_fn_load_state_fp32")
-            if name not in self._names:
-                self._names.append(name)
+            self._names[name] = None
 
     def close(self) -> None:
         if self._opt:

@@ -1,0 +1,131 @@
+"""The native loops of the Python face: which tensors they take and which they leave to the Python code (CPU), and that
+both ways give the same bits (GPU)."""
+import ctypes as C
+
+import pytest
+import torch
+from torch.overrides import BaseTorchFunctionMode
+
+from eridiffusion_amd import _lib as L
+from eridiffusion_amd import _torch_face
+
+
+class Sub(torch.Tensor):
+    pass
+
+
+def _handles(params):
+    arr = (C.c_void_p * len(params))()
+    for i, p in enumerate(params):
+        h = C.c_void_p()
+        tag = L.DTYPE_BF16 if p.dtype == torch.bfloat16 else L.DTYPE_F32
+        L.check(L.lib().eri_param_create(p.data_ptr() or 1, p.numel(), tag, C.byref(h)), "eri_param_create")
+        arr[i] = h
+    return arr
+
+
+def _gradient_forms(device):
+    """(parameter, gradient, taken natively) of every form the list optimizer accepts."""
+    bf, f32 = torch.bfloat16, torch.float32
+
+    def new(*shape, dtype=f32, seed=11):
+        return (torch.randn(*shape, generator=torch.Generator().manual_seed(sum(shape) + seed)) * 1e-3).to(dtype).to(device)
+    leaf = new(40, 64).requires_grad_()
+    param = torch.nn.Parameter(new(2049))
+    return [(new(40, 64), new(40, 64), True), (new(40, 64, dtype=bf), new(40, 64, dtype=bf), True),
+            (new(40, 64, dtype=bf), new(40, 64), True),              # fp32 gradient of a bf16 parameter
+            (new(40, 64), new(40, 64, dtype=bf), False),             # cast to the parameter's dtype
+            (new(40, 64), new(64, 40).t(), False),                   # transposed
+            (new(64), new(64, 2)[:, 0], False),                      # strided
+            (new(40, 64), new(40, 64).as_subclass(Sub), False),      # a subclass may redefine what it is asked
+            (new(40, 64).as_subclass(Sub), new(40, 64), False),
+            (new(2048)[16:], new(2032), True),                       # a view with an offset
+            (new(40, 64), None, True), (leaf, new(40, 64), True), (param, new(2049), True)]
+
+
+def _with_grads(forms):
+    params = []
+    for p, g, _ in forms:
+        if g is not None and g.dtype != p.dtype:
+            p.grad_dtype = None  # a gradient of another dtype may be assigned
+        p.grad = g
+        params.append(p)
+    return params
+
+
+def test_what_bind_takes():
+    forms = _gradient_forms("cpu")
+    params = _with_grads(forms)
+    handles = _handles(params)
+    held, rest = _torch_face.bind(params, C.addressof(handles))
+    assert rest == [i for i, (_, _, taken) in enumerate(forms) if not taken]
+    with BaseTorchFunctionMode():
+        assert _torch_face.bind(params, C.addressof(handles))[1] == list(range(len(params)))
+    product = params[10] * 2  # not a leaf: asking for its gradient warns, in Python code
+    assert _torch_face.bind([product], C.addressof(handles))[1] == [0]
+    assert _torch_face.bind([torch.empty(0)], C.addressof(handles))[1] == [0]  # no address: the C call refuses it by name
+    with pytest.raises(TypeError):
+        _torch_face.bind(tuple(params), C.addressof(handles))
+    for h in handles:
+        L.lib().eri_param_release(h)
+
+
+def test_what_update_many_leaves_to_python():
+    a, g = torch.zeros(8), torch.zeros(8)
+    leave = [({}, {}), ({"a": a}, {"b": g}), ({"a": a.double()}, {"a": g}), ({"a": a}, {"a": g.bfloat16()}),
+             ({"a": torch.zeros(4, 4).t()[1:]}, {"a": torch.zeros(3, 4)}), ({"a": a}, {"a": torch.zeros(16)[::2]}),
+             ({"a": a.as_subclass(Sub)}, {"a": g}), ({3: a}, {3: g}), ({"a": a.to_sparse()}, {"a": g})]
+    for params, grads in leave:
+        assert _torch_face.update_many(1, params, grads) is None
+    with BaseTorchFunctionMode():
+        assert _torch_face.update_many(1, {"a": a}, {"a": g}) is None
+
+
+@pytest.mark.gpu
+def test_native_and_python_loops_step_alike():
+    from eridiffusion_amd.adam8bit import Adam8bit, Adam8bitConfig, Adam8bitFunctional, update_params_8bit
+    results = []
+    for general in (False, True):
+        forms = _gradient_forms("cuda")
+        params = _with_grads(forms)
+        opt = Adam8bit(params, Adam8bitConfig(lr=1e-3))
+        for _ in range(2):
+            if general:
+                with BaseTorchFunctionMode():
+                    assert opt.step() == 1
+            else:
+                assert opt.step() == 1
+        named = {"t%d" % i: p.detach().clone() for i, (p, g, _) in enumerate(forms) if g is not None}
+        grads = {"t%d" % i: g for i, (_, g, _) in enumerate(forms) if g is not None}
+        plain = {n for i, (_, g, taken) in enumerate(forms) for n in ["t%d" % i] if taken and g is not None}
+        outs = []
+        for keep in (plain, set(named)):  # the plain ones alone take the native loop, all together the Python one
+            fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+            now = {n: t for n, t in named.items() if n in keep}
+            for _ in range(2):
+                if general:
+                    with BaseTorchFunctionMode():
+                        update_params_8bit(fn, now, grads)
+                else:
+                    update_params_8bit(fn, now, grads)
+                fn.step()
+            assert list(fn.get_state_as_tensors()) == list(now)
+            outs += [t.clone() for t in now.values()]
+        torch.cuda.synchronize()
+        results.append([p.detach().clone() for p in params] + outs)
+    for a, b in zip(*results):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_update_many_refusals_keep_their_codes():
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    fn.update_many({"a": torch.zeros(64, device="cuda")}, {"a": torch.zeros(64, device="cuda")})
+    with pytest.raises(L.EriError) as e:  # a state of another size under the same name
+        fn.update_many({"a": torch.zeros(128, device="cuda")}, {"a": torch.zeros(128, device="cuda")})
+    assert e.value.code == -6
+    with pytest.raises(L.EriError) as e:
+        fn.update_many({"b": torch.zeros(0, device="cuda")}, {"b": torch.zeros(0, device="cuda")})
+    assert e.value.code in (-1, -3)
+    assert list(fn.get_state_as_tensors()) == ["a"]
