@@ -136,10 +136,21 @@ int launch_step_pipelined_f32(int mode, bool wd, bool gs, const DevTensor *rows,
 int launch_quant_error(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, int layout,
                        const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, double *err,
                        uint32_t grid, void *stream);
-/* Gradient norm: one f64 partial per wave (grid * 4 of them), then norm and clip factor into out[0], out[1]. */
+/* Gradient norm: one f64 pair per workgroup (sum of squares, count of non-finite elements), then norm and clip factor
+ * into out[0], out[1].  A pass covers up to two tables, a group per layout each. */
 constexpr uint32_t kNormWavesPerCu = 32; // persistent waves of the gradient-norm pass per compute unit
-int launch_grad_sumsq(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, bool grad_bf16,
-                      double *partial, uint32_t grid, void *stream);
+struct NormGroup {
+    const DevTensor *rows;
+    uint32_t n_rows, total_blocks, n_tails;
+    uint32_t first_wg, wgs; // the launch's workgroups that take this group
+    uint32_t chunks;        // ranges the block list is cut into, as the step over the same group cuts it
+    uint32_t grad_bf16;
+};
+struct NormGroups {
+    NormGroup g[2 * kLayouts];
+    uint32_t n;
+};
+int launch_grad_sumsq(const NormGroups &groups, double *partial, void *stream);
 int launch_grad_norm_finish(const double *partial, uint32_t n, float max_norm, float denom_eps, float *out,
                             void *stream);
 /* Diagnostics: reads and rewrites (unchanged) every full block of a group of bf16 rows as the step does. */

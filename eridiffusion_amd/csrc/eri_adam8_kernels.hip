@@ -344,9 +344,8 @@ int launch_quantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const
 // ------------------------------------------------------------------------------------------
 // global gradient norm over the launch table (the trainers' clip_gradients,
 // src/trainers/pipeline_flux_lora_sequential.rs:1198-1213,1939-1950), without a host round trip:
-// pass 1 forms one fp32 sum of squares per block and adds a wave's blocks in f64, pass 2 adds the waves'
-// partials and writes the norm and
-// the clip factor to device memory, where the step kernel reads it.
+// pass 1 forms one fp32 sum of squares per block and adds a workgroup's blocks in f64, pass 2 adds the workgroups'
+// partials and writes the norm and the clip factor to device memory, where the step kernel reads it.
 // ------------------------------------------------------------------------------------------
 
 /* 1.0 for NaN and +-infinity, else 0.0 */
@@ -365,120 +364,158 @@ __device__ __forceinline__ float wave_sum(float x) {
     return r;
 }
 
+__device__ __forceinline__ double wave_sum_f64(double x) {
+    for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
+    return x;
+}
+
+/* One wave's blocks of one group of rows: partial last blocks follow the full ones in the same list, and the wave
+ * takes its share from the last to the first, one block's loads ahead. */
 template <bool BF16>
-__global__ __launch_bounds__(1024) void grad_sumsq_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,
-                                                         uint32_t total_blocks, double *__restrict__ partial,
-                                                         uint32_t chunks) {
-    // persistent: every wave adds the fp32 sums of its blocks in f64 and leaves one partial
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t waves_per_wg = blockDim.x / kWave;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
-    const uint32_t stride = gridDim.x * waves_per_wg;
-    double total = 0.0, bad = 0.0;
-    for (uint32_t r = wave; r < n_rows; r += stride) { // partial last blocks
-        const DevTensor t = rows[r];
-        const uint32_t n = (uint32_t)(t.numel % kBlock);
-        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-        float acc = 0.0f, nf = 0.0f;
-        for (uint32_t i = lane; i < n; i += kWave) {
-            const float g = load1<BF16>(t.g, e0 + i);
-            acc += g * g;
-            nf += not_finite(g);
-        }
-        total += (double)wave_sum(acc);
-        bad += (double)wave_sum(nf);
-    }
-    // full blocks, one load ahead: the next block's four words are in flight while this one is reduced
-    const BlockWalk walk(total_blocks, chunks);
-    if (walk.first < walk.end) {
-        uint32_t ti = 0, t_end = 0;
-        DevTensor t;
-        Raw8<BF16> raw[4];
-        const BlockRowMap map(rows, n_rows);
-        {
-            map.seek(rows, walk.first, ti, t, t_end);
-            const size_t e0 = (size_t)(walk.first - t.full_start) * kBlock;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) raw[c].load(static_cast<const char *>(t.g) + e0 * (BF16 ? 2 : 4), c * 512 + lane * 8);
-        }
-        for (uint32_t blk = walk.first; blk < walk.end; blk += walk.stride) {
-            Raw8<BF16> cur[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) cur[c] = raw[c];
-            const uint32_t nblk = blk + walk.stride;
-            if (nblk < walk.end) {
-                map.seek(rows, nblk, ti, t, t_end);
-                const size_t e0 = (size_t)(nblk - t.full_start) * kBlock;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) raw[c].load(static_cast<const char *>(t.g) + e0 * (BF16 ? 2 : 4), c * 512 + lane * 8);
+__device__ __forceinline__ void grad_sumsq_walk(const NormGroup &g, uint32_t wg, uint32_t wave_in_wg, uint32_t lane,
+                                                double &total, double &bad) {
+    const BlockRowMap map(g.rows, g.n_rows);
+    const uint32_t units = g.total_blocks + g.n_tails;
+    const uint32_t per_chunk = (units + g.chunks - 1) / g.chunks;
+    const uint32_t lo = (wg % g.chunks) * per_chunk;
+    const uint32_t end = lo + per_chunk < units ? lo + per_chunk : units;
+    const uint32_t stride = (g.wgs / g.chunks) * kNormWaves;
+    const uint32_t first = lo + (wg / g.chunks) * kNormWaves + wave_in_wg;
+    if (first >= end) return;
+    uint32_t left = (end - first + stride - 1) / stride; // blocks of this wave, counted down
+    uint32_t unit = first + (left - 1) * stride;
+    // full blocks [row_start, row_start + row_blocks) belong to the row at hand, whose gradients start at row_g
+    uint32_t row_start = 0, row_blocks = 0;
+    const char *row_g = nullptr;
+    Raw8<BF16> raw[4];
+    auto request = [&](uint32_t u) {
+        if (u < g.total_blocks) {
+            if (u - row_start >= row_blocks) {
+                const DevTensor &t = g.rows[map.row_of[u]];
+                row_g = static_cast<const char *>(t.g);
+                row_start = t.full_start;
+                row_blocks = (uint32_t)(t.numel / kBlock);
             }
-            float acc = 0.0f;
+            const char *base = row_g + (size_t)(u - row_start) * kBlock * (BF16 ? 2 : 4);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) raw[c].load(base, c * 512 + lane * 8);
+        } else {
+            const DevTensor &t = g.rows[map.tail_row(g.total_blocks, u - g.total_blocks)];
+            const uint32_t n = (uint32_t)(t.numel % kBlock);
+            const char *base = static_cast<const char *>(t.g) + (size_t)(t.numel / kBlock) * kBlock * (BF16 ? 2 : 4);
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                float g[8];
-                cur[c].unpack(g);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) acc += g[k] * g[k];
-            }
-            const float block_sum = wave_sum(acc);
-            total += (double)block_sum;
-            if (not_finite(block_sum) != 0.0f) { // rare: count the NaN / infinite elements of this block
-                float nf = 0.0f;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    float g[8];
-                    cur[c].unpack(g);
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) nf += not_finite(g[k]);
-                }
-                bad += (double)wave_sum(nf);
+                const uint32_t o = c * 512 + lane * 8;
+                const uint32_t count = lane_count(o, n);
+                if (count == 8) raw[c].load(base, o);
+                else raw[c].load_some(base, o, count);
             }
         }
+    };
+    request(unit);
+    while (true) {
+        Raw8<BF16> cur[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) cur[c] = raw[c];
+        const bool more = left > 1;
+        if (more) {
+            unit -= stride;
+            request(unit);
+        }
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float x[8];
+            cur[c].unpack(x);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc += x[k] * x[k];
+        }
+        const float block_sum = wave_sum(acc);
+        total += (double)block_sum;
+        if (not_finite(block_sum) != 0.0f) { // rare: count the NaN / infinite elements of this block
+            float nf = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float x[8];
+                cur[c].unpack(x);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) nf += not_finite(x[k]);
+            }
+            bad += (double)wave_sum(nf);
+        }
+        if (!more) break;
+        --left;
     }
+}
+
+/* All groups of rows of a pass in one launch: workgroups [first_wg, first_wg + wgs) take a group.  Reading the
+ * gradients once is the bound (6.2 TB/s on 10.3 GB); on the tables of an adapter the launches count as much, so there
+ * is one whatever the tables hold.  Measured, this pass and the one behind it, before (a launch per group, a pair per
+ * wave, partial blocks element by element) and after:
+ *   256 short tensors in two tables  5.3 + 5.3 + 3.0 -> 4.1 + 2.4 us
+ *   608 tensors, 306 MB of bf16      47.6 + 6.7 -> 48.2 + 5.4 us, and the step behind it 303 -> 299 us (it starts on
+ *                                    gradients that the last-level cache still holds: the walk goes backwards)
+ *   1,680 tensors, 10.3 GB of fp32   1,655 + 7.2 -> 1,640 + 4.7 us */
+__global__ __launch_bounds__(kNormWaves * kWave) void grad_sumsq_kernel(NormGroups groups, double *__restrict__ partial) {
+    __shared__ double sums[kNormWaves][2];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint32_t gi = 0;
+    while (gi + 1 < groups.n && blockIdx.x >= groups.g[gi + 1].first_wg) ++gi;
+    const NormGroup &g = groups.g[gi];
+    double total = 0.0, bad = 0.0;
+    if (g.grad_bf16) grad_sumsq_walk<true>(g, blockIdx.x - g.first_wg, wave_in_wg, lane, total, bad);
+    else grad_sumsq_walk<false>(g, blockIdx.x - g.first_wg, wave_in_wg, lane, total, bad);
     if (lane == 0) {
-        partial[2 * wave] = total;
-        partial[2 * wave + 1] = bad;
+        sums[wave_in_wg][0] = total;
+        sums[wave_in_wg][1] = bad;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double x = 0.0;
+        for (uint32_t w = 0; w < kNormWaves; ++w) x += sums[w][threadIdx.x];
+        partial[2 * blockIdx.x + threadIdx.x] = x;
     }
 }
 
 __global__ __launch_bounds__(1024) void grad_norm_finish_kernel(const double *__restrict__ partial, uint32_t n,
                                                                 float max_norm, float denom_eps,
                                                                 float *__restrict__ out /* norm, scale, u64 count */) {
-    // partial holds, per wave of the first pass, the sum of squares and the count of non-finite elements
-    __shared__ double sh[1024], shb[1024];
+    // partial holds, per workgroup of the first pass, the sum of squares and the count of non-finite elements
+    __shared__ double sums[16][2];
     double acc = 0.0, bad = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < n; i += 1024) {
         acc += partial[2 * i];
         bad += partial[2 * i + 1];
     }
-    sh[threadIdx.x] = acc;
-    shb[threadIdx.x] = bad;
-    __syncthreads();
-    for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            sh[threadIdx.x] += sh[threadIdx.x + s];
-            shb[threadIdx.x] += shb[threadIdx.x + s];
-        }
-        __syncthreads();
+    acc = wave_sum_f64(acc);
+    bad = wave_sum_f64(bad);
+    if (threadIdx.x % kWave == 0) {
+        sums[threadIdx.x / kWave][0] = acc;
+        sums[threadIdx.x / kWave][1] = bad;
     }
+    __syncthreads();
     if (threadIdx.x == 0) {
-        const float norm = (float)sqrt(sh[0]);
+        acc = bad = 0.0;
+        for (int w = 0; w < 16; ++w) {
+            acc += sums[w][0];
+            bad += sums[w][1];
+        }
+        const float norm = (float)sqrt(acc);
         float scale = 1.0f;
         // clip only a finite norm above the limit (crates/training/src/optimizer.rs:79-84)
         if (max_norm > 0.0f && norm > max_norm && norm <= 3.4028234e38f) scale = max_norm / (norm + denom_eps);
         out[0] = norm;
         out[1] = scale;
-        *reinterpret_cast<unsigned long long *>(out + 2) = (unsigned long long)shb[0];
+        *reinterpret_cast<unsigned long long *>(out + 2) = (unsigned long long)bad;
     }
 }
 
-int launch_grad_sumsq(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, bool grad_bf16, double *partial,
-                      uint32_t grid, void *stream) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!grad_bf16)
-        hipLaunchKernelGGL(grad_sumsq_kernel<false>, dim3(grid), dim3(kNormWaves * kWave), 0, s, rows, n_rows, total_blocks, partial, chunks_for(grid));
-    else
-        hipLaunchKernelGGL(grad_sumsq_kernel<true>, dim3(grid), dim3(kNormWaves * kWave), 0, s, rows, n_rows, total_blocks, partial, chunks_for(grid));
+int launch_grad_sumsq(const NormGroups &groups, double *partial, void *stream) {
+    const NormGroup &last = groups.g[groups.n - 1];
+    hipLaunchKernelGGL(grad_sumsq_kernel, dim3(last.first_wg + last.wgs), dim3(kNormWaves * kWave), 0, static_cast<hipStream_t>(stream),
+                       groups, partial);
     return (int)hipGetLastError();
 }
 
@@ -495,11 +532,6 @@ int launch_grad_norm_finish(const double *partial, uint32_t n, float max_norm, f
 // exactly as the step will, quantises them, and adds |value - dequantised value| per row in f64.
 // Diagnostics, not tuned: element by element, binary search.
 // ------------------------------------------------------------------------------------------
-
-__device__ __forceinline__ double wave_sum_f64(double x) {
-    for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
-    return x;
-}
 
 template <bool BF16, int MODE, bool WD, bool GS>
 __global__ __launch_bounds__(256) void quant_error_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,

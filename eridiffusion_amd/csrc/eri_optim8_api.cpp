@@ -205,11 +205,11 @@ const Tables &tables() {
 
 constexpr int kMaxDevices = 16;
 
-/* Scratch of eri_adam8_grad_norm_static: the per-wave partial sums of the gradient-norm pass, in device
+/* Scratch of eri_adam8_grad_norm_static: the partial sums of the gradient-norm pass, in device
  * memory that exists from the moment the library is loaded until the process ends (every device the
  * library runs on holds its own copy, 384 KiB).  The name below is a host-side stand-in, not a device
  * address: host code uses DeviceCtx::scratch_ptr, which hipGetSymbolAddress filled in for that device. */
-constexpr uint32_t kNormScratchPairs = 24576; // {sum of squares, non-finite count} per wave: 3 groups x 256 CUs x 32 waves
+constexpr uint32_t kNormScratchPairs = 24576; // {sum of squares, non-finite count} per workgroup: 3 groups x 256 CUs x 8 and room to spare
 static __device__ __align__(256) double scratch[2 * kNormScratchPairs];
 
 struct DeviceCtx {
@@ -317,12 +317,11 @@ struct EriAdam8Table {
     void *upload_stream = nullptr;  // stream of the last upload
     void *ordered_stream = nullptr; // another stream that has already been made to wait for that upload
     bool ordered_valid = false;
-    double *partial = nullptr; // one sum of squares per wave of the norm pass, per group
+    double *partial = nullptr; // per workgroup of the norm pass a sum of squares and a count
     float *norm_out = nullptr; // device: {norm, clip factor, 64-bit count}, owned by the table
     float *norm_last = nullptr; // where the last norm pass left its result: norm_out, the caller's buffer, or the
                                 // norm_out of the table this one was normed together with
     bool grads_only = false;    // rows carry gradients only: the table serves the norm pass and nothing else
-    uint32_t n_partial = 0;
     double *qerr = nullptr;    // device: per row {sum |m - deq m|, sum |v - deq v|}, groups back to back
     bool qerr_valid = false;
 };
@@ -1075,47 +1074,49 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
 }
 
 /* The launches of the gradient-norm pass over one table, or over two as if they were one (`also` may be null):
- * a sum-of-squares launch per group of rows, then one launch that adds the per-wave partial sums of all of them.
+ * one launch of sums of squares over all groups of rows, then one that adds its workgroups' partial sums.
  * `partial` holds room for `pairs` {sum, count} pairs. */
 static int grad_norm_launch(EriAdam8Table *t, EriAdam8Table *also, DeviceCtx *ctx, float max_norm, float denom_eps,
                             double *partial, uint32_t pairs, float *result, void *stream) {
     const uint32_t wpw = (uint32_t)eri::kNormWaves;
     const uint32_t grid_cap = ctx->cus * eri::kNormWavesPerCu / wpw; // persistent
     EriAdam8Table *tables[2] = {t, also};
-    uint32_t grids[2][eri::kLayouts] = {{0, 0, 0}, {0, 0, 0}}, need = 0;
-    for (int ti = 0; ti < 2; ++ti) {
-        if (!tables[ti]) continue;
-        for (int gi = 0; gi < eri::kLayouts; ++gi) {
-            const auto &g = tables[ti]->groups[gi];
+    eri::NormGroups groups;
+    groups.n = 0;
+    uint32_t wgs = 0;
+    for (EriAdam8Table *one : tables) {
+        if (!one) continue;
+        for (const auto &g : one->groups) {
             if (g.n == 0) continue;
-            const uint32_t work = g.total_blocks > g.n ? g.total_blocks : g.n;
-            uint32_t grid = (work + wpw - 1) / wpw;
-            if (grid > grid_cap) grid = grid_cap;
-            grids[ti][gi] = grid;
-            need += grid * wpw;
+            eri::NormGroup &ng = groups.g[groups.n++];
+            const uint32_t grid = (g.total_blocks + g.n_tails + wpw - 1) / wpw; // a row has one block at least
+            ng.rows = g.dev;
+            ng.n_rows = g.n;
+            ng.total_blocks = g.total_blocks;
+            ng.n_tails = g.n_tails;
+            ng.first_wg = wgs;
+            ng.wgs = grid > grid_cap ? grid_cap : grid;
+            // The step walks the larger groups in one range per die, the others in a common window; this pass takes
+            // the same way backwards, so that the gradients it read last, which the last-level cache still holds,
+            // are the first that the step reads.
+            ng.chunks = (uint64_t)g.total_blocks > (uint64_t)ctx->cus * eri::kPrefetchBlocksPerCu ? eri::chunks_for(ng.wgs) : 1u;
+            ng.grad_bf16 = eri::layout_grad_bf16(g.dtype) ? 1u : 0u;
+            wgs += ng.wgs;
         }
     }
-    if (need > pairs) {
+    if (wgs > pairs) {
         char buf[160];
-        std::snprintf(buf, sizeof buf, "the gradient-norm pass of this table needs %u per-wave partial sums, the scratch holds %u",
-                      need, pairs);
+        std::snprintf(buf, sizeof buf, "the gradient-norm pass of this table needs %u partial sums, the scratch holds %u", wgs, pairs);
         return fail(ERI_ERR_TOO_LARGE, buf);
     }
-    uint32_t off = 0;
-    for (int ti = 0; ti < 2; ++ti) {
-        if (!tables[ti]) continue;
-        int rc = order_after_upload(tables[ti], stream);
+    for (EriAdam8Table *one : tables) {
+        if (!one) continue;
+        int rc = order_after_upload(one, stream);
         if (rc) return rc;
-        for (int gi = 0; gi < eri::kLayouts; ++gi) {
-            auto &g = tables[ti]->groups[gi];
-            if (g.n == 0) continue;
-            rc = eri::launch_grad_sumsq(g.dev, g.n, g.total_blocks, eri::layout_grad_bf16(g.dtype), partial + 2 * off, grids[ti][gi], stream);
-            if (rc) return hip_fail((hipError_t)rc, "gradient sum-of-squares launch");
-            off += grids[ti][gi] * wpw;
-        }
     }
-    t->n_partial = off;
-    int rc = eri::launch_grad_norm_finish(partial, off, max_norm, denom_eps, result, stream);
+    int rc = eri::launch_grad_sumsq(groups, partial, stream);
+    if (rc) return hip_fail((hipError_t)rc, "gradient sum-of-squares launch");
+    rc = eri::launch_grad_norm_finish(partial, wgs, max_norm, denom_eps, result, stream);
     if (rc) return hip_fail((hipError_t)rc, "gradient norm launch");
     t->norm_last = result;
     if (also) also->norm_last = result;
@@ -1128,8 +1129,8 @@ static int grad_norm(EriAdam8Table *t, EriAdam8Table *also, float max_norm, floa
     DeviceCtx *ctx = nullptr;
     int rc = get_ctx_on(t->device, &ctx);
     if (rc) return rc;
-    // per table one group per layout at most, and per wave a sum of squares and a count; room for two tables
-    const uint32_t pairs = 2 * eri::kLayouts * ctx->cus * eri::kNormWavesPerCu;
+    // per table one group per layout at most, and per workgroup a sum of squares and a count; room for two tables
+    const uint32_t pairs = 2 * eri::kLayouts * ctx->cus * eri::kNormWavesPerCu / eri::kNormWaves;
     if (!t->partial) ERI_HIP(hipMalloc((void **)&t->partial, sizeof(double) * 2 * pairs));
     if (!t->norm_out) ERI_HIP(hipMalloc((void **)&t->norm_out, sizeof(float) * 4)); // norm, scale, 64-bit count
     return grad_norm_launch(t, also, ctx, max_norm, denom_eps, t->partial, pairs, t->norm_out, stream);

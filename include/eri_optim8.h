@@ -273,8 +273,8 @@ int eri_adam8_grad_norm_joint(EriAdam8Table *table, EriAdam8Table *also, float m
 int eri_adam8_grad_norm_scale_ptr(const EriAdam8Table *table, const float **dev_scale);
 /* The same pass for callers that cannot allocate (code under HIP graph capture, serving loops, harnesses
  * that forbid hipMalloc).  It has no counterpart in the reference.  eri_adam8_grad_norm allocates the
- * per-wave partial sums and the result words on a table's first call; this variant allocates nothing:
- * the partial sums go to a static device array of the library (384 KiB per device, 24,576 per-wave
+ * partial sums and the result words on a table's first call; this variant allocates nothing:
+ * the partial sums go to a static device array of the library (384 KiB per device, 24,576
  * pairs; a table whose pass needs more is refused with ERI_ERR_TOO_LARGE -- none does on a 256-CU
  * MI355X) and the result to `result`, 16 bytes of device memory the caller owns, 8-byte aligned:
  * {float norm, float scale, uint64 count of non-finite elements}.  A following step with

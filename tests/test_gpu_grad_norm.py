@@ -221,3 +221,44 @@ def test_joint_norm_over_a_step_table_and_a_gradient_only_table():
     assert abs(norm2.value - only) <= 2e-6 * only and scale2.value == 1.0
     L.lib().eri_adam8_table_destroy(gtable)
     L.lib().eri_adam8_table_destroy(table)
+
+
+@pytest.mark.parametrize("repeat", [1, 40], ids=["a-wave-each", "many-blocks-per-wave"])
+def test_one_launch_over_every_layout_and_partial_block(repeat):
+    """Two tables with groups of all three layouts, last blocks of every shape, NaN in the words behind every gradient:
+    none of those is read, and the norm is that of all gradients."""
+    import torch
+    L = _L()
+    rng = np.random.default_rng(321)
+    ends = [1, 7, 8, 9, 505, 512, 513, 1543, 2041, 2047, 2048, 3 * 2048, 2048 + 5]
+    layouts = [(L.DTYPE_F32, 0), (L.DTYPE_BF16, 0), (L.DTYPE_BF16, 1)]
+    total, keep, tables = 0.0, [], []
+    for part in range(2):
+        rows = (L.TensorRow * (len(ends) * repeat * 3))()
+        start = 0
+        for i in range(len(rows)):
+            n = ends[(i // 3) % len(ends)] * (9 if repeat > 1 and i % 7 == 0 else 1)
+            tag, grad_f32 = layouts[(i + part) % 3]
+            g = (rng.standard_normal(n + 16) * 1e-3).astype(np.float32)
+            g[n:] = np.nan
+            t = torch.from_numpy(g).cuda()
+            if tag == L.DTYPE_BF16 and not grad_f32:
+                t = t.bfloat16()
+            keep.append(t)
+            total += float((t[:n].double() ** 2).sum())
+            r = rows[i]
+            r.p = r.g = t.data_ptr()
+            r.numel, r.block_start, r.dtype_tag, r.grad_f32, r.grad_scale = n, start, tag, grad_f32, 1.0
+            start += (n + 2047) // 2048
+        table = C.c_void_p()
+        L.check(L.lib().eri_adam8_grad_table_create(rows, len(rows), None, C.byref(table)), "grad_table_create")
+        tables.append(table)
+    for _ in range(2):
+        L.check(L.lib().eri_adam8_grad_norm_joint(tables[0], tables[1], 1.0, 0.0, None), "grad_norm_joint")
+        norm, scale, bad = C.c_float(), C.c_float(), C.c_uint64()
+        L.check(L.lib().eri_adam8_grad_norm_read(tables[1], C.byref(norm), C.byref(scale), None), "read")
+        L.check(L.lib().eri_adam8_grad_nonfinite_read(tables[0], C.byref(bad), None), "nonfinite_read")
+        want = np.sqrt(total)
+        assert bad.value == 0 and abs(norm.value - want) <= 2e-6 * want
+    for t in tables:
+        L.lib().eri_adam8_table_destroy(t)
