@@ -95,8 +95,15 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_bloc
                 uint32_t compute_units, void *stream);
 
 constexpr uint32_t kChunks = 8;           /* contiguous ranges the block list is cut into: one per accelerator die */
-constexpr uint32_t kSplitBlocksPerCu = 64; /* tables of at most this many full blocks per compute unit take the
-                                              four-waves-per-block kernel */
+/* Tables of at most this many blocks per compute unit (partial ones counted) take the four-waves-per-block kernel: one
+ * round of its four teams.  Beyond it that kernel pays a barrier and a trip to memory per round, and a wave per block
+ * fills the chip by itself.  us per launch on 256 units, four waves per block | one:
+ *   blocks      1,024        1,536         2,816         8,192
+ *   bf16       7.6 | 8.9  10.6 | 10.5  15.7 | 15.1   38.4 | 33.7
+ *   fp32       9.0 | 10.1 14.4 | 12.8  23.9 | 20.8   53.3 | 50.3
+ *   bf16, fp32 gradients, functional update
+ *              8.2 | 8.9  12.5 | 10.9  17.3 | 15.1   44.0 | 35.3 */
+constexpr uint32_t kSplitBlocksPerCu = 4;
 constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* bf16 tables take the prefetching kernel above this many full blocks
                                                    per compute unit; up to it, sixteen waves without a prefetch are
                                                    2-4 % faster than twelve with one (measured at 292-876 per unit,
@@ -119,8 +126,9 @@ int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, 
 int launch_step_split(int layout, int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows,
                       uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                       uint32_t grid, uint32_t teams, void *stream);
-/* Whether launch_step would run this group on the prefetching kernel with the EMA update inside it. */
-bool step_fuses_ema(uint32_t total_full_blocks, int layout, const EriAdam8Hyper &h, uint32_t compute_units);
+/* Whether launch_step would run this group on the prefetching kernel with the EMA update inside it.  units: full blocks
+ * and partial ones. */
+bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units);
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream);

@@ -519,6 +519,12 @@ __device__ __forceinline__ void store_codes_some(uint8_t *codes, const u32x2 w, 
         if (k < count) as_global(codes)[k] = (uint8_t)((k < 4 ? w.x : w.y) >> (8 * (k & 3)));
 }
 
+template <bool PARTIAL>
+__device__ __forceinline__ void store_codes(uint8_t *codes, const u32x2 w, uint32_t count) {
+    if (!PARTIAL || count == 8) __builtin_nontemporal_store(w, as_global(reinterpret_cast<u32x2 *>(codes)));
+    else store_codes_some(codes, w, count);
+}
+
 __device__ __forceinline__ uint32_t byte_of(const u32x2 w, int k) {
     const uint32_t d = k < 4 ? w.x : w.y;
     return (d >> (8 * (k & 3))) & 0xffu;
@@ -635,9 +641,11 @@ __device__ __forceinline__ void requant8(const float *mf, const float *vf, const
 /* `mine` is the wave's own pair of 256-entry tables in LDS.  The block opens by filling them with
  * (MAP[c] * absmax) * beta for every code c -- the first two operations of both moment updates, done once
  * per code (eight per lane) instead of once per element (64 per lane); a wave's LDS operations complete in
- * order, so its reads below see its own writes without a barrier. */
-template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16>
-__device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint32_t lane, const StepHyper &h,
+ * order, so its reads below see its own writes without a barrier.
+ * PARTIAL: a row's last block of n < 2048 elements; lanes past the end are off (see tail_block for what stands in for
+ * the elements that are missing). */
+template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16, bool PARTIAL = false>
+__device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint32_t n, uint32_t lane, const StepHyper &h,
                                            float gscale, const BlockDiv &dbc1, const BlockDiv &dbc2, const Lds &L,
                                            float (*mine)[256]) {
     const size_t e0 = (size_t)lb * kBlock;
@@ -665,7 +673,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     float lm = 0.0f, lv = 0.0f;
     // Issue the loads of DEPTH passes before touching the first value: the wave then waits once per
     // DEPTH passes, with 48 * DEPTH bytes per lane in flight (bf16; fp32 values hold twice the registers).
-    constexpr int DEPTH = (BF16 && GBF16) ? 4 : 2;
+    constexpr int DEPTH = ((BF16 && GBF16) ? 4 : 2) / (PARTIAL ? 2 : 1);
 #pragma unroll
     for (int c0 = 0; c0 < 4; c0 += DEPTH) {
         Raw8<BF16> pr[DEPTH];
@@ -674,10 +682,18 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const uint32_t o = (c0 + d) * 512 + lane * 8;
-            pr[d].load(p_in, o);
-            gr[d].load(g, o);
-            mr[d] = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(mc + o)));
-            vr[d] = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(vc + o)));
+            const uint32_t count = lane_count(o, n);
+            if (!PARTIAL || count == 8) {
+                pr[d].load(p_in, o);
+                gr[d].load(g, o);
+                mr[d] = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(mc + o)));
+                vr[d] = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(vc + o)));
+            } else {
+                pr[d].load_some(p_in, o, count);
+                gr[d].load_some(g, o, count);
+                mr[d] = load_codes_some(mc + o, count, kZeroCodesS);
+                vr[d] = load_codes_some(vc + o, count, kZeroCodesU);
+            }
         }
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
@@ -708,7 +724,8 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
                     if (redo.lanes[k] && redo.mine(k))
                         pn[k] = param_exact<MODE, WD, BF16>(pv[k], mf[c * 8 + k], vf[c * 8 + k], h, dbc1, dbc2);
             }
-            store8<BF16>(p, o, pn);
+            if (!PARTIAL || lane_count(o, n) == 8) store8<BF16>(p, o, pn);
+            else store_some<BF16>(p, o, pn, lane_count(o, n));
         }
     }
     float nam = lm, nav = lv;
@@ -725,8 +742,8 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<true, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
-            __builtin_nontemporal_store(mw, as_global(reinterpret_cast<u32x2 *>(mc + o)));
-            __builtin_nontemporal_store(vw, as_global(reinterpret_cast<u32x2 *>(vc + o)));
+            store_codes<PARTIAL>(mc + o, mw, lane_count(o, n));
+            store_codes<PARTIAL>(vc + o, vw, lane_count(o, n));
         }
     } else {
 #pragma unroll
@@ -734,8 +751,8 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
-            __builtin_nontemporal_store(mw, as_global(reinterpret_cast<u32x2 *>(mc + o)));
-            __builtin_nontemporal_store(vw, as_global(reinterpret_cast<u32x2 *>(vc + o)));
+            store_codes<PARTIAL>(mc + o, mw, lane_count(o, n));
+            store_codes<PARTIAL>(vc + o, vw, lane_count(o, n));
         }
     }
 }

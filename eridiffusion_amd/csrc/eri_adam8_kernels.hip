@@ -9,10 +9,10 @@ namespace eri {
 
 /* The one case in which the EMA runs inside the step kernel: the prefetching kernel in mode ERI, on bf16
  * parameters (with bf16 or fp32 gradients). */
-bool step_fuses_ema(uint32_t total_blocks, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
+bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
     if ((h.flags & ERI_ADAM8_FLAG_EMA) == 0 || !layout_param_bf16(layout) || h.mode != ERI_ADAM8_MODE_ERI) return false;
     if (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) return false;
-    const bool few = (uint64_t)total_blocks <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
+    const bool few = (uint64_t)units <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
     return (h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || !few;
 }
 
@@ -34,14 +34,14 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     // have no binary-search variant of the one-wave kernel and stay on this one for those flags.
     const bool one_wave = (h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0;
     const bool kernel_named = (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) != 0;
-    const bool few = (uint64_t)total_blocks <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
+    const uint32_t units = total_blocks + n_tails; // a partial block costs what a full one does
+    const bool few = (uint64_t)units <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
     if ((mixed && (h.flags & ERI_ADAM8_FLAG_BSEARCH) != 0) || (!kernel_named && !one_wave && few)) {
         const bool bnb = h.mode == ERI_ADAM8_MODE_BNB;
         const bool wd_s = bnb ? h.weight_decay != 1.0f : h.weight_decay > 0.0f;
         const bool exact_s = !bf16 || (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
         // Up to four blocks per workgroup at a time (a team of four waves each), but no more than it takes to
         // give every compute unit a workgroup: 512 blocks on 256 units run as 256 workgroups of two teams.
-        const uint32_t units = total_blocks + n_tails; // a partial block counts like a full one here
         uint32_t teams = (units + compute_units - 1) / compute_units;
         teams = teams < 1 ? 1 : teams > 4 ? 4 : teams;
         uint32_t need = (units + teams - 1) / teams;
@@ -54,7 +54,7 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
         const bool wd_m = h.mode == ERI_ADAM8_MODE_BNB ? h.weight_decay != 1.0f : h.weight_decay > 0.0f;
         if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
             return launch_step_pipelined_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs,
-                                                  step_fuses_ema(total_blocks, layout, h, compute_units), rows, n_rows,
+                                                  step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                                   total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_bf16(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs, true, true, rows, n_rows,
                                       total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
@@ -76,7 +76,7 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
         return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     if (!bf16) return launch_step_plain_f32(h.mode, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
-        return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(total_blocks, layout, h, compute_units), rows, n_rows,
+        return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
 }

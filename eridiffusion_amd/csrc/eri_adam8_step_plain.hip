@@ -1,7 +1,10 @@
 /*
- * The plain step kernel (one wave per block, no cross-block prefetch): large tables of fp32 parameters and
- * of bf16 parameters with fp32 gradients, bf16 tables in the functional update's arithmetic, and any table
- * with ERI_ADAM8_FLAG_BSEARCH, ERI_ADAM8_FLAG_NO_PIPELINE or ERI_ADAM8_FLAG_ONE_WAVE.  Compiled twice,
+ * The plain step kernel (one wave per block, no cross-block prefetch): tables of every layout and mode between the
+ * four-waves-per-block kernel's (kSplitBlocksPerCu) and the prefetching kernel's (kPrefetchBlocksPerCu), and any table
+ * with ERI_ADAM8_FLAG_BSEARCH or ERI_ADAM8_FLAG_NO_PIPELINE.  HBM traffic bounds it, with the launch's start and its
+ * last round on the smaller tables.  A row's partial last block is one more block of the walk, with the lanes past its
+ * end off and one trip less in flight: as a two-sweep chain on one wave each it made 300 odd bf16 tensors with 14 M
+ * parameters 32.8 us, 28.3 so; 1,400 LoRA tensors 93.9 -> 92.1 us.  Compiled twice,
  * once per parameter dtype (-DERI_PLAIN_BF16=0|1), so that the two halves build in parallel.
  */
 #include "eri_adam8_inline.h"
@@ -49,34 +52,34 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     const uint32_t stride = gridDim.x * waves_per_wg;
     const BlockDiv dbc1(h.bc1), dbc2(h.bc2);
 
-    // Full blocks: round k gives wave w block k * stride + w, and the blocks left over when the list does not
-    // divide (fewer than one per wave) go one to each workgroup in turn -- workgroup i takes left-over blocks
-    // i, i + grid, i + 2 grid, ... on its first waves -- so that the short last round runs on every compute
-    // unit instead of filling the first few (2-3 % of the launch on tables of 5-20 blocks per wave).
+    // The blocks, partial last ones behind the full ones: round k gives wave w block k * stride + w, and the blocks
+    // left over when the list does not divide (fewer than one per wave) go one to each workgroup in turn -- workgroup
+    // i takes left-over blocks i, i + grid, i + 2 grid, ... on its first waves -- so that the short last round runs on
+    // every compute unit instead of filling the first few (2-3 % of the launch on tables of 5-20 blocks per wave).
+    const uint32_t units = total_blocks + n_tails;
     const uint32_t wave_in_wg = threadIdx.x / kWave;
-    const uint32_t rounds = total_blocks / stride;
+    const uint32_t rounds = units / stride;
     const uint32_t left_first = rounds * stride;
     const uint32_t left_mine = wave_in_wg * gridDim.x + blockIdx.x;
-    const bool has_left = left_first + left_mine < total_blocks;
+    const bool has_left = left_first + left_mine < units;
 
-    // partial last blocks first, one to each workgroup in turn, from a workgroup's last wave backwards: those are
-    // the waves without a left-over block, so the slower two-sweep tail lands where there is slack
-    const BlockRowMap map(rows, n_rows);
-    for (uint32_t i = blockIdx.x + (waves_per_wg - 1 - wave_in_wg) * gridDim.x; i < n_tails; i += stride) {
-        const DevTensor t = rows[map.tail_row(total_blocks, i)];
-        const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
-        tail_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, (uint32_t)(t.numel / kBlock), (uint32_t)(t.numel % kBlock), lane,
-                                                             h, gscale, dbc1, dbc2, L);
-    }
     uint32_t ti = 0, t_end = 0;
     DevTensor t;
+    const BlockRowMap map(rows, n_rows);
     const uint32_t trips = rounds + (has_left ? 1u : 0u);
     for (uint32_t k = 0; k < trips; ++k) {
-        const uint32_t blk = k < rounds ? k * stride + wave : left_first + left_mine;
-        map.seek(rows, blk, ti, t, t_end);
-        const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
-        full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, blk - t.full_start, lane, h, gscale, dbc1, dbc2, L,
-                                                             decayed[threadIdx.x / kWave]);
+        const uint32_t unit = __builtin_amdgcn_readfirstlane(k < rounds ? k * stride + wave : left_first + left_mine);
+        if (unit < total_blocks) {
+            map.seek(rows, unit, ti, t, t_end);
+            const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
+            full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, unit - t.full_start, kBlock, lane, h, gscale, dbc1, dbc2, L,
+                                                                 decayed[threadIdx.x / kWave]);
+        } else {
+            t = rows[map.tail_row(total_blocks, unit - total_blocks)];
+            const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
+            full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16, true>(t, (uint32_t)(t.numel / kBlock), (uint32_t)(t.numel % kBlock),
+                                                                       lane, h, gscale, dbc1, dbc2, L, decayed[threadIdx.x / kWave]);
+        }
     }
 }
 

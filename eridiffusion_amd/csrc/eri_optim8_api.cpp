@@ -1033,7 +1033,7 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
         // spread over every compute unit instead of filling a few of them.
         uint32_t waves_per_wg = ctx->wg / eri::kWave;
         const uint32_t slots = ctx->cus * ctx->wg_per_cu;
-        const uint32_t work = g.total_blocks > g.n ? g.total_blocks : g.n; // full blocks, or one tail per row
+        const uint32_t work = g.total_blocks + g.n_tails;
         const uint32_t per_slot = (work + slots - 1) / slots;
         if (per_slot < waves_per_wg) waves_per_wg = per_slot < 4 ? 4 : per_slot;
         uint32_t grid = slots;
@@ -1051,7 +1051,7 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
         }
         rc = eri::launch_step(g.dev, g.n, g.total_blocks, g.n_tails, g.dtype, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
         if (rc) return hip_fail((hipError_t)rc, "adam8 step launch");
-        if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(g.total_blocks, g.dtype, hh, ctx->cus)) {
+        if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(g.total_blocks + g.n_tails, g.dtype, hh, ctx->cus)) {
             // not the kernel that carries the EMA: this group's shadows join the plain sweep that follows the step
             for (uint32_t j = 0; j < g.n; ++j) {
                 const eri::DevTensor &d = g.pinned[j];
