@@ -190,13 +190,30 @@ struct ElemRow {
 };
 static_assert(sizeof(ElemRow) == 56, "ElemRow must stay 56 bytes");
 
-/* scaled: every gradient is first multiplied by (grad_scale * row.scale) * (*dev_scale, 1 if null), as the 8-bit
- * step does with ERI_ADAM8_FLAG_GRAD_SCALE. */
-int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_full_blocks, int dtype_tag,
-                   const EriAdamW32Hyper &h, bool scaled, float grad_scale, const float *dev_scale, uint32_t grid,
+/* One block of a small sweep: block `block` of row `row`.  The small kernels take one per workgroup, a quarter per wave:
+ * with a wave per block a table of few blocks lasts as long as one wave's chain of a row search, a partial block and a
+ * full one. */
+struct SweepUnit {
+    uint32_t row, block;
+};
+/* Sweeps of at most this many blocks per compute unit take the small kernels.  us per call, a wave per block | a quarter,
+ * 64 tensors, 256 units:
+ *   blocks                    64          512        2,048        8,192         16,384
+ *   32-bit step, bf16     6.0 | 4.0    7.1 | 5.8   19.0 | 16.0  59.7 | 59.5   118 | 112
+ *   ... with masters      6.7 | 3.9    9.4 | 7.0   23.7 | 22.6  94.5 | 78.5   199 | 171
+ *   ... 1,027 more each  12.4 | 4.5   14.1 | 7.2   24.6 | 18.2  60.9 | 60.1   113 | 112
+ *   EMA, fp32             4.0 | 3.7    4.2 | 4.1    8.4 |  7.1  31.5 | 29.4   57.5 | 56.8
+ * Above it the list itself (8 bytes per block, uploaded when the rows change) is no longer small. */
+constexpr uint32_t kSmallSweepBlocksPerCu = 64;
+
+/* units: the list of blocks, n_units of them, for the small kernels; null for the persistent ones, which take `grid`
+ * workgroups.  scaled: every gradient is first multiplied by (grad_scale * row.scale) * (*dev_scale, 1 if null), as the
+ * 8-bit step does with ERI_ADAM8_FLAG_GRAD_SCALE. */
+int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_full_blocks, const SweepUnit *units, uint32_t n_units,
+                   int dtype_tag, const EriAdamW32Hyper &h, bool scaled, float grad_scale, const float *dev_scale, uint32_t grid,
                    void *stream);
-int launch_ema(const ElemRow *rows, uint32_t n_rows, uint32_t total_full_blocks, int dtype_tag, float decay,
-               uint32_t grid, void *stream);
+int launch_ema(const ElemRow *rows, uint32_t n_rows, uint32_t total_full_blocks, const SweepUnit *units, uint32_t n_units,
+               int dtype_tag, float decay, uint32_t grid, void *stream);
 
 } // namespace eri
 #endif

@@ -632,7 +632,10 @@ int launch_quant_error(const DevTensor *rows, uint32_t n_rows, uint32_t total_bl
 
 // ------------------------------------------------------------------------------------------
 // plain element-wise sweeps over a row table: 32-bit AdamW and EMA.  One wave per 2048-element
-// block, 8 elements per lane and pass, partial last blocks element by element.  HBM-bound:
+// block, 8 elements per lane and pass, all of a block's loads in flight at once; in a partial last block the
+// lanes past the end are off and the one lane the end falls into moves its elements singly.  Sweeps of few blocks
+// take a quarter block per wave (kSmallSweepBlocksPerCu): the 32-bit step over the 87 tensors of 1,280 to 2,560
+// elements of a small adapter 14.2 -> 4.1 us.  HBM-bound:
 // AdamW bf16 22 B/param (read 2+2+4+4, write 2+4+4), fp32 28 B/param; EMA 3 x element size.
 // ------------------------------------------------------------------------------------------
 
@@ -654,17 +657,23 @@ __device__ __forceinline__ void adamw32_elem(float p, float g, float &m, float &
     pn = p + step;
 }
 
-template <bool BF16>
-__device__ __forceinline__ void store1(void *base, size_t i, float x) {
-    if (BF16) as_global(static_cast<uint16_t *>(base))[i] = (uint16_t)bf16_bits(x);
-    else as_global(static_cast<float *>(base))[i] = x;
+/* Eight elements of a lane of which `count` exist; of a full block (PARTIAL false) all do. */
+template <bool BF16, bool PARTIAL>
+__device__ __forceinline__ void sweep_load(Raw8<BF16> &r, const void *base, uint32_t o, uint32_t count) {
+    if (!PARTIAL || count == 8) r.load(base, o);
+    else r.load_some(base, o, count);
+}
+template <bool BF16, bool PARTIAL>
+__device__ __forceinline__ void sweep_store(void *base, uint32_t o, const float (&x)[8], uint32_t count) {
+    if (!PARTIAL || count == 8) store8<BF16>(base, o, x);
+    else store_some<BF16>(base, o, x, count);
 }
 
-/* One full block of the 32-bit step.  MASTER: the parameter value comes from, and goes back to, an fp32
+/* One block of the 32-bit step, of n elements.  MASTER: the parameter value comes from, and goes back to, an fp32
  * master copy; the tensor itself only receives the rounded result (mixed precision,
  * src/kernels/fused_adam.cu:151-193, with the arithmetic of adamw.rs). */
-template <bool BF16, bool MASTER, bool GS>
-__device__ __forceinline__ void adamw32_block(const ElemRow &t, size_t e0, uint32_t lane, const EriAdamW32Hyper &h,
+template <bool BF16, bool MASTER, bool GS, bool PARTIAL>
+__device__ __forceinline__ void adamw32_block(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, const EriAdamW32Hyper &h,
                                               float omb1, float omb2, float neg_lr, float gscale) {
     char *p = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
     const char *g = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
@@ -676,11 +685,12 @@ __device__ __forceinline__ void adamw32_block(const ElemRow &t, size_t e0, uint3
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const uint32_t o = c * 512 + lane * 8;
-        if (MASTER) wr[c].load(w, o);
-        else pr[c].load(p, o);
-        gr[c].load(g, o);
-        mr[c].load(m, o);
-        vr[c].load(v, o);
+        const uint32_t count = lane_count(o, n);
+        if (MASTER) sweep_load<false, PARTIAL>(wr[c], w, o, count);
+        else sweep_load<BF16, PARTIAL>(pr[c], p, o, count);
+        sweep_load<BF16, PARTIAL>(gr[c], g, o, count);
+        sweep_load<false, PARTIAL>(mr[c], m, o, count);
+        sweep_load<false, PARTIAL>(vr[c], v, o, count);
     }
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -693,10 +703,56 @@ __device__ __forceinline__ void adamw32_block(const ElemRow &t, size_t e0, uint3
         vr[c].unpack(vv);
 #pragma unroll
         for (int k = 0; k < 8; ++k) adamw32_elem(pv[k], GS ? gv[k] * gscale : gv[k], mv[k], vv[k], h, omb1, omb2, neg_lr, pn[k]);
-        store8<BF16>(p, o, pn);
-        if (MASTER) store8<false>(w, o, pn);
-        store8<false>(m, o, mv);
-        store8<false>(v, o, vv);
+        const uint32_t count = lane_count(o, n);
+        sweep_store<BF16, PARTIAL>(p, o, pn, count);
+        if (MASTER) sweep_store<false, PARTIAL>(w, o, pn, count);
+        sweep_store<false, PARTIAL>(m, o, mv, count);
+        sweep_store<false, PARTIAL>(v, o, vv, count);
+    }
+}
+
+/* A workgroup of the small sweeps: one block, partial or not, a quarter of it per wave (nothing crosses lanes here).
+ * The list of blocks rides behind the rows, so a wave finds its row with one load instead of a search. */
+struct SweepQuarter {
+    ElemRow t;
+    size_t e0;
+    uint32_t o, count; // this lane's eight elements and how many of them exist
+    __device__ __forceinline__ SweepQuarter(const ElemRow *rows, const SweepUnit &u)
+        : t(rows[u.row]), e0((size_t)u.block * kBlock), o(threadIdx.x * 8), count(t.numel - e0 >= kBlock ? 8u : lane_count(o, (uint32_t)(t.numel - e0))) {}
+};
+
+template <bool BF16, bool GS>
+__global__ __launch_bounds__(256) void adamw32_small_kernel(const ElemRow *__restrict__ rows, const SweepUnit *__restrict__ units,
+                                                            uint32_t n_units, EriAdamW32Hyper h, float grad_scale,
+                                                            const float *__restrict__ dev_scale) {
+    const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
+    const float omb1 = 1.0f - h.beta1, omb2 = 1.0f - h.beta2, neg_lr = -h.lr; // adamw.rs:36,42,53
+    for (uint32_t i = blockIdx.x; i < n_units; i += gridDim.x) {
+        const SweepQuarter q(rows, units[i]);
+        if (q.count == 0) continue;
+        char *p = static_cast<char *>(q.t.a) + q.e0 * (BF16 ? 2 : 4);
+        float *m = static_cast<float *>(q.t.c) + q.e0, *v = static_cast<float *>(q.t.d) + q.e0;
+        float *w = q.t.e ? static_cast<float *>(q.t.e) + q.e0 : nullptr; // fp32 master copy
+        Raw8<BF16> pr, gr;
+        Raw8<false> mr, vr, wr;
+        if (w) sweep_load<false, true>(wr, w, q.o, q.count);
+        else sweep_load<BF16, true>(pr, p, q.o, q.count);
+        sweep_load<BF16, true>(gr, static_cast<const char *>(q.t.b) + q.e0 * (BF16 ? 2 : 4), q.o, q.count);
+        sweep_load<false, true>(mr, m, q.o, q.count);
+        sweep_load<false, true>(vr, v, q.o, q.count);
+        const float gscale = GS ? (grad_scale * q.t.scale) * tscale : 1.0f;
+        float pv[8], gv[8], mv[8], vv[8], pn[8];
+        if (w) wr.unpack(pv);
+        else pr.unpack(pv);
+        gr.unpack(gv);
+        mr.unpack(mv);
+        vr.unpack(vv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) adamw32_elem(pv[k], GS ? gv[k] * gscale : gv[k], mv[k], vv[k], h, omb1, omb2, neg_lr, pn[k]);
+        sweep_store<BF16, true>(p, q.o, pn, q.count);
+        if (w) sweep_store<false, true>(w, q.o, pn, q.count);
+        sweep_store<false, true>(m, q.o, mv, q.count);
+        sweep_store<false, true>(v, q.o, vv, q.count);
     }
 }
 
@@ -714,21 +770,11 @@ __global__ __launch_bounds__(256) void adamw32_kernel(const ElemRow *__restrict_
     for (uint32_t r = wave; r < n_rows; r += stride) {
         const ElemRow t = rows[r];
         const uint32_t n = (uint32_t)(t.numel % kBlock);
+        if (n == 0) continue;
         const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-        ERI_GLOBAL float *mp = as_global(static_cast<float *>(t.c));
-        ERI_GLOBAL float *vp = as_global(static_cast<float *>(t.d));
-        ERI_GLOBAL float *wp = as_global(static_cast<float *>(t.e)); // fp32 master copy, or null
         const float gscale = GS ? (grad_scale * t.scale) * tscale : 1.0f; // the order of the 8-bit step's factors
-        for (uint32_t i = lane; i < n; i += kWave) {
-            float m = mp[e0 + i], v = vp[e0 + i], pn;
-            const float pf = wp ? wp[e0 + i] : load1<BF16>(t.a, e0 + i);
-            const float gf = load1<BF16>(t.b, e0 + i);
-            adamw32_elem(pf, GS ? gf * gscale : gf, m, v, h, omb1, omb2, neg_lr, pn);
-            mp[e0 + i] = m;
-            vp[e0 + i] = v;
-            if (wp) wp[e0 + i] = pn;
-            store1<BF16>(t.a, e0 + i, pn);
-        }
+        if (t.e) adamw32_block<BF16, true, GS, true>(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale);
+        else adamw32_block<BF16, false, GS, true>(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale);
     }
     uint32_t ti = 0, t_end = 0;
     ElemRow t;
@@ -737,8 +783,8 @@ __global__ __launch_bounds__(256) void adamw32_kernel(const ElemRow *__restrict_
         seek_row(rows, n_rows, blk, ti, t, t_end);
         const size_t e0 = (size_t)(blk - t.full_start) * kBlock;
         const float gscale = GS ? (grad_scale * t.scale) * tscale : 1.0f;
-        if (t.e) adamw32_block<BF16, true, GS>(t, e0, lane, h, omb1, omb2, neg_lr, gscale);
-        else adamw32_block<BF16, false, GS>(t, e0, lane, h, omb1, omb2, neg_lr, gscale);
+        if (t.e) adamw32_block<BF16, true, GS, false>(t, e0, kBlock, lane, h, omb1, omb2, neg_lr, gscale);
+        else adamw32_block<BF16, false, GS, false>(t, e0, kBlock, lane, h, omb1, omb2, neg_lr, gscale);
     }
 }
 
@@ -747,6 +793,49 @@ __device__ __forceinline__ float ema_elem(float shadow, float p, float decay, fl
     float a = shadow * decay;
     float b = p * omd;
     return a + b;
+}
+
+template <bool BF16, bool PARTIAL>
+__device__ __forceinline__ void ema_block(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, float decay, float omd) {
+    char *s = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
+    const char *p = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
+    Raw8<BF16> sr[4], pr[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t o = c * 512 + lane * 8;
+        sweep_load<BF16, PARTIAL>(sr[c], s, o, lane_count(o, n));
+        sweep_load<BF16, PARTIAL>(pr[c], p, o, lane_count(o, n));
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const uint32_t o = c * 512 + lane * 8;
+        float sv[8], pv[8], out[8];
+        sr[c].unpack(sv);
+        pr[c].unpack(pv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
+        sweep_store<BF16, PARTIAL>(s, o, out, lane_count(o, n));
+    }
+}
+
+template <bool BF16>
+__global__ __launch_bounds__(256) void ema_small_kernel(const ElemRow *__restrict__ rows, const SweepUnit *__restrict__ units,
+                                                        uint32_t n_units, float decay) {
+    const float omd = 1.0f - decay; // ema_enhanced.rs:96
+    for (uint32_t i = blockIdx.x; i < n_units; i += gridDim.x) {
+        const SweepQuarter q(rows, units[i]);
+        if (q.count == 0) continue;
+        char *s = static_cast<char *>(q.t.a) + q.e0 * (BF16 ? 2 : 4);
+        Raw8<BF16> sr, pr;
+        sweep_load<BF16, true>(sr, s, q.o, q.count);
+        sweep_load<BF16, true>(pr, static_cast<const char *>(q.t.b) + q.e0 * (BF16 ? 2 : 4), q.o, q.count);
+        float sv[8], pv[8], out[8];
+        sr.unpack(sv);
+        pr.unpack(pv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
+        sweep_store<BF16, true>(s, q.o, out, q.count);
+    }
 }
 
 template <bool BF16>
@@ -760,9 +849,7 @@ __global__ __launch_bounds__(256) void ema_kernel(const ElemRow *__restrict__ ro
     for (uint32_t r = wave; r < n_rows; r += stride) {
         const ElemRow t = rows[r];
         const uint32_t n = (uint32_t)(t.numel % kBlock);
-        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-        for (uint32_t i = lane; i < n; i += kWave)
-            store1<BF16>(t.a, e0 + i, ema_elem(load1<BF16>(t.a, e0 + i), load1<BF16>(t.b, e0 + i), decay, omd));
+        if (n != 0) ema_block<BF16, true>(t, (size_t)(t.numel / kBlock) * kBlock, n, lane, decay, omd);
     }
     uint32_t ti = 0, t_end = 0;
     ElemRow t;
@@ -770,31 +857,23 @@ __global__ __launch_bounds__(256) void ema_kernel(const ElemRow *__restrict__ ro
     for (uint32_t blk = walk.first; blk < walk.end; blk += walk.stride) {
         seek_row(rows, n_rows, blk, ti, t, t_end);
         const size_t e0 = (size_t)(blk - t.full_start) * kBlock;
-        char *s = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
-        const char *p = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
-        Raw8<BF16> sr[4], pr[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            sr[c].load(s, c * 512 + lane * 8);
-            pr[c].load(p, c * 512 + lane * 8);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            float sv[8], pv[8], out[8];
-            sr[c].unpack(sv);
-            pr[c].unpack(pv);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
-            store8<BF16>(s, c * 512 + lane * 8, out);
-        }
+        ema_block<BF16, false>(t, e0, kBlock, lane, decay, omd);
     }
 }
 
-int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, int dtype_tag,
-                   const EriAdamW32Hyper &h, bool scaled, float grad_scale, const float *dev_scale, uint32_t grid,
+int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, const SweepUnit *units, uint32_t n_units,
+                   int dtype_tag, const EriAdamW32Hyper &h, bool scaled, float grad_scale, const float *dev_scale, uint32_t grid,
                    void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_GO(B, G) hipLaunchKernelGGL((adamw32_kernel<B, G>), dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, h, grad_scale, dev_scale, chunks_for(grid))
+#define ERI_GO(B, G)                                                                                                     \
+    do {                                                                                                                 \
+        if (units)                                                                                                       \
+            hipLaunchKernelGGL((adamw32_small_kernel<B, G>), dim3(n_units), dim3(256), 0, s, rows, units, n_units, h,     \
+                               grad_scale, dev_scale);                                                                   \
+        else                                                                                                             \
+            hipLaunchKernelGGL((adamw32_kernel<B, G>), dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, h,        \
+                               grad_scale, dev_scale, chunks_for(grid));                                                 \
+    } while (0)
     if (dtype_tag == ERI_DTYPE_F32) {
         if (scaled) ERI_GO(false, true);
         else ERI_GO(false, false);
@@ -806,10 +885,14 @@ int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, 
     return (int)hipGetLastError();
 }
 
-int launch_ema(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, int dtype_tag, float decay,
-               uint32_t grid, void *stream) {
+int launch_ema(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, const SweepUnit *units, uint32_t n_units,
+               int dtype_tag, float decay, uint32_t grid, void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype_tag == ERI_DTYPE_F32)
+    if (units && dtype_tag == ERI_DTYPE_F32)
+        hipLaunchKernelGGL(ema_small_kernel<false>, dim3(n_units), dim3(256), 0, s, rows, units, n_units, decay);
+    else if (units)
+        hipLaunchKernelGGL(ema_small_kernel<true>, dim3(n_units), dim3(256), 0, s, rows, units, n_units, decay);
+    else if (dtype_tag == ERI_DTYPE_F32)
         hipLaunchKernelGGL(ema_kernel<false>, dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, decay, chunks_for(grid));
     else
         hipLaunchKernelGGL(ema_kernel<true>, dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, decay, chunks_for(grid));

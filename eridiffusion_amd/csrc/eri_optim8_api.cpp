@@ -1362,8 +1362,9 @@ namespace {
  * was uploaded on is ordered after the upload by an event wait on that stream. */
 struct ElemCache {
     struct Group {
-        eri::ElemRow *dev = nullptr, *pinned = nullptr;
-        uint32_t cap = 0, n = 0;
+        eri::ElemRow *dev = nullptr, *pinned = nullptr; // n rows, then the list of n_units blocks of a small sweep
+        size_t cap = 0;                                 // bytes
+        uint32_t n = 0, n_units = 0;
     };
     struct Slot {
         Group groups[2]; // F32, BF16
@@ -1378,7 +1379,8 @@ struct ElemCache {
                 if (g.dev) (void)hipFree(g.dev);
                 if (g.pinned) (void)hipHostFree(g.pinned);
                 g.dev = g.pinned = nullptr;
-                g.cap = g.n = 0;
+                g.cap = 0;
+                g.n = g.n_units = 0;
             }
             if (ev) (void)hipEventDestroy(ev);
             ev = nullptr;
@@ -1401,7 +1403,7 @@ struct ElemCache {
         }
         return sl.used != 0;
     }
-    int sync(void *stream, uint32_t cus, int (*launch)(const eri::ElemRow *, uint32_t, uint32_t, int, uint32_t, void *, const void *),
+    int sync(void *stream, uint32_t cus, int (*launch)(const eri::ElemRow *, uint32_t, uint32_t, const eri::SweepUnit *, uint32_t, int, uint32_t, void *, const void *),
              const void *extra) {
         int dev = 0;
         ERI_HIP(hipGetDevice(&dev));
@@ -1443,18 +1445,27 @@ struct ElemCache {
                 const uint32_t n = (uint32_t)rows[gi].size();
                 g.n = 0;
                 if (n == 0) continue;
-                if (g.cap < n) {
+                uint64_t units = 0;
+                for (const auto &r : rows[gi]) units += blocks_of(r.numel);
+                g.n_units = units <= (uint64_t)cus * eri::kSmallSweepBlocksPerCu ? (uint32_t)units : 0;
+                const size_t bytes = sizeof(eri::ElemRow) * n + sizeof(eri::SweepUnit) * g.n_units;
+                if (g.cap < bytes) {
                     if (g.dev) (void)hipFree(g.dev);
                     if (g.pinned) (void)hipHostFree(g.pinned);
                     g.dev = g.pinned = nullptr;
                     g.cap = 0; // stays 0 if an allocation below fails: the next call starts over
-                    const uint32_t cap = n + n / 2 + 16;
-                    ERI_HIP(hipMalloc((void **)&g.dev, sizeof(eri::ElemRow) * cap));
-                    ERI_HIP(hipHostMalloc((void **)&g.pinned, sizeof(eri::ElemRow) * cap, hipHostMallocDefault));
+                    const size_t cap = bytes + bytes / 2 + 1024;
+                    ERI_HIP(hipMalloc((void **)&g.dev, cap));
+                    ERI_HIP(hipHostMalloc((void **)&g.pinned, cap, hipHostMallocDefault));
                     g.cap = cap;
                 }
                 std::memcpy(g.pinned, rows[gi].data(), n * sizeof(eri::ElemRow));
-                ERI_HIP(hipMemcpyAsync(g.dev, g.pinned, n * sizeof(eri::ElemRow), hipMemcpyHostToDevice,
+                if (g.n_units) {
+                    eri::SweepUnit *u = reinterpret_cast<eri::SweepUnit *>(g.pinned + n);
+                    for (uint32_t j = 0; j < n; ++j)
+                        for (uint32_t b = 0, end = (uint32_t)blocks_of(rows[gi][j].numel); b < end; ++b) *u++ = {j, b};
+                }
+                ERI_HIP(hipMemcpyAsync(g.dev, g.pinned, bytes, hipMemcpyHostToDevice,
                                        static_cast<hipStream_t>(stream)));
                 g.n = n;
             }
@@ -1472,7 +1483,8 @@ struct ElemCache {
             const uint32_t work = total > n ? total : n;
             uint32_t grid = (work + 3) / 4;
             if (grid > cus * 16) grid = cus * 16;
-            int rc = launch(g.dev, n, total, gi == 0 ? ERI_DTYPE_F32 : ERI_DTYPE_BF16, grid, stream, extra);
+            const eri::SweepUnit *units = g.n_units ? reinterpret_cast<const eri::SweepUnit *>(g.dev + n) : nullptr;
+            int rc = launch(g.dev, n, total, units, g.n_units, gi == 0 ? ERI_DTYPE_F32 : ERI_DTYPE_BF16, grid, stream, extra);
             if (rc) return hip_fail((hipError_t)rc, "element-wise sweep launch");
         }
         return 0;
@@ -1496,12 +1508,12 @@ struct AdamW32Extra {
     float grad_scale;
     const float *dev_scale; // device, or null for 1
 };
-int adamw32_launch(const eri::ElemRow *rows, uint32_t n, uint32_t total, int dtype, uint32_t grid, void *stream, const void *extra) {
+int adamw32_launch(const eri::ElemRow *rows, uint32_t n, uint32_t total, const eri::SweepUnit *units, uint32_t n_units, int dtype, uint32_t grid, void *stream, const void *extra) {
     const AdamW32Extra &x = *static_cast<const AdamW32Extra *>(extra);
-    return eri::launch_adamw32(rows, n, total, dtype, x.h, x.scaled, x.grad_scale, x.dev_scale, grid, stream);
+    return eri::launch_adamw32(rows, n, total, units, n_units, dtype, x.h, x.scaled, x.grad_scale, x.dev_scale, grid, stream);
 }
-int ema_launch(const eri::ElemRow *rows, uint32_t n, uint32_t total, int dtype, uint32_t grid, void *stream, const void *extra) {
-    return eri::launch_ema(rows, n, total, dtype, *static_cast<const float *>(extra), grid, stream);
+int ema_launch(const eri::ElemRow *rows, uint32_t n, uint32_t total, const eri::SweepUnit *units, uint32_t n_units, int dtype, uint32_t grid, void *stream, const void *extra) {
+    return eri::launch_ema(rows, n, total, units, n_units, dtype, *static_cast<const float *>(extra), grid, stream);
 }
 
 } // namespace

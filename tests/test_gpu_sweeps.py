@@ -264,3 +264,59 @@ def test_traffic_probe_moves_the_bytes_and_changes_none():
     assert L.lib().eri_adam8_traffic_probe(t32, None) == -6
     L.lib().eri_adam8_table_destroy(t32)
     assert L.lib().eri_adam8_traffic_probe(None, None) == -1
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("more", [0, 64 * 256 * 2048], ids=["small-kernels", "persistent-kernels"])
+def test_partial_blocks_of_every_shape(bf16, more):
+    """Last blocks that end inside a lane's eight elements, on a lane's edge and one short of a block, in the 32-bit step
+    (every other row with a master copy where there is one) and the EMA sweep; nothing is written past a tensor."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    rng = np.random.default_rng(400 + bf16)
+    ends = [1, 7, 8, 9, 505, 512, 513, 1023, 1536, 1543, 2041, 2047]
+    sizes = ends + [2048 + e for e in ends] + [2048] + ([more] if more else [])  # one tensor takes the table over the line
+    tag, dt = (2, np.uint16) if bf16 else (0, np.float32)
+
+    def normal(n, std):  # the large one repeats itself
+        return np.resize((rng.standard_normal(min(n, 100003)) * std).astype(np.float32), n)
+
+    def host(n, std):
+        return onp.f32_to_bf16(normal(n, std)) if bf16 else normal(n, std)
+
+    def guarded(a):  # 64 poisoned bytes on both sides
+        raw = np.full(a.nbytes + 128, 0xA5, np.uint8)
+        raw[64:64 + a.nbytes] = a.view(np.uint8)
+        return torch.from_numpy(raw).cuda()
+
+    def back(t, dtype):
+        raw = t.cpu().numpy()
+        assert np.all(raw[:64] == 0xA5) and np.all(raw[-64:] == 0xA5)
+        return raw[64:-64].copy().view(dtype)
+
+    ps, gs, sh = [host(n, 0.02) for n in sizes], [host(n, 1e-3) for n in sizes], [host(n, 0.02) for n in sizes]
+    ms, vs = [normal(n, 1e-4) for n in sizes], [normal(n, 1e-3) ** 2 for n in sizes]
+    ws = [onp.bf16_to_f32(p).astype(np.float32) if bf16 and i % 2 else None for i, p in enumerate(ps)]
+    dp, dg, dm, dv, ds = [[guarded(a) for a in xs] for xs in (ps, gs, ms, vs, sh)]
+    dw = [guarded(w) if w is not None else None for w in ws]
+    rows, erows = (L.AdamW32Row * len(sizes))(), (L.EmaRow * len(sizes))()
+    for i, n in enumerate(sizes):
+        r, e = rows[i], erows[i]
+        r.p, r.g, r.m, r.v = [d[i].data_ptr() + 64 for d in (dp, dg, dm, dv)]
+        r.master = dw[i].data_ptr() + 64 if dw[i] is not None else None
+        r.numel, r.dtype_tag = n, tag
+        e.shadow, e.p, e.numel, e.dtype_tag = ds[i].data_ptr() + 64, r.p, n, tag
+        oc.lib().eri_oracle_adamw32_step(oc.ptr(ps[i]), oc.ptr(gs[i]), oc.ptr(ms[i]), oc.ptr(vs[i]), n, tag, 1e-3, 0.9, 0.999, 1e-8,
+                                         0.01, oc.ptr(ws[i]) if ws[i] is not None else None)
+        oc.lib().eri_oracle_ema_update(oc.ptr(sh[i]), oc.ptr(ps[i]), n, tag, 0.999)
+    stream = torch.cuda.current_stream().cuda_stream
+    h = L.AdamW32Hyper(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    L.check(L.lib().eri_adamw32_step_multi(rows, len(sizes), C.byref(h), stream), "adamw32")
+    L.check(L.lib().eri_ema_update_multi(erows, len(sizes), 0.999, stream), "ema")
+    torch.cuda.synchronize()
+    for i in range(len(sizes)):
+        assert np.array_equal(back(dp[i], dt), ps[i]), sizes[i]
+        assert np.array_equal(back(dg[i], dt), gs[i]) and np.array_equal(back(ds[i], dt), sh[i]), sizes[i]
+        assert np.array_equal(back(dm[i], np.float32), ms[i]) and np.array_equal(back(dv[i], np.float32), vs[i]), sizes[i]
+        if ws[i] is not None:
+            assert np.array_equal(back(dw[i], np.float32), ws[i]), sizes[i]
