@@ -369,16 +369,40 @@ __device__ __forceinline__ double wave_sum_f64(double x) {
     return x;
 }
 
-/* One wave's blocks of one group of rows: partial last blocks follow the full ones in the same list, and the wave
- * takes its share from the last to the first, one block's loads ahead. */
+/* One wave's blocks of one group of rows: its partial last blocks, then its full ones from the last to the first, one
+ * block's loads ahead.  The order of the additions within a block is part of the result's bits: a lane adds groups of
+ * eight of a full block and every 64th element of a partial one. */
 template <bool BF16>
 __device__ __forceinline__ void grad_sumsq_walk(const NormGroup &g, uint32_t wg, uint32_t wave_in_wg, uint32_t lane,
                                                 double &total, double &bad) {
     const BlockRowMap map(g.rows, g.n_rows);
-    const uint32_t units = g.total_blocks + g.n_tails;
-    const uint32_t per_chunk = (units + g.chunks - 1) / g.chunks;
+    // dealt from the group's last wave backwards: the waves that have a block less, or none
+    const uint32_t waves = g.wgs * kNormWaves;
+    for (uint32_t i = waves - 1 - (wg * kNormWaves + wave_in_wg); i < g.n_tails; i += waves) {
+        const DevTensor &t = g.rows[map.tail_row(g.total_blocks, i)];
+        const uint32_t n = (uint32_t)(t.numel % kBlock);
+        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
+        const void *tail_g = t.g;
+        float acc = 0.0f, nf = 0.0f;
+        for (uint32_t c = 0; c < n; c += 8 * kWave) { // eight loads in flight
+            float x[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t e = c + k * kWave + lane;
+                x[k] = e < n ? load1<BF16>(tail_g, e0 + e) : 0.0f;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                acc += x[k] * x[k];
+                nf += not_finite(x[k]);
+            }
+        }
+        total += (double)wave_sum(acc);
+        bad += (double)wave_sum(nf);
+    }
+    const uint32_t per_chunk = (g.total_blocks + g.chunks - 1) / g.chunks;
     const uint32_t lo = (wg % g.chunks) * per_chunk;
-    const uint32_t end = lo + per_chunk < units ? lo + per_chunk : units;
+    const uint32_t end = lo + per_chunk < g.total_blocks ? lo + per_chunk : g.total_blocks;
     const uint32_t stride = (g.wgs / g.chunks) * kNormWaves;
     const uint32_t first = lo + (wg / g.chunks) * kNormWaves + wave_in_wg;
     if (first >= end) return;
@@ -389,28 +413,15 @@ __device__ __forceinline__ void grad_sumsq_walk(const NormGroup &g, uint32_t wg,
     const char *row_g = nullptr;
     Raw8<BF16> raw[4];
     auto request = [&](uint32_t u) {
-        if (u < g.total_blocks) {
-            if (u - row_start >= row_blocks) {
-                const DevTensor &t = g.rows[map.row_of[u]];
-                row_g = static_cast<const char *>(t.g);
-                row_start = t.full_start;
-                row_blocks = (uint32_t)(t.numel / kBlock);
-            }
-            const char *base = row_g + (size_t)(u - row_start) * kBlock * (BF16 ? 2 : 4);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) raw[c].load(base, c * 512 + lane * 8);
-        } else {
-            const DevTensor &t = g.rows[map.tail_row(g.total_blocks, u - g.total_blocks)];
-            const uint32_t n = (uint32_t)(t.numel % kBlock);
-            const char *base = static_cast<const char *>(t.g) + (size_t)(t.numel / kBlock) * kBlock * (BF16 ? 2 : 4);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const uint32_t o = c * 512 + lane * 8;
-                const uint32_t count = lane_count(o, n);
-                if (count == 8) raw[c].load(base, o);
-                else raw[c].load_some(base, o, count);
-            }
+        if (u - row_start >= row_blocks) {
+            const DevTensor &t = g.rows[map.row_of[u]];
+            row_g = static_cast<const char *>(t.g);
+            row_start = t.full_start;
+            row_blocks = (uint32_t)(t.numel / kBlock);
         }
+        const char *base = row_g + (size_t)(u - row_start) * kBlock * (BF16 ? 2 : 4);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) raw[c].load(base, c * 512 + lane * 8);
     };
     request(unit);
     while (true) {
@@ -451,9 +462,9 @@ __device__ __forceinline__ void grad_sumsq_walk(const NormGroup &g, uint32_t wg,
 /* All groups of rows of a pass in one launch: workgroups [first_wg, first_wg + wgs) take a group.  Reading the
  * gradients once is the bound (6.2 TB/s on 10.3 GB); on the tables of an adapter the launches count as much, so there
  * is one whatever the tables hold.  Measured, this pass and the one behind it, before (a launch per group, a pair per
- * wave, partial blocks element by element) and after:
- *   256 short tensors in two tables  5.3 + 5.3 + 3.0 -> 4.1 + 2.4 us
- *   608 tensors, 306 MB of bf16      47.6 + 6.7 -> 48.2 + 5.4 us, and the step behind it 303 -> 299 us (it starts on
+ * wave, partial blocks one load at a time) and after:
+ *   256 short tensors in two tables  5.4 + 5.4 + 3.1 -> 5.8 + 2.6 us
+ *   608 tensors, 306 MB of bf16      47.7 + 6.8 -> 49.5 + 5.8 us, and the step behind it 306 -> 300 us (it starts on
  *                                    gradients that the last-level cache still holds: the walk goes backwards)
  *   1,680 tensors, 10.3 GB of fp32   1,655 + 7.2 -> 1,640 + 4.7 us */
 __global__ __launch_bounds__(kNormWaves * kWave) void grad_sumsq_kernel(NormGroups groups, double *__restrict__ partial) {
