@@ -104,6 +104,12 @@ constexpr uint32_t kChunks = 8;           /* contiguous ranges the block list is
  *   bf16, fp32 gradients, functional update
  *              8.2 | 8.9  12.5 | 10.9  17.3 | 15.1   44.0 | 35.3 */
 constexpr uint32_t kSplitBlocksPerCu = 4;
+/* Tables of both parameter dtypes with at most this many blocks per compute unit in all take one launch: it saves the
+ * start of a second one, and on larger tables the two kernels' code side by side costs as much.  us, two launches of a
+ * wave per block | one, half of the blocks fp32, 256 units:
+ *   blocks   256         1,024       2,816       8,192       32,768
+ *         14.4 | 8.4  16.6 | 10.7  23.4 | 20.6  50.0 | 46.0  160.8 | 163 */
+constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
 constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* bf16 tables take the prefetching kernel above this many full blocks
                                                    per compute unit; up to it, sixteen waves without a prefetch are
                                                    2-4 % faster than twelve with one (measured at 292-876 per unit,
@@ -126,6 +132,14 @@ int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, 
 int launch_step_split(int layout, int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows,
                       uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                       uint32_t grid, uint32_t teams, void *stream);
+/* One group of rows of a launch. */
+struct StepGroup {
+    const DevTensor *rows;
+    uint32_t n_rows, total_blocks, n_tails;
+};
+/* The fp32 and the bf16 rows of one table (gradients of the parameters' dtypes) in one launch of a wave per block. */
+int launch_step_two(const StepGroup &f32, const StepGroup &bf16, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
+                    uint32_t grid, uint32_t wg, void *stream);
 /* Whether launch_step would run this group on the prefetching kernel with the EMA update inside it.  units: full blocks
  * and partial ones. */
 bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units);

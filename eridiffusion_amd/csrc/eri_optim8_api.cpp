@@ -1026,29 +1026,44 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
     }
     rc = order_after_upload(t, stream);
     if (rc) return rc;
-    std::vector<EriEmaTensor> ema_rest;
-    for (auto &g : t->groups) {
-        if (g.n == 0) continue;
-        // One wavefront per block.  A small table gets smaller workgroups so that its blocks still
-        // spread over every compute unit instead of filling a few of them.
-        uint32_t waves_per_wg = ctx->wg / eri::kWave;
+    EriAdam8Hyper hh = *h;
+    const float *dev_scale = nullptr;
+    if (clip) {
+        dev_scale = t->norm_last + 1;
+        if (!scaled) { // the scale path is needed; neutral host-side factors
+            hh.flags |= ERI_ADAM8_FLAG_GRAD_SCALE;
+            hh.grad_scale = 1.0f;
+        }
+    }
+    // One wavefront per block.  A small table gets smaller workgroups so that its blocks still
+    // spread over every compute unit instead of filling a few of them.
+    uint32_t waves_per_wg = 0, grid = 0;
+    auto shape = [&](uint32_t work) {
+        waves_per_wg = ctx->wg / eri::kWave;
         const uint32_t slots = ctx->cus * ctx->wg_per_cu;
-        const uint32_t work = g.total_blocks + g.n_tails;
         const uint32_t per_slot = (work + slots - 1) / slots;
         if (per_slot < waves_per_wg) waves_per_wg = per_slot < 4 ? 4 : per_slot;
-        uint32_t grid = slots;
+        grid = slots;
         const uint32_t need = (work + waves_per_wg - 1) / waves_per_wg;
         if (grid > need) grid = need;
         if (grid == 0) grid = 1;
-        EriAdam8Hyper hh = *h;
-        const float *dev_scale = nullptr;
-        if (clip) {
-            dev_scale = t->norm_last + 1;
-            if (!scaled) { // the scale path is needed; neutral host-side factors
-                hh.flags |= ERI_ADAM8_FLAG_GRAD_SCALE;
-                hh.grad_scale = 1.0f;
-            }
-        }
+    };
+    // fp32 and bf16 rows in one launch where that pays (kTwoDtypeBlocksPerCu); the flags that name a kernel, and the EMA,
+    // which the prefetching kernel carries, keep a launch per group
+    auto &f32 = t->groups[eri::kLayoutF32], &bf16 = t->groups[eri::kLayoutBF16];
+    const uint64_t both = (uint64_t)f32.total_blocks + f32.n_tails + bf16.total_blocks + bf16.n_tails;
+    const bool one_launch = f32.n != 0 && bf16.n != 0 && both <= (uint64_t)ctx->cus * eri::kTwoDtypeBlocksPerCu &&
+                            (h->flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE | ERI_ADAM8_FLAG_ONE_WAVE | ERI_ADAM8_FLAG_EMA)) == 0;
+    if (one_launch) {
+        shape((uint32_t)both);
+        rc = eri::launch_step_two({f32.dev, f32.n, f32.total_blocks, f32.n_tails}, {bf16.dev, bf16.n, bf16.total_blocks, bf16.n_tails}, hh,
+                                  ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, stream);
+        if (rc) return hip_fail((hipError_t)rc, "adam8 step launch");
+    }
+    std::vector<EriEmaTensor> ema_rest;
+    for (auto &g : t->groups) {
+        if (g.n == 0 || (one_launch && (&g == &f32 || &g == &bf16))) continue;
+        shape(g.total_blocks + g.n_tails);
         rc = eri::launch_step(g.dev, g.n, g.total_blocks, g.n_tails, g.dtype, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
         if (rc) return hip_fail((hipError_t)rc, "adam8 step launch");
         if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(g.total_blocks + g.n_tails, g.dtype, hh, ctx->cus)) {
