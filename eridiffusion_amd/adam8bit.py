@@ -113,10 +113,11 @@ class Adam8bit:
 
     def step(self) -> int:
         """One optimizer step; returns how many parameters were skipped for lack of a gradient."""
-        held, rest = _torch_face.bind(self.params, C.addressof(self._handles))
+        params = self.params if type(self.params) is list else list(self.params)
+        held, rest = _torch_face.bind(params, C.addressof(self._handles), len(self._handles))
         live = [held]
         for i in rest:
-            p = self.params[i]
+            p = params[i]
             g = p.grad
             if g is not None:
                 g = _usable_grad(g, p)

@@ -59,13 +59,18 @@ bool grad_as_is(const at::Tensor &g, const at::Tensor &p) {
            (g.scalar_type() == p.scalar_type() || (p.scalar_type() == at::kBFloat16 && g.scalar_type() == at::kFloat));
 }
 
-/* bind(params, handles) -> (held, rest): sets data and gradient of the EriParameter at handles[i] from params[i].
- * `handles` is the address of an array of len(params) pointers.  `held` keeps the gradients alive that were read;
+/* bind(params, handles, n) -> (held, rest): sets data and gradient of the EriParameter at handles[i] from params[i].
+ * `handles` is the address of an array of n pointers; a longer list is an IndexError, before anything is set.  `held` keeps the gradients alive that were read;
  * `rest` lists the indices that were left alone. */
 PyObject *face_bind(PyObject *, PyObject *args) {
     PyObject *params;
     unsigned long long handles_addr;
-    if (!PyArg_ParseTuple(args, "O!K", &PyList_Type, &params, &handles_addr)) return nullptr;
+    Py_ssize_t n_handles;
+    if (!PyArg_ParseTuple(args, "O!Kn", &PyList_Type, &params, &handles_addr, &n_handles)) return nullptr;
+    if (PyList_GET_SIZE(params) > n_handles) {
+        PyErr_SetString(PyExc_IndexError, "more parameters than the optimizer was made for");
+        return nullptr;
+    }
     EriParameter *const *handles = reinterpret_cast<EriParameter *const *>(handles_addr);
     PyObject *rest = PyList_New(0);
     if (!rest) return nullptr;

@@ -57,15 +57,17 @@ def test_what_bind_takes():
     forms = _gradient_forms("cpu")
     params = _with_grads(forms)
     handles = _handles(params)
-    held, rest = _torch_face.bind(params, C.addressof(handles))
+    held, rest = _torch_face.bind(params, C.addressof(handles), len(handles))
     assert rest == [i for i, (_, _, taken) in enumerate(forms) if not taken]
     with BaseTorchFunctionMode():
-        assert _torch_face.bind(params, C.addressof(handles))[1] == list(range(len(params)))
+        assert _torch_face.bind(params, C.addressof(handles), len(handles))[1] == list(range(len(params)))
     product = params[10] * 2  # not a leaf: asking for its gradient warns, in Python code
-    assert _torch_face.bind([product], C.addressof(handles))[1] == [0]
-    assert _torch_face.bind([torch.empty(0)], C.addressof(handles))[1] == [0]  # no address: the C call refuses it by name
+    assert _torch_face.bind([product], C.addressof(handles), len(handles))[1] == [0]
+    assert _torch_face.bind([torch.empty(0)], C.addressof(handles), len(handles))[1] == [0]  # no address: the C call refuses it by name
     with pytest.raises(TypeError):
-        _torch_face.bind(tuple(params), C.addressof(handles))
+        _torch_face.bind(tuple(params), C.addressof(handles), len(handles))
+    with pytest.raises(IndexError):  # a list that has grown since the optimizer was made
+        _torch_face.bind(params + [torch.zeros(8)], C.addressof(handles), len(handles))
     for h in handles:
         L.lib().eri_param_release(h)
 
