@@ -883,7 +883,7 @@ __device__ __forceinline__ void tail_block(const DevTensor &t, uint32_t lb, uint
  * made seven trips to the caches one behind the other.  Here every wave copies 1 KB pieces straight into LDS
  * (global_load_lds, 16 bytes per lane, no registers), all of them in flight at once, and the caller may request its
  * first block in between; stage_end waits and makes the image visible to the workgroup.
- *   60 bf16 tensors with fp32 gradients, 5.8 M parameters (split kernel): 25.7 -> 23.7 us per launch
+ *   60 bf16 tensors with fp32 gradients, 5.8 M parameters (on the split kernel): 25.7 -> 23.7 us per launch
  *   one fp32 tensor of 2^20 elements (split kernel): 7.3 -> 7.1 us
  *   1,400 bf16 tensors, 44.8 M parameters (plain kernel): 93.05 -> 91.98 us per step */
 constexpr uint32_t kStagePiece = kWave * 16;
