@@ -27,10 +27,20 @@ def _dtype_tag(t: torch.Tensor) -> int:
     raise TypeError("Unsupported: 8-bit Adam takes float32 or bfloat16 parameters, got %s" % t.dtype)
 
 
+def _reachable(t: torch.Tensor) -> bool:
+    """Whether a kernel can read t; ordinary host memory in a kernel faults the device."""
+    return t.is_cuda or (t.device.type == "cpu" and t.is_pinned())
+
+
 def _usable_grad(g: torch.Tensor, p: torch.Tensor) -> torch.Tensor:
     """The gradient as the step reads it.  A float32 gradient of a bfloat16 parameter goes in as it is: the
     reference casts gradients to F32 and never rounds them (adam8bit_enhanced.rs:231-235).  Any other
-    mismatch is cast to the parameter's dtype, which for bf16 -> f32 is exact."""
+    mismatch is cast to the parameter's dtype, which for bf16 -> f32 is exact.  The launch is sized by the
+    parameter and reads where the parameter is: a gradient of another size or on another device is refused."""
+    if g.numel() != p.numel():
+        raise ValueError("a gradient of %d elements for a parameter of %d" % (g.numel(), p.numel()))
+    if not _reachable(g) or (g.is_cuda and p.is_cuda and g.device != p.device):
+        raise ValueError("a gradient on %s, which the step of a parameter on %s cannot read" % (g.device, p.device))
     if g.dtype != p.dtype and not (p.dtype == torch.bfloat16 and g.dtype == torch.float32):
         g = g.to(p.dtype)
     return g.contiguous()
@@ -86,6 +96,11 @@ class Adam8bitConfig:
     min_8bit_size: int = 0  # pipeline_flux_lora_1024.rs:451 passes 4096; 0 keeps every parameter 8-bit
 
 
+class _Made(C.Structure):
+    """What a parameter was when its optimizer was made: its handle and its state are sized by it."""
+    _fields_ = [("numel", C.c_uint64), ("dtype_tag", C.c_int64)]
+
+
 class Adam8bit:
     """`step()` over a list of tensors that carry their gradients in `.grad`."""
 
@@ -96,10 +111,12 @@ class Adam8bit:
             if not p.is_contiguous():
                 raise ValueError("parameters must be contiguous")
         self._handles = (C.c_void_p * len(self.params))()
+        self._made = (_Made * len(self.params))()
         for i, p in enumerate(self.params):
             h = C.c_void_p()
             check(lib().eri_param_create(p.data_ptr(), p.numel(), _dtype_tag(p), C.byref(h)), "eri_param_create")
             self._handles[i] = h
+            self._made[i] = _Made(p.numel(), _dtype_tag(p))
         cfg = Adam8bitConfigC(config.lr, config.betas[0], config.betas[1], config.eps, config.weight_decay,
                               int(config.amsgrad), int(config.block_wise), config.percentile_clipping)
         self._opt = C.c_void_p()
@@ -110,15 +127,23 @@ class Adam8bit:
         if config.min_8bit_size:
             check(lib().eri_adam8bit_set_min_8bit_size(self._opt, config.min_8bit_size), "eri_adam8bit_set_min_8bit_size")
         self._live = []
+        self._ema = None
 
     def step(self) -> int:
         """One optimizer step; returns how many parameters were skipped for lack of a gradient."""
         params = self.params if type(self.params) is list else list(self.params)
-        held, rest = _torch_face.bind(params, C.addressof(self._handles), len(self._handles))
+        held, rest = _torch_face.bind(params, C.addressof(self._handles), len(self._handles), C.addressof(self._made))
         live = [held]
         for i in rest:
             p = params[i]
             g = p.grad
+            if g is not None or self._ema is not None:  # no launch touches it otherwise
+                if not p.is_contiguous():
+                    raise ValueError("parameters must be contiguous")
+                if (p.numel(), _dtype_tag(p)) != (self._made[i].numel, self._made[i].dtype_tag):
+                    raise ValueError("parameter %d has %d elements of %s: not what the optimizer was made for" % (i, p.numel(), p.dtype))
+                if not _reachable(p):
+                    raise ValueError("parameter %d is in host memory that the step cannot reach" % i)
             if g is not None:
                 g = _usable_grad(g, p)
                 live.append(g)
@@ -221,6 +246,12 @@ class Adam8bit:
             pass
 
 
+def _functional_param(t: torch.Tensor) -> torch.Tensor:
+    if not t.is_cuda:
+        raise ValueError("a parameter on %s: updates take device tensors" % t.device)
+    return t.detach().contiguous()
+
+
 class Adam8bitFunctional:
     """Per-tensor flavour keyed by name: update() returns the new parameter tensor, step() ends the step
     (adam8bit.rs:89-92,101-208).
@@ -273,7 +304,7 @@ class Adam8bitFunctional:
         return lib().eri_adam8bit_fn_get_step(self._opt)
 
     def update(self, name: str, param: torch.Tensor, grad: torch.Tensor) -> torch.Tensor:
-        p = param.detach().contiguous()
+        p = _functional_param(param)
         g = _usable_grad(grad, p)
         out = torch.empty_like(p)
         check(lib().eri_adam8bit_fn_update(self._opt, name.encode(), p.data_ptr(), g.data_ptr(), p.numel(),
@@ -296,7 +327,7 @@ class Adam8bitFunctional:
             return outs
         names = [n for n in params if n in grads]
         k = len(names)
-        ps = [params[n].detach().contiguous() for n in names]
+        ps = [_functional_param(params[n]) for n in names]
         gs = [_usable_grad(grads[n], p) for n, p in zip(names, ps)]
         outs = [torch.empty_like(p) for p in ps]
         c_names = (C.c_char_p * k)(*[n.encode() for n in names])
@@ -332,6 +363,8 @@ class Adam8bitFunctional:
         for name, (m, v) in state.items():
             m = m.detach().to(torch.float32).contiguous().view(-1)
             v = v.detach().to(torch.float32).contiguous().view(-1)
+            if m.numel() != v.numel():
+                raise ValueError("moments of %d and %d elements for '%s'" % (m.numel(), v.numel(), name))
             check(lib().eri_adam8bit_fn_load_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr(),
                                                         m.numel()), "eri_adam8bit_fn_load_state_fp32")
             self._names[name] = None

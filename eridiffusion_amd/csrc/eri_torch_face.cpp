@@ -50,28 +50,45 @@ int dtype_tag(const at::Tensor &t) {
     return t.scalar_type() == at::kFloat ? ERI_DTYPE_F32 : t.scalar_type() == at::kBFloat16 ? ERI_DTYPE_BF16 : -1;
 }
 
+/* Whether a kernel that works on `p` can read t: device memory beside p's, or pinned host memory.  Ordinary host memory
+ * in a kernel faults the device. */
+bool reachable(const at::Tensor &t, const at::Tensor &p) {
+    return t.is_cuda() ? !p.is_cuda() || t.device() == p.device() : t.is_cpu() && t.is_pinned();
+}
+
 /* Whether the step reads g as it is: a plain tensor (no subclass where it has a Python object already) of the
- * parameter's dtype, or float32 for a bfloat16 parameter. */
+ * parameter's dtype, or float32 for a bfloat16 parameter, with an element for each of the parameter's: the launch is
+ * sized by the parameter. */
 bool grad_as_is(const at::Tensor &g, const at::Tensor &p) {
     PyObject *known = g.unsafeGetTensorImpl()->pyobj_slot()->load_pyobj();
     return (!known || THPVariable_CheckTypeExact(Py_TYPE(known))) && !g.unsafeGetTensorImpl()->is_python_dispatch() && dtype_tag(g) >= 0 &&
-           g.layout() == at::kStrided && g.has_storage() && g.is_contiguous() &&
+           g.layout() == at::kStrided && g.has_storage() && g.is_contiguous() && g.numel() == p.numel() &&
            (g.scalar_type() == p.scalar_type() || (p.scalar_type() == at::kBFloat16 && g.scalar_type() == at::kFloat));
 }
 
-/* bind(params, handles, n) -> (held, rest): sets data and gradient of the EriParameter at handles[i] from params[i].
- * `handles` is the address of an array of n pointers; a longer list is an IndexError, before anything is set.  `held` keeps the gradients alive that were read;
- * `rest` lists the indices that were left alone. */
+/* What a parameter was when its optimizer was made; handles and states are sized by it. */
+struct Made {
+    uint64_t numel;
+    int64_t dtype_tag;
+};
+
+/* bind(params, handles, n[, made]) -> (held, rest): sets data and gradient of the EriParameter at handles[i] from
+ * params[i].  `handles` is the address of an array of n pointers; a longer list is an IndexError, before anything is set.
+ * `made` is the address of n records: a parameter that has another size or dtype by now, or that kernels cannot reach,
+ * is left alone, and so is one with such a gradient.  (Without `made` the caller vouches for that.)  `held` keeps the
+ * gradients alive that were read; `rest` lists the indices that were left alone. */
 PyObject *face_bind(PyObject *, PyObject *args) {
     PyObject *params;
     unsigned long long handles_addr;
+    unsigned long long made_addr = 0;
     Py_ssize_t n_handles;
-    if (!PyArg_ParseTuple(args, "O!Kn", &PyList_Type, &params, &handles_addr, &n_handles)) return nullptr;
+    if (!PyArg_ParseTuple(args, "O!Kn|K", &PyList_Type, &params, &handles_addr, &n_handles, &made_addr)) return nullptr;
     if (PyList_GET_SIZE(params) > n_handles) {
         PyErr_SetString(PyExc_IndexError, "more parameters than the optimizer was made for");
         return nullptr;
     }
     EriParameter *const *handles = reinterpret_cast<EriParameter *const *>(handles_addr);
+    const Made *made = reinterpret_cast<const Made *>(made_addr);
     PyObject *rest = PyList_New(0);
     if (!rest) return nullptr;
     try {
@@ -82,12 +99,13 @@ PyObject *face_bind(PyObject *, PyObject *args) {
         for (Py_ssize_t i = 0; i < n; ++i) {
             const at::Tensor *p = general ? nullptr : plain(PyList_GET_ITEM(params, i));
             bool done = false;
-            if (p && p->is_leaf()) { // asking for another tensor's gradient warns
+            const bool fits = p && (!made || (made[i].numel == (uint64_t)p->numel() && made[i].dtype_tag == dtype_tag(*p) && reachable(*p, *p)));
+            if (fits && p->is_leaf()) { // asking for another tensor's gradient warns
                 const at::Tensor &g = p->grad();
                 void *data = p->data_ptr();
                 if (!g.defined()) {
                     done = eri_param_set_data(handles[i], data) == 0 && eri_param_set_grad(handles[i], nullptr) == 0;
-                } else if (grad_as_is(g, *p)) {
+                } else if (grad_as_is(g, *p) && (!made || reachable(g, *p))) {
                     done = eri_param_set_data(handles[i], data) == 0 && eri_param_set_grad_typed(handles[i], g.data_ptr(), dtype_tag(g)) == 0;
                     if (done) held->push_back(g);
                 }
@@ -141,7 +159,7 @@ PyObject *face_update_many(PyObject *, PyObject *args) {
             }
             if (!grad) continue;
             const at::Tensor *p = plain(value), *g = plain(grad);
-            if (!p || !g || dtype_tag(*p) < 0 || !grad_as_is(*g, *p)) {
+            if (!p || !g || !p->is_cuda() || dtype_tag(*p) < 0 || !grad_as_is(*g, *p) || !reachable(*g, *p)) {
                 Py_DECREF(keys);
                 Py_RETURN_NONE;
             }

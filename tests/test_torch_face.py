@@ -83,6 +83,83 @@ def test_what_update_many_leaves_to_python():
         assert _torch_face.update_many(1, {"a": a}, {"a": g}) is None
 
 
+class _MadeOfTwo:
+    """Parameters whose handles were made for 40 x 64 float32 elements."""
+
+    def __init__(self):
+        from eridiffusion_amd.adam8bit import _Made
+        self.handles = _handles([torch.zeros(40, 64), torch.zeros(40, 64)])
+        self.made = (_Made * 2)(_Made(2560, L.DTYPE_F32), _Made(2560, L.DTYPE_F32))
+
+    def rest(self, *params):
+        return _torch_face.bind(list(params), C.addressof(self.handles), 2, C.addressof(self.made))[1]
+
+
+def test_bind_leaves_alone_what_a_kernel_would_overrun():
+    """A launch is sized by what the optimizer was made for: smaller data, another dtype, a gradient that no longer has
+    the parameter's size, and host memory stay out of it."""
+    two = _MadeOfTwo()
+    assert two.rest(torch.zeros(40, 64), torch.zeros(40, 64)) == [0, 1]  # ordinary host memory
+    small, wide = torch.zeros(40, 64), torch.zeros(40, 64)
+    small.data, wide.data = torch.zeros(16), torch.zeros(40, 64, dtype=torch.bfloat16)
+    assert two.rest(small, wide) == [0, 1]
+    shrunk = torch.zeros(40, 64, requires_grad=True)
+    shrunk.grad = torch.zeros(40, 64)
+    shrunk.grad.data = torch.zeros(16)
+    assert _torch_face.bind([shrunk], C.addressof(two.handles), 2)[1] == [0]
+    for h in two.handles:
+        L.lib().eri_param_release(h)
+
+
+def test_python_loops_refuse_what_a_kernel_would_overrun(monkeypatch):
+    """No launch is queued for any of these; on a device the first two are faults."""
+    from eridiffusion_amd import adam8bit
+    monkeypatch.setattr(adam8bit, "_stream_ptr", lambda: 0)
+    a, b = torch.zeros(4096), torch.zeros(16)
+    assert _torch_face.update_many(1, {"a": a}, {"a": a}) is None
+    opt = adam8bit.Adam8bitFunctional()
+    for call in (lambda p, g: opt.update("a", p, g), lambda p, g: opt.update_many({"a": p}, {"a": g})):
+        with pytest.raises(ValueError, match="device tensors"):
+            call(a, a)
+    with pytest.raises(ValueError, match="16 elements for a parameter of 4096"):
+        adam8bit._usable_grad(b, a)
+    with pytest.raises(ValueError, match="cannot read"):
+        adam8bit._usable_grad(a, a)
+    with pytest.raises(ValueError, match="moments of 4096 and 16"):
+        opt.load_state_from_tensors({"a": (a, b)})
+    lists = adam8bit.Adam8bit([torch.zeros(4096), torch.zeros(4096)])
+    lists.params[0].grad = torch.zeros(4096)
+    with pytest.raises(ValueError, match="host memory"):
+        lists.step()
+    for data, message in ((b, "16 elements"), (a.bfloat16(), "bfloat16"), (b[:1].expand(4096), "contiguous")):
+        lists = adam8bit.Adam8bit([torch.zeros(4096)])
+        lists.params[0].data = data
+        assert lists.step() == 1  # nothing to step: it is left alone
+        lists.params[0].grad = data.clone()
+        with pytest.raises(ValueError, match=message):
+            lists.step()
+
+
+@pytest.mark.gpu
+def test_sizes_and_devices_are_looked_at_before_a_launch():
+    from eridiffusion_amd.adam8bit import Adam8bit, Adam8bitConfig, Adam8bitFunctional
+    p, g = torch.randn(4096, device="cuda"), torch.randn(4096, device="cuda") * 1e-3
+    fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    for bad in (g[:16], g.cpu()):
+        for call in (lambda: fn.update_many({"a": p}, {"a": bad}), lambda: fn.update("a", p, bad)):
+            with pytest.raises(ValueError):
+                call()
+    assert fn.get_state_as_tensors() == {}
+    want = fn.update_many({"a": p}, {"a": g})["a"].clone()
+    other = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    assert torch.equal(other.update_many({"a": p}, {"a": g.cpu().pin_memory()})["a"], want)  # pinned memory is read where it is
+    opt = Adam8bit([p.clone()], Adam8bitConfig(lr=1e-3))
+    opt.params[0].data = p[:16].clone()
+    opt.params[0].grad = g[:16].clone()
+    with pytest.raises(ValueError):
+        opt.step()
+
+
 @pytest.mark.gpu
 def test_native_and_python_loops_step_alike():
     from eridiffusion_amd.adam8bit import Adam8bit, Adam8bitConfig, Adam8bitFunctional, update_params_8bit
