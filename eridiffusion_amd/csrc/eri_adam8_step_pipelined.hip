@@ -35,15 +35,14 @@ constexpr uint32_t kPipeThreads = kGradBf16 ? 768 : 512;
 #define ERI_PIPE_KERNEL adam8_step_pipelined_f32_kernel
 #endif
 
-/* One lane's eight shadow values of one quarter block: shadow = d*shadow + (1-d)*p', each operation rounded
- * on its own, the result rounded to bf16. */
-__device__ __forceinline__ void ema_quarter(void *shadow, size_t e0, int c, uint32_t lane, const u32x4 &old, const u32x4 &pnew,
-                                            float decay) {
+/* Eight shadow values of a lane: shadow = d*shadow + (1-d)*p', each operation rounded on its own; the store rounds the
+ * result to bf16. */
+__device__ __forceinline__ void ema_eight(const u32x4 &old, const u32x4 &pnew, float decay, float (&out)[8]) {
     const float omd = 1.0f - decay; // ema_enhanced.rs:96
     Raw8<true> so, pn;
     so.w = old;
     pn.w = pnew;
-    float sv[8], pv[8], out[8];
+    float sv[8], pv[8];
     so.unpack(sv);
     pn.unpack(pv);
 #pragma unroll
@@ -52,7 +51,30 @@ __device__ __forceinline__ void ema_quarter(void *shadow, size_t e0, int c, uint
         float b = pv[k] * omd;
         out[k] = a + b;
     }
-    store8<true>(static_cast<char *>(shadow) + e0 * 2, c * 512 + lane * 8, out);
+}
+
+/* The shadow of a row's partial last block of n elements.  A lane takes the eight elements that it has just stored as
+ * parameters (tail_block), so that what it reads back are its own stores: nothing orders them before another lane's
+ * loads. */
+__device__ __forceinline__ void ema_tail(const DevTensor &t, uint32_t n, uint32_t lane, float decay) {
+    const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
+    char *shadow = static_cast<char *>(t.shadow) + e0 * 2;
+    const char *p = static_cast<const char *>(t.p) + e0 * 2;
+    for (uint32_t o = lane * 8; o < n; o += 8 * kWave) {
+        const uint32_t count = lane_count(o, n);
+        Raw8<true> so, pn;
+        float out[8];
+        if (count == 8) {
+            so.load(shadow, o);
+            pn.load(p, o);
+        } else {
+            so.load_some(shadow, o, count);
+            pn.load_some(p, o, count);
+        }
+        ema_eight(so.w, pn.w, decay, out);
+        if (count == 8) store8<true>(shadow, o, out);
+        else store_some<true>(shadow, o, out, count);
+    }
 }
 
 struct RawBlock {
@@ -145,15 +167,7 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         const uint32_t n = (uint32_t)(t.numel % kBlock);
         const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
         tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
-        if (EMA && t.shadow != nullptr) { // the partial block's shadow, element by element, from the parameters just stored
-            const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-            const float omd = 1.0f - h.ema_decay;
-            for (uint32_t j = lane; j < n; j += kWave) {
-                const float a = load1<true>(t.shadow, e0 + j) * h.ema_decay;
-                const float b = load1<true>(t.p, e0 + j) * omd;
-                as_global(static_cast<uint16_t *>(t.shadow))[e0 + j] = (uint16_t)bf16_bits(a + b);
-            }
-        }
+        if (EMA && t.shadow != nullptr) ema_tail(t, n, lane, h.ema_decay);
     }
     const BlockWalk walk(total_blocks, chunks);
     uint32_t blk = walk.first;
@@ -257,7 +271,11 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
             } else { // fp32 parameters are final here (they take the exact chain): stored quarter by quarter
                 store8<false>(p, c * 512 + lane * 8, pn);
             }
-            if (EMA && with_shadow) ema_quarter(t.shadow, e0, c, lane, sh[c], pw[c], h.ema_decay);
+            if (EMA && with_shadow) {
+                float out[8];
+                ema_eight(sh[c], pw[c], h.ema_decay, out);
+                store8<true>(static_cast<char *>(t.shadow) + e0 * 2, c * 512 + lane * 8, out);
+            }
             if (kEarly) { // the quarter's raw words are dead: the next block's quarter takes their registers now
                 raw.issue_quarter(nt, pblk - nt.full_start, c, lane);
                 if (kParamBf16) __builtin_nontemporal_store(pw[c], as_global(reinterpret_cast<u32x4 *>(p) + c * 64 + lane));

@@ -79,6 +79,38 @@ def test_shadows_follow_the_updated_parameters(case):
     L.lib().eri_adam8_table_destroy(table)
 
 
+@pytest.mark.parametrize("grad_f32", [False, True], ids=["bf16-grads", "f32-grads"])
+def test_shadow_of_a_partial_block_follows_the_parameters_just_stored(grad_f32):
+    """Last blocks of every shape in the kernel that carries the EMA, decay 0: the shadow becomes the new parameter, so
+    a value read before its store would show as the old one.  Nothing past a shadow's end is written."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    ends = [1, 7, 8, 9, 63, 64, 65, 505, 511, 512, 513, 1023, 1031, 1536, 1543, 2041, 2047]
+    sizes = ends + [2048 + e for e in ends]
+    ps, gs = hs.make_inputs(sizes, True, 71)
+    if grad_f32:
+        gs = hs.fresh_grads(sizes, False, 72)
+    gt = hs.GpuTensors(ps, gs, hs.oracle_states(sizes), True)
+    shadows = [torch.full((n + 64,), 7.0, dtype=torch.bfloat16, device="cuda") for n in sizes]
+    rows = gt.rows()
+    for r, s in zip(rows, shadows):
+        r.ema_shadow = s.data_ptr()
+        r.grad_f32 = 1 if grad_f32 else 0
+    table = C.c_void_p()
+    L.check(L.lib().eri_adam8_table_create(rows, len(rows), None, C.byref(table)), "table_create")
+    for step in (1, 2, 3):
+        h = L.hyper_pack(1e-2, B1, B2, EPS, WD, step, L.MODE_ERI, L.FLAG_EXACT_PARAM | L.FLAG_EMA | L.FLAG_ONE_WAVE)
+        h.ema_decay = 0.0
+        L.check(L.lib().eri_adam8_step_table(table, C.byref(h), None), "step_table")
+        torch.cuda.synchronize()
+        got_p, _ = gt.fetch()
+        for p, s, n, old in zip(got_p, shadows, sizes, ps):
+            assert not np.array_equal(p, old)
+            assert np.array_equal(s[:n].cpu().view(torch.int16).numpy().view(np.uint16), p), n
+            assert bool((s[n:] == 7.0).all()), n
+    L.lib().eri_adam8_table_destroy(table)
+
+
 def test_attached_ema_model_equals_step_then_update():
     """Two identical trainers: one calls optimizer.step() and then ema.update(all parameters), as the reference's
     trainers do, the other attaches the EMA model to the optimizer and only calls step().  Parameters, states
