@@ -245,12 +245,13 @@ template <bool VEC>
 __global__ __launch_bounds__(kMomentThreads) void quantize_kernel(MomentArgs args, uint64_t numel, uint64_t nblocks,
                                                                   const unsigned char *__restrict__ image) {
     __shared__ float mid[256];
-    __shared__ unsigned char lo[kSKeyCount];
+    __shared__ uint4 lo_words[kSKeyCount / 16]; // bytes, staged in 16-byte words and aligned for them
+    const unsigned char *lo = reinterpret_cast<const unsigned char *>(lo_words);
     static_assert(kSKeyCount == kUKeyCount && kSKeyCount == 16 * kMomentThreads, "one 16-byte word per thread");
     const uint32_t which = blockIdx.y;
     const bool is_signed = args.is_signed[which] != 0;
     mid[threadIdx.x] = reinterpret_cast<const float *>(image + (is_signed ? kSmallMidS : kSmallMidU))[threadIdx.x];
-    reinterpret_cast<uint4 *>(lo)[threadIdx.x] = reinterpret_cast<const uint4 *>(image + (is_signed ? kSmallLoS : kSmallLoU))[threadIdx.x];
+    lo_words[threadIdx.x] = reinterpret_cast<const uint4 *>(image + (is_signed ? kSmallLoS : kSmallLoU))[threadIdx.x];
     __syncthreads();
     const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kMomentThreads / kWave) + threadIdx.x / kWave);
