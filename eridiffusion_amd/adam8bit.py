@@ -262,7 +262,8 @@ class Adam8bitFunctional:
 
     def __init__(self, learning_rate=1e-4, beta1=0.9, beta2=0.999, eps=1e-8, weight_decay=0.01, batched=False):
         self._opt = C.c_void_p()
-        check(lib().eri_adam8bit_fn_with_params(learning_rate, beta1, beta2, eps, weight_decay, _stream_ptr(),
+        self._stream = _stream_ptr()
+        check(lib().eri_adam8bit_fn_with_params(learning_rate, beta1, beta2, eps, weight_decay, self._stream,
                                                 C.byref(self._opt)), "eri_adam8bit_fn_with_params")
         self._names: Dict[str, None] = {}  # in the order the names came up
         self._live: List[torch.Tensor] = []
@@ -360,13 +361,22 @@ class Adam8bitFunctional:
         return out
 
     def load_state_from_tensors(self, state: Dict[str, Tuple[torch.Tensor, torch.Tensor]]) -> None:
+        """The moments are read on the optimizer's stream, in its order.  Called under another stream, the moments (and
+        the float32 copies made of them here) belong to that one: each is waited for before it is read, and the reading
+        before it may be freed or changed."""
+        here = _stream_ptr()
+        apart = here != self._stream
         for name, (m, v) in state.items():
             m = m.detach().to(torch.float32).contiguous().view(-1)
             v = v.detach().to(torch.float32).contiguous().view(-1)
             if m.numel() != v.numel():
                 raise ValueError("moments of %d and %d elements for '%s'" % (m.numel(), v.numel(), name))
+            if apart:
+                check(lib().eri_hip_stream_sync(here), "eri_hip_stream_sync")
             check(lib().eri_adam8bit_fn_load_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr(),
                                                         m.numel()), "eri_adam8bit_fn_load_state_fp32")
+            if apart:
+                check(lib().eri_hip_stream_sync(self._stream), "eri_hip_stream_sync")
             self._names[name] = None
 
     def close(self) -> None:

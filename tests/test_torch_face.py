@@ -208,3 +208,52 @@ def test_update_many_refusals_keep_their_codes():
         fn.update_many({"b": torch.zeros(0, device="cuda")}, {"b": torch.zeros(0, device="cuda")})
     assert e.value.code in (-1, -3)
     assert list(fn.get_state_as_tensors()) == ["a"]
+
+
+def test_moments_loaded_under_another_stream_are_waited_for(monkeypatch):
+    """Before they are read, and before the call lets go of them; on the optimizer's own stream nothing waits."""
+    from eridiffusion_amd import adam8bit
+    calls, stream = [], [11]
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *args: calls.append((name, args[0])) or 0
+    monkeypatch.setattr(adam8bit, "lib", lambda: Lib())
+    monkeypatch.setattr(adam8bit, "_stream_ptr", lambda: stream[0])
+    opt = adam8bit.Adam8bitFunctional()
+    del calls[:]
+    state = {"a": (torch.zeros(8), torch.zeros(8)), "b": (torch.zeros(8), torch.zeros(8))}
+    opt.load_state_from_tensors(state)
+    assert [name for name, _ in calls] == ["eri_adam8bit_fn_load_state_fp32"] * 2
+    del calls[:]
+    stream[0] = 12
+    opt.load_state_from_tensors(state)
+    assert [(name, args) for name, args in calls if "sync" in name] == [("eri_hip_stream_sync", 12), ("eri_hip_stream_sync", 11)] * 2
+    assert [name.endswith("fp32") for name, _ in calls] == [False, True, False] * 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pooled", [False, True])
+def test_reload_under_another_stream(pooled):
+    """Moments that a side stream is still making when they are loaded, float64 so that they are converted on the way,
+    and whose memory that stream hands out and overwrites right behind the call."""
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
+    n = (1 << 22) + 5
+    want, opt = Adam8bitFunctional(), Adam8bitFunctional()
+    if pooled:
+        opt.set_state_pool(DevicePool(64 << 20, 1), 0)
+    m, v = torch.randn(n, device="cuda"), torch.rand(n, device="cuda")
+    want.load_state_from_tensors({"w": (m, v)})
+    opt.load_state_from_tensors({"w": (v, m.square())})
+    busy = torch.randn(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(8):
+            busy = busy @ busy * 1e-2
+        opt.load_state_from_tensors({"w": (m.double(), v.double())})
+        trash = [torch.full((n,), 9.0, device="cuda") for _ in range(6)]
+    torch.cuda.synchronize()
+    for a, b in zip(opt.get_state_as_tensors()["w"], want.get_state_as_tensors()["w"]):
+        assert torch.equal(a, b)
+    assert len(trash) == 6
