@@ -277,7 +277,7 @@ class Adam8bitFunctional:
         return cls(learning_rate, beta1, beta2, eps, weight_decay)
 
     def set_state_pool(self, pool: Optional[DevicePool], lane: int = 0) -> None:
-        """States of names not seen yet come out of `lane` of the pool."""
+        """States of names not seen yet, and states that are loaded, come out of `lane` of the pool."""
         check(lib().eri_adam8bit_fn_set_state_pool(self._opt, pool._pool if pool else None, lane), "eri_adam8bit_fn_set_state_pool")
         self._pool = pool
 

@@ -44,6 +44,7 @@ int fail(int code, const std::string &msg) {
 struct State8 {
     void *base = nullptr;
     EriHipPool *pool = nullptr; // the pool the piece came from and goes back to (not owned), or null
+    uint32_t pool_lane = 0;
     uint64_t total = 0;         // bytes of the piece
     uint8_t *m = nullptr, *v = nullptr;
     float *absmax_m = nullptr, *absmax_v = nullptr;
@@ -62,6 +63,7 @@ struct State8 {
         if (rc) return rc;
         if (from) eri_hip_pool_retain(from); // the piece goes back to it, also if the caller destroys the pool first
         pool = from;
+        pool_lane = lane;
         total = bytes;
         char *b = static_cast<char *>(base);
         m = reinterpret_cast<uint8_t *>(b);
@@ -1623,11 +1625,12 @@ int eri_adam8bit_fn_load_state_fp32(EriAdam8bitFn *o, const char *name, const fl
     if (numel == 0) return fail(ERI_ERR_EMPTY, "InvalidOperation: Empty tensor for quantization");
     int rc = fn_flush(o);
     if (rc) return rc;
-    // A state of this size that exists already takes the new contents where it is, in stream order behind the steps
+    // A state of this size that exists already, where new states would be made too, takes the new contents where it is, in stream order behind the steps
     // that still use the old ones: no allocation and no release, each of which waits for the device (24 tensors of
     // 340 M parameters loaded and read back: 33.8 -> 1.34 ms).
     auto it = o->states.find(std::string_view(name));
-    if (it != o->states.end() && it->second->numel == numel) {
+    if (it != o->states.end() && it->second->numel == numel && it->second->pool == o->state_pool &&
+        (!o->state_pool || it->second->pool_lane == o->state_lane)) {
         State8 &s = *it->second;
         return eri_adam8_quantize_state(m, v, numel, s.m, s.v, s.absmax_m, s.absmax_v, o->stream);
     }

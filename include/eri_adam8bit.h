@@ -153,7 +153,8 @@ int eri_adam8bit_fn_destroy(EriAdam8bitFn *opt);
  * the reference's callers may assume (pipeline_sdxl_lora.rs:708-724 reads the new tensor at once). */
 int eri_adam8bit_fn_update(EriAdam8bitFn *opt, const char *name, const void *param, const void *grad, uint64_t numel,
                            int dtype_tag, int grad_dtype_tag, void *out);
-/* As eri_adam8bit_set_state_pool: states of names not seen yet come out of `lane` of the pool. */
+/* As eri_adam8bit_set_state_pool: states of names not seen yet, and states that are loaded, come out of `lane` of
+ * the pool. */
 int eri_adam8bit_fn_set_state_pool(EriAdam8bitFn *opt, EriHipPool *pool, uint32_t lane);
 /* Batching: with it enabled, update() only queues its row, and ONE launch over all queued rows runs at the
  * next eri_adam8bit_fn_step (which every trainer calls right after its loop of updates:

@@ -283,3 +283,34 @@ def test_parameters_and_gradients_in_lane_0_states_in_lane_2():
             assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), i
     L.lib().eri_adam8_table_destroy(table)
     L.check(L.lib().eri_hip_pool_destroy(pool), "destroy")
+
+
+def test_loading_moments_moves_a_state_into_the_pool_that_was_set_since():
+    """A state that is loaded goes where new states are made: into the pool, and into the lane named last; loaded again
+    it stays there."""
+    import torch
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
+    L = _L()
+    n = 2048 * 3 + 130
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    moments = {"w": (torch.randn(n, device="cuda", generator=gen) * 1e-3, torch.rand(n, device="cuda", generator=gen) * 1e-6)}
+    opt = Adam8bitFunctional()
+    opt.load_state_from_tensors(moments)
+    want = opt.get_state_as_tensors()["w"]
+    pool = DevicePool(64 * MiB, 2)
+
+    def used(lane):
+        out = C.c_size_t()
+        L.check(L.lib().eri_hip_pool_lane_used(pool._pool, lane, C.byref(out)), "lane_used")
+        return out.value
+    for lane in (0, 0, 1):
+        opt.set_state_pool(pool, lane)
+        opt.load_state_from_tensors(moments)
+        assert used(lane) >= 2 * n and used(1 - lane) == 0  # the piece left behind is given back
+        got = opt.get_state_as_tensors()["w"]
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    opt.set_state_pool(None)
+    opt.load_state_from_tensors(moments)
+    assert used(0) == 0 and used(1) == 0
+    got = opt.get_state_as_tensors()["w"]
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
