@@ -17,6 +17,7 @@
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <memory>
@@ -126,9 +127,9 @@ PyObject *face_bind(PyObject *, PyObject *args) {
             return nullptr;
         }
         return Py_BuildValue("NN", h, rest);
-    } catch (const std::exception &e) {
+    } catch (const std::exception &) {
         Py_DECREF(rest);
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }
@@ -219,10 +220,10 @@ PyObject *face_update_many(PyObject *, PyObject *args) {
             return nullptr;
         }
         return Py_BuildValue("iNN", rc, outs, h);
-    } catch (const std::exception &e) {
+    } catch (const std::exception &) { // out of memory reaches Python as torch.OutOfMemoryError, which trainers catch
         Py_XDECREF(keys);
         Py_XDECREF(outs);
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }

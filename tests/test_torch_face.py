@@ -257,3 +257,21 @@ def test_reload_under_another_stream(pooled):
     for a, b in zip(opt.get_state_as_tensors()["w"], want.get_state_as_tensors()["w"]):
         assert torch.equal(a, b)
     assert len(trash) == 6
+
+
+@pytest.mark.gpu
+def test_out_of_memory_for_the_outputs_is_torchs_own_exception():
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    n = 1 << 25
+    p, g = torch.randn(n, device="cuda"), torch.randn(n, device="cuda")
+    fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 20)) / total)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            fn.update_many({"w": p}, {"w": g})
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert fn.get_state_as_tensors() == {} and fn.memory_stats() == (0, 0)
+    assert fn.update_many({"w": p}, {"w": g})["w"].shape == p.shape
