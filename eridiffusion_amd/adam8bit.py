@@ -318,7 +318,7 @@ class Adam8bitFunctional:
 
     def update_many(self, params: Dict[str, torch.Tensor], grads: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
         """Every named parameter that has a gradient, in one launch; returns the new tensors by name."""
-        done = _torch_face.update_many(self._opt.value, params, grads) if type(params) is dict and type(grads) is dict else None
+        done = _torch_face.update_many(self._opt.value or 0, params, grads) if type(params) is dict and type(grads) is dict else None
         if done is not None:
             code, outs, held = done
             check(code, "eri_adam8bit_fn_update_many")

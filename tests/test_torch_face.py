@@ -275,3 +275,13 @@ def test_out_of_memory_for_the_outputs_is_torchs_own_exception():
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert fn.get_state_as_tensors() == {} and fn.memory_stats() == (0, 0)
     assert fn.update_many({"w": p}, {"w": g})["w"].shape == p.shape
+
+
+def test_a_closed_optimizer_answers_as_the_library_does(monkeypatch):
+    from eridiffusion_amd import adam8bit
+    monkeypatch.setattr(adam8bit, "_stream_ptr", lambda: 0)
+    opt = adam8bit.Adam8bitFunctional()
+    opt.close()
+    with pytest.raises(L.EriError) as e:
+        opt.update_many({}, {})
+    assert e.value.code == -1
