@@ -125,9 +125,13 @@ inline uint32_t chunks_for(uint32_t grid) { return grid % kChunks == 0 ? kChunks
 int launch_step_plain_f32(int mode, bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream);
-int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, bool grad_f32, const DevTensor *rows, uint32_t n_rows,
+int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows,
                            uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                            uint32_t grid, uint32_t wg, void *stream);
+/* bf16 parameters with fp32 gradients: slot tables only. */
+int launch_step_plain_grad_f32(int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks,
+                               uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid,
+                               uint32_t wg, void *stream);
 /* Four waves per block, for tables of few blocks; `grid` workgroups of 1024 threads. */
 int launch_step_split(int layout, int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows,
                       uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,

@@ -56,15 +56,15 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
             return launch_step_pipelined_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs,
                                                   step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                                   total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-        return launch_step_plain_bf16(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs, true, true, rows, n_rows,
-                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+        return launch_step_plain_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs, rows, n_rows,
+                                          total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     }
     if (h.mode == ERI_ADAM8_MODE_BNB) { // slot table only; the decay is a factor
         const bool wd = h.weight_decay != 1.0f;
         const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
         if (bf16 && !kernel_named && prefetch_pays(total_blocks, h, compute_units))
             return launch_step_pipelined(h.mode, exact, wd, gs, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-        if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+        if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         if (!kernel_named && prefetch_pays(total_blocks, h, compute_units))
             return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_f32(h.mode, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
@@ -78,7 +78,7 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
         return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-    return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
+    return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -4,26 +4,49 @@
  * with ERI_ADAM8_FLAG_BSEARCH or ERI_ADAM8_FLAG_NO_PIPELINE.  HBM traffic bounds it, with the launch's start and its
  * last round on the smaller tables.  A row's partial last block is one more block of the walk, with the lanes past its
  * end off and one trip less in flight: as a two-sweep chain on one wave each it made 300 odd bf16 tensors with 14 M
- * parameters 32.8 us, 28.3 so; 1,400 LoRA tensors 93.9 -> 92.1 us.  Compiled twice,
- * once per parameter dtype (-DERI_PLAIN_BF16=0|1), so that the two halves build in parallel.
+ * parameters 32.8 us, 28.3 so; 1,400 LoRA tensors 93.9 -> 92.1 us.  Compiled three times, once per layout of the
+ * rows (-DERI_PLAIN_LAYOUT=0: fp32, 1: bf16, 2: bf16 parameters with fp32 gradients), so that they build in parallel.
  */
 #include "eri_adam8_inline.h"
 
-#ifndef ERI_PLAIN_BF16
-#error "compile with -DERI_PLAIN_BF16=0 or 1"
+#if !defined(ERI_PLAIN_LAYOUT) || ERI_PLAIN_LAYOUT < 0 || ERI_PLAIN_LAYOUT > 2
+#error "compile with -DERI_PLAIN_LAYOUT=0, 1 or 2"
 #endif
-
 
 namespace eri {
 
+static_assert(kLayoutF32 == 0 && kLayoutBF16 == 1 && kLayoutBF16GradF32 == 2, "ERI_PLAIN_LAYOUT names a Layout");
+constexpr bool kBf16 = ERI_PLAIN_LAYOUT != kLayoutF32;
+constexpr bool kGradBf16 = ERI_PLAIN_LAYOUT == kLayoutBF16;
+
+/* Which tables an instantiation is for.  Only the first holds the code for partial blocks: beside it the loop over
+ * whole ones took 128 registers and up to 20 bytes of scratch, 109 to 127 and none without (2,816 bf16 blocks 14.1 ->
+ * 13.5 us, 15.1 -> 14.2 with fp32 gradients).
+ * The last two differ in where a block's row is looked up.  Through the scalar cache (kWhole, kTails) the lookup is
+ * short.  Through vector loads (kWholeLarge) it waits for the stores of the block before, because one counter holds
+ * a wave's loads and stores: the wave's reads and writes keep apart, which costs the short tables a round trip per
+ * block and gives the long ones, which HBM bounds, 1-2 %.  us per launch, kWhole | kWholeLarge, 256 units:
+ *   blocks                     8,192         16,384         24,576         32,768         49,152        131,072
+ *   bf16                 31.7 | 34.0    63.4 | 64.3    95.0 | 94.5    126 | 125    188 | 185    504 | 497
+ *   bf16, functional     32.6 | 32.3    64.4 | 63.7    96.9 | 95.8    128 | 127    190 | 188    509 | 503
+ *   ... fp32 gradients   37.6 | 39.4    71.6 | 73.3    102 | 106      134 | 137    237 | 231    634 | 623
+ *   bf16, mode BNB       32.3 | 37.1    63.7 | 68.1    95.3 | 96.6    126 | 126    188 | 187
+ *   fp32, functional     51.7 | 51.7    97.6 | 97.6     167 | 167     223 | 220    335 | 330    874 | 862
+ * fp32 parameters in the other modes do not tell them apart (842.3 | 842.6 us on 131,072 blocks) and always take
+ * kWhole. */
+enum Table { kTails, kWhole, kWholeLarge };
+constexpr uint32_t large_blocks_per_cu(int mode) { return ERI_PLAIN_LAYOUT == kLayoutBF16GradF32 || mode == ERI_ADAM8_MODE_BNB ? 128 : 96; }
+
 /* Threads per workgroup: sixteen waves per compute unit where the instantiation fits the 128 registers that
  * leaves each lane, twelve (170 registers) where it would spill: the coupled-decay mode with a gradient scale,
- * with fp32 gradients or with the binary search (12-30 spilled registers at sixteen waves). */
+ * with fp32 gradients or with the binary search (12-30 spilled registers at sixteen waves).  Instantiations of kWhole
+ * use no scratch, kTails of bf16 parameters up to 20 bytes per lane, kWholeLarge, whose rows lie in vector registers, up
+ * to 28 (64 in mode BNB). */
 constexpr uint32_t plain_threads(int mode, bool gs, bool keytab, bool gbf16) {
     return (mode == ERI_ADAM8_MODE_L2 && (gs || !keytab || !gbf16)) ? 768 : 1024;
 }
 
-template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16>
+template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16, Table TABLE>
 __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_step_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,
                                                           uint32_t total_blocks, uint32_t n_tails, EriAdam8Hyper h_in,
                                                           const uint4 *__restrict__ lds_image,
@@ -56,7 +79,7 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     // left over when the list does not divide (fewer than one per wave) go one to each workgroup in turn -- workgroup
     // i takes left-over blocks i, i + grid, i + 2 grid, ... on its first waves -- so that the short last round runs on
     // every compute unit instead of filling the first few (2-3 % of the launch on tables of 5-20 blocks per wave).
-    const uint32_t units = total_blocks + n_tails;
+    const uint32_t units = TABLE == kTails ? total_blocks + n_tails : total_blocks;
     const uint32_t wave_in_wg = threadIdx.x / kWave;
     const uint32_t rounds = units / stride;
     const uint32_t left_first = rounds * stride;
@@ -68,8 +91,9 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     const BlockRowMap map(rows, n_rows);
     const uint32_t trips = rounds + (has_left ? 1u : 0u);
     for (uint32_t k = 0; k < trips; ++k) {
-        const uint32_t unit = __builtin_amdgcn_readfirstlane(k < rounds ? k * stride + wave : left_first + left_mine);
-        if (unit < total_blocks) {
+        uint32_t unit = k < rounds ? k * stride + wave : left_first + left_mine;
+        if (TABLE != kWholeLarge) unit = __builtin_amdgcn_readfirstlane(unit);
+        if (TABLE != kTails || unit < total_blocks) {
             map.seek(rows, unit, ti, t, t_end);
             const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
             full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, unit - t.full_start, kBlock, lane, h, gscale, dbc1, dbc2, L,
@@ -85,13 +109,18 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
 
 namespace {
 
-constexpr bool kBf16 = ERI_PLAIN_BF16 != 0;
-
-template <int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16>
+template <int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB>
 int launch_one(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h,
                const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
-    auto k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, GBF16>;
-    if (wg > plain_threads(MODE, GS, KEYTAB, GBF16)) wg = plain_threads(MODE, GS, KEYTAB, GBF16);
+    auto k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kTails>;
+    if constexpr (KEYTAB) { // the binary search is a cross-check and has the one variant
+        // such a table's grid is one workgroup per compute unit
+        const bool large = (uint64_t)total_blocks > (uint64_t)grid * large_blocks_per_cu(MODE);
+        if (n_tails == 0) k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kWhole>;
+        if constexpr (kBf16 || MODE == ERI_ADAM8_MODE_L2)
+            if (n_tails == 0 && large) k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kWholeLarge>;
+    }
+    if (wg > plain_threads(MODE, GS, KEYTAB, kGradBf16)) wg = plain_threads(MODE, GS, KEYTAB, kGradBf16);
     // One common window for all dies (a grid-stride walk): on the tables this kernel takes, up to 1,024
     // blocks per compute unit, it measured 2 % ahead of one range per die with the arrays far apart in device
     // memory and 5 % with them adjacent; the tables of the prefetching kernel want the ranges.
@@ -100,11 +129,12 @@ int launch_one(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, ui
     return (int)hipGetLastError();
 }
 
-/* BSEARCH selects the cross-check variants (binary search of the midpoint table); mode BNB has none. */
-template <int MODE, bool EXACT, bool BSEARCH, bool GBF16 = kBf16>
+/* BSEARCH: the layout and mode have the cross-check variants (binary search of the midpoint table); mode BNB and fp32
+ * gradients of bf16 parameters have none. */
+template <int MODE, bool EXACT, bool BSEARCH>
 int launch_flags(bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                  const EriAdam8Hyper &h, const void *img, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
-#define ERI_GO(W, G, K) return launch_one<MODE, EXACT, W, G, K, GBF16>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s)
+#define ERI_GO(W, G, K) return launch_one<MODE, EXACT, W, G, K>(rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s)
     if (BSEARCH && !keytab) {
         if (wd) { if (gs) ERI_GO(true, true, !BSEARCH); ERI_GO(true, false, !BSEARCH); }
         if (gs) ERI_GO(false, true, !BSEARCH);
@@ -118,39 +148,36 @@ int launch_flags(bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t 
 
 } // namespace
 
-#if ERI_PLAIN_BF16
-int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, bool grad_f32, const DevTensor *rows,
+#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, static_cast<hipStream_t>(stream)
+#if ERI_PLAIN_LAYOUT == 1
+int launch_step_plain_bf16(int mode, bool exact, bool wd, bool gs, bool keytab, const DevTensor *rows,
                            uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img,
                            const float *dev_scale, uint32_t grid, uint32_t wg, void *stream) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s
-    if (grad_f32) { // fp32 gradients for bf16 parameters: slot-table variants only
-        if (!keytab) return (int)hipErrorInvalidValue;
-        if (mode == ERI_ADAM8_MODE_BNB)
-            return exact ? launch_flags<ERI_ADAM8_MODE_BNB, true, false, false>(ERI_ARGS)
-                         : launch_flags<ERI_ADAM8_MODE_BNB, false, false, false>(ERI_ARGS);
-        if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, true, false, false>(ERI_ARGS);
-        return exact ? launch_flags<ERI_ADAM8_MODE_ERI, true, false, false>(ERI_ARGS)
-                     : launch_flags<ERI_ADAM8_MODE_ERI, false, false, false>(ERI_ARGS);
-    }
     if (mode == ERI_ADAM8_MODE_BNB)
         return exact ? launch_flags<ERI_ADAM8_MODE_BNB, true, false>(ERI_ARGS) : launch_flags<ERI_ADAM8_MODE_BNB, false, false>(ERI_ARGS);
     if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, true, true>(ERI_ARGS); // always the IEEE chain
     return exact ? launch_flags<ERI_ADAM8_MODE_ERI, true, true>(ERI_ARGS) : launch_flags<ERI_ADAM8_MODE_ERI, false, true>(ERI_ARGS);
-#undef ERI_ARGS
+}
+#elif ERI_PLAIN_LAYOUT == 2
+int launch_step_plain_grad_f32(int mode, bool exact, bool wd, bool gs, const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks,
+                               uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale, uint32_t grid,
+                               uint32_t wg, void *stream) {
+    constexpr bool keytab = true;
+    if (mode == ERI_ADAM8_MODE_BNB)
+        return exact ? launch_flags<ERI_ADAM8_MODE_BNB, true, false>(ERI_ARGS) : launch_flags<ERI_ADAM8_MODE_BNB, false, false>(ERI_ARGS);
+    if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, true, false>(ERI_ARGS);
+    return exact ? launch_flags<ERI_ADAM8_MODE_ERI, true, false>(ERI_ARGS) : launch_flags<ERI_ADAM8_MODE_ERI, false, false>(ERI_ARGS);
 }
 #else
 /* fp32 parameters always take the IEEE square root and division. */
 int launch_step_plain_f32(int mode, bool wd, bool gs, bool keytab, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-#define ERI_ARGS wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, img, dev_scale, grid, wg, s
     if (mode == ERI_ADAM8_MODE_BNB) return launch_flags<ERI_ADAM8_MODE_BNB, true, false>(ERI_ARGS);
     if (mode == ERI_ADAM8_MODE_L2) return launch_flags<ERI_ADAM8_MODE_L2, true, true>(ERI_ARGS);
     return launch_flags<ERI_ADAM8_MODE_ERI, true, true>(ERI_ARGS);
-#undef ERI_ARGS
 }
 #endif
+#undef ERI_ARGS
 
 } // namespace eri

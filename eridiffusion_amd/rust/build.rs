@@ -28,8 +28,8 @@ fn main() {
         "-packed-fp32-ops".into(),
     ];
     let mut objects = Vec::new();
-    // (source, object name, extra define, compiled as HIP?) -- the plain step kernel is built once per
-    // parameter dtype
+    // (source, object name, extra define, compiled as HIP?) -- the pipelined and the plain step kernel
+    // are built once per layout of the rows
     for (file, obj_name, define, is_hip) in [
         ("eri_adam8_kernels.hip", "kernels", "", true),
         ("eri_adam8_step_split.hip", "step_split", "", true),
@@ -37,8 +37,9 @@ fn main() {
         ("eri_adam8_step_pipelined.hip", "step_pipelined", "-DERI_PIPE_LAYOUT=1", true),
         ("eri_adam8_step_pipelined.hip", "step_pipelined_grad_f32", "-DERI_PIPE_LAYOUT=2", true),
         ("eri_adam8_step_pipelined.hip", "step_pipelined_f32", "-DERI_PIPE_LAYOUT=0", true),
-        ("eri_adam8_step_plain.hip", "step_plain_bf16", "-DERI_PLAIN_BF16=1", true),
-        ("eri_adam8_step_plain.hip", "step_plain_f32", "-DERI_PLAIN_BF16=0", true),
+        ("eri_adam8_step_plain.hip", "step_plain_bf16", "-DERI_PLAIN_LAYOUT=1", true),
+        ("eri_adam8_step_plain.hip", "step_plain_grad_f32", "-DERI_PLAIN_LAYOUT=2", true),
+        ("eri_adam8_step_plain.hip", "step_plain_f32", "-DERI_PLAIN_LAYOUT=0", true),
         ("eri_optim8_api.cpp", "api", "", true),
         ("eri_adam8bit_host.cpp", "host", "", false),
     ] {

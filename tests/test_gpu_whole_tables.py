@@ -1,0 +1,52 @@
+"""Tables without partial blocks, which the plain kernel runs without the code for them, below and above the size from
+which it looks its rows up through vector loads: every layout and mode against the prefetching kernel (which the parity
+tests hold against the oracle) on the same inputs, bit for bit."""
+import ctypes as C
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+BLOCK = 2048
+
+
+def _run(layout, mode, lengths, flags, scale):
+    """Two steps over tensors of `lengths` blocks; returns everything the step writes."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    stream = torch.cuda.current_stream().cuda_stream
+    blocks = sum(lengths)
+    gen = torch.Generator(device="cuda").manual_seed(blocks + mode)
+    pdt = torch.float32 if layout == "f32" else torch.bfloat16
+    gdt = torch.bfloat16 if layout == "bf16" else torch.float32
+    p = (torch.randn(blocks * BLOCK, device="cuda", generator=gen) * 0.02).to(pdt)
+    gs = [(torch.randn(blocks * BLOCK, device="cuda", generator=gen) * 1e-3).to(gdt) for _ in range(2)]
+    m, v = (torch.empty(blocks * BLOCK, dtype=torch.uint8, device="cuda") for _ in range(2))
+    am, av = (torch.empty(blocks, device="cuda") for _ in range(2))
+    L.check(L.lib().eri_adam8_state_init(m.data_ptr(), v.data_ptr(), am.data_ptr(), av.data_ptr(), m.numel(), stream), "init")
+    for step, g in enumerate(gs, 1):
+        rows, at = (L.TensorRow * len(lengths))(), 0
+        for r, n in zip(rows, lengths):
+            r.p, r.g = p.data_ptr() + at * BLOCK * p.element_size(), g.data_ptr() + at * BLOCK * g.element_size()
+            r.m, r.v, r.absmax_m, r.absmax_v = m.data_ptr() + at * BLOCK, v.data_ptr() + at * BLOCK, am.data_ptr() + 4 * at, av.data_ptr() + 4 * at
+            r.numel, r.block_start, r.grad_scale = n * BLOCK, at, 1.0
+            r.dtype_tag, r.grad_f32 = (L.DTYPE_F32 if layout == "f32" else L.DTYPE_BF16), int(layout == "bf16-f32-grads")
+            at += n
+        h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, step - (mode == L.MODE_L2), mode, L.FLAG_EXACT_PARAM | flags, scale)
+        L.check(L.lib().eri_adam8_step_multi(rows, len(rows), C.byref(h), stream), "step_multi")
+    torch.cuda.synchronize()
+    return p, m, v, am, av
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2], ids=["eri", "l2", "bnb"])
+@pytest.mark.parametrize("layout", ["bf16", "bf16-f32-grads", "f32"])
+@pytest.mark.parametrize("blocks,scale", [(1, None), (4097, 0.5), (96 * 256 + 300, None), (128 * 256 + 300, 0.5)])
+def test_plain_kernel_over_whole_blocks(layout, mode, blocks, scale):
+    import torch
+    from eridiffusion_amd import _lib as L
+    lengths = []
+    while sum(lengths) < blocks:
+        lengths.append(min(1 + len(lengths) * 7 % 53, blocks - sum(lengths)))
+    want = _run(layout, mode, lengths, L.FLAG_ONE_WAVE, scale)
+    got = _run(layout, mode, lengths, L.FLAG_NO_PIPELINE if blocks == 1 else 0, scale)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
