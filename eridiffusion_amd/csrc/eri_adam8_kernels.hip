@@ -8,18 +8,29 @@
 namespace eri {
 
 /* The one case in which the EMA runs inside the step kernel: the prefetching kernel in mode ERI, on bf16
- * parameters (with bf16 or fp32 gradients). */
+ * parameters (with bf16 or fp32 gradients).  With bf16 gradients that kernel has twelve waves per compute unit against
+ * the plain kernel's sixteen, and between one round of them and the tables that HBM bounds, the plain kernel and the
+ * sweep behind it are faster.  us per step and EMA, prefetching kernel | plain kernel and sweep, 256 units:
+ *   blocks               1,088        2,816        3,584        4,096        8,192       16,384       32,768
+ *   bf16           12.0 | 13.3  21.0 | 20.9  32.9 | 25.3  33.0 | 28.4  54.3 | 50.6   105 | 97.8    199 | 204
+ *   fp32 gradients 11.9 | 13.0  23.7 | 22.8  26.9 | 28.2  28.5 | 34.3  49.2 | 59.6  92.6 | 107     201 | 210 */
+constexpr uint32_t kFusedEmaOneRound = 12; // bf16 gradients: blocks per unit up to which
+constexpr uint32_t kFusedEmaLarge = 64;    // and beyond which the EMA runs inside the step
 bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
     if ((h.flags & ERI_ADAM8_FLAG_EMA) == 0 || !layout_param_bf16(layout) || h.mode != ERI_ADAM8_MODE_ERI) return false;
     if (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) return false;
     const bool few = (uint64_t)units <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
-    return (h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || !few;
+    if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0) return true;
+    if (few) return false;
+    return !layout_grad_bf16(layout) || units <= compute_units * kFusedEmaOneRound ||
+           (uint64_t)units > (uint64_t)compute_units * kFusedEmaLarge;
 }
 
-/* Whether a bf16 table that qualifies for the prefetching kernel is large enough to gain from it.  A step
- * that carries the EMA stays on the prefetching kernel at every size: it is the one that fuses it. */
-static bool prefetch_pays(uint32_t total_blocks, const EriAdam8Hyper &h, uint32_t compute_units) {
-    if (h.flags & (ERI_ADAM8_FLAG_ONE_WAVE | ERI_ADAM8_FLAG_EMA)) return true;
+/* Whether a table that qualifies for the prefetching kernel is large enough to gain from it, or has its EMA inside that
+ * kernel.  A step whose EMA is a sweep of its own runs as it would without one: on the prefetching kernel all the same,
+ * mode BNB took 38.1 us for 4,096 bf16 blocks instead of 29.0, and fp32 parameters 39 for 2,816 instead of 31.5. */
+static bool prefetch_pays(uint32_t total_blocks, uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
+    if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || step_fuses_ema(units, layout, h, compute_units)) return true;
     return (uint64_t)total_blocks > (uint64_t)compute_units * (uint64_t)kPrefetchBlocksPerCu;
 }
 
@@ -52,7 +63,7 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     }
     if (mixed) {
         const bool wd_m = h.mode == ERI_ADAM8_MODE_BNB ? h.weight_decay != 1.0f : h.weight_decay > 0.0f;
-        if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
+        if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, units, layout, h, compute_units))
             return launch_step_pipelined_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs,
                                                   step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                                   total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
@@ -62,20 +73,20 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     if (h.mode == ERI_ADAM8_MODE_BNB) { // slot table only; the decay is a factor
         const bool wd = h.weight_decay != 1.0f;
         const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
-        if (bf16 && !kernel_named && prefetch_pays(total_blocks, h, compute_units))
+        if (bf16 && !kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
             return launch_step_pipelined(h.mode, exact, wd, gs, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-        if (!kernel_named && prefetch_pays(total_blocks, h, compute_units))
+        if (!kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
             return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_f32(h.mode, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     }
     const bool wd = h.weight_decay > 0.0f;
     const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
     const bool keytab = (h.flags & ERI_ADAM8_FLAG_BSEARCH) == 0;
-    if (!bf16 && !kernel_named && prefetch_pays(total_blocks, h, compute_units))
+    if (!bf16 && !kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
         return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     if (!bf16) return launch_step_plain_f32(h.mode, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-    if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, h, compute_units))
+    if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, units, layout, h, compute_units))
         return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);

@@ -9,8 +9,9 @@ pytestmark = pytest.mark.gpu
 BLOCK = 2048
 
 
-def _run(layout, mode, lengths, flags, scale):
-    """Two steps over tensors of `lengths` blocks; returns everything the step writes."""
+def _run(layout, mode, lengths, flags, scale, ema=False):
+    """Two steps over tensors of `lengths` blocks, every other one with a shadow if `ema`; returns everything the steps
+    write."""
     import torch
     from eridiffusion_amd import _lib as L
     stream = torch.cuda.current_stream().cuda_stream
@@ -22,6 +23,7 @@ def _run(layout, mode, lengths, flags, scale):
     gs = [(torch.randn(blocks * BLOCK, device="cuda", generator=gen) * 1e-3).to(gdt) for _ in range(2)]
     m, v = (torch.empty(blocks * BLOCK, dtype=torch.uint8, device="cuda") for _ in range(2))
     am, av = (torch.empty(blocks, device="cuda") for _ in range(2))
+    shadow = p * 0.5
     L.check(L.lib().eri_adam8_state_init(m.data_ptr(), v.data_ptr(), am.data_ptr(), av.data_ptr(), m.numel(), stream), "init")
     for step, g in enumerate(gs, 1):
         rows, at = (L.TensorRow * len(lengths))(), 0
@@ -30,11 +32,14 @@ def _run(layout, mode, lengths, flags, scale):
             r.m, r.v, r.absmax_m, r.absmax_v = m.data_ptr() + at * BLOCK, v.data_ptr() + at * BLOCK, am.data_ptr() + 4 * at, av.data_ptr() + 4 * at
             r.numel, r.block_start, r.grad_scale = n * BLOCK, at, 1.0
             r.dtype_tag, r.grad_f32 = (L.DTYPE_F32 if layout == "f32" else L.DTYPE_BF16), int(layout == "bf16-f32-grads")
+            if ema and at % 2 == 0:
+                r.ema_shadow = shadow.data_ptr() + at * BLOCK * p.element_size()
             at += n
-        h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, step - (mode == L.MODE_L2), mode, L.FLAG_EXACT_PARAM | flags, scale)
+        h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, step - (mode == L.MODE_L2), mode, L.FLAG_EXACT_PARAM | flags | (L.FLAG_EMA if ema else 0), scale)
+        h.ema_decay = 0.9
         L.check(L.lib().eri_adam8_step_multi(rows, len(rows), C.byref(h), stream), "step_multi")
     torch.cuda.synchronize()
-    return p, m, v, am, av
+    return p, m, v, am, av, shadow
 
 
 @pytest.mark.parametrize("mode", [0, 1, 2], ids=["eri", "l2", "bnb"])
@@ -49,4 +54,19 @@ def test_plain_kernel_over_whole_blocks(layout, mode, blocks, scale):
     want = _run(layout, mode, lengths, L.FLAG_ONE_WAVE, scale)
     got = _run(layout, mode, lengths, L.FLAG_NO_PIPELINE if blocks == 1 else 0, scale)
     for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layout,mode", [("bf16", 0), ("bf16-f32-grads", 0), ("f32", 0), ("bf16", 2), ("f32", 2)])
+@pytest.mark.parametrize("blocks", [1024, 1025, 12 * 256, 12 * 256 + 1, 64 * 256, 64 * 256 + 1])
+def test_every_route_of_a_step_with_an_ema(layout, mode, blocks):
+    """On both sides of each line between the kernels that take such a step."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    lengths = []
+    while sum(lengths) < blocks:
+        lengths.append(min(1 + len(lengths) * 7 % 53, blocks - sum(lengths)))
+    want = _run(layout, mode, lengths, L.FLAG_ONE_WAVE, None, ema=True)
+    assert not torch.equal(want[5], _run(layout, mode, lengths, 0, None)[5])
+    for a, b in zip(_run(layout, mode, lengths, 0, None, ema=True), want):
         assert torch.equal(a, b)
