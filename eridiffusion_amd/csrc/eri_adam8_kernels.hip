@@ -476,9 +476,15 @@ __device__ __forceinline__ void grad_sumsq_walk(const NormGroup &g, uint32_t wg,
  * is one whatever the tables hold.  Measured, this pass and the one behind it, before (a launch per group, a pair per
  * wave, partial blocks one load at a time) and after:
  *   256 short tensors in two tables  5.4 + 5.4 + 3.1 -> 5.8 + 2.6 us
- *   608 tensors, 306 MB of bf16      47.7 + 6.8 -> 49.5 + 5.8 us, and the step behind it 306 -> 300 us (it starts on
+ * and both kernels together, over the same arrays:
+ *   608 tensors, 306 MB of bf16      52.3 -> 49.9 us, and with the clipped step behind it 334.6 -> 331.5 (it starts on
  *                                    gradients that the last-level cache still holds: the walk goes backwards)
- *   1,680 tensors, 10.3 GB of fp32   1,655 + 7.2 -> 1,640 + 4.7 us */
+ *   608 tensors, 1.23 GB of bf16     187.8 -> 186.1 us
+ *   1,680 tensors, 10.3 GB of fp32   1,721 -> 1,680 us
+ * A pass over gradients of one dtype has an instantiation of its own: beside the fp32 walk the bf16 one took 75
+ * registers for 57, six waves per SIMD for eight, and 197.6 us on those 1.23 GB. */
+enum NormDtypes { kNormF32, kNormBF16, kNormBoth };
+template <NormDtypes GRADS>
 __global__ __launch_bounds__(kNormWaves * kWave) void grad_sumsq_kernel(NormGroups groups, double *__restrict__ partial) {
     __shared__ double sums[kNormWaves][2];
     const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -487,7 +493,7 @@ __global__ __launch_bounds__(kNormWaves * kWave) void grad_sumsq_kernel(NormGrou
     while (gi + 1 < groups.n && blockIdx.x >= groups.g[gi + 1].first_wg) ++gi;
     const NormGroup &g = groups.g[gi];
     double total = 0.0, bad = 0.0;
-    if (g.grad_bf16) grad_sumsq_walk<true>(g, blockIdx.x - g.first_wg, wave_in_wg, lane, total, bad);
+    if (GRADS == kNormBF16 || (GRADS == kNormBoth && g.grad_bf16 != 0)) grad_sumsq_walk<true>(g, blockIdx.x - g.first_wg, wave_in_wg, lane, total, bad);
     else grad_sumsq_walk<false>(g, blockIdx.x - g.first_wg, wave_in_wg, lane, total, bad);
     if (lane == 0) {
         sums[wave_in_wg][0] = total;
@@ -537,7 +543,10 @@ __global__ __launch_bounds__(1024) void grad_norm_finish_kernel(const double *__
 
 int launch_grad_sumsq(const NormGroups &groups, double *partial, void *stream) {
     const NormGroup &last = groups.g[groups.n - 1];
-    hipLaunchKernelGGL(grad_sumsq_kernel, dim3(last.first_wg + last.wgs), dim3(kNormWaves * kWave), 0, static_cast<hipStream_t>(stream),
+    bool f32 = false, bf16 = false;
+    for (uint32_t i = 0; i < groups.n; ++i) (groups.g[i].grad_bf16 ? bf16 : f32) = true;
+    const auto k = f32 ? (bf16 ? grad_sumsq_kernel<kNormBoth> : grad_sumsq_kernel<kNormF32>) : grad_sumsq_kernel<kNormBF16>;
+    hipLaunchKernelGGL(k, dim3(last.first_wg + last.wgs), dim3(kNormWaves * kWave), 0, static_cast<hipStream_t>(stream),
                        groups, partial);
     return (int)hipGetLastError();
 }
