@@ -221,7 +221,7 @@ struct SweepUnit {
  *   ... with masters      6.7 | 3.9    9.4 | 7.0   23.7 | 22.6  94.5 | 78.5   199 | 171
  *   ... 1,027 more each  12.4 | 4.5   14.1 | 7.2   24.6 | 18.2  60.9 | 60.1   113 | 112
  *   EMA, fp32             4.0 | 3.7    4.2 | 4.1    8.4 |  7.1  31.5 | 29.4   57.5 | 56.8
- * Above it the list itself (8 bytes per block, uploaded when the rows change) is no longer small. */
+ * Above it the list itself (8 bytes per block, uploaded when the rows' sizes change) is no longer small. */
 constexpr uint32_t kSmallSweepBlocksPerCu = 64;
 
 /* units: the list of blocks, n_units of them, for the small kernels; null for the persistent ones, which take `grid`

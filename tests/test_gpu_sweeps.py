@@ -320,3 +320,50 @@ def test_partial_blocks_of_every_shape(bf16, more):
         assert np.array_equal(back(dm[i], np.float32), ms[i]) and np.array_equal(back(dv[i], np.float32), vs[i]), sizes[i]
         if ws[i] is not None:
             assert np.array_equal(back(dw[i], np.float32), ws[i]), sizes[i]
+
+
+def test_row_sets_that_change_addresses_and_sizes():
+    """The small sweeps' list of blocks is kept where only addresses change: more row sets than are kept, of the same
+    sizes, of the same sizes in another order, of fewer rows and of both dtypes, every call against the same sweep of
+    each tensor alone."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    stream = torch.cuda.current_stream().cuda_stream
+    sizes = [5, 2048, 2048 * 7 + 9, 4096, 300, 2048 * 3 - 1]
+    orders = [sizes] * 6 + [sizes[::-1], sizes, sizes[1:], sizes, sizes[::-1], sizes[::-1], [n + 2048 for n in sizes], sizes]
+    gen = torch.Generator(device="cuda").manual_seed(8)
+
+    def tensor(n, dt):
+        return torch.randn(n, device="cuda", generator=gen).to(dt)
+    keep = []
+    for call, order in enumerate(orders):
+        dts = [torch.bfloat16 if (i + call // 7) % 2 else torch.float32 for i in range(len(order))]
+        sh, ps = [tensor(n, dt) for n, dt in zip(order, dts)], [tensor(n, dt) for n, dt in zip(order, dts)]
+        ms, vs = [tensor(n, torch.float32) for n in order], [tensor(n, torch.float32).square() for n in order]
+        alone = [[t.clone() for t in ts] for ts in (sh, ps, ms, vs)]
+        keep.append((sh, ps, ms, vs, alone))  # their addresses stay taken: every call brings new ones
+
+        def sweep(which, sh, ps, ms, vs):
+            tags = [L.DTYPE_BF16 if dts[i] == torch.bfloat16 else L.DTYPE_F32 for i in which]
+            erows, rows = (L.EmaRow * len(which))(), (L.AdamW32Row * len(which))()
+            for e, r, i, tag in zip(erows, rows, which, tags):
+                e.shadow, e.p, e.numel, e.dtype_tag = sh[i].data_ptr(), ps[i].data_ptr(), order[i], tag
+                r.p, r.g, r.m, r.v = sh[i].data_ptr(), ps[i].data_ptr(), ms[i].data_ptr(), vs[i].data_ptr()
+                r.numel, r.dtype_tag = order[i], tag
+            L.check(L.lib().eri_ema_update_multi(erows, len(which), 0.9, stream), "ema")
+            h = L.AdamW32Hyper(1e-3, 0.9, 0.999, 1e-8, 0.01)
+            L.check(L.lib().eri_adamw32_step_multi(rows, len(which), C.byref(h), stream), "adamw32")
+        sweep(range(len(order)), sh, ps, ms, vs)
+        if call >= 6:  # the first sets follow one another without a single row in between
+            for i in range(len(order)):
+                sweep([i], *alone)
+    for call, order in enumerate(orders[:6]):
+        sh, ps, ms, vs, alone = keep[call]
+        dts = [t.dtype for t in sh]
+        for i in range(len(order)):
+            sweep([i], *alone)
+    torch.cuda.synchronize()
+    for call, (sh, ps, ms, vs, alone) in enumerate(keep):
+        for got, want in zip((sh, ps, ms, vs), alone):
+            for a, b in zip(got, want):
+                assert torch.equal(a, b), call
