@@ -223,7 +223,7 @@ def test_joint_norm_over_a_step_table_and_a_gradient_only_table():
     L.lib().eri_adam8_table_destroy(table)
 
 
-@pytest.mark.parametrize("repeat", [1, 40], ids=["a-wave-each", "many-blocks-per-wave"])
+@pytest.mark.parametrize("repeat", [1, 40], ids=["few-rows", "a-block-per-wave"])
 def test_one_launch_over_every_layout_and_partial_block(repeat):
     """Two tables with groups of all three layouts, last blocks of every shape, NaN in the words behind every gradient:
     none of those is read, and the norm is that of all gradients."""
@@ -262,3 +262,42 @@ def test_one_launch_over_every_layout_and_partial_block(repeat):
         assert bad.value == 0 and abs(norm.value - want) <= 2e-6 * want
     for t in tables:
         L.lib().eri_adam8_table_destroy(t)
+
+
+@pytest.mark.parametrize("layouts", [[0], [1], [0, 1, 2]], ids=["f32", "bf16", "all"])
+def test_waves_that_walk_several_blocks(layouts):
+    """Groups of 9,000 to 10,000 blocks over 104 rows, more than the 8,192 waves of a pass: a wave's second block, with
+    its loads ahead and its row another one.  NaN behind every gradient is not read; NaN and infinity in the first row
+    (the walk goes from the last block to the first) and in the last are counted."""
+    import torch
+    L = _L()
+    ends = [0, 1, 7, 8, 9, 505, 512, 513, 1543, 2041, 2047, 5, 1024]
+    forms = [(L.DTYPE_F32, 0, torch.float32), (L.DTYPE_BF16, 0, torch.bfloat16), (L.DTYPE_BF16, 1, torch.float32)]
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    rows, total, keep, start = (L.TensorRow * (104 * len(layouts)))(), 0.0, [], 0
+    for i, r in enumerate(rows):
+        tag, grad_f32, dt = forms[layouts[i % len(layouts)]]
+        n = 2048 * (80 + i // len(layouts) % 17) + ends[i // len(layouts) % len(ends)]
+        g = (torch.randn(n + 16, device="cuda", generator=gen) * 1e-3).to(dt)
+        g[n:] = float("nan")
+        keep.append(g)
+        total += float((g[:n].double() ** 2).sum())
+        r.p = r.g = g.data_ptr()
+        r.numel, r.block_start, r.dtype_tag, r.grad_f32, r.grad_scale = n, start, tag, grad_f32, 1.0
+        start += (n + 2047) // 2048
+    table = C.c_void_p()
+    L.check(L.lib().eri_adam8_grad_table_create(rows, len(rows), None, C.byref(table)), "grad_table_create")
+
+    def read():
+        norm, scale, bad = C.c_float(), C.c_float(), C.c_uint64()
+        L.check(L.lib().eri_adam8_grad_norm(table, 1.0, 0.0, None), "grad_norm")
+        L.check(L.lib().eri_adam8_grad_norm_read(table, C.byref(norm), C.byref(scale), None), "read")
+        L.check(L.lib().eri_adam8_grad_nonfinite_read(table, C.byref(bad), None), "nonfinite_read")
+        return norm.value, bad.value
+    want = np.sqrt(total)
+    norm, bad = read()
+    assert bad == 0 and abs(norm - want) <= 2e-6 * want
+    keep[0][3000], keep[0][2048 * 70 + 1], keep[-1][2048 * 5] = float("nan"), float("inf"), float("-inf")
+    norm, bad = read()
+    assert bad == 3 and not np.isfinite(norm)
+    L.lib().eri_adam8_table_destroy(table)

@@ -148,18 +148,20 @@ def test_adamw32_and_ema_over_rows_of_both_dtypes():
 
 @pytest.mark.parametrize("mode", [0, 1, 2], ids=["eri", "l2", "bnb"])
 @pytest.mark.parametrize("scaled", [False, True])
-def test_both_parameter_dtypes_in_one_launch(mode, scaled):
-    """Blocks of every shape of both dtypes in one table: more than a wave each and fewer, with and without a gradient
-    scale; every tensor as if it had been stepped in a table of its dtype."""
+@pytest.mark.parametrize("exact,wd", [(True, 0.01), (False, 0.0)], ids=["exact-decay", "fast-no-decay"])
+def test_both_parameter_dtypes_in_one_launch(mode, scaled, exact, wd):
+    """Blocks of every shape of both dtypes in one table, with and without a gradient scale; every tensor as if it had
+    been stepped in a table of its dtype.  The larger table has 5,702 blocks: a whole round of the 4,096 waves (3,072 in
+    mode L2) that ends among the bf16 blocks, so that waves go from an fp32 block to a bf16 one, and blocks left over."""
     import ctypes as C
     import torch
     import harness as hs
     import oracle_c as oc
     from eridiffusion_amd import _lib as L
     ends = [1, 7, 8, 9, 505, 512, 1023, 1543, 2047, 2048, 2048 * 2 + 3, 2048 * 5]
-    for repeat in (1, 40):
+    for repeat in (1, 200):
         sizes = {True: ends * repeat, False: (ends[::-1] * repeat)[: 7 * repeat]}
-        parts, args = {}, lambda t: (1e-4, 0.9, 0.999, 1e-8, 0.01, t - 1 if mode == 1 else t)
+        parts, args = {}, lambda t: (1e-4, 0.9, 0.999, 1e-8, wd, t - 1 if mode == 1 else t)
         omode = {0: oc.MODE_ERI, 1: oc.MODE_L2, 2: oc.MODE_BNB}[mode]
         for bf16 in (True, False):
             ps, gs = hs.make_inputs(sizes[bf16], bf16, 900 + 10 * mode + bf16)
@@ -172,10 +174,11 @@ def test_both_parameter_dtypes_in_one_launch(mode, scaled):
         for r in rows:
             r.block_start = start
             start += (r.numel + 2047) // 2048
-        h = L.hyper_pack(*args(2), mode, L.FLAG_EXACT_PARAM, 0.5 if scaled else None)
+        h = L.hyper_pack(*args(2), mode, L.FLAG_EXACT_PARAM if exact else 0, 0.5 if scaled else None)
         L.check(L.lib().eri_adam8_step_multi(rows, len(rows), C.byref(h), torch.cuda.current_stream().cuda_stream), "step_multi")
         torch.cuda.synchronize()
         for bf16, (ps, gs, states, gt) in parts.items():
             hs.oracle_step(ps, gs, states, args(2), bf16, omode, 0.5 if scaled else None)
             got_p, got_st = gt.fetch()
-            assert hs.compare(got_p, got_st, ps, states, bf16, True, "both dtypes, bf16=%s" % bf16)["code_mismatch"] == 0
+            stats = hs.compare(got_p, got_st, ps, states, bf16, exact or mode == 1, "both dtypes, bf16=%s" % bf16)
+            assert stats["code_mismatch"] == 0

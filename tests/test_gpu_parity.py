@@ -564,6 +564,7 @@ def test_partial_blocks_of_every_shape(mode, bf16):
 
 
 def test_more_partial_blocks_than_waves():
-    # 4,500 tensors of which every other one is a partial block and nothing else: more of them than four per workgroup
-    sizes = [(5 * i) % 61 + 1 if i % 2 else 2048 for i in range(4500)]
+    # 9,000 tensors of which every other one is a partial block and nothing else: 4,500 of them for the 3,072 waves of the
+    # prefetching kernel and the 4,096 of the plain one
+    sizes = [(5 * i) % 61 + 1 if i % 2 else 2048 for i in range(9000)]
     run_case(sizes, True, 4200, steps=1, flags=2, prior=1, label="many partial blocks")
