@@ -428,6 +428,35 @@ bool is_capturing(void *stream) {
     return cs == hipStreamCaptureStatusActive;
 }
 
+/* The streams whose kernels read device memory that is overwritten later, for caches that a caller does not see and so
+ * cannot order.  `ev` is an event of the memory's owner. */
+struct Readers {
+    static constexpr size_t kMax = 8;
+    std::vector<void *> on;
+    /* Orders what follows on `stream` after what the others have queued by now; `stream` then stands for them. */
+    int settle(hipEvent_t ev, void *stream) {
+        for (void *r : on) {
+            if (r == stream || is_capturing(r)) continue; // an event of a capture would draw `stream` into it
+            hipError_t e = hipEventRecord(ev, static_cast<hipStream_t>(r));
+            // a capture cannot wait for an event from outside it
+            if (e == hipSuccess) e = is_capturing(stream) ? hipEventSynchronize(ev) : hipStreamWaitEvent(static_cast<hipStream_t>(stream), ev, 0);
+            if (e != hipSuccess) { // a stream that has been destroyed since
+                (void)hipGetLastError();
+                ERI_HIP(hipDeviceSynchronize());
+            }
+        }
+        on.assign(1, stream);
+        return 0;
+    }
+    int add(hipEvent_t ev, void *stream) {
+        for (void *r : on)
+            if (r == stream) return 0;
+        if (on.size() >= kMax) return settle(ev, stream);
+        on.push_back(stream);
+        return 0;
+    }
+};
+
 /* Work that reads the device rows must run after their upload.  On the upload's own stream that is stream
  * order; another stream is made to wait for the upload's event (no host wait).  A stream that is being
  * captured into a graph cannot wait for an event outside the graph, so there the host waits for the
@@ -1378,7 +1407,8 @@ namespace {
  * parameters outside the 8-bit table), the same sets step after step, so the last four distinct sets are kept:
  * rows found in one of them are not uploaded again.  A set is uploaded through its own pinned mirror, whose
  * previous copy is waited for before it is overwritten; a set that is used on another stream than the one it
- * was uploaded on is ordered after the upload by an event wait on that stream. */
+ * was uploaded on is ordered after the upload by an event wait on that stream, and the upload of a set that takes
+ * its place after the kernels that other streams have queued on it. */
 struct ElemCache {
     struct Group {
         eri::ElemRow *dev = nullptr, *pinned = nullptr; // n rows, then the list of n_units blocks of a small sweep
@@ -1391,6 +1421,7 @@ struct ElemCache {
         hipEvent_t ev = nullptr;
         bool pending = false;
         void *stream = nullptr; // of the last upload
+        Readers readers;        // of the device rows
         uint64_t used = 0;
         void drop() {
             if (pending && ev) (void)hipEventSynchronize(ev);
@@ -1404,6 +1435,7 @@ struct ElemCache {
             }
             if (ev) (void)hipEventDestroy(ev);
             ev = nullptr;
+            readers.on.clear();
             used = 0;
         }
     };
@@ -1456,6 +1488,8 @@ struct ElemCache {
             }
             sl->used = 0; // not a set to come back to until the upload below is complete
             const bool capturing = is_capturing(stream); // a captured copy runs at each replay and not now
+            const int rc = sl->readers.settle(sl->ev, stream);
+            if (rc) return rc;
             for (int gi = 0; gi < 2; ++gi) {
                 Group &g = sl->groups[gi];
                 const uint32_t n = (uint32_t)rows[gi].size();
@@ -1498,6 +1532,8 @@ struct ElemCache {
             sl->stream = stream;
         }
         sl->used = ++tick;
+        const int rc = sl->readers.add(sl->ev, stream);
+        if (rc) return rc;
         for (int gi = 0; gi < 2; ++gi) {
             const Group &g = sl->groups[gi];
             const uint32_t n = g.n;
@@ -1508,7 +1544,7 @@ struct ElemCache {
             uint32_t grid = (work + 3) / 4;
             if (grid > cus * 16) grid = cus * 16;
             const eri::SweepUnit *units = g.n_units ? reinterpret_cast<const eri::SweepUnit *>(g.dev + n) : nullptr;
-            int rc = launch(g.dev, n, total, units, g.n_units, gi == 0 ? ERI_DTYPE_F32 : ERI_DTYPE_BF16, grid, stream, extra);
+            const int rc = launch(g.dev, n, total, units, g.n_units, gi == 0 ? ERI_DTYPE_F32 : ERI_DTYPE_BF16, grid, stream, extra);
             if (rc) return hip_fail((hipError_t)rc, "element-wise sweep launch");
         }
         return 0;

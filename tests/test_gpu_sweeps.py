@@ -367,3 +367,52 @@ def test_row_sets_that_change_addresses_and_sizes():
         for got, want in zip((sh, ps, ms, vs), alone):
             for a, b in zip(got, want):
                 assert torch.equal(a, b), call
+
+
+def test_row_sets_on_several_streams():
+    """A row set that a queued kernel of another stream has still to read stays what it was: four sets (all that are
+    kept) wait on one stream while four others come in on a second one, and then one set comes in on more streams than
+    are remembered.  Every tensor against the same sweeps alone on one stream."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    sets = []
+    for i in range(8):
+        sizes = [2048 * (i + 1) + 3 * i, 77 + i, 4096 * (8 - i)]
+        sets.append([(torch.randn(n, device="cuda", generator=gen), torch.randn(n, device="cuda", generator=gen)) for n in sizes])
+    alone = [[(sh.clone(), p) for sh, p in one] for one in sets]
+
+    def sweep(one, stream):
+        rows = (L.EmaRow * len(one))()
+        for r, (sh, p) in zip(rows, one):
+            r.shadow, r.p, r.numel, r.dtype_tag = sh.data_ptr(), p.data_ptr(), sh.numel(), L.DTYPE_F32
+        L.check(L.lib().eri_ema_update_multi(rows, len(one), 0.9, stream.cuda_stream), "ema")
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for one in sets[:4]:
+        sweep(one, a)
+    a.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(5000000)
+    for one in sets[:4]:
+        sweep(one, a)
+    for one in sets[4:] + sets[4:]:
+        sweep(one, b)
+    last, more = b, [torch.cuda.Stream() for _ in range(10)]
+    for s in more:
+        s.wait_stream(last)
+        sweep(sets[7], s)
+        last = s
+    for one in sets[:4]:  # takes the places of the others again
+        a.wait_stream(last)
+        sweep(one, a)
+    torch.cuda.synchronize()
+    default = torch.cuda.current_stream()
+    for i, one in enumerate(alone):
+        for _ in range(3 if i < 4 else 2 if i < 7 else 12):
+            for t in one:
+                sweep([t], default)
+    torch.cuda.synchronize()
+    for i, (one, want) in enumerate(zip(sets, alone)):
+        for (x, _), (y, _) in zip(one, want):
+            assert torch.equal(x, y), i
