@@ -1312,7 +1312,19 @@ int eri_adam8_step_multi(const EriAdam8Tensor *rows, uint32_t n, const EriAdam8H
     struct Cache {
         EriAdam8Table *table = nullptr;
         std::vector<EriAdam8Tensor> last;
-        ~Cache() { destroy_table(table); }
+        Readers readers;         // of the table's device rows
+        hipEvent_t ev = nullptr; // theirs
+        int device = -1;         // of ev
+        void drop() {
+            destroy_table(table);
+            table = nullptr;
+            last.clear();
+            readers.on.clear();
+        }
+        ~Cache() {
+            drop();
+            if (ev) (void)hipEventDestroy(ev);
+        }
     };
     thread_local Cache cache;
     if (!rows || !h) return fail(ERI_ERR_NULL, "rows or hyper is NULL");
@@ -1324,17 +1336,25 @@ int eri_adam8_step_multi(const EriAdam8Tensor *rows, uint32_t n, const EriAdam8H
             same_shape = rows[i].numel == cache.table->numel[i] && layout_of(rows[i]) == cache.table->dtype[i];
     int rc = 0;
     if (!same_shape) {
-        destroy_table(cache.table);
-        cache.table = nullptr;
-        cache.last.clear();
+        cache.drop();
+        if (cache.ev && cache.device != dev) {
+            (void)hipEventDestroy(cache.ev);
+            cache.ev = nullptr;
+        }
+        if (!cache.ev) ERI_HIP(hipEventCreateWithFlags(&cache.ev, hipEventDisableTiming));
+        cache.device = dev;
         rc = eri_adam8_table_create(rows, n, stream, &cache.table);
         if (rc) return rc;
         cache.last.assign(rows, rows + n);
     } else if (std::memcmp(cache.last.data(), rows, sizeof(EriAdam8Tensor) * n) != 0) {
+        rc = cache.readers.settle(cache.ev, stream);
+        if (rc) return rc;
         rc = eri_adam8_table_update(cache.table, rows, n, stream);
         if (rc) return rc;
         cache.last.assign(rows, rows + n);
     }
+    rc = cache.readers.add(cache.ev, stream);
+    if (rc) return rc;
     return eri_adam8_step_table(cache.table, h, stream);
 }
 

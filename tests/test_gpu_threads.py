@@ -68,3 +68,53 @@ def test_two_threads_two_streams_each_bit_exact(bf16):
     for t in threads:
         t.join(timeout=100)
     assert out == {0: "ok", 1: "ok"}, out
+
+
+def test_step_multi_on_two_streams_of_one_thread():
+    """The launch table behind eri_adam8_step_multi is not given other rows while a step that is queued on another
+    stream has still to read it.  Both sets of rows against the same steps on one stream."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    sizes = [2048 * 5, 2048 + 9, 640]
+    gen = torch.Generator(device="cuda").manual_seed(4)
+
+    def make():
+        one = []
+        for n in sizes:
+            nb = (n + 2047) // 2048
+            t = [torch.randn(n, device="cuda", generator=gen), torch.randn(n, device="cuda", generator=gen),
+                 torch.empty(n, dtype=torch.uint8, device="cuda"), torch.empty(n, dtype=torch.uint8, device="cuda"),
+                 torch.empty(nb, device="cuda"), torch.empty(nb, device="cuda")]
+            L.check(L.lib().eri_adam8_state_init(*[x.data_ptr() for x in t[2:]], n, None), "state_init")
+            one.append(t)
+        return one
+
+    def step(one, t, stream):
+        rows, start = (L.TensorRow * len(sizes))(), 0
+        for r, n, x in zip(rows, sizes, one):
+            r.p, r.g, r.m, r.v, r.absmax_m, r.absmax_v = [y.data_ptr() for y in x]
+            r.numel, r.block_start, r.dtype_tag, r.grad_scale = n, start, L.DTYPE_F32, 1.0
+            start += (n + 2047) // 2048
+        h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, t, L.MODE_ERI, 0)
+        L.check(L.lib().eri_adam8_step_multi(rows, len(rows), C.byref(h), stream.cuda_stream), "step_multi")
+    sets = [make(), make()]
+    torch.cuda.synchronize()
+    want = [[[x.clone() for x in t] for t in one] for one in sets]
+    a, b, default = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    step(sets[0], 1, a)
+    a.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(5000000)
+    step(sets[0], 2, a)
+    step(sets[1], 1, b)
+    step(sets[0], 3, a)
+    step(sets[1], 2, b)
+    torch.cuda.synchronize()
+    for one, steps in zip(want, (3, 2)):
+        for t in range(steps):
+            step(one, t + 1, default)
+    torch.cuda.synchronize()
+    for got, expected in zip(sets, want):
+        for x, y in zip(got, expected):
+            assert all(torch.equal(u, v) for u, v in zip(x, y))
