@@ -102,7 +102,11 @@ constexpr uint32_t kChunks = 8;           /* contiguous ranges the block list is
  *   bf16       7.6 | 8.9  10.6 | 10.5  15.7 | 15.1   38.4 | 33.7
  *   fp32       9.0 | 10.1 14.4 | 12.8  23.9 | 20.8   53.3 | 50.3
  *   bf16, fp32 gradients, functional update
- *              8.2 | 8.9  12.5 | 10.9  17.3 | 15.1   44.0 | 35.3 */
+ *              8.2 | 8.9  12.5 | 10.9  17.3 | 15.1   44.0 | 35.3
+ * and with partial blocks of 1,027 elements behind the full ones, just past the line and further:
+ *   blocks  1,024 + 64   1,024 + 512   1,536 + 64    2,048 + 64    2,816 + 64
+ *   bf16   13.2 | 13.3   13.6 | 14.2   13.8 | 14.2   18.0 | 16.1   18.2 | 17.2
+ *   fp32   13.4 | 13.6   14.4 | 14.1   15.3 | 14.7   21.0 | 18.2   23.6 | 20.3 */
 constexpr uint32_t kSplitBlocksPerCu = 4;
 /* Tables of both parameter dtypes with at most this many blocks per compute unit in all take one launch: it saves the
  * start of a second one, and on larger tables the two kernels' code side by side costs as much.  us, two launches of a

@@ -669,6 +669,10 @@ int launch_quant_error(const DevTensor *rows, uint32_t n_rows, uint32_t total_bl
 // take a quarter block per wave (kSmallSweepBlocksPerCu): the 32-bit step over the 87 tensors of 1,280 to 2,560
 // elements of a small adapter 14.2 -> 4.1 us.  HBM-bound:
 // AdamW bf16 22 B/param (read 2+2+4+4, write 2+4+4), fp32 28 B/param; EMA 3 x element size.
+// The code for partial blocks takes the persistent kernels to 168-173 registers (32-bit step: two and three waves per
+// SIMD) and 68-96 (EMA).  With one pass of a partial block at a time they are 116-128 and 50-73 (four waves, and six
+// and eight), and that is no faster; over the same arrays, 1.31 G parameters, us as it is | so:
+//   32-bit step bf16 5,780 | 5,781, fp32 7,352 | 7,452, with masters 7,280 | 7,537; EMA bf16 1,467 | 1,467, fp32 3,103 | 3,105
 // ------------------------------------------------------------------------------------------
 
 /* crates/common/optim/src/adamw.rs:34-54, one rounded operation per line */

@@ -13,6 +13,9 @@
  * are followed in the same walk by the rows that have one.  (As a serial chain of one wave each, in front of the
  * loop, 64 element-wise trips to memory where the size is odd, they were the larger half of the launch: 64 bf16 tensors
  * of 2,048 * 4 + 1,027 elements 16.6 -> 6.9 us, fp32 17.9 -> 6.0 us.)
+ * A launch is one round of the teams up to kSplitBlocksPerCu.  The loop over rounds, with the next round's quarters
+ * requested behind the barrier and two sets of maxima in turn, serves bf16 rows with fp32 gradients under
+ * ERI_ADAM8_FLAG_BSEARCH: no other kernel has a variant for these, and they come here at any size.
  * Arithmetic, rounding and results are those of the other two kernels.
  */
 #include "eri_adam8_inline.h"
