@@ -282,7 +282,7 @@ int eri_adam8_grad_norm_scale_ptr(const EriAdam8Table *table, const float **dev_
  * of the table: the caller keeps it allocated that long (the library holds the bare address and cannot
  * tell whether it still is).  All calls on one device share the array: two such
  * calls that overlap in time on one device (different streams, different tables) race.  Nothing in
- * the array has to start at zero (every wave of a pass writes its pair before the pair is read). */
+ * the array has to start at zero (every workgroup of a pass writes its pair before the pair is read). */
 int eri_adam8_grad_norm_static(EriAdam8Table *table, float max_norm, float denom_eps, void *result, void *stream);
 /* Copies the last norm and clip factor to the host; waits for `stream`. */
 int eri_adam8_grad_norm_read(EriAdam8Table *table, float *norm, float *scale, void *stream);
