@@ -29,6 +29,9 @@ struct DevTensor {
     void *shadow;     /* EMA shadow of the parameter, or null */
 };
 static_assert(sizeof(DevTensor) == 80, "DevTensor must stay 80 bytes");
+/* In front of the rows of a launch table on the device: the counter its launches take their rounds from, zero between
+ * launches, alone in its cache line. */
+constexpr uint32_t kTableHead = 256;
 
 /* How the elements of one group of rows are stored: parameters and gradients F32, both BF16, or BF16
  * parameters with F32 gradients (the reference casts every gradient to F32 and never rounds it). */
@@ -114,10 +117,7 @@ constexpr uint32_t kSplitBlocksPerCu = 4;
  *   blocks   256         1,024       2,816       8,192       32,768
  *         14.4 | 8.4  16.6 | 10.7  23.4 | 20.6  50.0 | 46.0  160.8 | 163 */
 constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
-constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* bf16 tables take the prefetching kernel above this many full blocks
-                                                   per compute unit; up to it, sixteen waves without a prefetch are
-                                                   2-4 % faster than twelve with one (measured at 292-876 per unit,
-                                                   the other way round from 1,168) */
+constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* tables take the prefetching kernel above this many full blocks per unit */
 constexpr uint32_t kNormWaves = 4;        /* waves per workgroup of the gradient-norm pass */
 
 /* The chunked walk (BlockWalk) needs the same number of workgroups in every chunk. */
@@ -173,7 +173,7 @@ struct NormGroup {
     const DevTensor *rows;
     uint32_t n_rows, total_blocks, n_tails;
     uint32_t first_wg, wgs; // the launch's workgroups that take this group
-    uint32_t chunks;        // ranges the block list is cut into, as the step over the same group cuts it
+    uint32_t chunks;        // ranges the block list is cut into
     uint32_t grad_bf16;
 };
 struct NormGroups {

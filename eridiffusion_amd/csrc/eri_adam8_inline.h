@@ -13,8 +13,8 @@
  * p, g, m, v crosses HBM once in each direction.
  *
  * The grid is persistent: workgroups stage the lookup tables into LDS once, then their waves walk
- * the global block list -- cut into one contiguous range per accelerator die, see BlockWalk -- with
- * the stride of their die's waves, so consecutive waves touch consecutive blocks.
+ * the global block list, long lists in rounds of one block per wave that are handed out by ticket
+ * (Tickets), so consecutive waves touch consecutive blocks.
  * The tensor that owns a block is found by a scalar binary search over the launch table.
  *
  * Arithmetic: every fp32 operation of the update is written as its own statement and the file is
@@ -930,6 +930,11 @@ __device__ __forceinline__ void seek_row(const Row *rows, uint32_t n_rows, uint3
     }
 }
 
+/* The ticket counter of a launch table (kTableHead). */
+__device__ __forceinline__ uint32_t *table_ticket(const DevTensor *rows) {
+    return reinterpret_cast<uint32_t *>(reinterpret_cast<uintptr_t>(rows) - kTableHead);
+}
+
 struct BlockRowMap {
     const uint32_t *row_of; // row_of[b] = index of the row that owns full block b
     __device__ __forceinline__ BlockRowMap(const DevTensor *rows, uint32_t n_rows)
@@ -944,6 +949,35 @@ struct BlockRowMap {
     /* Row of partial block i: behind the map stands the list of the rows that have one. */
     __device__ __forceinline__ uint32_t tail_row(uint32_t total_blocks, uint32_t i) const { return row_of[total_blocks + i]; }
 };
+
+/* Rounds of blocks handed out by ticket.  Nothing bounds how far the waves of a static walk drift apart; after a few
+ * thousand blocks each they read and write all over the arrays, and what HBM then gives depends on where the arrays
+ * lie.  Here a workgroup takes one block per wave at a time, the next `waves` blocks of the list from a counter in front
+ * of the table's rows, and waits for its slowest wave in between: all workgroups stay within one window of the list.
+ * Reads and writes of a step without its arithmetic, 2.57 G bf16 parameters, arrays side by side | in 48 GiB lanes:
+ *   static walk 5.15 | 6.2 TB/s; a barrier per round alone 5.36 | 6.36; by ticket 6.3-6.6 | 6.6
+ * One address takes 80 M atomics per second: a ticket per wave was 3.4 times as slow as the static walk.
+ * The first round of a workgroup is its own number; it asks for the one after next when the one at hand begins, so the
+ * answer has a round's time to arrive.  Every round asks exactly once, so the answer rounds - 1 is the last of the
+ * launch, and whoever gets it puts the counter back to zero for the next launch on the stream. */
+struct Tickets {
+    uint32_t *counter;
+    uint32_t rounds, first; // first: rounds that are not asked for
+    __device__ __forceinline__ Tickets(const DevTensor *rows, uint32_t units, uint32_t waves)
+        : counter(table_ticket(rows)), rounds((units + waves - 1) / waves), first(gridDim.x < rounds ? gridDim.x : rounds) {}
+    __device__ __forceinline__ uint32_t ask() const { return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    /* The round that the answer stands for; `rounds` or more: none is left. */
+    __device__ __forceinline__ uint32_t round_of(uint32_t answer) const {
+        if (answer == rounds - 1) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return first + answer;
+    }
+};
+/* All waves of the workgroup are here and see each other's LDS writes; requests to memory stay in flight. */
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 
 /* The full blocks one wave walks.  Workgroup i of a launch runs on accelerator die (XCD) i mod 8.  The
  * block list is cut into `chunks` contiguous ranges and workgroup i walks range i mod chunks, so with

@@ -114,21 +114,31 @@ __global__ void state_init_kernel(uint8_t *m, uint8_t *v, float *am, float *av, 
 // ------------------------------------------------------------------------------------------
 
 /* Every full block of the table is read and written as the step kernel reads and writes it -- the launch shape
- * of the prefetching kernel (one workgroup of 768 threads per compute unit, one range of the block list per die),
+ * of the prefetching kernel (one workgroup of 512 threads per compute unit, rounds of blocks by ticket),
  * 128-bit non-temporal loads of parameters and gradients, 64-bit ones of the two code arrays, the two absmax
  * words, all of a block's loads in flight before its first store -- with no arithmetic between load and store.
  * Parameters, codes and absmax are written back with the bits they had (`zero` is 0 at run time, which the
  * compiler cannot know, so neither the loads of the gradients nor the stores fall away).  What this launch takes
  * is what the memory system gives the step's mix of four read and three written streams in the placement at
- * hand; the step kernel cannot be faster than that. */
-__global__ __launch_bounds__(768) void traffic_probe_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,
-                                                            uint32_t total_blocks, uint32_t chunks, uint32_t zero) {
+ * hand. */
+constexpr uint32_t kProbeThreads = 512;
+__global__ __launch_bounds__(kProbeThreads) void traffic_probe_kernel(const DevTensor *__restrict__ rows, uint32_t n_rows,
+                                                            uint32_t total_blocks, uint32_t zero) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const BlockWalk walk(total_blocks, chunks);
+    const uint32_t waves_per_wg = blockDim.x / kWave;
+    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const Tickets tickets(rows, total_blocks, waves_per_wg);
+    if (blockIdx.x >= tickets.rounds) return;
     const BlockRowMap map(rows, n_rows);
+    __shared__ uint32_t coming[2];
     uint32_t ti = 0, t_end = 0;
     DevTensor t;
-    for (uint32_t blk = walk.first; blk < walk.end; blk += walk.stride) {
+    uint32_t round = blockIdx.x;
+    for (uint32_t slot = 0; round < tickets.rounds; slot ^= 1) {
+        uint32_t answer = 0;
+        if (threadIdx.x == 0) answer = tickets.ask();
+        const uint32_t blk = round * waves_per_wg + wave_in_wg;
+        if (blk >= total_blocks) break; // in the last round, which is a workgroup's last
         map.seek(rows, blk, ti, t, t_end);
         const uint32_t lb = blk - t.full_start;
         const size_t e0 = (size_t)lb * kBlock;
@@ -156,12 +166,15 @@ __global__ __launch_bounds__(768) void traffic_probe_kernel(const DevTensor *__r
             as_global(t.absmax_m)[lb] = u2f(a_m ^ zero);
             as_global(t.absmax_v)[lb] = u2f(a_v ^ zero);
         }
+        if (threadIdx.x == 0) coming[slot] = tickets.round_of(answer);
+        lds_barrier();
+        round = __builtin_amdgcn_readfirstlane(coming[slot]);
     }
 }
 
 int launch_traffic_probe(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t grid, void *stream) {
-    hipLaunchKernelGGL(traffic_probe_kernel, dim3(grid), dim3(768), 0, static_cast<hipStream_t>(stream), rows, n_rows,
-                       total_blocks, chunks_for(grid), 0u);
+    hipLaunchKernelGGL(traffic_probe_kernel, dim3(grid), dim3(kProbeThreads), 0, static_cast<hipStream_t>(stream), rows, n_rows,
+                       total_blocks, 0u);
     return (int)hipGetLastError();
 }
 

