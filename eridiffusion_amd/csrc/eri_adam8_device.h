@@ -29,8 +29,8 @@ struct DevTensor {
     void *shadow;     /* EMA shadow of the parameter, or null */
 };
 static_assert(sizeof(DevTensor) == 80, "DevTensor must stay 80 bytes");
-/* In front of the rows of a launch table on the device: the counter its launches take their rounds from, zero between
- * launches, alone in its cache line. */
+/* In front of the rows of a launch table or a sweep on the device: the counter its launches take their rounds from, zero
+ * between launches, alone in its cache line. */
 constexpr uint32_t kTableHead = 256;
 
 /* How the elements of one group of rows are stored: parameters and gradients F32, both BF16, or BF16
@@ -97,7 +97,7 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_bloc
                 const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg,
                 uint32_t compute_units, void *stream);
 
-constexpr uint32_t kChunks = 8;           /* contiguous ranges the block list is cut into: one per accelerator die */
+constexpr uint32_t kChunks = 8;           /* contiguous ranges the gradient-norm pass cuts long block lists into: one per accelerator die */
 /* Tables of at most this many blocks per compute unit (partial ones counted) take the four-waves-per-block kernel: one
  * round of its four teams.  Beyond it that kernel pays a barrier and a trip to memory per round, and a wave per block
  * fills the chip by itself.  us per launch on 256 units, four waves per block | one:
@@ -120,7 +120,7 @@ constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
 constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* tables take the prefetching kernel above this many full blocks per unit */
 constexpr uint32_t kNormWaves = 4;        /* waves per workgroup of the gradient-norm pass */
 
-/* The chunked walk (BlockWalk) needs the same number of workgroups in every chunk. */
+/* Such a walk needs the same number of workgroups in every range. */
 inline uint32_t chunks_for(uint32_t grid) { return grid % kChunks == 0 ? kChunks : 1u; }
 
 /* The step's kernels live in translation units of their own (they build in parallel); launch_step
@@ -218,15 +218,16 @@ static_assert(sizeof(ElemRow) == 56, "ElemRow must stay 56 bytes");
 struct SweepUnit {
     uint32_t row, block;
 };
-/* Sweeps of at most this many blocks per compute unit take the small kernels.  us per call, a wave per block | a quarter,
- * 64 tensors, 256 units:
- *   blocks                    64          512        2,048        8,192         16,384
- *   32-bit step, bf16     6.0 | 4.0    7.1 | 5.8   19.0 | 16.0  59.7 | 59.5   118 | 112
- *   ... with masters      6.7 | 3.9    9.4 | 7.0   23.7 | 22.6  94.5 | 78.5   199 | 171
- *   ... 1,027 more each  12.4 | 4.5   14.1 | 7.2   24.6 | 18.2  60.9 | 60.1   113 | 112
- *   EMA, fp32             4.0 | 3.7    4.2 | 4.1    8.4 |  7.1  31.5 | 29.4   57.5 | 56.8
+/* Sweeps of at most this many blocks per compute unit take the small kernels, whose workgroups the hardware starts in the
+ * order of the list, many to a unit.  us per call over the same arrays, a quarter block per wave | by ticket, 256 units:
+ *   blocks                 2,048     8,192      16,824      23,639      31,398     72,781       639,470
+ *   32-bit step, bf16    16 | 24    59 | 70  119 | 137   168 | 189   236 | 269   554 | 564   5,205 | 4,791
+ *   ... fp32                                 159 | 164   229 | 226   313 | 309   749 | 673   6,692 | 5,879
+ *   ... with masters                         157 | 166   223 | 230               731 | 685   6,784 | 5,992
+ *   EMA, bf16           4.5 | 8.5   17 | 24   31 | 41     44 | 53     58 | 71    133 | 147   1,193 | 1,217
+ *   ... fp32                                  62 | 71     89 | 96    120 | 126   287 | 277   2,606 | 2,364
  * Above it the list itself (8 bytes per block, uploaded when the rows' sizes change) is no longer small. */
-constexpr uint32_t kSmallSweepBlocksPerCu = 64;
+constexpr uint32_t kSmallSweepBlocksPerCu = 128;
 
 /* units: the list of blocks, n_units of them, for the small kernels; null for the persistent ones, which take `grid`
  * workgroups.  scaled: every gradient is first multiplied by (grad_scale * row.scale) * (*dev_scale, 1 if null), as the

@@ -902,10 +902,16 @@ __device__ __forceinline__ void stage_end() {
 }
 
 /* Row owning full block `blk`: the last row whose full_start is <= blk (rows without full blocks
- * share their successor's full_start and are skipped by taking the last).  All wave-uniform. */
+ * share their successor's full_start and are skipped by taking the last).  All wave-uniform.  The rows behind `from`
+ * are tried in growing steps first: a walk that moves on finds its row near the last one. */
 template <typename Row>
 __device__ __forceinline__ uint32_t find_row(const Row *rows, uint32_t n_rows, uint32_t from, uint32_t blk) {
-    uint32_t lo = from, hi = n_rows; // rows[lo].full_start <= blk
+    uint32_t lo = from, hi = from + 1; // rows[lo].full_start <= blk
+    for (uint32_t step = 1; hi < n_rows && rows[hi].full_start <= blk; step *= 2) {
+        lo = hi;
+        hi = lo + 2 * step;
+    }
+    if (hi > n_rows) hi = n_rows;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
         if (rows[mid].full_start <= blk) lo = mid; else hi = mid;
@@ -930,8 +936,9 @@ __device__ __forceinline__ void seek_row(const Row *rows, uint32_t n_rows, uint3
     }
 }
 
-/* The ticket counter of a launch table (kTableHead). */
-__device__ __forceinline__ uint32_t *table_ticket(const DevTensor *rows) {
+/* The ticket counter of a table of rows (kTableHead). */
+template <typename Row>
+__device__ __forceinline__ uint32_t *table_ticket(const Row *rows) {
     return reinterpret_cast<uint32_t *>(reinterpret_cast<uintptr_t>(rows) - kTableHead);
 }
 
@@ -963,8 +970,10 @@ struct BlockRowMap {
 struct Tickets {
     uint32_t *counter;
     uint32_t rounds, first; // first: rounds that are not asked for
-    __device__ __forceinline__ Tickets(const DevTensor *rows, uint32_t units, uint32_t waves)
-        : counter(table_ticket(rows)), rounds((units + waves - 1) / waves), first(gridDim.x < rounds ? gridDim.x : rounds) {}
+    /* `per_round` of the list's units make a round */
+    template <typename Row>
+    __device__ __forceinline__ Tickets(const Row *rows, uint32_t units, uint32_t per_round)
+        : counter(table_ticket(rows)), rounds((units + per_round - 1) / per_round), first(gridDim.x < rounds ? gridDim.x : rounds) {}
     __device__ __forceinline__ uint32_t ask() const { return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
     /* The round that the answer stands for; `rounds` or more: none is left. */
     __device__ __forceinline__ uint32_t round_of(uint32_t answer) const {
@@ -978,24 +987,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
-
-/* The full blocks one wave walks.  Workgroup i of a launch runs on accelerator die (XCD) i mod 8.  The
- * block list is cut into `chunks` contiguous ranges and workgroup i walks range i mod chunks, so with
- * chunks == 8 each die sweeps its own part of every buffer instead of all dies advancing through one
- * common window; on MI355X that made the sweep both a little faster and much less dependent on where
- * the buffers happen to lie physically.  chunks == 1 is the plain grid-stride walk. */
-struct BlockWalk {
-    uint32_t first, end, stride;
-    __device__ __forceinline__ BlockWalk(uint32_t total_blocks, uint32_t chunks) {
-        const uint32_t waves_per_wg = blockDim.x / kWave;
-        const uint32_t per_chunk = (total_blocks + chunks - 1) / chunks;
-        const uint32_t lo = (blockIdx.x % chunks) * per_chunk;
-        end = lo + per_chunk < total_blocks ? lo + per_chunk : total_blocks;
-        stride = (gridDim.x / chunks) * waves_per_wg;
-        first = __builtin_amdgcn_readfirstlane(lo + (blockIdx.x / chunks) * waves_per_wg + threadIdx.x / kWave);
-    }
-};
-
 
 } // namespace eri
 #endif /* ERI_ADAM8_INLINE_H */

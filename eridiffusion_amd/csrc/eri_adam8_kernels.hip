@@ -676,16 +676,21 @@ int launch_quant_error(const DevTensor *rows, uint32_t n_rows, uint32_t total_bl
 }
 
 // ------------------------------------------------------------------------------------------
-// plain element-wise sweeps over a row table: 32-bit AdamW and EMA.  One wave per 2048-element
-// block, 8 elements per lane and pass, all of a block's loads in flight at once; in a partial last block the
-// lanes past the end are off and the one lane the end falls into moves its elements singly.  Sweeps of few blocks
-// take a quarter block per wave (kSmallSweepBlocksPerCu): the 32-bit step over the 87 tensors of 1,280 to 2,560
-// elements of a small adapter 14.2 -> 4.1 us.  HBM-bound:
-// AdamW bf16 22 B/param (read 2+2+4+4, write 2+4+4), fp32 28 B/param; EMA 3 x element size.
-// The code for partial blocks takes the persistent kernels to 168-173 registers (32-bit step: two and three waves per
-// SIMD) and 68-96 (EMA).  With one pass of a partial block at a time they are 116-128 and 50-73 (four waves, and six
-// and eight), and that is no faster; over the same arrays, 1.31 G parameters, us as it is | so:
-//   32-bit step bf16 5,780 | 5,781, fp32 7,352 | 7,452, with masters 7,280 | 7,537; EMA bf16 1,467 | 1,467, fp32 3,103 | 3,105
+// plain element-wise sweeps over a row table: 32-bit AdamW and EMA.  HBM-bound: AdamW bf16 22 B/param (read 2+2+4+4,
+// write 2+4+4), fp32 28 B/param; EMA 3 x element size.
+//
+// The persistent kernels run one workgroup of eight waves per compute unit and take rounds of blocks by ticket (Tickets:
+// what HBM gives depends on how close together the launch reads and writes).  A lane holds four consecutive elements per
+// pass, so that every access of either dtype is whole cache lines over the wave and nothing is read twice: streamed.
+// A round is what keeps the counter's rate low and the window narrow, about 200 KB per workgroup.  us over the same arrays
+// side by side, 1.31 G parameters: 64 waves per unit on a static walk, eight elements per lane, fp32 in two half-line
+// words | by ticket:
+//   32-bit step bf16 5,784 | 4,791 (6.0 TB/s), fp32 7,393 | 5,879 (6.2), with masters 7,322 | 5,992
+//   EMA bf16 1,470 | 1,217 (6.5), fp32 3,100 | 2,364 (6.7)
+// Traffic of the 32-bit step alone by what a round holds, 8 waves: half a block per wave 4,476, a block 4,783, two 4,817.
+// Sweeps of few blocks take a quarter block per wave (kSmallSweepBlocksPerCu): the 32-bit step over the 87 tensors of
+// 1,280 to 2,560 elements of a small adapter 14.2 -> 4.1 us with a wave per block before; whole-line words there
+// (4,678 blocks): bf16 37.6 -> 33.7, with masters 48.3 -> 42.8, EMA fp32 18.9 -> 16.8.
 // ------------------------------------------------------------------------------------------
 
 /* crates/common/optim/src/adamw.rs:34-54, one rounded operation per line */
@@ -706,135 +711,243 @@ __device__ __forceinline__ void adamw32_elem(float p, float g, float &m, float &
     pn = p + step;
 }
 
-/* Eight elements of a lane of which `count` exist; of a full block (PARTIAL false) all do. */
-template <bool BF16, bool PARTIAL>
-__device__ __forceinline__ void sweep_load(Raw8<BF16> &r, const void *base, uint32_t o, uint32_t count) {
-    if (!PARTIAL || count == 8) r.load(base, o);
-    else r.load_some(base, o, count);
-}
-template <bool BF16, bool PARTIAL>
-__device__ __forceinline__ void sweep_store(void *base, uint32_t o, const float (&x)[8], uint32_t count) {
-    if (!PARTIAL || count == 8) store8<BF16>(base, o, x);
-    else store_some<BF16>(base, o, x, count);
-}
+/* Four consecutive elements of a lane as they come from memory; `count` of them exist. */
+template <bool BF16>
+struct Raw4;
+template <>
+struct Raw4<true> {
+    u32x2 w;
+    template <bool PARTIAL>
+    __device__ __forceinline__ void load(const void *base, uint32_t elem, uint32_t count) {
+        ERI_GLOBAL const uint16_t *q = as_global(static_cast<const uint16_t *>(base) + elem);
+        if (!PARTIAL || count == 4) {
+            w = __builtin_nontemporal_load((ERI_GLOBAL const u32x2 *)q);
+            return;
+        }
+        uint32_t x[3] = {0, 0, 0};
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+            if (k < count) x[k] = q[k];
+        w = u32x2{x[0] | x[1] << 16, x[2]};
+    }
+    __device__ __forceinline__ f32x4 unpack() const { return f32x4{bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y)}; }
+    template <bool PARTIAL>
+    static __device__ __forceinline__ void store(void *base, uint32_t elem, const f32x4 &v, uint32_t count) {
+        ERI_GLOBAL uint16_t *q = as_global(static_cast<uint16_t *>(base) + elem);
+        if (!PARTIAL || count == 4) {
+            __builtin_nontemporal_store(u32x2{bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)}, (ERI_GLOBAL u32x2 *)q);
+            return;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+            if (k < count) q[k] = (uint16_t)bf16_bits(v[k]);
+    }
+};
+template <>
+struct Raw4<false> {
+    f32x4 w;
+    template <bool PARTIAL>
+    __device__ __forceinline__ void load(const void *base, uint32_t elem, uint32_t count) {
+        ERI_GLOBAL const float *q = as_global(static_cast<const float *>(base) + elem);
+        if (!PARTIAL || count == 4) {
+            w = __builtin_nontemporal_load((ERI_GLOBAL const f32x4 *)q);
+            return;
+        }
+        w = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+            if (k < count) w[k] = q[k];
+    }
+    __device__ __forceinline__ f32x4 unpack() const { return w; }
+    template <bool PARTIAL>
+    static __device__ __forceinline__ void store(void *base, uint32_t elem, const f32x4 &v, uint32_t count) {
+        ERI_GLOBAL float *q = as_global(static_cast<float *>(base) + elem);
+        if (!PARTIAL || count == 4) {
+            __builtin_nontemporal_store(v, (ERI_GLOBAL f32x4 *)q);
+            return;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+            if (k < count) q[k] = v[k];
+    }
+};
 
-/* One block of the 32-bit step, of n elements.  MASTER: the parameter value comes from, and goes back to, an fp32
- * master copy; the tensor itself only receives the rounded result (mixed precision,
- * src/kernels/fused_adam.cu:151-193, with the arithmetic of adamw.rs). */
-template <bool BF16, bool MASTER, bool GS, bool PARTIAL>
-__device__ __forceinline__ void adamw32_block(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, const EriAdamW32Hyper &h,
-                                              float omb1, float omb2, float neg_lr, float gscale) {
-    char *p = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
-    const char *g = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
-    float *m = static_cast<float *>(t.c) + e0;
-    float *v = static_cast<float *>(t.d) + e0;
-    float *w = MASTER ? static_cast<float *>(t.e) + e0 : nullptr;
-    Raw8<BF16> pr[4], gr[4];
-    Raw8<false> mr[4], vr[4], wr[4];
+constexpr uint32_t kSweepThreads = 512;
+constexpr uint32_t kPass = 4 * kWave; // elements of a wave's pass
+/* Of the four elements of a lane that begin at o, how many exist in a piece of n. */
+__device__ __forceinline__ uint32_t lane_count4(uint32_t o, uint32_t n) { return o + 4 <= n ? 4u : o < n ? n - o : 0u; }
+
+/* Up to PASSES * kPass elements of one tensor from e0 on, n of them; PARTIAL: fewer than that.  Requested whole, then
+ * worked off, so that the caller can look up its next row in between. */
+template <bool BF16, bool MASTER, bool GS, int PASSES, bool PARTIAL>
+struct AdamW32Piece {
+    Raw4<BF16> pr[PASSES], gr[PASSES];
+    Raw4<false> mr[PASSES], vr[PASSES], wr[PASSES];
+    __device__ __forceinline__ void request(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane) {
+        const char *p = static_cast<const char *>(t.a) + e0 * (BF16 ? 2 : 4), *g = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
+        const float *m = static_cast<const float *>(t.c) + e0, *v = static_cast<const float *>(t.d) + e0, *w = static_cast<const float *>(t.e) + (MASTER ? e0 : 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        const uint32_t count = lane_count(o, n);
-        if (MASTER) sweep_load<false, PARTIAL>(wr[c], w, o, count);
-        else sweep_load<BF16, PARTIAL>(pr[c], p, o, count);
-        sweep_load<BF16, PARTIAL>(gr[c], g, o, count);
-        sweep_load<false, PARTIAL>(mr[c], m, o, count);
-        sweep_load<false, PARTIAL>(vr[c], v, o, count);
+        for (int c = 0; c < PASSES; ++c) {
+            const uint32_t o = c * kPass + lane * 4, count = lane_count4(o, n);
+            if (MASTER) wr[c].template load<PARTIAL>(w, o, count);
+            else pr[c].template load<PARTIAL>(p, o, count);
+            gr[c].template load<PARTIAL>(g, o, count);
+            mr[c].template load<PARTIAL>(m, o, count);
+            vr[c].template load<PARTIAL>(v, o, count);
+        }
     }
+    /* MASTER: the parameter value comes from, and goes back to, an fp32 master copy; the tensor itself only receives the
+     * rounded result (mixed precision, src/kernels/fused_adam.cu:151-193, with the arithmetic of adamw.rs). */
+    __device__ __forceinline__ void step(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, const EriAdamW32Hyper &h, float omb1,
+                                         float omb2, float neg_lr, float gscale) {
+        char *p = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
+        float *m = static_cast<float *>(t.c) + e0, *v = static_cast<float *>(t.d) + e0, *w = static_cast<float *>(t.e) + (MASTER ? e0 : 0);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        float pv[8], gv[8], mv[8], vv[8], pn[8];
-        if (MASTER) wr[c].unpack(pv);
-        else pr[c].unpack(pv);
-        gr[c].unpack(gv);
-        mr[c].unpack(mv);
-        vr[c].unpack(vv);
+        for (int c = 0; c < PASSES; ++c) {
+            const uint32_t o = c * kPass + lane * 4, count = lane_count4(o, n);
+            const f32x4 pv = MASTER ? wr[c].unpack() : pr[c].unpack(), gv = gr[c].unpack();
+            f32x4 mv = mr[c].unpack(), vv = vr[c].unpack(), pn;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) adamw32_elem(pv[k], GS ? gv[k] * gscale : gv[k], mv[k], vv[k], h, omb1, omb2, neg_lr, pn[k]);
-        const uint32_t count = lane_count(o, n);
-        sweep_store<BF16, PARTIAL>(p, o, pn, count);
-        if (MASTER) sweep_store<false, PARTIAL>(w, o, pn, count);
-        sweep_store<false, PARTIAL>(m, o, mv, count);
-        sweep_store<false, PARTIAL>(v, o, vv, count);
+            for (int k = 0; k < 4; ++k) {
+                float a = mv[k], b = vv[k], x;
+                adamw32_elem(pv[k], GS ? gv[k] * gscale : gv[k], a, b, h, omb1, omb2, neg_lr, x);
+                mv[k] = a;
+                vv[k] = b;
+                pn[k] = x;
+            }
+            Raw4<BF16>::template store<PARTIAL>(p, o, pn, count);
+            if (MASTER) Raw4<false>::template store<PARTIAL>(w, o, pn, count);
+            Raw4<false>::template store<PARTIAL>(m, o, mv, count);
+            Raw4<false>::template store<PARTIAL>(v, o, vv, count);
+        }
     }
-}
+};
 
 /* A workgroup of the small sweeps: one block, partial or not, a quarter of it per wave (nothing crosses lanes here).
  * The list of blocks rides behind the rows, so a wave finds its row with one load instead of a search. */
 struct SweepQuarter {
     ElemRow t;
     size_t e0;
-    uint32_t o, count; // this lane's eight elements and how many of them exist
-    __device__ __forceinline__ SweepQuarter(const ElemRow *rows, const SweepUnit &u)
-        : t(rows[u.row]), e0((size_t)u.block * kBlock), o(threadIdx.x * 8), count(t.numel - e0 >= kBlock ? 8u : lane_count(o, (uint32_t)(t.numel - e0))) {}
+    uint32_t n; // elements of the quarter that exist
+    __device__ __forceinline__ SweepQuarter(const ElemRow *rows, const SweepUnit &u) : t(rows[u.row]) {
+        constexpr uint32_t kQuarter = kBlock / 4;
+        const uint32_t from = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * kQuarter;
+        const size_t b0 = (size_t)u.block * kBlock;
+        const uint32_t here = t.numel - b0 >= kBlock ? kBlock : (uint32_t)(t.numel - b0);
+        e0 = b0 + from;
+        n = here <= from ? 0u : here - from < kQuarter ? here - from : kQuarter;
+    }
+    static constexpr int kPasses = kBlock / 4 / kPass;
+    __device__ __forceinline__ bool whole() const { return n == kBlock / 4; }
 };
+
+template <bool BF16, bool MASTER, bool GS, bool PARTIAL>
+__device__ __forceinline__ void adamw32_quarter(const SweepQuarter &q, uint32_t lane, const EriAdamW32Hyper &h, float omb1, float omb2,
+                                                float neg_lr, float gscale) {
+    AdamW32Piece<BF16, MASTER, GS, SweepQuarter::kPasses, PARTIAL> x;
+    x.request(q.t, q.e0, q.n, lane);
+    x.step(q.t, q.e0, q.n, lane, h, omb1, omb2, neg_lr, gscale);
+}
 
 template <bool BF16, bool GS>
 __global__ __launch_bounds__(256) void adamw32_small_kernel(const ElemRow *__restrict__ rows, const SweepUnit *__restrict__ units,
-                                                            uint32_t n_units, EriAdamW32Hyper h, float grad_scale,
+                                                            EriAdamW32Hyper h, float grad_scale,
                                                             const float *__restrict__ dev_scale) {
     const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
     const float omb1 = 1.0f - h.beta1, omb2 = 1.0f - h.beta2, neg_lr = -h.lr; // adamw.rs:36,42,53
-    for (uint32_t i = blockIdx.x; i < n_units; i += gridDim.x) {
-        const SweepQuarter q(rows, units[i]);
-        if (q.count == 0) continue;
-        char *p = static_cast<char *>(q.t.a) + q.e0 * (BF16 ? 2 : 4);
-        float *m = static_cast<float *>(q.t.c) + q.e0, *v = static_cast<float *>(q.t.d) + q.e0;
-        float *w = q.t.e ? static_cast<float *>(q.t.e) + q.e0 : nullptr; // fp32 master copy
-        Raw8<BF16> pr, gr;
-        Raw8<false> mr, vr, wr;
-        if (w) sweep_load<false, true>(wr, w, q.o, q.count);
-        else sweep_load<BF16, true>(pr, p, q.o, q.count);
-        sweep_load<BF16, true>(gr, static_cast<const char *>(q.t.b) + q.e0 * (BF16 ? 2 : 4), q.o, q.count);
-        sweep_load<false, true>(mr, m, q.o, q.count);
-        sweep_load<false, true>(vr, v, q.o, q.count);
-        const float gscale = GS ? (grad_scale * q.t.scale) * tscale : 1.0f;
-        float pv[8], gv[8], mv[8], vv[8], pn[8];
-        if (w) wr.unpack(pv);
-        else pr.unpack(pv);
-        gr.unpack(gv);
-        mr.unpack(mv);
-        vr.unpack(vv);
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const SweepQuarter q(rows, units[blockIdx.x]);
+    if (q.n == 0) return;
+    const float gscale = GS ? (grad_scale * q.t.scale) * tscale : 1.0f;
+    if (q.t.e) {
+        if (q.whole()) adamw32_quarter<BF16, true, GS, false>(q, lane, h, omb1, omb2, neg_lr, gscale);
+        else adamw32_quarter<BF16, true, GS, true>(q, lane, h, omb1, omb2, neg_lr, gscale);
+    } else {
+        if (q.whole()) adamw32_quarter<BF16, false, GS, false>(q, lane, h, omb1, omb2, neg_lr, gscale);
+        else adamw32_quarter<BF16, false, GS, true>(q, lane, h, omb1, omb2, neg_lr, gscale);
+    }
+}
+
+/* A wave's way through a list of `units`, SUB of them per wave and round, `per_block` units to a block: at(row, unit,
+ * ahead) is called for each with the row that owns its block, and calls ahead() once its loads are on the way, which
+ * looks up the row of the unit after it. */
+template <uint32_t SUB, uint32_t PER_BLOCK, typename At>
+__device__ __forceinline__ void sweep_by_ticket(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t *coming, At at) {
+    const uint32_t units = total_blocks * PER_BLOCK, waves = blockDim.x / kWave;
+    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const Tickets tickets(rows, units, waves * SUB);
+    uint32_t round = blockIdx.x;
+    if (round >= tickets.rounds) return;
+    if (threadIdx.x == 0) coming[0] = tickets.round_of(tickets.ask());
+    auto unit_of = [&](uint32_t r, uint32_t sub) { return (r * SUB + sub) * waves + wave_in_wg; };
+    uint32_t ti = 0, t_end = 0;
+    ElemRow t;
+    if (unit_of(round, 0) < units) seek_row(rows, n_rows, unit_of(round, 0) / PER_BLOCK, ti, t, t_end);
+    lds_barrier();
+    uint32_t next = __builtin_amdgcn_readfirstlane(coming[0]);
+    for (uint32_t slot = 1;; slot ^= 1) {
+        const bool more = next < tickets.rounds;
+        uint32_t answer = 0;
+        if (more && threadIdx.x == 0) answer = tickets.ask(); // for the round after next
 #pragma unroll
-        for (int k = 0; k < 8; ++k) adamw32_elem(pv[k], GS ? gv[k] * gscale : gv[k], mv[k], vv[k], h, omb1, omb2, neg_lr, pn[k]);
-        sweep_store<BF16, true>(p, q.o, pn, q.count);
-        if (w) sweep_store<false, true>(w, q.o, pn, q.count);
-        sweep_store<false, true>(m, q.o, mv, q.count);
-        sweep_store<false, true>(v, q.o, vv, q.count);
+        for (uint32_t sub = 0; sub < SUB; ++sub) {
+            const uint32_t unit = unit_of(round, sub);
+            if (unit >= units) break; // in the last round
+            const uint32_t then = sub + 1 < SUB ? unit + waves : more ? unit_of(next, 0) : units;
+            const ElemRow here = t;
+            at(here, unit, [&] { if (then < units) seek_row(rows, n_rows, then / PER_BLOCK, ti, t, t_end); });
+        }
+        if (!more) break;
+        if (threadIdx.x == 0) coming[slot] = tickets.round_of(answer);
+        lds_barrier();
+        round = next;
+        next = __builtin_amdgcn_readfirstlane(coming[slot]);
     }
 }
 
 template <bool BF16, bool GS>
-__global__ __launch_bounds__(256) void adamw32_kernel(const ElemRow *__restrict__ rows, uint32_t n_rows,
-                                                      uint32_t total_blocks, EriAdamW32Hyper h, float grad_scale,
-                                                      const float *__restrict__ dev_scale, uint32_t chunks) {
+__global__ __launch_bounds__(kSweepThreads) void adamw32_kernel(const ElemRow *__restrict__ rows, uint32_t n_rows,
+                                                                uint32_t total_blocks, EriAdamW32Hyper h, float grad_scale,
+                                                                const float *__restrict__ dev_scale) {
+    constexpr int kPasses = 4; // half a block per wave
+    constexpr uint32_t kPiece = kPasses * kPass;
+    __shared__ uint32_t coming[2];
     // the clip factor left on the device by the gradient-norm pass (1.0 when there is none)
     const float tscale = (GS && dev_scale) ? *dev_scale : 1.0f;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t waves_per_wg = blockDim.x / kWave;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
-    const uint32_t stride = gridDim.x * waves_per_wg;
     const float omb1 = 1.0f - h.beta1, omb2 = 1.0f - h.beta2, neg_lr = -h.lr; // adamw.rs:36,42,53
-    for (uint32_t r = wave; r < n_rows; r += stride) {
-        const ElemRow t = rows[r];
-        const uint32_t n = (uint32_t)(t.numel % kBlock);
-        if (n == 0) continue;
-        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
-        const float gscale = GS ? (grad_scale * t.scale) * tscale : 1.0f; // the order of the 8-bit step's factors
-        if (t.e) adamw32_block<BF16, true, GS, true>(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale);
-        else adamw32_block<BF16, false, GS, true>(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale);
+    auto gscale_of = [&](const ElemRow &t) { return GS ? (grad_scale * t.scale) * tscale : 1.0f; }; // the order of the 8-bit step's factors
+    const uint32_t waves = blockDim.x / kWave;
+    for (uint32_t i = __builtin_amdgcn_readfirstlane(blockIdx.x * waves + threadIdx.x / kWave); i < 2 * n_rows; i += gridDim.x * waves) {
+        const ElemRow t = rows[i / 2];
+        const uint32_t tail = (uint32_t)(t.numel % kBlock), from = (i & 1) * kPiece;
+        if (tail <= from) continue;
+        const uint32_t n = tail - from < kPiece ? tail - from : kPiece;
+        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock + from;
+        if (t.e) {
+            AdamW32Piece<BF16, true, GS, kPasses, true> x;
+            x.request(t, e0, n, lane);
+            x.step(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale_of(t));
+        } else {
+            AdamW32Piece<BF16, false, GS, kPasses, true> x;
+            x.request(t, e0, n, lane);
+            x.step(t, e0, n, lane, h, omb1, omb2, neg_lr, gscale_of(t));
+        }
     }
-    uint32_t ti = 0, t_end = 0;
-    ElemRow t;
-    const BlockWalk walk(total_blocks, chunks);
-    for (uint32_t blk = walk.first; blk < walk.end; blk += walk.stride) {
-        seek_row(rows, n_rows, blk, ti, t, t_end);
-        const size_t e0 = (size_t)(blk - t.full_start) * kBlock;
-        const float gscale = GS ? (grad_scale * t.scale) * tscale : 1.0f;
-        if (t.e) adamw32_block<BF16, true, GS, false>(t, e0, kBlock, lane, h, omb1, omb2, neg_lr, gscale);
-        else adamw32_block<BF16, false, GS, false>(t, e0, kBlock, lane, h, omb1, omb2, neg_lr, gscale);
-    }
+    sweep_by_ticket<1, 2>(rows, n_rows, total_blocks, coming, [&](const ElemRow &t, uint32_t unit, auto ahead) {
+        const size_t e0 = (size_t)(unit / 2 - t.full_start) * kBlock + (unit & 1) * kPiece;
+        if (t.e) {
+            AdamW32Piece<BF16, true, GS, kPasses, false> x;
+            x.request(t, e0, kPiece, lane);
+            ahead();
+            x.step(t, e0, kPiece, lane, h, omb1, omb2, neg_lr, gscale_of(t));
+        } else {
+            AdamW32Piece<BF16, false, GS, kPasses, false> x;
+            x.request(t, e0, kPiece, lane);
+            ahead();
+            x.step(t, e0, kPiece, lane, h, omb1, omb2, neg_lr, gscale_of(t));
+        }
+    });
 }
 
 /* src/trainers/ema_enhanced.rs:91-100 */
@@ -844,70 +957,74 @@ __device__ __forceinline__ float ema_elem(float shadow, float p, float decay, fl
     return a + b;
 }
 
+/* Up to PASSES * kPass elements from e0 on, requested whole. */
+template <bool BF16, int PASSES, bool PARTIAL>
+struct EmaPiece {
+    static constexpr int kPasses = PASSES;
+    Raw4<BF16> sr[kPasses], pr[kPasses];
+    __device__ __forceinline__ void request(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane) {
+        const char *s = static_cast<const char *>(t.a) + e0 * (BF16 ? 2 : 4), *p = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
+#pragma unroll
+        for (int c = 0; c < kPasses; ++c) {
+            const uint32_t o = c * kPass + lane * 4, count = lane_count4(o, n);
+            sr[c].template load<PARTIAL>(s, o, count);
+            pr[c].template load<PARTIAL>(p, o, count);
+        }
+    }
+    __device__ __forceinline__ void update(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, float decay, float omd) {
+        char *s = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
+#pragma unroll
+        for (int c = 0; c < kPasses; ++c) {
+            const uint32_t o = c * kPass + lane * 4;
+            const f32x4 sv = sr[c].unpack(), pv = pr[c].unpack();
+            f32x4 out;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
+            Raw4<BF16>::template store<PARTIAL>(s, o, out, lane_count4(o, n));
+        }
+    }
+};
+
 template <bool BF16, bool PARTIAL>
-__device__ __forceinline__ void ema_block(const ElemRow &t, size_t e0, uint32_t n, uint32_t lane, float decay, float omd) {
-    char *s = static_cast<char *>(t.a) + e0 * (BF16 ? 2 : 4);
-    const char *p = static_cast<const char *>(t.b) + e0 * (BF16 ? 2 : 4);
-    Raw8<BF16> sr[4], pr[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        sweep_load<BF16, PARTIAL>(sr[c], s, o, lane_count(o, n));
-        sweep_load<BF16, PARTIAL>(pr[c], p, o, lane_count(o, n));
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        float sv[8], pv[8], out[8];
-        sr[c].unpack(sv);
-        pr[c].unpack(pv);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
-        sweep_store<BF16, PARTIAL>(s, o, out, lane_count(o, n));
-    }
+__device__ __forceinline__ void ema_quarter(const SweepQuarter &q, uint32_t lane, float decay, float omd) {
+    EmaPiece<BF16, SweepQuarter::kPasses, PARTIAL> x;
+    x.request(q.t, q.e0, q.n, lane);
+    x.update(q.t, q.e0, q.n, lane, decay, omd);
 }
 
 template <bool BF16>
 __global__ __launch_bounds__(256) void ema_small_kernel(const ElemRow *__restrict__ rows, const SweepUnit *__restrict__ units,
-                                                        uint32_t n_units, float decay) {
+                                                        float decay) {
     const float omd = 1.0f - decay; // ema_enhanced.rs:96
-    for (uint32_t i = blockIdx.x; i < n_units; i += gridDim.x) {
-        const SweepQuarter q(rows, units[i]);
-        if (q.count == 0) continue;
-        char *s = static_cast<char *>(q.t.a) + q.e0 * (BF16 ? 2 : 4);
-        Raw8<BF16> sr, pr;
-        sweep_load<BF16, true>(sr, s, q.o, q.count);
-        sweep_load<BF16, true>(pr, static_cast<const char *>(q.t.b) + q.e0 * (BF16 ? 2 : 4), q.o, q.count);
-        float sv[8], pv[8], out[8];
-        sr.unpack(sv);
-        pr.unpack(pv);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) out[k] = ema_elem(sv[k], pv[k], decay, omd);
-        sweep_store<BF16, true>(s, q.o, out, q.count);
-    }
+    const SweepQuarter q(rows, units[blockIdx.x]);
+    if (q.n == 0) return;
+    if (q.whole()) ema_quarter<BF16, false>(q, threadIdx.x & (kWave - 1), decay, omd);
+    else ema_quarter<BF16, true>(q, threadIdx.x & (kWave - 1), decay, omd);
 }
 
 template <bool BF16>
-__global__ __launch_bounds__(256) void ema_kernel(const ElemRow *__restrict__ rows, uint32_t n_rows,
-                                                  uint32_t total_blocks, float decay, uint32_t chunks) {
+__global__ __launch_bounds__(kSweepThreads) void ema_kernel(const ElemRow *__restrict__ rows, uint32_t n_rows,
+                                                            uint32_t total_blocks, float decay) {
+    __shared__ uint32_t coming[2];
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t waves_per_wg = blockDim.x / kWave;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
-    const uint32_t stride = gridDim.x * waves_per_wg;
     const float omd = 1.0f - decay; // ema_enhanced.rs:96
-    for (uint32_t r = wave; r < n_rows; r += stride) {
+    const uint32_t waves = blockDim.x / kWave;
+    for (uint32_t r = __builtin_amdgcn_readfirstlane(blockIdx.x * waves + threadIdx.x / kWave); r < n_rows; r += gridDim.x * waves) {
         const ElemRow t = rows[r];
         const uint32_t n = (uint32_t)(t.numel % kBlock);
-        if (n != 0) ema_block<BF16, true>(t, (size_t)(t.numel / kBlock) * kBlock, n, lane, decay, omd);
+        if (n == 0) continue;
+        const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
+        EmaPiece<BF16, kBlock / kPass, true> x;
+        x.request(t, e0, n, lane);
+        x.update(t, e0, n, lane, decay, omd);
     }
-    uint32_t ti = 0, t_end = 0;
-    ElemRow t;
-    const BlockWalk walk(total_blocks, chunks);
-    for (uint32_t blk = walk.first; blk < walk.end; blk += walk.stride) {
-        seek_row(rows, n_rows, blk, ti, t, t_end);
+    sweep_by_ticket<BF16 ? 2 : 1, 1>(rows, n_rows, total_blocks, coming, [&](const ElemRow &t, uint32_t blk, auto ahead) {
         const size_t e0 = (size_t)(blk - t.full_start) * kBlock;
-        ema_block<BF16, false>(t, e0, kBlock, lane, decay, omd);
-    }
+        EmaPiece<BF16, kBlock / kPass, false> x;
+        x.request(t, e0, kBlock, lane);
+        ahead();
+        x.update(t, e0, kBlock, lane, decay, omd);
+    });
 }
 
 int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, const SweepUnit *units, uint32_t n_units,
@@ -917,11 +1034,10 @@ int launch_adamw32(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, 
 #define ERI_GO(B, G)                                                                                                     \
     do {                                                                                                                 \
         if (units)                                                                                                       \
-            hipLaunchKernelGGL((adamw32_small_kernel<B, G>), dim3(n_units), dim3(256), 0, s, rows, units, n_units, h,     \
-                               grad_scale, dev_scale);                                                                   \
+            hipLaunchKernelGGL((adamw32_small_kernel<B, G>), dim3(n_units), dim3(256), 0, s, rows, units, h, grad_scale, dev_scale); \
         else                                                                                                             \
-            hipLaunchKernelGGL((adamw32_kernel<B, G>), dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, h,        \
-                               grad_scale, dev_scale, chunks_for(grid));                                                 \
+            hipLaunchKernelGGL((adamw32_kernel<B, G>), dim3(grid), dim3(kSweepThreads), 0, s, rows, n_rows, total_blocks, h, \
+                               grad_scale, dev_scale);                                                                   \
     } while (0)
     if (dtype_tag == ERI_DTYPE_F32) {
         if (scaled) ERI_GO(false, true);
@@ -938,13 +1054,13 @@ int launch_ema(const ElemRow *rows, uint32_t n_rows, uint32_t total_blocks, cons
                int dtype_tag, float decay, uint32_t grid, void *stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (units && dtype_tag == ERI_DTYPE_F32)
-        hipLaunchKernelGGL(ema_small_kernel<false>, dim3(n_units), dim3(256), 0, s, rows, units, n_units, decay);
+        hipLaunchKernelGGL(ema_small_kernel<false>, dim3(n_units), dim3(256), 0, s, rows, units, decay);
     else if (units)
-        hipLaunchKernelGGL(ema_small_kernel<true>, dim3(n_units), dim3(256), 0, s, rows, units, n_units, decay);
+        hipLaunchKernelGGL(ema_small_kernel<true>, dim3(n_units), dim3(256), 0, s, rows, units, decay);
     else if (dtype_tag == ERI_DTYPE_F32)
-        hipLaunchKernelGGL(ema_kernel<false>, dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, decay, chunks_for(grid));
+        hipLaunchKernelGGL(ema_kernel<false>, dim3(grid), dim3(kSweepThreads), 0, s, rows, n_rows, total_blocks, decay);
     else
-        hipLaunchKernelGGL(ema_kernel<true>, dim3(grid), dim3(256), 0, s, rows, n_rows, total_blocks, decay, chunks_for(grid));
+        hipLaunchKernelGGL(ema_kernel<true>, dim3(grid), dim3(kSweepThreads), 0, s, rows, n_rows, total_blocks, decay);
     return (int)hipGetLastError();
 }
 

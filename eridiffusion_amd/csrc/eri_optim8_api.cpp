@@ -1436,10 +1436,19 @@ namespace {
  * its place after the kernels that other streams have queued on it. */
 struct ElemCache {
     struct Group {
-        eri::ElemRow *dev = nullptr, *pinned = nullptr; // n rows, then the list of n_units blocks of a small sweep
-        size_t cap = 0;                                 // bytes
+        // kTableHead bytes, then n rows, then the list of n_units blocks of a small sweep; dev and pinned are the rows'
+        char *mem = nullptr, *mirror = nullptr;
+        eri::ElemRow *dev = nullptr, *pinned = nullptr;
+        size_t cap = 0; // bytes
         uint32_t n = 0, n_units = 0;
         uint32_t listed = 0;                            // rows in the mirror whose list is on the device, 0 if it may not be
+        void release() {
+            if (mem) (void)hipFree(mem);
+            if (mirror) (void)hipHostFree(mirror);
+            mem = mirror = nullptr;
+            dev = pinned = nullptr;
+            cap = 0;
+        }
     };
     struct Slot {
         Group groups[2]; // F32, BF16
@@ -1452,10 +1461,7 @@ struct ElemCache {
             if (pending && ev) (void)hipEventSynchronize(ev);
             pending = false;
             for (auto &g : groups) {
-                if (g.dev) (void)hipFree(g.dev);
-                if (g.pinned) (void)hipHostFree(g.pinned);
-                g.dev = g.pinned = nullptr;
-                g.cap = 0;
+                g.release();
                 g.n = g.n_units = g.listed = 0;
             }
             if (ev) (void)hipEventDestroy(ev);
@@ -1529,16 +1535,16 @@ struct ElemCache {
                 bool keep_list = small && !capturing && g.listed == n;
                 for (uint32_t j = 0; keep_list && j < n; ++j) keep_list = g.pinned[j].numel == rows[gi][j].numel;
                 g.n_units = small ? (uint32_t)units : 0;
-                const size_t bytes = sizeof(eri::ElemRow) * n + sizeof(eri::SweepUnit) * g.n_units;
+                const size_t rows_bytes = eri::kTableHead + sizeof(eri::ElemRow) * n, bytes = rows_bytes + sizeof(eri::SweepUnit) * g.n_units;
                 if (!keep_list) g.listed = 0;
                 if (g.cap < bytes) {
-                    if (g.dev) (void)hipFree(g.dev);
-                    if (g.pinned) (void)hipHostFree(g.pinned);
-                    g.dev = g.pinned = nullptr;
-                    g.cap = 0; // stays 0 if an allocation below fails: the next call starts over
+                    g.release(); // the capacity stays 0 if an allocation below fails: the next call starts over
                     const size_t cap = bytes + bytes / 2 + 1024;
-                    ERI_HIP(hipMalloc((void **)&g.dev, cap));
-                    ERI_HIP(hipHostMalloc((void **)&g.pinned, cap, hipHostMallocDefault));
+                    ERI_HIP(hipMalloc((void **)&g.mem, cap));
+                    ERI_HIP(hipHostMalloc((void **)&g.mirror, cap, hipHostMallocDefault));
+                    std::memset(g.mirror, 0, eri::kTableHead); // every upload sets the counter to zero
+                    g.dev = reinterpret_cast<eri::ElemRow *>(g.mem + eri::kTableHead);
+                    g.pinned = reinterpret_cast<eri::ElemRow *>(g.mirror + eri::kTableHead);
                     g.cap = cap;
                 }
                 std::memcpy(g.pinned, rows[gi].data(), n * sizeof(eri::ElemRow));
@@ -1547,7 +1553,7 @@ struct ElemCache {
                     for (uint32_t j = 0; j < n; ++j)
                         for (uint32_t b = 0, end = (uint32_t)blocks_of(rows[gi][j].numel); b < end; ++b) *u++ = {j, b};
                 }
-                ERI_HIP(hipMemcpyAsync(g.dev, g.pinned, keep_list ? sizeof(eri::ElemRow) * n : bytes, hipMemcpyHostToDevice,
+                ERI_HIP(hipMemcpyAsync(g.mem, g.mirror, keep_list ? rows_bytes : bytes, hipMemcpyHostToDevice,
                                        static_cast<hipStream_t>(stream)));
                 g.n = n;
                 if (small && !capturing) g.listed = n;
@@ -1565,9 +1571,8 @@ struct ElemCache {
             if (n == 0) continue;
             const eri::ElemRow &last = rows[gi].back();
             const uint32_t total = last.full_start + (uint32_t)(last.numel / eri::kBlock);
-            const uint32_t work = total > n ? total : n;
-            uint32_t grid = (work + 3) / 4;
-            if (grid > cus * 16) grid = cus * 16;
+            uint32_t grid = total > n ? total : n; // of the persistent kernels: a workgroup per unit
+            if (grid > cus) grid = cus;
             const eri::SweepUnit *units = g.n_units ? reinterpret_cast<const eri::SweepUnit *>(g.dev + n) : nullptr;
             const int rc = launch(g.dev, n, total, units, g.n_units, gi == 0 ? ERI_DTYPE_F32 : ERI_DTYPE_BF16, grid, stream, extra);
             if (rc) return hip_fail((hipError_t)rc, "element-wise sweep launch");

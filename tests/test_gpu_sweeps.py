@@ -267,7 +267,7 @@ def test_traffic_probe_moves_the_bytes_and_changes_none():
 
 
 @pytest.mark.parametrize("bf16", [True, False])
-@pytest.mark.parametrize("more", [0, 64 * 256 * 2048], ids=["small-kernels", "persistent-kernels"])
+@pytest.mark.parametrize("more", [0, 64 * 256 * 2048, 128 * 256 * 2048], ids=["small-kernels", "long-list", "persistent-kernels"])
 def test_partial_blocks_of_every_shape(bf16, more):
     """Last blocks that end inside a lane's eight elements, on a lane's edge and one short of a block, in the 32-bit step
     (every other row with a master copy where there is one) and the EMA sweep; nothing is written past a tensor."""

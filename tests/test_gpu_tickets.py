@@ -31,3 +31,44 @@ def test_step_by_ticket(bf16, blocks):
     got_p, got_st = gt.fetch()
     assert hs.compare(got_p, got_st, ps, states, bf16, True, "blocks %d" % blocks)["code_mismatch"] == 0
     L.lib().eri_adam8_table_destroy(table)
+
+
+@pytest.mark.parametrize("dtype,master", [("bf16", False), ("bf16", True), ("f32", False)])
+@pytest.mark.parametrize("extra", [1, 5, 4 * UNITS + 3])
+def test_sweeps_by_ticket(dtype, master, extra):
+    """The 32-bit step and the EMA over lists just longer than the small kernels take, against the small kernels over the
+    same rows in two calls, bit for bit; twice, so that the counter has been put back once."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    line = 128 * UNITS
+    halves = [[(line // 2 + extra) * 2048 + 1500, 700, 2048 * 2 + 3], [(line // 2) * 2048 - 2048 * 3 + 1027]]
+    sizes = halves[0] + halves[1]
+    dt, tag = (torch.bfloat16, L.DTYPE_BF16) if dtype == "bf16" else (torch.float32, L.DTYPE_F32)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(groups):
+        gen = torch.Generator(device="cuda").manual_seed(extra)
+        at, total = [], 0
+        for n in sizes:
+            at.append(total)
+            total += (n + 15) // 16 * 16
+        p, g = [(torch.randn(total, device="cuda", generator=gen) * s).to(dt) for s in (0.02, 1e-3)]
+        m, v = torch.randn(total, device="cuda", generator=gen) * 1e-3, torch.rand(total, device="cuda", generator=gen) * 1e-6
+        w, shadow = p.float() * 1.0001, p * 0.5
+        for _ in range(2):
+            for ids in groups:
+                rows, ema = (L.AdamW32Row * len(ids))(), (L.EmaRow * len(ids))()
+                for r, e, i in zip(rows, ema, ids):
+                    o = at[i]
+                    r.p, r.g, r.m, r.v = p[o:].data_ptr(), g[o:].data_ptr(), m[o:].data_ptr(), v[o:].data_ptr()
+                    r.master = w[o:].data_ptr() if master else None
+                    r.numel, r.dtype_tag = sizes[i], tag
+                    e.shadow, e.p, e.numel, e.dtype_tag = shadow[o:].data_ptr(), p[o:].data_ptr(), sizes[i], tag
+                h = L.AdamW32Hyper(1e-3, 0.9, 0.999, 1e-8, 0.01)
+                L.check(L.lib().eri_adamw32_step_multi(rows, len(ids), C.byref(h), stream), "adamw32")
+                L.check(L.lib().eri_ema_update_multi(ema, len(ids), 0.9, stream), "ema")
+        torch.cuda.synchronize()
+        return p, m, v, w, shadow
+
+    for a, b in zip(run([[0, 1, 2, 3]]), run([[0, 1, 2], [3]])):
+        assert torch.equal(a, b)
