@@ -117,7 +117,26 @@ constexpr uint32_t kSplitBlocksPerCu = 4;
  *   blocks   256         1,024       2,816       8,192       32,768
  *         14.4 | 8.4  16.6 | 10.7  23.4 | 20.6  50.0 | 46.0  160.8 | 163 */
 constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
-constexpr uint32_t kPrefetchBlocksPerCu = 1024; /* tables take the prefetching kernel above this many full blocks per unit */
+/* Tables take the prefetching kernel above this many full blocks per compute unit.  Its eight waves by ticket get more out
+ * of HBM, the plain kernel's sixteen start and end sooner and hide more arithmetic: mode L2's recomputed elements, the
+ * IEEE chain of fp32 parameters.  us per launch, prefetching kernel | plain, 256 units, no two launches on the same data:
+ *   blocks                 8,192      12,288      16,896      21,997      37,392      74,784     157,651
+ *   bf16                 38 | 34     52 | 50     67 | 68     86 | 93   138 | 143   267 | 294   547 | 671
+ *   ... fp32 gradients   41 | 39     59 | 60     77 | 83   100 | 111   160 | 176   310 | 351   637 | 775
+ *   fp32                 62 | 58     86 | 84   114 | 114   145 | 150   235 | 245   453 | 482  939 | 1,026
+ *   bf16, mode L2        43 | 37     56 | 53     71 | 70     96 | 95   146 | 146   274 | 302   561 | 684
+ *   ... fp32 gradients   45 | 37     62 | 62     80 | 85   107 | 110   165 | 179   314 | 360   642 | 770
+ *   fp32, mode L2        70 | 61     96 | 90   127 | 120   164 | 156   259 | 253   488 | 504 1,006 | 1,068
+ *   bf16, mode BNB       42 | 36     58 | 52     73 | 70     98 | 95   148 | 150   280 | 301   573 | 682
+ *   ... fp32 gradients   45 | 39     63 | 62     81 | 84   107 | 115   166 | 180   321 | 350   655 | 781
+ *   fp32, mode BNB       65 | 58     90 | 85   117 | 115   150 | 152   243 | 246   463 | 489   957 | 1,036 */
+inline uint32_t prefetch_blocks_per_cu(int mode, int layout) {
+    if (mode == ERI_ADAM8_MODE_L2) return layout == kLayoutF32 ? 160 : layout == kLayoutBF16 ? 96 : 48;
+    if (mode == ERI_ADAM8_MODE_BNB) return layout == kLayoutF32 ? 80 : layout == kLayoutBF16 ? 128 : 56;
+    return layout == kLayoutF32 ? 64 : 48;
+}
+/* Above this many full blocks per compute unit the gradient-norm pass cuts its list into ranges. */
+constexpr uint32_t kNormRangesBlocksPerCu = 1024;
 constexpr uint32_t kNormWaves = 4;        /* waves per workgroup of the gradient-norm pass */
 
 /* Such a walk needs the same number of workgroups in every range. */

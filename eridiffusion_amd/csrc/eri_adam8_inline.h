@@ -44,6 +44,20 @@ __device__ __forceinline__ ERI_GLOBAL T *as_global(T *p) {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+/* Tables that do not change during a launch, at wave-uniform addresses: declared constant, they are read through the
+ * scalar cache.  As ordinary loads the compiler reads them through the vector path wherever it sees a store, a barrier or
+ * an atomic before them, and a vector load is waited for together with every load and store that the wave has in flight. */
+#define ERI_CONSTANT __attribute__((address_space(4)))
+template <typename T>
+__device__ __forceinline__ T load_constant(const T *p) {
+    static_assert(sizeof(T) % 4 == 0, "read word by word");
+    struct Words { uint32_t w[sizeof(T) / 4]; } words;
+    const ERI_CONSTANT uint32_t *q = (const ERI_CONSTANT uint32_t *)p;
+#pragma unroll
+    for (uint32_t i = 0; i < sizeof(T) / 4; ++i) words.w[i] = q[i];
+    return __builtin_bit_cast(T, words);
+}
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t f2u(float x) { return __builtin_bit_cast(uint32_t, x); }
@@ -907,14 +921,14 @@ __device__ __forceinline__ void stage_end() {
 template <typename Row>
 __device__ __forceinline__ uint32_t find_row(const Row *rows, uint32_t n_rows, uint32_t from, uint32_t blk) {
     uint32_t lo = from, hi = from + 1; // rows[lo].full_start <= blk
-    for (uint32_t step = 1; hi < n_rows && rows[hi].full_start <= blk; step *= 2) {
+    for (uint32_t step = 1; hi < n_rows && load_constant(&rows[hi].full_start) <= blk; step *= 2) {
         lo = hi;
         hi = lo + 2 * step;
     }
     if (hi > n_rows) hi = n_rows;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (rows[mid].full_start <= blk) lo = mid; else hi = mid;
+        if (load_constant(&rows[mid].full_start) <= blk) lo = mid; else hi = mid;
     }
     return lo;
 }
@@ -931,15 +945,15 @@ __device__ __forceinline__ void seek_row(const Row *rows, uint32_t n_rows, uint3
                                          uint32_t &t_end) {
     if (blk >= t_end) {
         ti = find_row(rows, n_rows, ti, blk);
-        t = rows[ti];
+        t = load_constant(rows + ti);
         t_end = t.full_start + (uint32_t)(t.numel / kBlock);
     }
 }
 
 /* The ticket counter of a table of rows (kTableHead). */
 template <typename Row>
-__device__ __forceinline__ uint32_t *table_ticket(const Row *rows) {
-    return reinterpret_cast<uint32_t *>(reinterpret_cast<uintptr_t>(rows) - kTableHead);
+__device__ __forceinline__ ERI_GLOBAL uint32_t *table_ticket(const Row *rows) {
+    return (ERI_GLOBAL uint32_t *)(reinterpret_cast<uintptr_t>(rows) - kTableHead);
 }
 
 struct BlockRowMap {
@@ -948,13 +962,13 @@ struct BlockRowMap {
         : row_of(reinterpret_cast<const uint32_t *>(rows + n_rows)) {}
     __device__ __forceinline__ void seek(const DevTensor *rows, uint32_t blk, uint32_t &ti, DevTensor &t, uint32_t &t_end) const {
         if (blk >= t_end) {
-            ti = row_of[blk];
-            t = rows[ti];
+            ti = load_constant(row_of + blk);
+            t = load_constant(rows + ti);
             t_end = t.full_start + (uint32_t)(t.numel / kBlock);
         }
     }
     /* Row of partial block i: behind the map stands the list of the rows that have one. */
-    __device__ __forceinline__ uint32_t tail_row(uint32_t total_blocks, uint32_t i) const { return row_of[total_blocks + i]; }
+    __device__ __forceinline__ uint32_t tail_row(uint32_t total_blocks, uint32_t i) const { return load_constant(row_of + total_blocks + i); }
 };
 
 /* Rounds of blocks handed out by ticket.  Nothing bounds how far the waves of a static walk drift apart; after a few
@@ -966,20 +980,19 @@ struct BlockRowMap {
  * One address takes 80 M atomics per second: a ticket per wave was 3.4 times as slow as the static walk.
  * The first round of a workgroup is its own number; it asks for the one after next when the one at hand begins, so the
  * answer has a round's time to arrive.  Every round asks exactly once, so the answer rounds - 1 is the last of the
- * launch, and whoever gets it puts the counter back to zero for the next launch on the stream. */
+ * launch, and with it the counter wraps to zero for the next launch on the stream. */
 struct Tickets {
-    uint32_t *counter;
+    ERI_GLOBAL uint32_t *counter;
     uint32_t rounds, first; // first: rounds that are not asked for
     /* `per_round` of the list's units make a round */
     template <typename Row>
     __device__ __forceinline__ Tickets(const Row *rows, uint32_t units, uint32_t per_round)
         : counter(table_ticket(rows)), rounds((units + per_round - 1) / per_round), first(gridDim.x < rounds ? gridDim.x : rounds) {}
-    __device__ __forceinline__ uint32_t ask() const { return __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    /* One lane of the workgroup.  (Not a fetch_add: the compiler would fold that over the lanes of the wave and wait for
+     * the answer on the spot.) */
+    __device__ __forceinline__ uint32_t ask() const { return __builtin_amdgcn_atomic_inc32(counter, rounds - 1, __ATOMIC_RELAXED, "agent"); }
     /* The round that the answer stands for; `rounds` or more: none is left. */
-    __device__ __forceinline__ uint32_t round_of(uint32_t answer) const {
-        if (answer == rounds - 1) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return first + answer;
-    }
+    __device__ __forceinline__ uint32_t round_of(uint32_t answer) const { return first + answer; }
 };
 /* All waves of the workgroup are here and see each other's LDS writes; requests to memory stay in flight. */
 __device__ __forceinline__ void lds_barrier() {

@@ -8,22 +8,18 @@
 namespace eri {
 
 /* The one case in which the EMA runs inside the step kernel: the prefetching kernel in mode ERI, on bf16
- * parameters (with bf16 or fp32 gradients).  With bf16 gradients that kernel has twelve waves per compute unit against
- * the plain kernel's sixteen, and between one round of them and the tables that HBM bounds, the plain kernel and the
- * sweep behind it are faster.  us per step and EMA, prefetching kernel | plain kernel and sweep, 256 units:
- *   blocks               1,088        2,816        3,584        4,096        8,192       16,384       32,768
- *   bf16           12.0 | 13.3  21.0 | 20.9  32.9 | 25.3  33.0 | 28.4  54.3 | 50.6   105 | 97.8    199 | 204
- *   fp32 gradients 11.9 | 13.0  23.7 | 22.8  26.9 | 28.2  28.5 | 34.3  49.2 | 59.6  92.6 | 107     201 | 210 */
-constexpr uint32_t kFusedEmaOneRound = 12; // bf16 gradients: blocks per unit up to which
-constexpr uint32_t kFusedEmaLarge = 64;    // and beyond which the EMA runs inside the step
+ * parameters (with bf16 or fp32 gradients).  On tables that its eight waves per compute unit go through in a few rounds
+ * the plain kernel and the sweep behind it are faster.  us per step and EMA, prefetching kernel | plain kernel and sweep,
+ * 256 units, no two launches on the same data:
+ *   blocks               1,025        2,560        4,096        8,192       12,288       16,896       74,784
+ *   bf16           13.5 | 13.1  23.7 | 21.2  31.5 | 29.9  49.1 | 51.5  68.1 | 74.6   88.9 | 100    354 | 417
+ *   fp32 gradients 14.2 | 14.1  25.7 | 23.0  32.3 | 33.4  50.6 | 57.9  75.5 | 86.5    100 | 111    408 | 467 */
+constexpr uint32_t kFusedEmaBlocksPerCu = 24, kFusedEmaBlocksPerCuGradF32 = 14;
 bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
     if ((h.flags & ERI_ADAM8_FLAG_EMA) == 0 || !layout_param_bf16(layout) || h.mode != ERI_ADAM8_MODE_ERI) return false;
     if (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) return false;
-    const bool few = (uint64_t)units <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
     if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0) return true;
-    if (few) return false;
-    return !layout_grad_bf16(layout) || units <= compute_units * kFusedEmaOneRound ||
-           (uint64_t)units > (uint64_t)compute_units * kFusedEmaLarge;
+    return (uint64_t)units > (uint64_t)compute_units * (layout_grad_bf16(layout) ? kFusedEmaBlocksPerCu : kFusedEmaBlocksPerCuGradF32);
 }
 
 /* Whether a table that qualifies for the prefetching kernel is large enough to gain from it, or has its EMA inside that
@@ -31,7 +27,7 @@ bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t
  * mode BNB took 38.1 us for 4,096 bf16 blocks instead of 29.0, and fp32 parameters 39 for 2,816 instead of 31.5. */
 static bool prefetch_pays(uint32_t total_blocks, uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
     if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || step_fuses_ema(units, layout, h, compute_units)) return true;
-    return (uint64_t)total_blocks > (uint64_t)compute_units * (uint64_t)kPrefetchBlocksPerCu;
+    return (uint64_t)total_blocks > (uint64_t)compute_units * prefetch_blocks_per_cu(h.mode, layout);
 }
 
 int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, int layout,
@@ -685,7 +681,7 @@ int launch_quant_error(const DevTensor *rows, uint32_t n_rows, uint32_t total_bl
 // A round is what keeps the counter's rate low and the window narrow, about 200 KB per workgroup.  us over the same arrays
 // side by side, 1.31 G parameters: 64 waves per unit on a static walk, eight elements per lane, fp32 in two half-line
 // words | by ticket:
-//   32-bit step bf16 5,784 | 4,791 (6.0 TB/s), fp32 7,393 | 5,879 (6.2), with masters 7,322 | 5,992
+//   32-bit step bf16 5,784 | 4,563 (6.3 TB/s), fp32 7,393 | 5,840 (6.3), with masters 7,322 | 5,992
 //   EMA bf16 1,470 | 1,217 (6.5), fp32 3,100 | 2,364 (6.7)
 // Traffic of the 32-bit step alone by what a round holds, 8 waves: half a block per wave 4,476, a block 4,783, two 4,817.
 // Sweeps of few blocks take a quarter block per wave (kSmallSweepBlocksPerCu): the 32-bit step over the 87 tensors of
@@ -919,7 +915,7 @@ __global__ __launch_bounds__(kSweepThreads) void adamw32_kernel(const ElemRow *_
     auto gscale_of = [&](const ElemRow &t) { return GS ? (grad_scale * t.scale) * tscale : 1.0f; }; // the order of the 8-bit step's factors
     const uint32_t waves = blockDim.x / kWave;
     for (uint32_t i = __builtin_amdgcn_readfirstlane(blockIdx.x * waves + threadIdx.x / kWave); i < 2 * n_rows; i += gridDim.x * waves) {
-        const ElemRow t = rows[i / 2];
+        const ElemRow t = load_constant(rows + i / 2);
         const uint32_t tail = (uint32_t)(t.numel % kBlock), from = (i & 1) * kPiece;
         if (tail <= from) continue;
         const uint32_t n = tail - from < kPiece ? tail - from : kPiece;
@@ -1010,7 +1006,7 @@ __global__ __launch_bounds__(kSweepThreads) void ema_kernel(const ElemRow *__res
     const float omd = 1.0f - decay; // ema_enhanced.rs:96
     const uint32_t waves = blockDim.x / kWave;
     for (uint32_t r = __builtin_amdgcn_readfirstlane(blockIdx.x * waves + threadIdx.x / kWave); r < n_rows; r += gridDim.x * waves) {
-        const ElemRow t = rows[r];
+        const ElemRow t = load_constant(rows + r);
         const uint32_t n = (uint32_t)(t.numel % kBlock);
         if (n == 0) continue;
         const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;

@@ -142,6 +142,10 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     const uint32_t waves_per_wg = blockDim.x / kWave;
     const Tickets tickets(rows, total_blocks, waves_per_wg);
     __shared__ uint32_t coming[2];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const BlockRowMap map(rows, n_rows);
+    uint32_t blk = blockIdx.x * waves_per_wg + wave_in_wg;
     stage_begin<kLdsImageBytes>(lds_raw, lds_image);
     if (threadIdx.x == 0 && blockIdx.x < tickets.rounds) coming[0] = tickets.round_of(tickets.ask());
     stage_end();
@@ -154,25 +158,19 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     L.key_s = base + kOffKeyS;
     L.key_u = base + kOffKeyU;
 
-    const uint32_t lane = threadIdx.x & (kWave - 1);
     const uint32_t stride = gridDim.x * waves_per_wg;
     const BlockDiv dbc1(h.bc1), dbc2(h.bc2);
     float(*const mine)[256] = decayed[threadIdx.x / kWave];
 
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * waves_per_wg + threadIdx.x / kWave);
     // partial last blocks first, handed out from the last wave backwards; their workgroups come to the tickets later
-    const BlockRowMap map(rows, n_rows);
-    for (uint32_t i = stride - 1 - wave; i < n_tails; i += stride) {
-        const DevTensor t = rows[map.tail_row(total_blocks, i)];
+    for (uint32_t i = stride - 1 - blk; i < n_tails; i += stride) {
+        const DevTensor t = load_constant(rows + map.tail_row(total_blocks, i));
         const uint32_t n = (uint32_t)(t.numel % kBlock);
         const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
         tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
         if (EMA && t.shadow != nullptr) ema_tail(t, n, lane, h.ema_decay);
     }
-    if (blockIdx.x >= tickets.rounds) return;
-    const uint32_t wave_in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     uint32_t next_round = __builtin_amdgcn_readfirstlane(coming[0]);
-    uint32_t blk = blockIdx.x * waves_per_wg + wave_in_wg;
     // the last round may have fewer blocks than the workgroup has waves, and is a workgroup's last: a wave without one ends
     if (blk >= total_blocks) return;
     const f32x4 base_s = reinterpret_cast<const f32x4 *>(L.map_s)[lane]; // codes 4*lane .. 4*lane + 3
@@ -181,10 +179,10 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
     uint32_t ti = 0, t_end = 0;
     DevTensor t;
     map.seek(rows, blk, ti, t, t_end);
-    uint32_t nti = ti, nt_end = t_end;
-    DevTensor nt = t;
     RawBlock raw;
     raw.issue(t, blk - t.full_start, lane);
+    uint32_t nti = ti, nt_end = t_end;
+    DevTensor nt = t;
     for (uint32_t slot = 1;; slot ^= 1) {
         const bool more = next_round < tickets.rounds;
         uint32_t answer = 0;

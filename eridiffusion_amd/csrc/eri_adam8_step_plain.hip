@@ -1,6 +1,6 @@
 /*
  * The plain step kernel (one wave per block, no cross-block prefetch): tables of every layout and mode between the
- * four-waves-per-block kernel's (kSplitBlocksPerCu) and the prefetching kernel's (kPrefetchBlocksPerCu), and any table
+ * four-waves-per-block kernel's (kSplitBlocksPerCu) and the prefetching kernel's (prefetch_blocks_per_cu), and any table
  * with ERI_ADAM8_FLAG_BSEARCH or ERI_ADAM8_FLAG_NO_PIPELINE.  HBM traffic bounds it, with the launch's start and its
  * last round on the smaller tables.  A row's partial last block is one more block of the walk, with the lanes past its
  * end off and one trip less in flight: as a two-sweep chain on one wave each it made 300 odd bf16 tensors with 14 M
@@ -21,27 +21,13 @@ constexpr bool kGradBf16 = ERI_PLAIN_LAYOUT == kLayoutBF16;
 
 /* Which tables an instantiation is for.  Only the first holds the code for partial blocks: beside it the loop over
  * whole ones took 128 registers and up to 20 bytes of scratch, 109 to 127 and none without (2,816 bf16 blocks 14.1 ->
- * 13.5 us, 15.1 -> 14.2 with fp32 gradients).
- * The last two differ in where a block's row is looked up.  Through the scalar cache (kWhole, kTails) the lookup is
- * short.  Through vector loads (kWholeLarge) it waits for the stores of the block before, because one counter holds
- * a wave's loads and stores: the wave's reads and writes keep apart, which costs the short tables a round trip per
- * block and gives the long ones, which HBM bounds, 1-2 %.  us per launch, kWhole | kWholeLarge, 256 units:
- *   blocks                     8,192         16,384         24,576         32,768         49,152        131,072
- *   bf16                 31.7 | 34.0    63.4 | 64.3    95.0 | 94.5    126 | 125    188 | 185    504 | 497
- *   bf16, functional     32.6 | 32.3    64.4 | 63.7    96.9 | 95.8    128 | 127    190 | 188    509 | 503
- *   ... fp32 gradients   37.6 | 39.4    71.6 | 73.3    102 | 106      134 | 137    237 | 231    634 | 623
- *   bf16, mode BNB       32.3 | 37.1    63.7 | 68.1    95.3 | 96.6    126 | 126    188 | 187
- *   fp32, functional     51.7 | 51.7    97.6 | 97.6     167 | 167     223 | 220    335 | 330    874 | 862
- * fp32 parameters in the other modes do not tell them apart (842.3 | 842.6 us on 131,072 blocks) and always take
- * kWhole. */
-enum Table { kTails, kWhole, kWholeLarge };
-constexpr uint32_t large_blocks_per_cu(int mode) { return ERI_PLAIN_LAYOUT == kLayoutBF16GradF32 || mode == ERI_ADAM8_MODE_BNB ? 128 : 96; }
+ * 13.5 us, 15.1 -> 14.2 with fp32 gradients). */
+enum Table { kTails, kWhole };
 
 /* Threads per workgroup: sixteen waves per compute unit where the instantiation fits the 128 registers that
  * leaves each lane, twelve (170 registers) where it would spill: the coupled-decay mode with a gradient scale,
  * with fp32 gradients or with the binary search (12-30 spilled registers at sixteen waves).  Instantiations of kWhole
- * use no scratch, kTails of bf16 parameters up to 20 bytes per lane, kWholeLarge, whose rows lie in vector registers, up
- * to 28 (64 in mode BNB). */
+ * use no scratch, kTails of bf16 parameters up to 20 bytes per lane. */
 constexpr uint32_t plain_threads(int mode, bool gs, bool keytab, bool gbf16) {
     return (mode == ERI_ADAM8_MODE_L2 && (gs || !keytab || !gbf16)) ? 768 : 1024;
 }
@@ -92,14 +78,14 @@ __global__ __launch_bounds__(plain_threads(MODE, GS, KEYTAB, GBF16)) void adam8_
     const uint32_t trips = rounds + (has_left ? 1u : 0u);
     for (uint32_t k = 0; k < trips; ++k) {
         uint32_t unit = k < rounds ? k * stride + wave : left_first + left_mine;
-        if (TABLE != kWholeLarge) unit = __builtin_amdgcn_readfirstlane(unit);
+        unit = __builtin_amdgcn_readfirstlane(unit);
         if (TABLE != kTails || unit < total_blocks) {
             map.seek(rows, unit, ti, t, t_end);
             const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
             full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16>(t, unit - t.full_start, kBlock, lane, h, gscale, dbc1, dbc2, L,
                                                                  decayed[threadIdx.x / kWave]);
         } else {
-            t = rows[map.tail_row(total_blocks, unit - total_blocks)];
+            t = load_constant(rows + map.tail_row(total_blocks, unit - total_blocks));
             const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
             full_block<BF16, MODE, EXACT, WD, GS, KEYTAB, GBF16, true>(t, (uint32_t)(t.numel / kBlock), (uint32_t)(t.numel % kBlock),
                                                                        lane, h, gscale, dbc1, dbc2, L, decayed[threadIdx.x / kWave]);
@@ -113,17 +99,10 @@ template <int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB>
 int launch_one(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h,
                const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg, hipStream_t s) {
     auto k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kTails>;
-    if constexpr (KEYTAB) { // the binary search is a cross-check and has the one variant
-        // such a table's grid is one workgroup per compute unit
-        const bool large = (uint64_t)total_blocks > (uint64_t)grid * large_blocks_per_cu(MODE);
+    if constexpr (KEYTAB) // the binary search is a cross-check and has the one variant
         if (n_tails == 0) k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kWhole>;
-        if constexpr (kBf16 || MODE == ERI_ADAM8_MODE_L2)
-            if (n_tails == 0 && large) k = adam8_step_kernel<kBf16, MODE, EXACT, WD, GS, KEYTAB, kGradBf16, kWholeLarge>;
-    }
     if (wg > plain_threads(MODE, GS, KEYTAB, kGradBf16)) wg = plain_threads(MODE, GS, KEYTAB, kGradBf16);
-    // One common window for all dies (a grid-stride walk): on the tables this kernel takes, up to 1,024
-    // blocks per compute unit, it measured 2 % ahead of one range per die with the arrays far apart in device
-    // memory and 5 % with them adjacent; the tables of the prefetching kernel want the ranges.
+    // One common window for all dies (a grid-stride walk).
     hipLaunchKernelGGL(k, dim3(grid), dim3(wg), 0, s, rows, n_rows, total_blocks, n_tails, h,
                        static_cast<const uint4 *>(lds_image), dev_scale);
     return (int)hipGetLastError();

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(1024) void adam8_step_split_kernel(const DevTensor 
             q.lb = unit - q.t.full_start;
             q.n = kBlock;
         } else {
-            q.t = rows[map.tail_row(total_blocks, unit - total_blocks)];
+            q.t = load_constant(rows + map.tail_row(total_blocks, unit - total_blocks));
             q.lb = (uint32_t)(q.t.numel / kBlock);
             q.n = (uint32_t)(q.t.numel % kBlock);
         }

@@ -52,7 +52,7 @@ __global__ __launch_bounds__(two_threads(MODE)) void adam8_step_two_kernel(StepG
         if (!is_f32) unit -= f32_units;
         // a full block's row or, behind those, the row of a partial one: one list (BlockRowMap)
         const BlockRowMap map(g.rows, g.n_rows);
-        const DevTensor t = g.rows[map.row_of[unit]];
+        const DevTensor t = load_constant(g.rows + load_constant(map.row_of + unit));
         const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
         const bool partial = unit >= g.total_blocks;
         const uint32_t lb = partial ? (uint32_t)(t.numel / kBlock) : unit - t.full_start;

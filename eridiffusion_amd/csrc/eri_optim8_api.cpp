@@ -1152,7 +1152,7 @@ static int grad_norm_launch(EriAdam8Table *t, EriAdam8Table *also, DeviceCtx *ct
             // The pass goes backwards, so that the gradients it read last, which the last-level cache still holds, are
             // the first that the step reads.  Of the larger groups that cache holds next to nothing, and one range per
             // die reads these faster: 10.3 GB of fp32 in 1,620 us, in a common window 1,670.
-            ng.chunks = (uint64_t)g.total_blocks > (uint64_t)ctx->cus * eri::kPrefetchBlocksPerCu ? eri::chunks_for(ng.wgs) : 1u;
+            ng.chunks = (uint64_t)g.total_blocks > (uint64_t)ctx->cus * eri::kNormRangesBlocksPerCu ? eri::chunks_for(ng.wgs) : 1u;
             ng.grad_bf16 = eri::layout_grad_bf16(g.dtype) ? 1u : 0u;
             wgs += ng.wgs;
         }

@@ -6,6 +6,7 @@ import ctypes as C
 import pytest
 
 import harness as hs
+import test_gpu_whole_tables as whole
 
 pytestmark = pytest.mark.gpu
 WAVES, UNITS = 8, 256
@@ -71,4 +72,30 @@ def test_sweeps_by_ticket(dtype, master, extra):
         return p, m, v, w, shadow
 
     for a, b in zip(run([[0, 1, 2, 3]]), run([[0, 1, 2], [3]])):
+        assert torch.equal(a, b)
+
+
+LINES = {("bf16", 0): 48, ("bf16", 1): 96, ("bf16", 2): 128, ("bf16-f32-grads", 0): 48, ("bf16-f32-grads", 1): 48,
+         ("bf16-f32-grads", 2): 56, ("f32", 0): 64, ("f32", 1): 160, ("f32", 2): 80}
+
+
+@pytest.mark.parametrize("layout,mode", sorted(LINES), ids=str)
+@pytest.mark.parametrize("over,tail", [(0, 0), (1, 0), (1, 515)])
+def test_both_sides_of_the_line_to_the_prefetching_kernel(layout, mode, over, tail):
+    """The dispatch's own choice just below and above, against the plain kernel, bit for bit."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    sizes = whole._sizes(LINES[layout, mode] * UNITS + over, tail)
+    for a, b in zip(whole._run(layout, mode, sizes, 0, 0.5), whole._run(layout, mode, sizes, L.FLAG_NO_PIPELINE, 0.5)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layout,line", [("bf16", 24), ("bf16-f32-grads", 14)])
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("tail", [0, 515])
+def test_both_sides_of_the_line_to_the_step_that_carries_the_ema(layout, line, over, tail):
+    import torch
+    from eridiffusion_amd import _lib as L
+    sizes = whole._sizes(line * UNITS + over, tail)
+    for a, b in zip(whole._run(layout, 0, sizes, 0, None, ema=True), whole._run(layout, 0, sizes, L.FLAG_NO_PIPELINE, None, ema=True)):
         assert torch.equal(a, b)

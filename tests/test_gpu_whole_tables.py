@@ -55,11 +55,11 @@ def _run(layout, mode, sizes, flags, scale, ema=False):
 @pytest.mark.parametrize("layout", ["bf16", "bf16-f32-grads", "f32"])
 @pytest.mark.parametrize("blocks,scale", [(1, None), (4097, 0.5), (96 * 256 + 300, None), (128 * 256 + 300, 0.5)])
 def test_plain_kernel_over_whole_blocks(layout, mode, blocks, scale):
-    """Without the code for partial blocks, below and above the size from which rows are looked up through vector loads."""
+    """Without the code for partial blocks, on tables of its own size and of the prefetching kernel's."""
     import torch
     from eridiffusion_amd import _lib as L
     want = _run(layout, mode, _sizes(blocks), L.FLAG_ONE_WAVE, scale)
-    got = _run(layout, mode, _sizes(blocks), L.FLAG_NO_PIPELINE if blocks == 1 else 0, scale)
+    got = _run(layout, mode, _sizes(blocks), L.FLAG_NO_PIPELINE, scale)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
 
