@@ -123,17 +123,17 @@ constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
  *   blocks                 8,192      12,288      16,896      21,997      37,392      74,784     157,651
  *   bf16                 38 | 34     52 | 50     67 | 68     86 | 93   138 | 143   267 | 294   547 | 671
  *   ... fp32 gradients   41 | 39     59 | 60     77 | 83   100 | 111   160 | 176   310 | 351   637 | 775
- *   fp32                 62 | 58     86 | 84   114 | 114   145 | 150   235 | 245   453 | 482  939 | 1,026
+ *   fp32                 58 | 58     82 | 84   108 | 114   132 | 146   216 | 235   420 | 482  865 | 1,026
  *   bf16, mode L2        43 | 37     56 | 53     71 | 70     96 | 95   146 | 146   274 | 302   561 | 684
  *   ... fp32 gradients   45 | 37     62 | 62     80 | 85   107 | 110   165 | 179   314 | 360   642 | 770
- *   fp32, mode L2        70 | 61     96 | 90   127 | 120   164 | 156   259 | 253   488 | 504 1,006 | 1,068
+ *   fp32, mode L2        65 | 61     90 | 90                           242 | 256
  *   bf16, mode BNB       42 | 36     58 | 52     73 | 70     98 | 95   148 | 150   280 | 301   573 | 682
  *   ... fp32 gradients   45 | 39     63 | 62     81 | 84   107 | 115   166 | 180   321 | 350   655 | 781
- *   fp32, mode BNB       65 | 58     90 | 85   117 | 115   150 | 152   243 | 246   463 | 489   957 | 1,036 */
+ *   fp32, mode BNB       60 | 58     84 | 84                           220 | 241 */
 inline uint32_t prefetch_blocks_per_cu(int mode, int layout) {
-    if (mode == ERI_ADAM8_MODE_L2) return layout == kLayoutF32 ? 160 : layout == kLayoutBF16 ? 96 : 48;
-    if (mode == ERI_ADAM8_MODE_BNB) return layout == kLayoutF32 ? 80 : layout == kLayoutBF16 ? 128 : 56;
-    return layout == kLayoutF32 ? 64 : 48;
+    if (mode == ERI_ADAM8_MODE_L2) return layout == kLayoutBF16 ? 96 : 48;
+    if (mode == ERI_ADAM8_MODE_BNB) return layout == kLayoutBF16 ? 128 : layout == kLayoutBF16GradF32 ? 56 : 48;
+    return layout == kLayoutF32 ? 40 : 48;
 }
 /* Above this many full blocks per compute unit the gradient-norm pass cuts its list into ranges. */
 constexpr uint32_t kNormRangesBlocksPerCu = 1024;

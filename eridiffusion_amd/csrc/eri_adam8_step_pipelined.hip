@@ -28,9 +28,9 @@ constexpr bool kGradBf16 = ERI_PIPE_LAYOUT == kLayoutBF16;
 //   bf16, 2.57 G                            5,060 |  4,832 |  4,216
 //   ... with the EMA                        7,170 |  7,624 |  5,699 (the next block requested quarter by quarter;
 //                                                                    5,867 after the update half, as it was)
-//   bf16 with fp32 gradients, 2.57 G        5,980 |        |  4,930
+//   bf16 with fp32 gradients, 2.57 G        5,980 |        |  4,924
 //   ... with the EMA                        8,140 |        |  6,627 (6,848 after the update half)
-//   fp32, 2.57 G                            8,031 |        |  7,348
+//   fp32, 2.57 G                            8,031 |        |  7,348 (6,785 in whole lines)
 // ------------------------------------------------------------------------------------------
 
 constexpr uint32_t kPipeThreads = 512;
@@ -84,34 +84,82 @@ __device__ __forceinline__ void ema_tail(const DevTensor &t, uint32_t n, uint32_
     }
 }
 
+/* A lane's eight elements of a quarter block (512 elements).  Where everything is bf16 they are consecutive: one 128-bit
+ * word each of parameters and gradients, 64 bits of codes.  Beside fp32 they are four of the quarter's first half and four
+ * of its second, so that an access of either dtype is whole cache lines over the wave and can be streamed; as two half-line
+ * words of eight consecutive fp32 values, every line was asked for twice and had to stay in the caches in between.
+ *   fp32, 2.57 G parameters 7,302 -> 6,785 us; bf16 with fp32 gradients 4,979 -> 4,924, with the EMA level */
+constexpr bool kHalves = !kGradBf16;
+__device__ __forceinline__ u32x4 load_bf16_quarter(const void *block, int c, uint32_t lane) {
+    if (kHalves) {
+        ERI_GLOBAL const u32x2 *q = as_global(static_cast<const u32x2 *>(block)) + c * 128 + lane;
+        const u32x2 a = __builtin_nontemporal_load(q), b = __builtin_nontemporal_load(q + 64);
+        return u32x4{a.x, a.y, b.x, b.y};
+    }
+    return __builtin_nontemporal_load(as_global(static_cast<const u32x4 *>(block)) + c * 64 + lane);
+}
+__device__ __forceinline__ void store_bf16_quarter(const u32x4 &w, void *block, int c, uint32_t lane) {
+    if (kHalves) {
+        ERI_GLOBAL u32x2 *q = as_global(static_cast<u32x2 *>(block)) + c * 128 + lane;
+        __builtin_nontemporal_store(u32x2{w.x, w.y}, q);
+        __builtin_nontemporal_store(u32x2{w.z, w.w}, q + 64);
+    } else {
+        __builtin_nontemporal_store(w, as_global(static_cast<u32x4 *>(block)) + c * 64 + lane);
+    }
+}
+/* Parameters and gradients by how many words a lane's eight elements take: bf16 one, fp32 two. */
+__device__ __forceinline__ void load_quarter(u32x4 (&w)[1], const void *block, int c, uint32_t lane) { w[0] = load_bf16_quarter(block, c, lane); }
+__device__ __forceinline__ void load_quarter(u32x4 (&w)[2], const void *block, int c, uint32_t lane) {
+    ERI_GLOBAL const u32x4 *q = as_global(static_cast<const u32x4 *>(block)) + c * 128 + lane;
+    w[0] = __builtin_nontemporal_load(q);
+    w[1] = __builtin_nontemporal_load(q + 64);
+}
+__device__ __forceinline__ void unpack_quarter(const u32x4 (&w)[1], float (&out)[8]) {
+    Raw8<true> r;
+    r.w = w[0];
+    r.unpack(out);
+}
+__device__ __forceinline__ void unpack_quarter(const u32x4 (&w)[2], float (&out)[8]) {
+    Raw8<false> r;
+    r.a = __builtin_bit_cast(f32x4, w[0]);
+    r.b = __builtin_bit_cast(f32x4, w[1]);
+    r.unpack(out);
+}
+__device__ __forceinline__ void store_f32_quarter(const float (&v)[8], void *block, int c, uint32_t lane) {
+    ERI_GLOBAL f32x4 *q = as_global(static_cast<f32x4 *>(block)) + c * 128 + lane;
+    __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, q);
+    __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, q + 64);
+}
+__device__ __forceinline__ u32x2 load_codes_quarter(const uint8_t *block, int c, uint32_t lane) {
+    if (kHalves) {
+        ERI_GLOBAL const uint32_t *q = as_global(reinterpret_cast<const uint32_t *>(block)) + c * 128 + lane;
+        return u32x2{__builtin_nontemporal_load(q), __builtin_nontemporal_load(q + 64)};
+    }
+    return __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(block)) + c * 64 + lane);
+}
+__device__ __forceinline__ void store_codes_quarter(const u32x2 &w, uint8_t *block, int c, uint32_t lane) {
+    if (kHalves) {
+        ERI_GLOBAL uint32_t *q = as_global(reinterpret_cast<uint32_t *>(block)) + c * 128 + lane;
+        __builtin_nontemporal_store(w.x, q);
+        __builtin_nontemporal_store(w.y, q + 64);
+    } else {
+        __builtin_nontemporal_store(w, as_global(reinterpret_cast<u32x2 *>(block)) + c * 64 + lane);
+    }
+}
+
 struct RawBlock {
-    u32x4 p[kParamBf16 ? 4 : 8]; // bf16: one word per quarter block; fp32: two (elements 8*lane .. +3 and +4 .. +7)
-    u32x4 g[kGradBf16 ? 4 : 8];
+    u32x4 p[4][kParamBf16 ? 1 : 2]; // per quarter block
+    u32x4 g[4][kGradBf16 ? 1 : 2];
     u32x2 m[4], v[4];
     float a_m, a_v;
     /* Requests quarter c of block lb; the block's two absmax words ride with quarter 0. */
     __device__ __forceinline__ void issue_quarter(const DevTensor &t, uint32_t lb, int c, uint32_t lane) {
         const size_t e0 = (size_t)lb * kBlock;
-        ERI_GLOBAL const u32x4 *pp = as_global(reinterpret_cast<const u32x4 *>(static_cast<const char *>(t.p_in) + e0 * (kParamBf16 ? 2 : 4)));
-        ERI_GLOBAL const u32x4 *gp = as_global(reinterpret_cast<const u32x4 *>(static_cast<const char *>(t.g) + e0 * (kGradBf16 ? 2 : 4)));
-        ERI_GLOBAL const u32x2 *mp = as_global(reinterpret_cast<const u32x2 *>(t.m + e0));
-        ERI_GLOBAL const u32x2 *vp = as_global(reinterpret_cast<const u32x2 *>(t.v + e0));
-        if (kParamBf16) {
-            p[c] = __builtin_nontemporal_load(&pp[c * 64 + lane]); // each byte is touched once per step
-        } else {
-            p[2 * c] = pp[c * 128 + 2 * lane];
-            p[2 * c + 1] = pp[c * 128 + 2 * lane + 1];
-        }
-        if (kGradBf16) {
-            g[c] = __builtin_nontemporal_load(&gp[c * 64 + lane]);
-        } else {
-            // a lane's two words share cache lines with its neighbours' across the two instructions, so
-            // these stay ordinary loads: streamed, the second instruction would fetch every line again
-            g[2 * c] = gp[c * 128 + 2 * lane];
-            g[2 * c + 1] = gp[c * 128 + 2 * lane + 1];
-        }
-        m[c] = __builtin_nontemporal_load(&mp[c * 64 + lane]);
-        v[c] = __builtin_nontemporal_load(&vp[c * 64 + lane]);
+        const char *pp = static_cast<const char *>(t.p_in) + e0 * (kParamBf16 ? 2 : 4), *gp = static_cast<const char *>(t.g) + e0 * (kGradBf16 ? 2 : 4);
+        load_quarter(p[c], pp, c, lane);
+        load_quarter(g[c], gp, c, lane);
+        m[c] = load_codes_quarter(t.m + e0, c, lane);
+        v[c] = load_codes_quarter(t.v + e0, c, lane);
         if (c == 0) {
             a_m = as_global(t.absmax_m)[lb];
             a_v = as_global(t.absmax_v)[lb];
@@ -218,31 +266,14 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         u32x4 sh[4];
         const bool with_shadow = EMA && t.shadow != nullptr;
         if (EMA && with_shadow) {
-            ERI_GLOBAL const u32x4 *sp = as_global(reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(t.shadow) + e0));
 #pragma unroll
-            for (int c = 0; c < 4; ++c) sh[c] = __builtin_nontemporal_load(&sp[c * 64 + lane]);
+            for (int c = 0; c < 4; ++c) sh[c] = load_bf16_quarter(static_cast<const char *>(t.shadow) + e0 * 2, c, lane);
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             float pv[8], gv[8], pn[8];
-            if (kParamBf16) {
-                Raw8<true> pr;
-                pr.w = raw.p[c];
-                pr.unpack(pv);
-            } else {
-                const u32x4 pa = raw.p[kParamBf16 ? c : 2 * c], pb = raw.p[kParamBf16 ? c : 2 * c + 1];
-                pv[0] = u2f(pa.x); pv[1] = u2f(pa.y); pv[2] = u2f(pa.z); pv[3] = u2f(pa.w);
-                pv[4] = u2f(pb.x); pv[5] = u2f(pb.y); pv[6] = u2f(pb.z); pv[7] = u2f(pb.w);
-            }
-            if (kGradBf16) {
-                Raw8<true> gr;
-                gr.w = raw.g[c];
-                gr.unpack(gv);
-            } else {
-                const u32x4 ga = raw.g[kGradBf16 ? c : 2 * c], gb = raw.g[kGradBf16 ? c : 2 * c + 1];
-                gv[0] = u2f(ga.x); gv[1] = u2f(ga.y); gv[2] = u2f(ga.z); gv[3] = u2f(ga.w);
-                gv[4] = u2f(gb.x); gv[5] = u2f(gb.y); gv[6] = u2f(gb.z); gv[7] = u2f(gb.w);
-            }
+            unpack_quarter(raw.p[c], pv);
+            unpack_quarter(raw.g[c], gv);
             // one flag per element: flagged elements are put right quarter by quarter (before the shadow uses
             // them), and the exact chain runs for the flagged positions only
             Redo8 redo;
@@ -272,16 +303,17 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
                 pw[c].z = bf16_pair(pn[4], pn[5]);
                 pw[c].w = bf16_pair(pn[6], pn[7]);
             } else { // fp32 parameters are final here (they take the exact chain): stored quarter by quarter
-                store8<false>(p, c * 512 + lane * 8, pn);
+                store_f32_quarter(pn, p, c, lane);
             }
             if (EMA && with_shadow) {
                 float out[8];
                 ema_eight(sh[c], pw[c], h.ema_decay, out);
-                store8<true>(static_cast<char *>(t.shadow) + e0 * 2, c * 512 + lane * 8, out);
+                const u32x4 w = {bf16_pair(out[0], out[1]), bf16_pair(out[2], out[3]), bf16_pair(out[4], out[5]), bf16_pair(out[6], out[7])};
+                store_bf16_quarter(w, static_cast<char *>(t.shadow) + e0 * 2, c, lane);
             }
             // the quarter's raw words are dead: the next block's quarter takes their registers now
             raw.issue_quarter(nt, pblk - nt.full_start, c, lane);
-            if (kParamBf16) __builtin_nontemporal_store(pw[c], as_global(reinterpret_cast<u32x4 *>(p) + c * 64 + lane));
+            if (kParamBf16) store_bf16_quarter(pw[c], p, c, lane);
         }
         float nam = lm, nav = lv;
         wave_max2(nam, nav);
@@ -293,19 +325,17 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         if (dm.fast && dv.fast) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const uint32_t o = c * 512 + lane * 8;
                 u32x2 mw, vw;
                 requant8<true, true, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
-                __builtin_nontemporal_store(mw, as_global(reinterpret_cast<u32x2 *>(mc + o)));
-                __builtin_nontemporal_store(vw, as_global(reinterpret_cast<u32x2 *>(vc + o)));
+                store_codes_quarter(mw, mc, c, lane);
+                store_codes_quarter(vw, vc, c, lane);
             }
         } else {
             for (int c = 0; c < 4; ++c) {
-                const uint32_t o = c * 512 + lane * 8;
                 u32x2 mw, vw;
                 requant8<false, true, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
-                __builtin_nontemporal_store(mw, as_global(reinterpret_cast<u32x2 *>(mc + o)));
-                __builtin_nontemporal_store(vw, as_global(reinterpret_cast<u32x2 *>(vc + o)));
+                store_codes_quarter(mw, mc, c, lane);
+                store_codes_quarter(vw, vc, c, lane);
             }
         }
         if (!more) break;

@@ -76,7 +76,7 @@ def test_sweeps_by_ticket(dtype, master, extra):
 
 
 LINES = {("bf16", 0): 48, ("bf16", 1): 96, ("bf16", 2): 128, ("bf16-f32-grads", 0): 48, ("bf16-f32-grads", 1): 48,
-         ("bf16-f32-grads", 2): 56, ("f32", 0): 64, ("f32", 1): 160, ("f32", 2): 80}
+         ("bf16-f32-grads", 2): 56, ("f32", 0): 40, ("f32", 1): 48, ("f32", 2): 48}
 
 
 @pytest.mark.parametrize("layout,mode", sorted(LINES), ids=str)
