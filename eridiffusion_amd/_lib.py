@@ -50,6 +50,10 @@ class EmaRow(C.Structure):
                 ("reserved", C.c_int32)]
 
 
+class MomentRow(C.Structure):  # EriMomentTensor
+    _fields_ = [(n, C.c_void_p) for n in ("m32", "v32", "m", "v", "absmax_m", "absmax_v")] + [("numel", C.c_uint64)]
+
+
 class MemoryReportC(C.Structure):
     _fields_ = [("num_params", C.c_uint64), ("param_memory_gb", C.c_double), ("state_memory_gb", C.c_double),
                 ("total_memory_gb", C.c_double), ("memory_reduction_percent", C.c_double), ("has_reduction", C.c_int32),
@@ -116,6 +120,8 @@ EXPORTS = {
     "eri_adam8_quantize": (C.c_int, [C.c_void_p, C.c_int, C.c_uint64, C.c_void_p, C.c_void_p, C.c_void_p]),
     "eri_adam8_dequantize_state": (C.c_int, [C.c_void_p] * 4 + [C.c_uint64] + [C.c_void_p] * 3),
     "eri_adam8_quantize_state": (C.c_int, [C.c_void_p] * 2 + [C.c_uint64] + [C.c_void_p] * 5),
+    "eri_adam8_dequantize_states": (C.c_int, [C.POINTER(MomentRow), C.c_uint32, C.c_void_p]),
+    "eri_adam8_quantize_states": (C.c_int, [C.POINTER(MomentRow), C.c_uint32, C.c_void_p]),
     "eri_adamw32_step_multi": (C.c_int, [C.POINTER(AdamW32Row), C.c_uint32, C.POINTER(AdamW32Hyper), C.c_void_p]),
     "eri_adamw32_step_multi_scaled": (C.c_int, [C.POINTER(AdamW32Row), C.c_uint32, C.POINTER(AdamW32Hyper), C.c_float,
                                               C.c_void_p, C.c_void_p]),
@@ -185,6 +191,9 @@ EXPORTS = {
     "eri_adam8bit_fn_state_numel": (C.c_int, [C.c_void_p, C.c_char_p, C.POINTER(C.c_uint64)]),
     "eri_adam8bit_fn_get_state_fp32": (C.c_int, [C.c_void_p, C.c_char_p, C.c_void_p, C.c_void_p]),
     "eri_adam8bit_fn_load_state_fp32": (C.c_int, [C.c_void_p, C.c_char_p, C.c_void_p, C.c_void_p, C.c_uint64]),
+    "eri_adam8bit_fn_get_states_fp32": (C.c_int, [C.c_void_p, C.POINTER(C.c_char_p), C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.c_uint32]),
+    "eri_adam8bit_fn_load_states_fp32": (C.c_int, [C.c_void_p, C.POINTER(C.c_char_p), C.POINTER(C.c_void_p), C.POINTER(C.c_void_p),
+                                                   C.POINTER(C.c_uint64), C.c_uint32]),
 }
 
 _lib = None

@@ -354,23 +354,31 @@ class Adam8bitFunctional:
             numel = C.c_uint64()
             check(lib().eri_adam8bit_fn_state_numel(self._opt, name.encode(), C.byref(numel)), "state_numel")
             m = torch.empty(numel.value, dtype=torch.float32, device="cuda")
-            v = torch.empty_like(m)
-            check(lib().eri_adam8bit_fn_get_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr()),
-                  "eri_adam8bit_fn_get_state_fp32")
-            out[name] = (m, v)
+            out[name] = (m, torch.empty_like(m))
+        k = len(out)
+        if k:
+            check(lib().eri_adam8bit_fn_get_states_fp32(self._opt, (C.c_char_p * k)(*[n.encode() for n in out]),
+                                                        (C.c_void_p * k)(*[m.data_ptr() for m, _ in out.values()]),
+                                                        (C.c_void_p * k)(*[v.data_ptr() for _, v in out.values()]), k),
+                  "eri_adam8bit_fn_get_states_fp32")
         return out
 
     def load_state_from_tensors(self, state: Dict[str, Tuple[torch.Tensor, torch.Tensor]]) -> None:
         """The moments are read on the optimizer's stream, in its order.  Called under another stream, the moments (and
         the float32 copies made of them here) belong to that one: each is waited for before it is read, and the reading
-        before it may be freed or changed."""
+        before it may be freed or changed.  Otherwise device tensors that are read as they are share a launch."""
         here = _stream_ptr()
         apart = here != self._stream
+        together = []
         for name, (m, v) in state.items():
+            as_is = [m, v]
             m = m.detach().to(torch.float32).contiguous().view(-1)
             v = v.detach().to(torch.float32).contiguous().view(-1)
             if m.numel() != v.numel():
                 raise ValueError("moments of %d and %d elements for '%s'" % (m.numel(), v.numel(), name))
+            if not apart and all(a.is_cuda and a.data_ptr() == b.data_ptr() for a, b in zip(as_is, (m, v))):
+                together.append((name, m, v))
+                continue
             if apart:
                 check(lib().eri_hip_stream_sync(here), "eri_hip_stream_sync")
             check(lib().eri_adam8bit_fn_load_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr(),
@@ -378,6 +386,15 @@ class Adam8bitFunctional:
             if apart:
                 check(lib().eri_hip_stream_sync(self._stream), "eri_hip_stream_sync")
             self._names[name] = None
+        k = len(together)
+        if k:
+            check(lib().eri_adam8bit_fn_load_states_fp32(self._opt, (C.c_char_p * k)(*[n.encode() for n, _, _ in together]),
+                                                         (C.c_void_p * k)(*[m.data_ptr() for _, m, _ in together]),
+                                                         (C.c_void_p * k)(*[v.data_ptr() for _, _, v in together]),
+                                                         (C.c_uint64 * k)(*[m.numel() for _, m, _ in together]), k),
+                  "eri_adam8bit_fn_load_states_fp32")
+            for name, _, _ in together:
+                self._names[name] = None
 
     def close(self) -> None:
         if self._opt:

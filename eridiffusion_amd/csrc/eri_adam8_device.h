@@ -207,16 +207,17 @@ int launch_traffic_probe(const DevTensor *rows, uint32_t n_rows, uint32_t total_
 /* Clears `bytes` bytes at `p`; both multiples of 16. */
 int launch_fill_zero(void *p, size_t bytes, void *stream);
 int launch_state_init(uint8_t *m, uint8_t *v, float *absmax_m, float *absmax_v, uint64_t numel, void *stream);
-/* fp32 moments <-> codes and absmax, one or two moments of `numel` elements in one launch; `small_image` is the device
- * copy of the kSmallImageBytes image. */
-struct MomentArgs {
-    float *x[2];       /* fp32 values: read by quantize, written by dequantize */
-    uint8_t *codes[2];
-    float *absmax[2];
-    int32_t is_signed[2];
+/* fp32 moments <-> codes and absmax, any number of moments in one launch; `small_image` is the device copy of the
+ * kSmallImageBytes image. */
+struct Moment {
+    float *x; /* fp32 values: read by quantize, written by dequantize */
+    uint8_t *codes;
+    float *absmax;
+    uint64_t numel;
+    bool is_signed;
 };
-int launch_dequantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream);
-int launch_quantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream);
+int launch_dequantize(const Moment *moments, uint32_t n, const void *small_image, void *stream);
+int launch_quantize(const Moment *moments, uint32_t n, const void *small_image, void *stream);
 
 /* Row of the plain element-wise sweeps (32-bit AdamW, EMA): up to five streams of one tensor. */
 struct ElemRow {

@@ -200,12 +200,32 @@ int launch_state_init(uint8_t *m, uint8_t *v, float *absmax_m, float *absmax_v, 
 }
 
 /* Checkpoint traffic: fp32 moments to codes and absmax and back.  HBM is the bound, 5 bytes per element (4 of fp32, 1 of
- * code) each way; blockIdx.y is the moment, so that both moments of a tensor are one launch.  One wave takes a
- * 2048-element block: lane l of pass c holds elements c*256 + 4l .. +3, which is one 128-bit access of fp32 and one
- * 32-bit access of codes per lane, both contiguous over the wave.
- * Measured on both moments of 24 tensors, 340 M parameters: quantise 2.84 -> 0.69 ms in all, dequantise 1.51 -> 0.68 ms,
- * 5.0 TB/s each (before: one element per access, IEEE division, an eight-step search, a launch per moment). */
+ * code) each way.  One wave takes a 2048-element block: lane l of pass c holds elements c*256 + 4l .. +3, which is one
+ * 128-bit access of fp32 and one 32-bit access of codes per lane, both contiguous over the wave.
+ * All moments of a call are one launch, their rows in its arguments, a workgroup per four blocks: the hardware starts these
+ * in the order of the list, which keeps the reads and writes of the launch close together.  How close is a matter of how
+ * many run at once, which the LDS they ask for sets: 28,000 bytes beside their tables leave four and five to a unit.
+ * us, quantise and dequantise, both moments; a launch per tensor with a persistent grid | one launch, no LDS beside the
+ * tables | 28,000 bytes | 60,000:
+ *   24 tensors, 340 M parameters   683 + 660 | 570 + 643 | 529 + 600 (6.4 and 5.7 TB/s) | 682 + 656
+ *   30 tensors of a rank-128 adapter, 27 M   175 + 119 |  48 +  49 |  49 +  48 |  65 +  50
+ *   20 tensors of a rank-16 adapter, 2.3 M    97 +  99 |  12 +  13 |  12 +  13 |  13 +  12 */
 constexpr uint32_t kMomentThreads = 256;
+constexpr uint32_t kMomentLds = 28000;
+/* One moment as a launch carries it. */
+struct MomentRow {
+    float *x;
+    uint8_t *codes;
+    float *absmax;
+    uint64_t numel;
+    uint32_t first_wg; // of the launch's workgroups, the first that takes this row
+    uint32_t is_signed;
+};
+constexpr uint32_t kMomentRows = 96; // 3.8 KB of arguments
+struct MomentRows {
+    MomentRow row[kMomentRows];
+    uint32_t n;
+};
 
 /* Pass c of a block of n elements: whole = this lane's four elements exist, else the ones below n - o do. */
 template <bool VEC>
@@ -225,11 +245,8 @@ __device__ __forceinline__ uint32_t small_code(float xs, uint32_t half, const un
 }
 
 template <bool VEC, bool SIGNED>
-__device__ __forceinline__ void quantize_block(const float *x, uint8_t *codes, float *absmax, uint32_t n, uint32_t lane,
+__device__ __forceinline__ void quantize_block(const f32x4 (&v)[8], uint8_t *codes, float *absmax, uint32_t n, uint32_t lane,
                                                const unsigned char *lo, const float *mid) {
-    f32x4 v[8];
-#pragma unroll
-    for (uint32_t c = 0; c < 8; ++c) v[c] = moment_load<VEC>(x, c * 256 + lane * 4, n);
     float a = 0.0f;
 #pragma unroll
     for (uint32_t c = 0; c < 8; ++c)
@@ -261,105 +278,127 @@ __device__ __forceinline__ void quantize_block(const float *x, uint8_t *codes, f
     if (lane == 0) *as_global(absmax) = a;
 }
 
+/* The row of this workgroup and the block of this wave in it. */
+struct MomentBlock {
+    MomentRow row;
+    uint64_t block;
+    size_t e0;
+    uint32_t n; // elements of the block, 0 past the row's last
+    __device__ __forceinline__ explicit MomentBlock(const MomentRows &rows) {
+        uint32_t lo = 0, hi = rows.n; // row[lo].first_wg <= blockIdx.x
+        while (hi - lo > 1) {
+            const uint32_t at = (lo + hi) >> 1;
+            if (rows.row[at].first_wg <= blockIdx.x) lo = at; else hi = at;
+        }
+        row = rows.row[lo];
+        block = (uint64_t)(blockIdx.x - row.first_wg) * (kMomentThreads / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        e0 = block * kBlock;
+        n = e0 >= row.numel ? 0u : row.numel - e0 < kBlock ? (uint32_t)(row.numel - e0) : kBlock;
+    }
+};
+
 template <bool VEC>
-__global__ __launch_bounds__(kMomentThreads) void quantize_kernel(MomentArgs args, uint64_t numel, uint64_t nblocks,
-                                                                  const unsigned char *__restrict__ image) {
+__global__ __launch_bounds__(kMomentThreads) void quantize_kernel(MomentRows rows, const unsigned char *__restrict__ image) {
     __shared__ float mid[256];
     __shared__ uint4 lo_words[kSKeyCount / 16]; // bytes, staged in 16-byte words and aligned for them
     const unsigned char *lo = reinterpret_cast<const unsigned char *>(lo_words);
     static_assert(kSKeyCount == kUKeyCount && kSKeyCount == 16 * kMomentThreads, "one 16-byte word per thread");
-    const uint32_t which = blockIdx.y;
-    const bool is_signed = args.is_signed[which] != 0;
+    const MomentBlock b(rows);
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    f32x4 v[8];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) v[c] = moment_load<VEC>(b.row.x + b.e0, c * 256 + lane * 4, b.n);
+    const bool is_signed = b.row.is_signed != 0;
     mid[threadIdx.x] = reinterpret_cast<const float *>(image + (is_signed ? kSmallMidS : kSmallMidU))[threadIdx.x];
     lo_words[threadIdx.x] = reinterpret_cast<const uint4 *>(image + (is_signed ? kSmallLoS : kSmallLoU))[threadIdx.x];
     __syncthreads();
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kMomentThreads / kWave) + threadIdx.x / kWave);
-    const uint64_t stride = (uint64_t)gridDim.x * (kMomentThreads / kWave);
-    for (uint64_t b = wave; b < nblocks; b += stride) {
-        const uint64_t e0 = b * kBlock;
-        const uint32_t n = (uint32_t)((numel - e0) < kBlock ? (numel - e0) : kBlock);
-        if (is_signed) quantize_block<VEC, true>(args.x[which] + e0, args.codes[which] + e0, args.absmax[which] + b, n, lane, lo, mid);
-        else quantize_block<VEC, false>(args.x[which] + e0, args.codes[which] + e0, args.absmax[which] + b, n, lane, lo, mid);
-    }
+    if (b.n == 0) return;
+    if (is_signed) quantize_block<VEC, true>(v, b.row.codes + b.e0, b.row.absmax + b.block, b.n, lane, lo, mid);
+    else quantize_block<VEC, false>(v, b.row.codes + b.e0, b.row.absmax + b.block, b.n, lane, lo, mid);
 }
 
 template <bool VEC>
-__global__ __launch_bounds__(kMomentThreads) void dequantize_kernel(MomentArgs args, uint64_t numel, uint64_t nblocks,
-                                                                    const unsigned char *__restrict__ image) {
+__global__ __launch_bounds__(kMomentThreads) void dequantize_kernel(MomentRows rows, const unsigned char *__restrict__ image) {
     __shared__ float map[256];
-    const uint32_t which = blockIdx.y;
-    map[threadIdx.x] = reinterpret_cast<const float *>(image + (args.is_signed[which] ? kSmallMapS : kSmallMapU))[threadIdx.x];
-    __syncthreads();
+    const MomentBlock b(rows);
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint64_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (kMomentThreads / kWave) + threadIdx.x / kWave);
-    const uint64_t stride = (uint64_t)gridDim.x * (kMomentThreads / kWave);
-    for (uint64_t b = wave; b < nblocks; b += stride) {
-        const uint64_t e0 = b * kBlock;
-        const uint32_t n = (uint32_t)((numel - e0) < kBlock ? (numel - e0) : kBlock);
-        const uint8_t *codes = args.codes[which] + e0;
-        float *out = args.x[which] + e0;
-        const float a = as_global(args.absmax[which])[b];
-        uint32_t w[8];
+    const uint8_t *codes = b.row.codes + b.e0;
+    uint32_t w[8];
 #pragma unroll
-        for (uint32_t c = 0; c < 8; ++c) {
-            const uint32_t o = c * 256 + lane * 4;
-            if (VEC && o + 4 <= n) {
-                w[c] = __builtin_nontemporal_load(as_global(reinterpret_cast<const uint32_t *>(codes + o)));
-            } else {
-                w[c] = 0;
+    for (uint32_t c = 0; c < 8; ++c) {
+        const uint32_t o = c * 256 + lane * 4;
+        w[c] = 0;
+        if (VEC && o + 4 <= b.n) {
+            w[c] = __builtin_nontemporal_load(as_global(reinterpret_cast<const uint32_t *>(codes + o)));
+        } else {
 #pragma unroll
-                for (uint32_t k = 0; k < 4; ++k)
-                    if (o + k < n) w[c] |= (uint32_t)as_global(codes)[o + k] << (8 * k);
-            }
+            for (uint32_t k = 0; k < 4; ++k)
+                if (o + k < b.n) w[c] |= (uint32_t)as_global(codes)[o + k] << (8 * k);
         }
+    }
+    map[threadIdx.x] = reinterpret_cast<const float *>(image + (b.row.is_signed ? kSmallMapS : kSmallMapU))[threadIdx.x];
+    __syncthreads();
+    if (b.n == 0) return;
+    const float a = as_global(b.row.absmax)[b.block];
+    float *out = b.row.x + b.e0;
 #pragma unroll
-        for (uint32_t c = 0; c < 8; ++c) {
-            const uint32_t o = c * 256 + lane * 4;
-            const f32x4 r = {map[w[c] & 0xffu] * a, map[(w[c] >> 8) & 0xffu] * a, map[(w[c] >> 16) & 0xffu] * a, map[w[c] >> 24] * a};
-            if (VEC && o + 4 <= n) {
-                __builtin_nontemporal_store(r, as_global(reinterpret_cast<f32x4 *>(out + o)));
-            } else {
+    for (uint32_t c = 0; c < 8; ++c) {
+        const uint32_t o = c * 256 + lane * 4;
+        const f32x4 r = {map[w[c] & 0xffu] * a, map[(w[c] >> 8) & 0xffu] * a, map[(w[c] >> 16) & 0xffu] * a, map[w[c] >> 24] * a};
+        if (VEC && o + 4 <= b.n) {
+            __builtin_nontemporal_store(r, as_global(reinterpret_cast<f32x4 *>(out + o)));
+        } else {
 #pragma unroll
-                for (uint32_t k = 0; k < 4; ++k)
-                    if (o + k < n) as_global(out)[o + k] = r[k];
-            }
+            for (uint32_t k = 0; k < 4; ++k)
+                if (o + k < b.n) as_global(out)[o + k] = r[k];
         }
     }
 }
 
 /* Whole words need fp32 pointers on 16 bytes and code pointers on 4 (the optimizers' states and every allocator's
- * buffers are); other addresses take the same kernels element by element. */
-static bool moments_aligned(const MomentArgs &a, uint32_t moments) {
+ * buffers are); a launch with other addresses takes the same kernels element by element. */
+static bool moments_aligned(const MomentRows &rows) {
     uintptr_t wide = 0, codes = 0;
-    for (uint32_t i = 0; i < moments; ++i) {
-        wide |= (uintptr_t)a.x[i];
-        codes |= (uintptr_t)a.codes[i];
+    for (uint32_t i = 0; i < rows.n; ++i) {
+        wide |= (uintptr_t)rows.row[i].x;
+        codes |= (uintptr_t)rows.row[i].codes;
     }
     return (wide & 15u) == 0 && (codes & 3u) == 0;
 }
 
-/* Workgroups of four waves, up to eight per compute unit over both moments: 32 waves fill its wave slots. */
-static dim3 moments_grid(uint64_t nblocks, uint32_t moments, uint32_t compute_units) {
-    uint64_t grid = (nblocks + 3) / 4;
-    const uint64_t cap = (uint64_t)compute_units * 8 / moments;
-    return dim3((uint32_t)(grid < cap ? grid : cap), moments);
+/* Rows as far as they fit one launch's arguments and grid, then the rest. */
+static int launch_moments(bool quantize, const Moment *moments, uint32_t n, const void *small_image, hipStream_t s) {
+    constexpr uint64_t kWgBlocks = kMomentThreads / kWave, kMaxWgs = 0x7fffffffu / kMomentThreads;
+    const unsigned char *image = static_cast<const unsigned char *>(small_image);
+    uint32_t i = 0;
+    while (i < n) {
+        MomentRows rows;
+        rows.n = 0;
+        uint64_t wgs = 0;
+        for (; i < n && rows.n < kMomentRows; ++i) {
+            const uint64_t need = ((moments[i].numel + kBlock - 1) / kBlock + kWgBlocks - 1) / kWgBlocks;
+            if (wgs + need > kMaxWgs) {
+                if (rows.n == 0) return (int)hipErrorInvalidValue; // one moment of 2^36 elements and more
+                break;
+            }
+            rows.row[rows.n++] = {moments[i].x, moments[i].codes, moments[i].absmax, moments[i].numel, (uint32_t)wgs, moments[i].is_signed ? 1u : 0u};
+            wgs += need;
+        }
+        const bool vec = moments_aligned(rows);
+        const auto k = quantize ? (vec ? quantize_kernel<true> : quantize_kernel<false>) : (vec ? dequantize_kernel<true> : dequantize_kernel<false>);
+        hipLaunchKernelGGL(k, dim3((uint32_t)wgs), dim3(kMomentThreads), kMomentLds, s, rows, image);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+    }
+    return 0;
 }
 
-int launch_dequantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream) {
-    const uint64_t nblocks = (numel + kBlock - 1) / kBlock;
-    const auto k = moments_aligned(a, moments) ? dequantize_kernel<true> : dequantize_kernel<false>;
-    hipLaunchKernelGGL(k, moments_grid(nblocks, moments, compute_units), dim3(kMomentThreads), 0, static_cast<hipStream_t>(stream), a, numel,
-                       nblocks, static_cast<const unsigned char *>(small_image));
-    return (int)hipGetLastError();
+int launch_dequantize(const Moment *moments, uint32_t n, const void *small_image, void *stream) {
+    return launch_moments(false, moments, n, small_image, static_cast<hipStream_t>(stream));
 }
 
-int launch_quantize(const MomentArgs &a, uint32_t moments, uint64_t numel, const void *small_image, uint32_t compute_units, void *stream) {
-    const uint64_t nblocks = (numel + kBlock - 1) / kBlock;
-    const auto k = moments_aligned(a, moments) ? quantize_kernel<true> : quantize_kernel<false>;
-    hipLaunchKernelGGL(k, moments_grid(nblocks, moments, compute_units), dim3(kMomentThreads), 0, static_cast<hipStream_t>(stream), a, numel,
-                       nblocks, static_cast<const unsigned char *>(small_image));
-    return (int)hipGetLastError();
+int launch_quantize(const Moment *moments, uint32_t n, const void *small_image, void *stream) {
+    return launch_moments(true, moments, n, small_image, static_cast<hipStream_t>(stream));
 }
 
 // ------------------------------------------------------------------------------------------

@@ -1611,37 +1611,82 @@ int eri_adam8bit_fn_state_numel(const EriAdam8bitFn *o, const char *name, uint64
 
 int eri_adam8bit_fn_get_state_fp32(EriAdam8bitFn *o, const char *name, float *m_out, float *v_out) {
     if (!o || !name || !m_out || !v_out) return fail(ERI_ERR_NULL, "NULL argument");
+    return eri_adam8bit_fn_get_states_fp32(o, &name, &m_out, &v_out, 1);
+}
+
+int eri_adam8bit_fn_get_states_fp32(EriAdam8bitFn *o, const char *const *names, float *const *m_out, float *const *v_out, uint32_t n) {
+    if (!o || !names || !m_out || !v_out) return fail(ERI_ERR_NULL, "NULL argument");
+    if (n == 0) return 0;
     int rc = fn_flush(o);
     if (rc) return rc;
-    auto it = o->states.find(std::string_view(name));
-    if (it == o->states.end()) return fail(ERI_ERR_ARG, std::string("no optimizer state named '") + name + "'");
-    State8 &s = *it->second;
-    return eri_adam8_dequantize_state(s.m, s.v, s.absmax_m, s.absmax_v, s.numel, m_out, v_out, o->stream);
+    std::vector<EriMomentTensor> rows;
+    rows.reserve(n);
+    for (uint32_t i = 0; i < n; ++i) {
+        if (!names[i] || !m_out[i] || !v_out[i]) return fail(ERI_ERR_NULL, "NULL argument");
+        auto it = o->states.find(std::string_view(names[i]));
+        if (it == o->states.end()) return fail(ERI_ERR_ARG, std::string("no optimizer state named '") + names[i] + "'");
+        State8 &s = *it->second;
+        rows.push_back({m_out[i], v_out[i], s.m, s.v, s.absmax_m, s.absmax_v, s.numel});
+    }
+    return eri_adam8_dequantize_states(rows.data(), n, o->stream);
 }
 
 int eri_adam8bit_fn_load_state_fp32(EriAdam8bitFn *o, const char *name, const float *m, const float *v,
                                     uint64_t numel) {
     if (!o || !name || !m || !v) return fail(ERI_ERR_NULL, "NULL argument");
-    if (numel == 0) return fail(ERI_ERR_EMPTY, "InvalidOperation: Empty tensor for quantization");
+    return eri_adam8bit_fn_load_states_fp32(o, &name, &m, &v, &numel, 1);
+}
+
+int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names, const float *const *m, const float *const *v,
+                                     const uint64_t *numels, uint32_t n) {
+    if (!o || !names || !m || !v || !numels) return fail(ERI_ERR_NULL, "NULL argument");
+    for (uint32_t i = 0; i < n; ++i) {
+        if (!names[i] || !m[i] || !v[i]) return fail(ERI_ERR_NULL, "NULL argument");
+        if (numels[i] == 0) return fail(ERI_ERR_EMPTY, "InvalidOperation: Empty tensor for quantization");
+    }
+    if (n == 0) return 0;
     int rc = fn_flush(o);
     if (rc) return rc;
-    // A state of this size that exists already, where new states would be made too, takes the new contents where it is, in stream order behind the steps
-    // that still use the old ones: no allocation and no release, each of which waits for the device (24 tensors of
-    // 340 M parameters loaded and read back: 33.8 -> 1.34 ms).
-    auto it = o->states.find(std::string_view(name));
-    if (it != o->states.end() && it->second->numel == numel && it->second->pool == o->state_pool &&
-        (!o->state_pool || it->second->pool_lane == o->state_lane)) {
-        State8 &s = *it->second;
-        return eri_adam8_quantize_state(m, v, numel, s.m, s.v, s.absmax_m, s.absmax_v, o->stream);
+    // A state of this size that exists already, where new states would be made too, takes the new contents where it is,
+    // in stream order behind the steps that still use the old ones: no allocation and no release, each of which waits for
+    // the device (24 tensors of 340 M parameters loaded and read back: 33.8 -> 1.34 ms).  The others get a new state,
+    // which takes its name once the conversion has been launched.
+    std::vector<EriMomentTensor> rows;
+    std::vector<std::pair<uint32_t, std::unique_ptr<FnState>>> made;
+    const uint64_t loading = ++o->generation; // no row of the last batch is queued any more (fn_flush)
+    auto launch = [&]() -> int {
+        if (rows.empty()) return 0;
+        const int e = eri_adam8_quantize_states(rows.data(), (uint32_t)rows.size(), o->stream);
+        if (e) return e;
+        if (!made.empty()) o->last_order.clear(); // it may hold a state that is replaced here
+        for (auto &kv : made) o->states[names[kv.first]] = std::move(kv.second);
+        rows.clear();
+        made.clear();
+        return 0;
+    };
+    for (uint32_t i = 0; i < n; ++i) {
+        auto it = o->states.find(std::string_view(names[i]));
+        bool again = it != o->states.end() && it->second->queued_in == loading;
+        for (size_t k = 0; !again && k < made.size(); ++k) again = std::strcmp(names[made[k].first], names[i]) == 0;
+        if (again) { // a name twice in one call: the first contents are replaced in order
+            rc = launch();
+            if (rc) return rc;
+            it = o->states.find(std::string_view(names[i]));
+        }
+        FnState *s = it == o->states.end() ? nullptr : it->second.get();
+        if (!s || s->numel != numels[i] || s->pool != o->state_pool || (o->state_pool && s->pool_lane != o->state_lane)) {
+            std::unique_ptr<FnState> fresh(new FnState());
+            rc = fresh->allocate(numels[i], o->stream, o->state_pool, o->state_lane);
+            if (rc) return rc;
+            s = fresh.get();
+            made.emplace_back(i, std::move(fresh));
+        }
+        s->queued_in = loading;
+        rows.push_back({const_cast<float *>(m[i]), const_cast<float *>(v[i]), s->m, s->v, s->absmax_m, s->absmax_v, numels[i]});
     }
-    o->last_order.clear(); // it may hold the state that is replaced below
-    std::unique_ptr<FnState> s(new FnState());
-    rc = s->allocate(numel, o->stream, o->state_pool, o->state_lane);
-    if (rc) return rc;
-    rc = eri_adam8_quantize_state(m, v, numel, s->m, s->v, s->absmax_m, s->absmax_v, o->stream);
-    if (rc) return rc;
-    o->states[name] = std::move(s);
-    return 0;
+    rc = launch();
+    o->generation += 1; // the marks above are not those of the next batch
+    return rc;
 }
 
 // ---- helpers beside the optimizers ------------------------------------------------------------

@@ -1363,63 +1363,67 @@ int eri_adam8_step_multi(const EriAdam8Tensor *rows, uint32_t n, const EriAdam8H
     return eri_adam8_step_table(cache.table, h, stream);
 }
 
-static int dequantize(const eri::MomentArgs &a, uint32_t moments, uint64_t numel, void *stream) {
-    for (uint32_t i = 0; i < moments; ++i)
-        if (!a.codes[i] || !a.absmax[i] || !a.x[i]) return fail(ERI_ERR_NULL, "dequantize with NULL pointer");
-    if (numel == 0) return fail(ERI_ERR_EMPTY, "Empty quantized data");
+/* Everything is checked before the first launch: a refused call converts nothing. */
+static int convert_moments(bool quantize, const std::vector<eri::Moment> &moments, void *stream) {
+    const char *what = quantize ? "quantize" : "dequantize";
+    for (const auto &m : moments) {
+        if (!m.x || !m.codes || !m.absmax) return fail(ERI_ERR_NULL, std::string(what) + " with NULL pointer");
+        if (m.numel == 0) return fail(ERI_ERR_EMPTY, quantize ? "Empty tensor for quantization" : "Empty quantized data");
+    }
     DeviceCtx *ctx = nullptr;
     int rc = get_ctx(&ctx);
-    for (uint32_t i = 0; i < moments && rc == 0; ++i) {
-        rc = require_kernel_visible(a.codes[i], "dequantize: codes");
-        if (rc == 0) rc = require_kernel_visible(a.absmax[i], "dequantize: absmax");
-        if (rc == 0) rc = require_kernel_visible(a.x[i], "dequantize: out");
+    for (const auto &m : moments) {
+        if (rc == 0) rc = require_kernel_visible(m.x, quantize ? "quantize: x" : "dequantize: out");
+        if (rc == 0) rc = require_kernel_visible(m.codes, quantize ? "quantize: codes" : "dequantize: codes");
+        if (rc == 0) rc = require_kernel_visible(m.absmax, quantize ? "quantize: absmax" : "dequantize: absmax");
     }
     if (rc) return rc;
-    rc = eri::launch_dequantize(a, moments, numel, ctx->small_image, ctx->cus, stream);
-    if (rc) return hip_fail((hipError_t)rc, "dequantize launch");
-    return 0;
-}
-
-static int quantize(const eri::MomentArgs &a, uint32_t moments, uint64_t numel, void *stream) {
-    for (uint32_t i = 0; i < moments; ++i)
-        if (!a.x[i] || !a.codes[i] || !a.absmax[i]) return fail(ERI_ERR_NULL, "quantize with NULL pointer");
-    if (numel == 0) return fail(ERI_ERR_EMPTY, "Empty tensor for quantization");
-    DeviceCtx *ctx = nullptr;
-    int rc = get_ctx(&ctx);
-    for (uint32_t i = 0; i < moments && rc == 0; ++i) {
-        rc = require_kernel_visible(a.x[i], "quantize: x");
-        if (rc == 0) rc = require_kernel_visible(a.codes[i], "quantize: codes");
-        if (rc == 0) rc = require_kernel_visible(a.absmax[i], "quantize: absmax");
-    }
-    if (rc) return rc;
-    rc = eri::launch_quantize(a, moments, numel, ctx->small_image, ctx->cus, stream);
-    if (rc) return hip_fail((hipError_t)rc, "quantize launch");
+    rc = quantize ? eri::launch_quantize(moments.data(), (uint32_t)moments.size(), ctx->small_image, stream)
+                  : eri::launch_dequantize(moments.data(), (uint32_t)moments.size(), ctx->small_image, stream);
+    if (rc) return hip_fail((hipError_t)rc, quantize ? "quantize launch" : "dequantize launch");
     return 0;
 }
 
 int eri_adam8_dequantize(const uint8_t *codes, const float *absmax, int signed_map, uint64_t numel, float *out,
                          void *stream) {
-    const eri::MomentArgs a = {{out, nullptr}, {const_cast<uint8_t *>(codes), nullptr}, {const_cast<float *>(absmax), nullptr}, {signed_map != 0, 0}};
-    return dequantize(a, 1, numel, stream);
+    return convert_moments(false, {{out, const_cast<uint8_t *>(codes), const_cast<float *>(absmax), numel, signed_map != 0}}, stream);
 }
 
 int eri_adam8_quantize(const float *x, int signed_map, uint64_t numel, uint8_t *codes, float *absmax, void *stream) {
-    const eri::MomentArgs a = {{const_cast<float *>(x), nullptr}, {codes, nullptr}, {absmax, nullptr}, {signed_map != 0, 0}};
-    return quantize(a, 1, numel, stream);
+    return convert_moments(true, {{const_cast<float *>(x), codes, absmax, numel, signed_map != 0}}, stream);
+}
+
+static void both_moments(const EriMomentTensor &t, std::vector<eri::Moment> &out) {
+    out.push_back({t.m32, t.m, t.absmax_m, t.numel, true});
+    out.push_back({t.v32, t.v, t.absmax_v, t.numel, false});
 }
 
 int eri_adam8_dequantize_state(const uint8_t *m, const uint8_t *v, const float *absmax_m, const float *absmax_v, uint64_t numel,
                                float *m_out, float *v_out, void *stream) {
-    const eri::MomentArgs a = {{m_out, v_out}, {const_cast<uint8_t *>(m), const_cast<uint8_t *>(v)},
-                               {const_cast<float *>(absmax_m), const_cast<float *>(absmax_v)}, {1, 0}};
-    return dequantize(a, 2, numel, stream);
+    std::vector<eri::Moment> moments;
+    both_moments({m_out, v_out, const_cast<uint8_t *>(m), const_cast<uint8_t *>(v), const_cast<float *>(absmax_m), const_cast<float *>(absmax_v), numel}, moments);
+    return convert_moments(false, moments, stream);
 }
 
 int eri_adam8_quantize_state(const float *m_in, const float *v_in, uint64_t numel, uint8_t *m, uint8_t *v, float *absmax_m,
                              float *absmax_v, void *stream) {
-    const eri::MomentArgs a = {{const_cast<float *>(m_in), const_cast<float *>(v_in)}, {m, v}, {absmax_m, absmax_v}, {1, 0}};
-    return quantize(a, 2, numel, stream);
+    std::vector<eri::Moment> moments;
+    both_moments({const_cast<float *>(m_in), const_cast<float *>(v_in), m, v, absmax_m, absmax_v, numel}, moments);
+    return convert_moments(true, moments, stream);
 }
+
+static int convert_states(bool quantize, const EriMomentTensor *tensors, uint32_t n, void *stream) {
+    if (!tensors) return fail(ERI_ERR_NULL, "tensors is NULL");
+    if (n == 0) return fail(ERI_ERR_ARG, "no tensors");
+    std::vector<eri::Moment> moments;
+    moments.reserve(2 * (size_t)n);
+    for (uint32_t i = 0; i < n; ++i) both_moments(tensors[i], moments);
+    return convert_moments(quantize, moments, stream);
+}
+
+int eri_adam8_dequantize_states(const EriMomentTensor *tensors, uint32_t n, void *stream) { return convert_states(false, tensors, n, stream); }
+
+int eri_adam8_quantize_states(const EriMomentTensor *tensors, uint32_t n, void *stream) { return convert_states(true, tensors, n, stream); }
 
 } // extern "C"
 

@@ -56,6 +56,9 @@ pub struct EriEmaTensor { pub shadow: *mut c_void, pub p: *const c_void, pub num
 
 #[repr(C)]
 #[derive(Clone, Copy)]
+pub struct EriMomentTensor { pub m32: *mut f32, pub v32: *mut f32, pub m: *mut u8, pub v: *mut u8, pub absmax_m: *mut f32, pub absmax_v: *mut f32, pub numel: u64 }
+#[repr(C)]
+#[derive(Clone, Copy)]
 pub struct EriOptimizerMemoryReport { pub num_params: u64, pub param_memory_gb: f64, pub state_memory_gb: f64, pub total_memory_gb: f64,
     pub memory_reduction_percent: f64, pub has_reduction: i32, pub description: [c_char; 44] }
 
@@ -120,6 +123,8 @@ extern "C" {
     pub fn eri_adam8_dequantize(codes: *const u8, absmax: *const f32, signed_map: c_int, numel: u64, out: *mut f32, stream: *mut c_void) -> c_int;
     pub fn eri_adam8_quantize(x: *const f32, signed_map: c_int, numel: u64, codes: *mut u8, absmax: *mut f32, stream: *mut c_void) -> c_int;
     pub fn eri_adam8_dequantize_state(m: *const u8, v: *const u8, absmax_m: *const f32, absmax_v: *const f32, numel: u64, m_out: *mut f32, v_out: *mut f32, stream: *mut c_void) -> c_int;
+    pub fn eri_adam8_dequantize_states(tensors: *const EriMomentTensor, n: u32, stream: *mut c_void) -> c_int;
+    pub fn eri_adam8_quantize_states(tensors: *const EriMomentTensor, n: u32, stream: *mut c_void) -> c_int;
     pub fn eri_adam8_quantize_state(m_in: *const f32, v_in: *const f32, numel: u64, m: *mut u8, v: *mut u8, absmax_m: *mut f32, absmax_v: *mut f32, stream: *mut c_void) -> c_int;
     // 32-bit sibling and EMA sweep
     pub fn eri_adamw32_step_multi(rows: *const EriAdamW32Tensor, n: u32, hyper: *const EriAdamW32Hyper, stream: *mut c_void) -> c_int;
@@ -187,4 +192,6 @@ extern "C" {
     pub fn eri_adam8bit_fn_state_numel(opt: *const EriAdam8bitFn, name: *const c_char, numel: *mut u64) -> c_int;
     pub fn eri_adam8bit_fn_get_state_fp32(opt: *mut EriAdam8bitFn, name: *const c_char, m_out: *mut f32, v_out: *mut f32) -> c_int;
     pub fn eri_adam8bit_fn_load_state_fp32(opt: *mut EriAdam8bitFn, name: *const c_char, m: *const f32, v: *const f32, numel: u64) -> c_int;
+    pub fn eri_adam8bit_fn_get_states_fp32(opt: *mut EriAdam8bitFn, names: *const *const c_char, m_out: *const *mut f32, v_out: *const *mut f32, n: u32) -> c_int;
+    pub fn eri_adam8bit_fn_load_states_fp32(opt: *mut EriAdam8bitFn, names: *const *const c_char, m: *const *const f32, v: *const *const f32, numels: *const u64, n: u32) -> c_int;
 }

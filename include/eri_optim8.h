@@ -333,6 +333,19 @@ int eri_adam8_dequantize_state(const uint8_t *m, const uint8_t *v, const float *
                                uint64_t numel, float *m_out, float *v_out, void *stream);
 int eri_adam8_quantize_state(const float *m_in, const float *v_in, uint64_t numel, uint8_t *m, uint8_t *v,
                              float *absmax_m, float *absmax_v, void *stream);
+/* Both moments of any number of tensors, up to 48 of them in one launch.  Nothing is launched if any pointer is
+ * refused.  No two of the tensors may share what the call writes. */
+typedef struct EriMomentTensor {
+    float *m32;  /* fp32 moments: read by quantize, written by dequantize */
+    float *v32;
+    uint8_t *m;  /* the state: written by quantize, read by dequantize */
+    uint8_t *v;
+    float *absmax_m;
+    float *absmax_v;
+    uint64_t numel;
+} EriMomentTensor;
+int eri_adam8_dequantize_states(const EriMomentTensor *tensors, uint32_t n, void *stream);
+int eri_adam8_quantize_states(const EriMomentTensor *tensors, uint32_t n, void *stream);
 
 /* ---------------------------------------------------------------------------------------------
  * 32-bit sibling: fused multi-tensor AdamW with fp32 moments, for tensors kept out of the 8-bit

@@ -94,3 +94,53 @@ def test_loading_moments_of_the_same_size_keeps_the_state_where_it_is():
     assert L.lib().eri_adam8bit_fn_load_state_fp32(used._opt, b"w", p.data_ptr(), host.ctypes.data, n) == -6
     after = used.get_state_as_tensors()["w"]
     assert torch.equal(before[0], after[0]) and torch.equal(before[1], after[1])
+
+
+@pytest.mark.parametrize("names", [3, 48, 49, 130])
+@pytest.mark.parametrize("pooled", [False, True])
+def test_many_states_in_one_call(names, pooled):
+    """Fewer tensors than one launch takes, as many, one more, and three launches; sizes around the four blocks of a
+    workgroup, one pair of moments at an odd address; against the same calls name by name, bit for bit, on an optimizer
+    that has the states already and on one that makes them."""
+    import torch
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
+    gen = torch.Generator(device="cuda").manual_seed(names)
+    sizes = [(5, 2047, 2048, 2049, 4 * 2048, 4 * 2048 + 1, 8 * 2048 - 3)[i % 7] + 3 * i for i in range(names)]
+    state = {"n%d" % i: (torch.randn(n, device="cuda", generator=gen) * 1e-3, torch.rand(n, device="cuda", generator=gen) * 1e-6)
+             for i, n in enumerate(sizes)}
+    state["n1"] = tuple(torch.cat([x.new_zeros(1), x])[1:] for x in state["n1"])
+    one, many = Adam8bitFunctional(), Adam8bitFunctional()
+    if pooled:
+        many.set_state_pool(DevicePool(64 << 20, 1), 0)
+    for name, moments in state.items():
+        one.load_state_from_tensors({name: moments})
+    for _ in range(2):
+        many.load_state_from_tensors(state)
+        a, b = one.get_state_as_tensors(), many.get_state_as_tensors()
+        assert list(a) == list(b) == list(state)
+        for name in state:
+            assert torch.equal(a[name][0], b[name][0]) and torch.equal(a[name][1], b[name][1]), name
+
+
+def test_a_name_twice_in_one_load_keeps_its_last_contents():
+    import ctypes as C
+    import torch
+    from eridiffusion_amd import _lib as L
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    n = 5000
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    xs = [torch.rand(n, device="cuda", generator=gen) for _ in range(6)]
+    opt, want = Adam8bitFunctional(), Adam8bitFunctional()
+    names = (C.c_char_p * 3)(b"a", b"b", b"a")
+    ptr = [(C.c_void_p * 3)(*[x.data_ptr() for x in xs[k::2]]) for k in (0, 1)]
+    for _ in range(2):  # states that the call makes, then states that are there
+        L.check(L.lib().eri_adam8bit_fn_load_states_fp32(opt._opt, names, ptr[0], ptr[1], (C.c_uint64 * 3)(n, n, n), 3), "load")
+        opt._names.update({"a": None, "b": None})
+        want.load_state_from_tensors({"a": (xs[4], xs[5]), "b": (xs[2], xs[3])})
+        for name, moments in want.get_state_as_tensors().items():
+            assert all(torch.equal(x, y) for x, y in zip(opt.get_state_as_tensors()[name], moments)), name
+    out = torch.empty(n, device="cuda")
+    unknown = (C.c_void_p * 2)(out.data_ptr(), out.data_ptr())
+    out.fill_(5.0)
+    assert L.lib().eri_adam8bit_fn_get_states_fp32(opt._opt, (C.c_char_p * 2)(b"a", b"nobody"), unknown, unknown, 2) == -6
+    assert bool((out == 5.0).all())  # nothing of a refused call runs
