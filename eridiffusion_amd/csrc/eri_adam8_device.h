@@ -33,6 +33,16 @@ static_assert(sizeof(DevTensor) == 80, "DevTensor must stay 80 bytes");
  * between launches, alone in its cache line. */
 constexpr uint32_t kTableHead = 256;
 
+/* New addresses for rows of a launch table, as a launch carries them in its arguments. */
+struct RowAddresses {
+    void *p;
+    const void *p_in;
+    const void *g;
+};
+constexpr uint32_t kAddressRows = 160, kGradRows = 480; /* 3.8 KB of arguments either way */
+int launch_set_addresses(DevTensor *rows, const RowAddresses *a, uint32_t n, void *stream);
+int launch_set_gradients(DevTensor *rows, const void *const *g, uint32_t n, void *stream);
+
 /* How the elements of one group of rows are stored: parameters and gradients F32, both BF16, or BF16
  * parameters with F32 gradients (the reference casts every gradient to F32 and never rounds it). */
 enum Layout { kLayoutF32 = 0, kLayoutBF16 = 1, kLayoutBF16GradF32 = 2, kLayouts = 3 };

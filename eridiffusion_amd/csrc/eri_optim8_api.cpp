@@ -314,7 +314,8 @@ struct EriAdam8Table {
     std::vector<uint64_t> numel;
     std::vector<int32_t> dtype; // per row: its layout
     hipEvent_t uploaded = nullptr;
-    bool upload_pending = false;
+    bool upload_pending = false;    // the copy behind `uploaded` may still be on its way
+    bool set_pending = false;       // addresses have been set by a launch on upload_stream that `uploaded` does not cover yet
     void *upload_stream = nullptr;  // stream of the last upload
     void *ordered_stream = nullptr; // another stream that has already been made to wait for that upload
     bool ordered_valid = false;
@@ -415,6 +416,7 @@ int upload(EriAdam8Table *t, void *stream) {
     }
     ERI_HIP(hipEventRecord(t->uploaded, static_cast<hipStream_t>(stream)));
     t->upload_pending = true;
+    t->set_pending = false;
     t->upload_stream = stream;
     t->ordered_valid = false;
     return 0;
@@ -463,8 +465,18 @@ struct Readers {
  * captured into a graph cannot wait for an event outside the graph, so there the host waits for the
  * upload instead, once. */
 int order_after_upload(EriAdam8Table *t, void *stream) {
-    if (!t->upload_pending || stream == t->upload_stream) return 0;
+    if ((!t->upload_pending && !t->set_pending) || stream == t->upload_stream) return 0;
     if (t->ordered_valid && stream == t->ordered_stream) return 0;
+    if (t->set_pending) { // no event was recorded behind the launch: nobody but another stream needs one
+        if (hipEventRecord(t->uploaded, static_cast<hipStream_t>(t->upload_stream)) != hipSuccess) { // a stream destroyed since
+            (void)hipGetLastError();
+            ERI_HIP(hipDeviceSynchronize());
+            t->upload_pending = t->set_pending = false;
+            return 0;
+        }
+        t->upload_pending = true;
+        t->set_pending = false;
+    }
     if (is_capturing(stream)) {
         const hipError_t e = hipEventSynchronize(t->uploaded);
         if (e != hipSuccess) {
@@ -1027,9 +1039,44 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
         ERI_HIP(hipEventSynchronize(t->uploaded));
         t->upload_pending = false;
     }
+    // Where only addresses change, and in no more rows than two launches carry per group, a launch sets them: the rows
+    // need no copy, no event and no wait for the copy before.
+    bool set = true;
+    std::vector<eri::RowAddresses> to[eri::kLayouts];
+    bool grads_alone[eri::kLayouts];
+    for (int li = 0; li < eri::kLayouts && set; ++li) {
+        const auto &g = t->groups[li];
+        grads_alone[li] = true;
+        for (uint32_t j = 0; j < g.n && set; ++j) {
+            const EriAdam8Tensor &r = rows[g.src[j]];
+            const eri::DevTensor &d = g.pinned[j];
+            set = d.m == r.m && d.v == r.v && d.absmax_m == r.absmax_m && d.absmax_v == r.absmax_v && d.shadow == r.ema_shadow &&
+                  std::memcmp(&d.grad_scale, &r.grad_scale, sizeof d.grad_scale) == 0;
+            const void *p_in = r.p_src ? r.p_src : r.p;
+            if (d.p != r.p || d.p_in != p_in) grads_alone[li] = false;
+            to[li].push_back({r.p, p_in, r.g});
+        }
+        if (g.n > 2 * (grads_alone[li] ? eri::kGradRows : eri::kAddressRows)) set = false;
+    }
     for (auto &g : t->groups)
         if (g.n) fill_group(g, rows);
-    return upload(t, stream);
+    if (!set) return upload(t, stream);
+    for (int li = 0; li < eri::kLayouts; ++li) {
+        auto &g = t->groups[li];
+        if (g.n == 0) continue;
+        if (grads_alone[li]) {
+            std::vector<const void *> grads(g.n);
+            for (uint32_t j = 0; j < g.n; ++j) grads[j] = to[li][j].g;
+            rc = eri::launch_set_gradients(g.dev, grads.data(), g.n, stream);
+        } else {
+            rc = eri::launch_set_addresses(g.dev, to[li].data(), g.n, stream);
+        }
+        if (rc) return hip_fail((hipError_t)rc, "launch table update");
+    }
+    t->set_pending = true;
+    t->upload_stream = stream;
+    t->ordered_valid = false;
+    return 0;
 }
 
 int eri_adam8_table_destroy(EriAdam8Table *t) {
