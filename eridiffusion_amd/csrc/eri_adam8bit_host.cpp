@@ -422,6 +422,11 @@ struct EriAdam8bit {
     EriAdam8Table *grad_table = nullptr;     // gradients of the tensors kept in 32-bit moments, for the global norm
     std::vector<EriAdam8Tensor> grad_rows;
     EriAdam8Table *norm_table = nullptr;     // the table that holds the last norm: table or grad_table (not owned twice)
+    struct {                                 // the step at hand; kept for its memory
+        std::vector<uint32_t> ids;
+        std::vector<EriAdam8Tensor> rows, grad_rows;
+        std::vector<EriAdamW32Tensor> rows32;
+    } work;
 };
 
 /* One named state of the functional flavour with its own one-row launch table: updates of many
@@ -599,9 +604,14 @@ int eri_adam8bit_step(EriAdam8bit *o, uint32_t *skipped) {
 static int adam8bit_step_impl(EriAdam8bit *o, uint32_t *skipped) {
     o->step += 1; // :203
     uint32_t skip = 0;
-    std::vector<uint32_t> ids;
-    std::vector<EriAdam8Tensor> rows;
-    std::vector<EriAdamW32Tensor> rows32;
+    auto &ids = o->work.ids;
+    auto &rows = o->work.rows;
+    auto &rows32 = o->work.rows32;
+    ids.clear();
+    rows.clear();
+    rows32.clear();
+    ids.reserve(o->params.size());
+    rows.reserve(o->params.size());
     uint64_t start = 0;
     bool scaled = o->grad_scale != 1.0f;
     for (uint32_t i = 0; i < o->params.size(); ++i) {
@@ -721,7 +731,8 @@ static int adam8bit_step_impl(EriAdam8bit *o, uint32_t *skipped) {
     // (pipeline_flux_lora_1024.rs:691-697 clips every trainable gradient, then steps): their gradients go into
     // a gradient-only table that is normed together with the 8-bit table.
     if (clip && !rows32.empty()) {
-        std::vector<EriAdam8Tensor> grows(rows32.size());
+        auto &grows = o->work.grad_rows;
+        grows.resize(rows32.size());
         uint64_t gstart = 0;
         for (size_t k = 0; k < rows32.size(); ++k) {
             EriAdam8Tensor &g = grows[k];

@@ -16,7 +16,11 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/detail/CUDAHooksInterface.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -66,6 +70,26 @@ bool grad_as_is(const at::Tensor &g, const at::Tensor &p) {
            g.layout() == at::kStrided && g.has_storage() && g.is_contiguous() && g.numel() == p.numel() &&
            (g.scalar_type() == p.scalar_type() || (p.scalar_type() == at::kBFloat16 && g.scalar_type() == at::kFloat));
 }
+
+/* Whether nothing wants to see or to change the tensors that are made now: no dispatch mode, transform or tracer, no
+ * filling of uninitialised memory. */
+bool factories_are_plain() {
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
+    if (c10::impl::tls_local_dispatch_key_set().included_ != c10::default_included_set) return false;
+    return !(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
+}
+
+/* Tensors like others, on their devices: what at::empty_strided makes on a device, past the dispatcher. */
+struct Outputs {
+    const bool direct = factories_are_plain();
+    c10::Allocator *const allocator = direct ? at::detail::getCUDAHooks().getCUDADeviceAllocator() : nullptr;
+    c10::OptionalDeviceGuard guard;
+    at::Tensor like(const at::Tensor &t) {
+        if (!direct) return at::empty_strided(t.sizes(), t.strides(), t.options());
+        if (guard.current_device() != t.device()) guard.reset_device(t.device());
+        return at::detail::empty_strided_generic(t.sizes(), t.strides(), allocator, c10::DispatchKeySet(c10::DispatchKey::CUDA), t.scalar_type());
+    }
+};
 
 /* What a parameter was when its optimizer was made; handles and states are sized by it. */
 struct Made {
@@ -187,8 +211,13 @@ PyObject *face_update_many(PyObject *, PyObject *args) {
             Py_DECREF(keys);
             return nullptr;
         }
+        std::vector<at::Tensor> fresh(k);
+        {
+            Outputs made; // its device guard ends before the launch
+            for (size_t i = 0; i < k; ++i) fresh[i] = made.like(ps[i]);
+        }
         for (size_t i = 0; i < k; ++i) {
-            at::Tensor out = at::empty_strided(ps[i].sizes(), ps[i].strides(), ps[i].options()); // empty_like less its dispatch: 92 -> 80 us per 60
+            at::Tensor &out = fresh[i];
             p_ptr[i] = ps[i].data_ptr();
             g_ptr[i] = gs[i].data_ptr();
             o_ptr[i] = out.data_ptr();

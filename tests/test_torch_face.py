@@ -285,3 +285,33 @@ def test_a_closed_optimizer_answers_as_the_library_does(monkeypatch):
     with pytest.raises(L.EriError) as e:
         opt.update_many({}, {})
     assert e.value.code == -1
+
+
+@pytest.mark.gpu
+def test_outputs_of_named_updates_are_torchs_own():
+    """Storages of their own on the parameter's device, seen by the allocator's counters and by a dispatch mode, inference
+    tensors under inference mode, filled under deterministic algorithms as torch fills them."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
+    params = {"a": torch.randn(40, 64, device="cuda"), "b": torch.randn(2049, device="cuda").to(torch.bfloat16)}
+    grads = {k: torch.randn_like(v) for k, v in params.items()}
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    outs = fn.update_many(params, grads)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before >= 2
+    for k, v in outs.items():
+        assert type(v) is torch.Tensor and v.shape == params[k].shape and v.dtype == params[k].dtype and v.device == params[k].device
+        assert v.untyped_storage().nbytes() == v.numel() * v.element_size() and v.is_leaf and not v.requires_grad
+    assert outs["a"].untyped_storage().data_ptr() != outs["b"].untyped_storage().data_ptr()
+
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        fn.update_many(params, grads)
+    assert sum("empty" in s for s in seen) == 2
+    with torch.inference_mode():
+        assert all(v.is_inference() for v in fn.update_many(params, grads).values())
