@@ -289,8 +289,8 @@ def test_a_closed_optimizer_answers_as_the_library_does(monkeypatch):
 
 @pytest.mark.gpu
 def test_outputs_of_named_updates_are_torchs_own():
-    """Storages of their own on the parameter's device, seen by the allocator's counters and by a dispatch mode, inference
-    tensors under inference mode, filled under deterministic algorithms as torch fills them."""
+    """Storages of their own on the parameter's device, seen by the allocator's counters and by a dispatch mode, and
+    inference tensors under inference mode."""
     from torch.utils._python_dispatch import TorchDispatchMode
     from eridiffusion_amd.adam8bit import Adam8bitFunctional
     fn = Adam8bitFunctional.with_params(1e-3, 0.9, 0.999, 1e-8, 0.01)
