@@ -314,8 +314,9 @@ struct EriAdam8Table {
     std::vector<uint64_t> numel;
     std::vector<int32_t> dtype; // per row: its layout
     hipEvent_t uploaded = nullptr;
-    bool upload_pending = false;    // the copy behind `uploaded` may still be on its way
-    bool set_pending = false;       // addresses have been set by a launch on upload_stream that `uploaded` does not cover yet
+    bool upload_pending = false;    // the copy or the launch behind `uploaded` may still be on its way
+    bool mirror_read = false;       // it is a copy, and reads the pinned rows
+    bool mirror_ahead = true;       // the pinned rows are not known to be what the device rows become
     void *upload_stream = nullptr;  // stream of the last upload
     void *ordered_stream = nullptr; // another stream that has already been made to wait for that upload
     bool ordered_valid = false;
@@ -408,20 +409,6 @@ void fill_group(EriAdam8Table::Group &g, const EriAdam8Tensor *rows) {
     g.total_blocks = start;
 }
 
-int upload(EriAdam8Table *t, void *stream) {
-    for (auto &g : t->groups) {
-        if (g.n == 0) continue;
-        ERI_HIP(hipMemcpyAsync(g.dev, g.pinned, sizeof(eri::DevTensor) * g.n, hipMemcpyHostToDevice,
-                               static_cast<hipStream_t>(stream)));
-    }
-    ERI_HIP(hipEventRecord(t->uploaded, static_cast<hipStream_t>(stream)));
-    t->upload_pending = true;
-    t->set_pending = false;
-    t->upload_stream = stream;
-    t->ordered_valid = false;
-    return 0;
-}
-
 bool is_capturing(void *stream) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cs) != hipSuccess) {
@@ -429,6 +416,22 @@ bool is_capturing(void *stream) {
         cs = hipStreamCaptureStatusNone;
     }
     return cs == hipStreamCaptureStatusActive;
+}
+
+int upload(EriAdam8Table *t, void *stream) {
+    t->mirror_ahead = true; // until all of it is queued
+    for (auto &g : t->groups) {
+        if (g.n == 0) continue;
+        ERI_HIP(hipMemcpyAsync(g.dev, g.pinned, sizeof(eri::DevTensor) * g.n, hipMemcpyHostToDevice,
+                               static_cast<hipStream_t>(stream)));
+    }
+    ERI_HIP(hipEventRecord(t->uploaded, static_cast<hipStream_t>(stream)));
+    t->upload_pending = true;
+    t->mirror_read = true;
+    t->mirror_ahead = is_capturing(stream); // a copy that is captured runs with the graph
+    t->upload_stream = stream;
+    t->ordered_valid = false;
+    return 0;
 }
 
 /* The streams whose kernels read device memory that is overwritten later, for caches that a caller does not see and so
@@ -465,18 +468,8 @@ struct Readers {
  * captured into a graph cannot wait for an event outside the graph, so there the host waits for the
  * upload instead, once. */
 int order_after_upload(EriAdam8Table *t, void *stream) {
-    if ((!t->upload_pending && !t->set_pending) || stream == t->upload_stream) return 0;
+    if (!t->upload_pending || stream == t->upload_stream) return 0;
     if (t->ordered_valid && stream == t->ordered_stream) return 0;
-    if (t->set_pending) { // no event was recorded behind the launch: nobody but another stream needs one
-        if (hipEventRecord(t->uploaded, static_cast<hipStream_t>(t->upload_stream)) != hipSuccess) { // a stream destroyed since
-            (void)hipGetLastError();
-            ERI_HIP(hipDeviceSynchronize());
-            t->upload_pending = t->set_pending = false;
-            return 0;
-        }
-        t->upload_pending = true;
-        t->set_pending = false;
-    }
     if (is_capturing(stream)) {
         const hipError_t e = hipEventSynchronize(t->uploaded);
         if (e != hipSuccess) {
@@ -1035,13 +1028,15 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
     for (uint32_t i = 0; i < n; ++i)
         if (rows[i].numel != t->numel[i] || layout_of(rows[i]) != t->dtype[i])
             return fail(ERI_ERR_ARG, "table_update: numel or dtype differs from the table's");
-    if (t->upload_pending) { // the pinned mirror may still be the source of the previous copy
+    // The pinned mirror may still be the source of the previous copy, and the rows of one stream's update must not land
+    // behind those of a later one on another.
+    if (t->upload_pending && (t->mirror_read || stream != t->upload_stream)) {
         ERI_HIP(hipEventSynchronize(t->uploaded));
-        t->upload_pending = false;
+        t->upload_pending = t->mirror_read = false;
     }
     // Where only addresses change, and in no more rows than two launches carry per group, a launch sets them: the rows
-    // need no copy, no event and no wait for the copy before.
-    bool set = true;
+    // need no copy and no wait for the update before.  A graph gets the copy, which takes the rows of the time it runs.
+    bool set = !t->mirror_ahead && !is_capturing(stream);
     std::vector<eri::RowAddresses> to[eri::kLayouts];
     bool grads_alone[eri::kLayouts];
     for (int li = 0; li < eri::kLayouts && set; ++li) {
@@ -1061,6 +1056,7 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
     for (auto &g : t->groups)
         if (g.n) fill_group(g, rows);
     if (!set) return upload(t, stream);
+    t->mirror_ahead = true;
     for (int li = 0; li < eri::kLayouts; ++li) {
         auto &g = t->groups[li];
         if (g.n == 0) continue;
@@ -1073,7 +1069,9 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
         }
         if (rc) return hip_fail((hipError_t)rc, "launch table update");
     }
-    t->set_pending = true;
+    ERI_HIP(hipEventRecord(t->uploaded, static_cast<hipStream_t>(stream)));
+    t->upload_pending = true;
+    t->mirror_ahead = false;
     t->upload_stream = stream;
     t->ordered_valid = false;
     return 0;

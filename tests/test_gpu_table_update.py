@@ -67,3 +67,73 @@ def test_rows_at_new_addresses(what, n, mixed, other_stream):
 
     for a, b in zip(run(True), run(False)):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def _one(case, rows, k, stream):
+    from eridiffusion_amd import _lib as L
+    L.check(L.lib().eri_adam8_table_update(case, rows[k], len(rows[k]), stream.cuda_stream), "update")
+
+
+@pytest.mark.parametrize("how", ["two_streams", "captured", "before_a_capture"])
+def test_updates_follow_each_other(how):
+    """Rows of a stream's update stay behind those of a later one on another; an update that a graph holds leaves the next
+    one everything to set; and one in front of a capture on another stream is what the graph steps on."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    n, size = 40, 3000
+    main, side = torch.cuda.current_stream(), torch.cuda.Stream()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    total, blocks = n * ((size + 15) // 16 * 16), n * 2
+    ps = [torch.randn(2 * total, device="cuda", generator=gen).to(torch.bfloat16) for _ in range(2)]
+    gs = [torch.randn(2 * total, device="cuda", generator=gen).to(torch.bfloat16) for _ in range(3)]
+    h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, 1, L.MODE_ERI, L.FLAG_EXACT_PARAM)
+
+    def run(update):
+        s = (torch.zeros(total, dtype=torch.uint8, device="cuda"), torch.zeros(total, dtype=torch.uint8, device="cuda"),
+             torch.zeros(blocks, device="cuda"), torch.zeros(blocks, device="cuda"))
+        for i in range(n):
+            at = i * ((size + 15) // 16 * 16)
+            L.check(L.lib().eri_adam8_state_init(s[0].data_ptr() + at, s[1].data_ptr() + at, s[2].data_ptr() + 8 * i, s[3].data_ptr() + 8 * i,
+                                                 size, main.cuda_stream), "init")
+        p = [x.clone() for x in ps]
+        rows = [_rows([size] * n, [1] * n, p[a], gs[b], s) for a, b in ((0, 0), (1, 1), (1, 2))]
+        table, last = C.c_void_p(), 2 if how != "before_a_capture" else 1
+        L.check(L.lib().eri_adam8_table_create(rows[0 if update else last], n, main.cuda_stream, C.byref(table)), "create")
+
+        def step(stream):
+            L.check(L.lib().eri_adam8_step_table(table, C.byref(h), stream.cuda_stream), "step")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        if how == "two_streams":
+            if update:
+                _one(table, rows, 0, main)
+                torch.cuda._sleep(20_000_000)
+                _one(table, rows, 1, main)
+                _one(table, rows, 2, side)
+            step(side)
+            torch.cuda.synchronize()
+            step(side)
+        elif how == "captured":
+            if update:
+                with torch.cuda.graph(graph):
+                    _one(table, rows, 1, torch.cuda.current_stream())
+                _one(table, rows, 2, main)
+            step(main)
+            step(main)
+        else:
+            if update:
+                _one(table, rows, 1, main)
+                with torch.cuda.graph(graph):
+                    step(torch.cuda.current_stream())
+                for _ in range(2):
+                    graph.replay()
+                    torch.cuda.synchronize()
+            else:
+                step(main)
+                step(main)
+        torch.cuda.synchronize()
+        L.lib().eri_adam8_table_destroy(table)
+        return tuple(p) + s
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
