@@ -87,9 +87,9 @@ int eri_hip_pointer_kind(const void *p, int *kind);
 
 /* A device memory pool with lanes: ONE device allocation cut into `lanes` equal parts, each handing out
  * 256-byte aligned, zero-filled pieces from its start upwards.  It exists for placement.  On MI355X a kernel
- * that reads and writes several arrays at once (the optimizer step: parameters, gradients, two state arrays)
- * runs 10-17 % faster when the 8-bit states lie 32 GiB or more away from the parameters and gradients in
- * device memory than with everything adjacent, and separate hipMalloc calls give no say over that; inside
+ * that reads and writes several arrays at once on fixed shares per wave runs up to 17 % faster when the written
+ * arrays lie 32 GiB or more apart in device memory than with everything adjacent (the step over large tables, which
+ * keeps the chip within one window of them, 0-4 %), and separate hipMalloc calls give no say over that; inside
  * one allocation distances are what the caller makes them.  Meant as the backing store of the reference's
  * MemoryPool (crates/core/src/memory.rs:243-311 allocates one block per request through cuda_malloc_zeroed):
  * a lane per kind of tensor -- the reference already keeps one pool per dtype, so U8 states and BF16 parameters
