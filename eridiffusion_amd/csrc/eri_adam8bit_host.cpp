@@ -1658,6 +1658,14 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
     if (n == 0) return 0;
     int rc = fn_flush(o);
     if (rc) return rc;
+    for (uint32_t i = 0; i < n; ++i)
+        for (const float *x : {m[i], v[i]}) {
+            int kind = ERI_PTR_UNKNOWN;
+            rc = eri_hip_pointer_kind(x, &kind);
+            if (rc) return rc;
+            if (kind == ERI_PTR_UNKNOWN)
+                return fail(ERI_ERR_ARG, std::string("moments of '") + names[i] + "' are not in device, pinned or managed memory: kernels cannot reach them");
+        }
     // A state of this size that exists already, where new states would be made too, takes the new contents where it is,
     // in stream order behind the steps that still use the old ones: no allocation and no release, each of which waits for
     // the device (24 tensors of 340 M parameters loaded and read back: 33.8 -> 1.34 ms).  The others get a new state,

@@ -193,8 +193,9 @@ int eri_adam8bit_fn_state_numel(const EriAdam8bitFn *opt, const char *name, uint
 int eri_adam8bit_fn_get_state_fp32(EriAdam8bitFn *opt, const char *name, float *m_out, float *v_out);
 int eri_adam8bit_fn_load_state_fp32(EriAdam8bitFn *opt, const char *name, const float *m, const float *v,
                                     uint64_t numel);
-/* The same for n names in one call, whose conversions share a launch: row i is what the calls above take.  Every row is
- * checked before anything is launched, and a refused call converts nothing; states that a load creates stay. */
+/* The same for n names in one call, whose conversions share launches: row i is what the calls above take.  Every argument is
+ * checked before anything is launched, and a call that is refused for one converts nothing.  A load for whose states the
+ * memory does not suffice may have loaded names that stand before, as the calls in turn would. */
 int eri_adam8bit_fn_get_states_fp32(EriAdam8bitFn *opt, const char *const *names, float *const *m_out, float *const *v_out,
                                     uint32_t n);
 int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *opt, const char *const *names, const float *const *m,

@@ -144,3 +144,28 @@ def test_a_name_twice_in_one_load_keeps_its_last_contents():
     out.fill_(5.0)
     assert L.lib().eri_adam8bit_fn_get_states_fp32(opt._opt, (C.c_char_p * 2)(b"a", b"nobody"), unknown, unknown, 2) == -6
     assert bool((out == 5.0).all())  # nothing of a refused call runs
+
+
+def _load_many(opt, rows):
+    """rows: (name, m, v, numel) of eri_adam8bit_fn_load_states_fp32; addresses or tensors."""
+    import ctypes as C
+    from eridiffusion_amd import _lib as L
+    k = len(rows)
+    at = lambda x: x if isinstance(x, int) else x.data_ptr()
+    return L.lib().eri_adam8bit_fn_load_states_fp32(opt._opt, (C.c_char_p * k)(*[r[0].encode() for r in rows]), (C.c_void_p * k)(*[at(r[1]) for r in rows]),
+                                                    (C.c_void_p * k)(*[at(r[2]) for r in rows]), (C.c_uint64 * k)(*[r[3] for r in rows]), k)
+
+
+def test_a_load_refused_behind_a_repeated_name_converts_nothing():
+    import torch
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    n = 3000
+    x = [torch.rand(n, device="cuda") for _ in range(3)]
+    opt = Adam8bitFunctional()
+    opt.load_state_from_tensors({"a": (x[0], x[0])})
+    before = opt.get_state_as_tensors()["a"]
+    host = np.ones(n, dtype=np.float32)
+    assert _load_many(opt, [("a", x[1], x[1], n), ("b", x[2], x[2], n), ("a", x[2], x[2], n), ("c", x[1], host.ctypes.data, n)]) == -6
+    after = opt.get_state_as_tensors()["a"]
+    assert torch.equal(before[0], after[0]) and torch.equal(before[1], after[1])
+    assert opt.memory_stats()[0] == 1
