@@ -24,6 +24,7 @@
 #include <sstream>
 #include <string>
 #include <string_view>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/eri_adam8bit.h"
@@ -1672,9 +1673,10 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
     // which takes its name once the conversion has been launched.
     std::vector<EriMomentTensor> rows;
     std::vector<std::pair<uint32_t, std::unique_ptr<FnState>>> made;
-    const uint64_t loading = ++o->generation; // no row of the last batch is queued any more (fn_flush)
+    std::unordered_map<std::string_view, uint32_t> last; // of a name that comes up again only the last contents count
+    last.reserve(n);
+    for (uint32_t i = 0; i < n; ++i) last[names[i]] = i;
     auto launch = [&]() -> int {
-        if (rows.empty()) return 0;
         const int e = eri_adam8_quantize_states(rows.data(), (uint32_t)rows.size(), o->stream);
         if (e) return e;
         if (!made.empty()) o->last_order.clear(); // it may hold a state that is replaced here
@@ -1684,14 +1686,8 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
         return 0;
     };
     for (uint32_t i = 0; i < n; ++i) {
+        if (last[names[i]] != i) continue;
         auto it = o->states.find(std::string_view(names[i]));
-        bool again = it != o->states.end() && it->second->queued_in == loading;
-        for (size_t k = 0; !again && k < made.size(); ++k) again = std::strcmp(names[made[k].first], names[i]) == 0;
-        if (again) { // a name twice in one call: the first contents are replaced in order
-            rc = launch();
-            if (rc) return rc;
-            it = o->states.find(std::string_view(names[i]));
-        }
         FnState *s = it == o->states.end() ? nullptr : it->second.get();
         if (!s || s->numel != numels[i] || s->pool != o->state_pool || (o->state_pool && s->pool_lane != o->state_lane)) {
             std::unique_ptr<FnState> fresh(new FnState());
@@ -1700,12 +1696,9 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
             s = fresh.get();
             made.emplace_back(i, std::move(fresh));
         }
-        s->queued_in = loading;
         rows.push_back({const_cast<float *>(m[i]), const_cast<float *>(v[i]), s->m, s->v, s->absmax_m, s->absmax_v, numels[i]});
     }
-    rc = launch();
-    o->generation += 1; // the marks above are not those of the next batch
-    return rc;
+    return launch();
 }
 
 // ---- helpers beside the optimizers ------------------------------------------------------------
