@@ -1670,7 +1670,10 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
     // A state of this size that exists already, where new states would be made too, takes the new contents where it is,
     // in stream order behind the steps that still use the old ones: no allocation and no release, each of which waits for
     // the device (24 tensors of 340 M parameters loaded and read back: 33.8 -> 1.34 ms).  The others get a new state,
-    // which takes its name once the conversion has been launched.
+    // which takes its name once the conversion has been launched; the one that it replaces is held until then.  So that
+    // a load needs little more memory than the calls in turn, no more than this is held, and nothing when memory runs out.
+    constexpr uint64_t kReplacedBytes = 64u << 20;
+    uint64_t replaced = 0;
     std::vector<EriMomentTensor> rows;
     std::vector<std::pair<uint32_t, std::unique_ptr<FnState>>> made;
     std::unordered_map<std::string_view, uint32_t> last; // of a name that comes up again only the last contents count
@@ -1683,16 +1686,26 @@ int eri_adam8bit_fn_load_states_fp32(EriAdam8bitFn *o, const char *const *names,
         for (auto &kv : made) o->states[names[kv.first]] = std::move(kv.second);
         rows.clear();
         made.clear();
+        replaced = 0;
         return 0;
     };
     for (uint32_t i = 0; i < n; ++i) {
         if (last[names[i]] != i) continue;
+        if (replaced > kReplacedBytes) {
+            rc = launch();
+            if (rc) return rc;
+        }
         auto it = o->states.find(std::string_view(names[i]));
         FnState *s = it == o->states.end() ? nullptr : it->second.get();
         if (!s || s->numel != numels[i] || s->pool != o->state_pool || (o->state_pool && s->pool_lane != o->state_lane)) {
             std::unique_ptr<FnState> fresh(new FnState());
             rc = fresh->allocate(numels[i], o->stream, o->state_pool, o->state_lane);
+            if (rc && replaced) {
+                rc = launch();
+                if (rc == 0) rc = fresh->allocate(numels[i], o->stream, o->state_pool, o->state_lane);
+            }
             if (rc) return rc;
+            if (s) replaced += s->total;
             s = fresh.get();
             made.emplace_back(i, std::move(fresh));
         }

@@ -211,3 +211,39 @@ def test_loading_many_new_names_takes_time_by_their_number():
         assert _load_many(opt, rows) == 0
         times[k] = time.perf_counter() - start
     assert times[16000] < 14 * times[2000], times  # eight times as many names; 30 with a search through those before
+
+
+def test_states_of_other_sizes_take_the_room_of_those_they_replace():
+    """A lane that holds all states and one more (a piece goes to states of its size again), loaded with the sizes of
+    neighbours exchanged: name by name that fits."""
+    import torch
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
+    gen = torch.Generator(device="cuda").manual_seed(11)
+
+    def moments(sizes):
+        return {"w%d" % i: (torch.randn(n, device="cuda", generator=gen) * 1e-3, torch.rand(n, device="cuda", generator=gen) * 1e-6)
+                for i, n in enumerate(sizes)}
+    first, second = moments([200_000, 190_001] * 4), moments([190_001, 200_000] * 4)
+    tight, roomy = Adam8bitFunctional(), Adam8bitFunctional()
+    tight.set_state_pool(DevicePool(4 << 20, 1), 0)  # eight states take 3.1 MB
+    for opt in (tight, roomy):
+        opt.load_state_from_tensors(first)
+        opt.load_state_from_tensors(second)
+    a, b = tight.get_state_as_tensors(), roomy.get_state_as_tensors()
+    for name in second:
+        assert torch.equal(a[name][0], b[name][0]) and torch.equal(a[name][1], b[name][1]), name
+
+
+def test_a_load_holds_little_of_what_it_replaces():
+    """Twelve states of 24 MiB made anew, as above: how far up their lane they reach says how many were held at once."""
+    import torch
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
+    n, k = 12 << 20, 12
+    x = torch.rand(n, device="cuda") * 1e-3
+    opt, pool = Adam8bitFunctional(), DevicePool(1 << 30, 1)
+    base = pool.alloc_ptr(0, 256)
+    opt.set_state_pool(pool, 0)
+    for turn in (0, 1):
+        assert _load_many(opt, [("w%d" % i, x, x, n - 4096 * ((i + turn) % 2)) for i in range(k)]) == 0
+    top = pool.alloc_ptr(0, k * 24 << 20) - base  # larger than any hole: behind the highest piece in use
+    assert top < (k + 5) * 25 << 20
