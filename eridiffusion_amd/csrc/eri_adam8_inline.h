@@ -656,9 +656,17 @@ __device__ __forceinline__ void requant8(const float *mf, const float *vf, const
  * (MAP[c] * absmax) * beta for every code c -- the first two operations of both moment updates, done once
  * per code (eight per lane) instead of once per element (64 per lane); a wave's LDS operations complete in
  * order, so its reads below see its own writes without a barrier.
- * PARTIAL: a row's last block of n < 2048 elements; lanes past the end are off (see tail_block for what stands in for
- * the elements that are missing). */
-template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16, bool PARTIAL = false>
+ * PARTIAL: a row's last block of n < 2048 elements, with the lanes past the end off; the one lane the end falls into
+ * moves its up to seven elements one by one.  What is filled in for missing elements are zero moments and zero gradients,
+ * which make zero or NaN moments whatever the scalars are: neither moves a maximum, and nothing of them is stored.
+ * ROOMY: a partial block in a kernel with registers for all of its loads at once, in front of its main loop: one trip to
+ * memory, and no pass behind the end.  In the prefetching kernel, where a sweep for the maxima and a second one that read
+ * and computed all again stood before, a trip per 512 elements each; us, 16,384 tensors of a block and a part, before |
+ * the same with the code of the plain kernel | so:
+ *   a part of         101           952           1,027         2,047
+ *   bf16        118 | 177 | 108  124 | 164 | 122  177 | 156 | 140  227 | 161 | 170
+ *   fp32        152 | 181 | 136  174 | 189 | 164  227 | 192 | 181  284 | 223 | 233 */
+template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16, bool PARTIAL = false, bool ROOMY = false>
 __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint32_t n, uint32_t lane, const StepHyper &h,
                                            float gscale, const BlockDiv &dbc1, const BlockDiv &dbc2, const Lds &L,
                                            float (*mine)[256]) {
@@ -687,7 +695,9 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     float lm = 0.0f, lv = 0.0f;
     // Issue the loads of DEPTH passes before touching the first value: the wave then waits once per
     // DEPTH passes, with 48 * DEPTH bytes per lane in flight (bf16; fp32 values hold twice the registers).
-    constexpr int DEPTH = ((BF16 && GBF16) ? 4 : 2) / (PARTIAL ? 2 : 1);
+    static_assert(PARTIAL || !ROOMY, "a whole block has no end to stop at");
+    constexpr int DEPTH = ROOMY ? 4 : ((BF16 && GBF16) ? 4 : 2) / (PARTIAL ? 2 : 1);
+    const uint32_t passes = ROOMY ? (n + 511) / 512 : 4;
 #pragma unroll
     for (int c0 = 0; c0 < 4; c0 += DEPTH) {
         Raw8<BF16> pr[DEPTH];
@@ -695,6 +705,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
         u32x2 mr[DEPTH], vr[DEPTH];
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
+            if ((uint32_t)(c0 + d) >= passes) continue;
             const uint32_t o = (c0 + d) * 512 + lane * 8;
             const uint32_t count = lane_count(o, n);
             if (!PARTIAL || count == 8) {
@@ -712,6 +723,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const int c = c0 + d;
+            if ((uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             float pv[8], gv[8], pn[8];
             pr[d].unpack(pv);
@@ -753,6 +765,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     if (dm.fast && dv.fast) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            if ((uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<true, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
@@ -762,6 +775,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     } else {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            if ((uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
@@ -771,118 +785,10 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     }
 }
 
-// ------------------------------------------------------------------------------------------
-// the last, partial block of a tensor (n < 2048 elements, once per tensor at most)
-// ------------------------------------------------------------------------------------------
-
 template <bool BF16>
 __device__ __forceinline__ float load1(const void *base, size_t i) {
     if (BF16) return u2f((uint32_t)as_global(static_cast<const uint16_t *>(base))[i] << 16);
     return as_global(static_cast<const float *>(base))[i];
-}
-
-/* One wave, the 8-elements-per-lane accesses of a full block with the lanes past the end switched off; the one
- * lane the end falls into moves its up to seven elements one by one.  What is filled in for missing elements
- * are zero moments and zero gradients, which make zero or NaN moments whatever the scalars are: neither moves a
- * maximum, and nothing of them is stored.  What bounds it is latency, one trip to memory per 512 elements and
- * sweep: two sweeps, the second recomputing the moments, so that nothing but one pass of values is held -- this
- * code is inlined into kernels whose register budget belongs to their main loop. */
-template <bool BF16, int MODE, bool EXACT, bool WD, bool GS, bool KEYTAB, bool GBF16 = BF16>
-__device__ __forceinline__ void tail_block(const DevTensor &t, uint32_t lb, uint32_t n, uint32_t lane,
-                                        const StepHyper &h, float gscale, const BlockDiv &dbc1,
-                                        const BlockDiv &dbc2, const Lds &L) {
-    const size_t e0 = (size_t)lb * kBlock;
-    const float a_m = as_global(t.absmax_m)[lb];
-    const float a_v = as_global(t.absmax_v)[lb];
-    float lm = 0.0f, lv = 0.0f;
-    constexpr float ks = KEYTAB ? kKeyScale : 1.0f, ksi = KEYTAB ? kKeyScaleInv : 1.0f;
-    const size_t esz = BF16 ? 2 : 4;
-    char *p = static_cast<char *>(t.p) + e0 * esz;
-    const char *p_in = static_cast<const char *>(t.p_in) + e0 * esz;
-    const char *g = static_cast<const char *>(t.g) + e0 * (GBF16 ? 2 : 4);
-    const uint32_t passes = (n + 511) / 512;
-    for (uint32_t c = 0; c < passes; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        const uint32_t count = lane_count(o, n);
-        if (count != 0) {
-            Raw8<BF16> pr;
-            Raw8<GBF16> gr;
-            u32x2 mr, vr;
-            if (count == 8) {
-                pr.load(p_in, o);
-                gr.load(g, o);
-                mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
-                vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
-            } else {
-                pr.load_some(p_in, o, count);
-                gr.load_some(g, o, count);
-                mr = load_codes_some(t.m + e0 + o, count, kZeroCodesS);
-                vr = load_codes_some(t.v + e0 + o, count, kZeroCodesU);
-            }
-            float pv[8], gv[8];
-            pr.unpack(pv);
-            gr.unpack(gv);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                float m, v, pn;
-                uint64_t unused = 0;
-                adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
-                                                     L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m, v, pn, unused);
-                lm = fmaxf(lm, __builtin_fabsf(m));
-                lv = fmaxf(lv, __builtin_fabsf(v));
-            }
-        }
-    }
-    float nam = lm, nav = lv;
-    wave_max2(nam, nav);
-    const BlockDiv dm(nam, ks, ksi), dv(nav, ks, ksi);
-    for (uint32_t c = 0; c < passes; ++c) {
-        const uint32_t o = c * 512 + lane * 8;
-        const uint32_t count = lane_count(o, n);
-        if (count != 0) {
-            Raw8<BF16> pr;
-            Raw8<GBF16> gr;
-            u32x2 mr, vr;
-            if (count == 8) {
-                pr.load(p_in, o);
-                gr.load(g, o);
-                mr = *as_global(reinterpret_cast<const u32x2 *>(t.m + e0 + o));
-                vr = *as_global(reinterpret_cast<const u32x2 *>(t.v + e0 + o));
-            } else {
-                pr.load_some(p_in, o, count);
-                gr.load_some(g, o, count);
-                mr = load_codes_some(t.m + e0 + o, count, kZeroCodesS);
-                vr = load_codes_some(t.v + e0 + o, count, kZeroCodesU);
-            }
-            float pv[8], gv[8], pn[8], m[8], v[8];
-            pr.unpack(pv);
-            gr.unpack(gv);
-            uint64_t cancel = (BF16 && MODE == ERI_ADAM8_MODE_L2 && h.l2_all_exact) ? ~0ull : 0ull;
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                adam_elem<MODE, EXACT, BF16, WD, GS>(pv[k], gv[k], L.map_s[byte_of(mr, k)] * a_m,
-                                                     L.map_u[byte_of(vr, k)] * a_v, h, gscale, dbc1, dbc2, m[k], v[k], pn[k], cancel);
-            if (BF16 && __builtin_amdgcn_inverse_ballot_w64(cancel)) { // a lane with a flagged element redoes its eight
-#pragma unroll
-                for (int k = 0; k < 8; ++k) pn[k] = param_exact<MODE, WD, BF16>(pv[k], m[k], v[k], h, dbc1, dbc2);
-            }
-            u32x2 mw, vw;
-            requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(m, v, dm, dv, L, mw, vw);
-            if (count == 8) {
-                *as_global(reinterpret_cast<u32x2 *>(t.m + e0 + o)) = mw;
-                *as_global(reinterpret_cast<u32x2 *>(t.v + e0 + o)) = vw;
-                store8<BF16>(p, o, pn);
-            } else {
-                store_codes_some(t.m + e0 + o, mw, count);
-                store_codes_some(t.v + e0 + o, vw, count);
-                store_some<BF16>(p, o, pn, count);
-            }
-        }
-    }
-    if (lane == 0) {
-        as_global(t.absmax_m)[lb] = nam;
-        as_global(t.absmax_v)[lb] = nav;
-    }
 }
 
 // ------------------------------------------------------------------------------------------

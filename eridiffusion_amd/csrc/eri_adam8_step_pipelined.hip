@@ -61,7 +61,7 @@ __device__ __forceinline__ void ema_eight(const u32x4 &old, const u32x4 &pnew, f
 }
 
 /* The shadow of a row's partial last block of n elements.  A lane takes the eight elements that it has just stored as
- * parameters (tail_block), so that what it reads back are its own stores: nothing orders them before another lane's
+ * parameters (full_block), so that what it reads back are its own stores: nothing orders them before another lane's
  * loads. */
 __device__ __forceinline__ void ema_tail(const DevTensor &t, uint32_t n, uint32_t lane, float decay) {
     const size_t e0 = (size_t)(t.numel / kBlock) * kBlock;
@@ -215,7 +215,7 @@ __global__ __launch_bounds__(kPipeThreads) void ERI_PIPE_KERNEL(const DevTensor 
         const DevTensor t = load_constant(rows + map.tail_row(total_blocks, i));
         const uint32_t n = (uint32_t)(t.numel % kBlock);
         const float gscale = GS ? (h.grad_scale * t.grad_scale) * tscale : 1.0f;
-        tail_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L);
+        full_block<kParamBf16, MODE, EXACT, WD, GS, true, kGradBf16, true, true>(t, (uint32_t)(t.numel / kBlock), n, lane, h, gscale, dbc1, dbc2, L, mine);
         if (EMA && t.shadow != nullptr) ema_tail(t, n, lane, h.ema_decay);
     }
     uint32_t next_round = __builtin_amdgcn_readfirstlane(coming[0]);
@@ -384,7 +384,7 @@ int launch_flags(bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_r
 
 } // namespace
 
-/* All three modes, 190-250 registers, no scratch. */
+/* All three modes, 160-220 registers, no scratch. */
 #if ERI_PIPE_LAYOUT == 1
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *img, const float *dev_scale,

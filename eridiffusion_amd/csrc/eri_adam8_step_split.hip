@@ -78,7 +78,7 @@ __global__ __launch_bounds__(1024) void adam8_step_split_kernel(const DevTensor 
             q.gr.load(g, o);
             q.mr = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(q.t.m + e0 + o)));
             q.vr = __builtin_nontemporal_load(as_global(reinterpret_cast<const u32x2 *>(q.t.v + e0 + o)));
-        } else { // zero moments and gradients past the end: they move no maximum (see tail_block)
+        } else { // zero moments and gradients past the end: they move no maximum (see full_block)
             q.pr.load_some(p_in, o, count);
             q.gr.load_some(g, o, count);
             q.mr = load_codes_some(q.t.m + e0 + o, count, kZeroCodesS);
