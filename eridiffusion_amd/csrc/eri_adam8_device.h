@@ -101,11 +101,19 @@ constexpr uint32_t kSmallLoU = kSmallLoS + kSKeyCount;    /* kUKeyCount bytes */
 constexpr uint32_t kSmallImageBytes = kSmallLoU + kUKeyCount;
 static_assert(kSmallImageBytes % 1024 == 0, "the image is staged in pieces of 1 KB");
 
+/* What the choice of a step's kernel goes by, of the rows of one layout. */
+struct TableShape {
+    uint32_t total_blocks; // full ones
+    uint32_t n_tails;      // partial last blocks
+    uint32_t n_long;       // of these, the ones of more than half a block
+    int layout;
+    uint32_t units() const { return total_blocks + n_tails; } // a partial block costs about what a full one does
+};
+
 /* Launchers implemented in eri_adam8_kernels.hip; `stream` is a hipStream_t.  All return a
  * hipError_t as int.  `lds_image` is the device copy of the kLdsImageBytes table image. */
-int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_full_blocks, uint32_t n_tails, int layout,
-                const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg,
-                uint32_t compute_units, void *stream);
+int launch_step(const DevTensor *rows, uint32_t n_rows, const TableShape &t, const EriAdam8Hyper &h, const void *lds_image,
+                const float *dev_scale, uint32_t grid, uint32_t wg, uint32_t compute_units, void *stream);
 
 constexpr uint32_t kChunks = 8;           /* contiguous ranges the gradient-norm pass cuts long block lists into: one per accelerator die */
 /* Tables of at most this many blocks per compute unit (partial ones counted) take the four-waves-per-block kernel: one
@@ -145,6 +153,20 @@ inline uint32_t prefetch_blocks_per_cu(int mode, int layout) {
     if (mode == ERI_ADAM8_MODE_BNB) return layout == kLayoutBF16 ? 128 : layout == kLayoutBF16GradF32 ? 56 : 48;
     return layout == kLayoutF32 ? 40 : 48;
 }
+/* Partial blocks run in front of that kernel's tickets, a wave each without a prefetch, at what their length costs; the
+ * plain kernel takes them like whole ones.  With bf16 parameters it is the faster one where many of them are long.  us per
+ * launch, prefetching kernel | plain, 256 units, tensors of k blocks and a part of 1,501 elements:
+ *   blocks, k            16,384, 1   16,384, 2   16,384, 4   37,376, 1   37,376, 2   37,376, 4
+ *   bf16                 151 | 138   108 | 104     86 | 87   330 | 307   232 | 227   182 | 190
+ *   ... fp32 gradients   168 | 159   119 | 124    97 | 105   360 | 355   252 | 271   203 | 231
+ *   fp32                 200 | 215   153 | 163   124 | 139   432 | 478   324 | 363   263 | 308
+ *   bf16, mode L2                                            333 | 294   233 | 222   185 | 189
+ *   bf16, mode BNB                                           325 | 288   231 | 219   183 | 187
+ * and where all are short (952 elements, k = 1) it is not: 16,384 blocks bf16 122 | 137, 35,840 in mode L2 251 | 267. */
+inline bool long_tails_weigh(const TableShape &t) {
+    if (t.layout == kLayoutF32) return false;
+    return (uint64_t)t.n_long * (t.layout == kLayoutBF16 ? 3 : 2) > t.total_blocks;
+}
 /* Above this many full blocks per compute unit the gradient-norm pass cuts its list into ranges. */
 constexpr uint32_t kNormRangesBlocksPerCu = 1024;
 constexpr uint32_t kNormWaves = 4;        /* waves per workgroup of the gradient-norm pass */
@@ -179,7 +201,7 @@ int launch_step_two(const StepGroup &f32, const StepGroup &bf16, const EriAdam8H
                     uint32_t grid, uint32_t wg, void *stream);
 /* Whether launch_step would run this group on the prefetching kernel with the EMA update inside it.  units: full blocks
  * and partial ones. */
-bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units);
+bool step_fuses_ema(const TableShape &t, const EriAdam8Hyper &h, uint32_t compute_units);
 int launch_step_pipelined(int mode, bool exact, bool wd, bool gs, bool ema, const DevTensor *rows, uint32_t n_rows,
                           uint32_t total_blocks, uint32_t n_tails, const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale,
                           uint32_t grid, uint32_t wg, void *stream);

@@ -13,26 +13,29 @@ namespace eri {
  * 256 units, no two launches on the same data:
  *   blocks               1,025        2,560        4,096        8,192       12,288       16,896       74,784
  *   bf16           13.5 | 13.1  23.7 | 21.2  31.5 | 29.9  49.1 | 51.5  68.1 | 74.6   88.9 | 100    354 | 417
- *   fp32 gradients 14.2 | 14.1  25.7 | 23.0  32.3 | 33.4  50.6 | 57.9  75.5 | 86.5    100 | 111    408 | 467 */
+ *   fp32 gradients 14.2 | 14.1  25.7 | 23.0  32.3 | 33.4  50.6 | 57.9  75.5 | 86.5    100 | 111    408 | 467
+ * With partial blocks the same: 7,680 and 15,360 tensors of 1,501 elements 74 | 83 and 143 | 130, half as many of 3,075
+ * elements 57 | 76 and 101 | 117. */
 constexpr uint32_t kFusedEmaBlocksPerCu = 24, kFusedEmaBlocksPerCuGradF32 = 14;
-bool step_fuses_ema(uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
-    if ((h.flags & ERI_ADAM8_FLAG_EMA) == 0 || !layout_param_bf16(layout) || h.mode != ERI_ADAM8_MODE_ERI) return false;
+bool step_fuses_ema(const TableShape &t, const EriAdam8Hyper &h, uint32_t compute_units) {
+    if ((h.flags & ERI_ADAM8_FLAG_EMA) == 0 || !layout_param_bf16(t.layout) || h.mode != ERI_ADAM8_MODE_ERI) return false;
     if (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) return false;
     if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0) return true;
-    return (uint64_t)units > (uint64_t)compute_units * (layout_grad_bf16(layout) ? kFusedEmaBlocksPerCu : kFusedEmaBlocksPerCuGradF32);
+    return (uint64_t)t.units() > (uint64_t)compute_units * (layout_grad_bf16(t.layout) ? kFusedEmaBlocksPerCu : kFusedEmaBlocksPerCuGradF32);
 }
 
 /* Whether a table that qualifies for the prefetching kernel is large enough to gain from it, or has its EMA inside that
  * kernel.  A step whose EMA is a sweep of its own runs as it would without one: on the prefetching kernel all the same,
  * mode BNB took 38.1 us for 4,096 bf16 blocks instead of 29.0, and fp32 parameters 39 for 2,816 instead of 31.5. */
-static bool prefetch_pays(uint32_t total_blocks, uint32_t units, int layout, const EriAdam8Hyper &h, uint32_t compute_units) {
-    if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || step_fuses_ema(units, layout, h, compute_units)) return true;
-    return (uint64_t)total_blocks > (uint64_t)compute_units * prefetch_blocks_per_cu(h.mode, layout);
+static bool prefetch_pays(const TableShape &t, const EriAdam8Hyper &h, uint32_t compute_units) {
+    if ((h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0 || step_fuses_ema(t, h, compute_units)) return true;
+    return !long_tails_weigh(t) && (uint64_t)t.total_blocks > (uint64_t)compute_units * prefetch_blocks_per_cu(h.mode, t.layout);
 }
 
-int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, uint32_t n_tails, int layout,
-                const EriAdam8Hyper &h, const void *lds_image, const float *dev_scale, uint32_t grid, uint32_t wg,
-                uint32_t compute_units, void *stream) {
+int launch_step(const DevTensor *rows, uint32_t n_rows, const TableShape &t, const EriAdam8Hyper &h, const void *lds_image,
+                const float *dev_scale, uint32_t grid, uint32_t wg, uint32_t compute_units, void *stream) {
+    const uint32_t total_blocks = t.total_blocks, n_tails = t.n_tails, units = t.units();
+    const int layout = t.layout;
     const bool bf16 = layout_param_bf16(layout);
     const bool mixed = layout == kLayoutBF16GradF32; // F32 gradients for BF16 parameters
     const bool gs = (h.flags & ERI_ADAM8_FLAG_GRAD_SCALE) != 0;
@@ -41,7 +44,6 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     // have no binary-search variant of the one-wave kernel and stay on this one for those flags.
     const bool one_wave = (h.flags & ERI_ADAM8_FLAG_ONE_WAVE) != 0;
     const bool kernel_named = (h.flags & (ERI_ADAM8_FLAG_BSEARCH | ERI_ADAM8_FLAG_NO_PIPELINE)) != 0;
-    const uint32_t units = total_blocks + n_tails; // a partial block costs what a full one does
     const bool few = (uint64_t)units <= (uint64_t)compute_units * (uint64_t)kSplitBlocksPerCu;
     if ((mixed && (h.flags & ERI_ADAM8_FLAG_BSEARCH) != 0) || (!kernel_named && !one_wave && few)) {
         const bool bnb = h.mode == ERI_ADAM8_MODE_BNB;
@@ -59,9 +61,9 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     }
     if (mixed) {
         const bool wd_m = h.mode == ERI_ADAM8_MODE_BNB ? h.weight_decay != 1.0f : h.weight_decay > 0.0f;
-        if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, units, layout, h, compute_units))
+        if ((h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(t, h, compute_units))
             return launch_step_pipelined_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs,
-                                                  step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
+                                                  step_fuses_ema(t, h, compute_units), rows, n_rows,
                                                   total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_grad_f32(h.mode, (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0, wd_m, gs, rows, n_rows,
                                           total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
@@ -69,21 +71,21 @@ int launch_step(const DevTensor *rows, uint32_t n_rows, uint32_t total_blocks, u
     if (h.mode == ERI_ADAM8_MODE_BNB) { // slot table only; the decay is a factor
         const bool wd = h.weight_decay != 1.0f;
         const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
-        if (bf16 && !kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
+        if (bf16 && !kernel_named && prefetch_pays(t, h, compute_units))
             return launch_step_pipelined(h.mode, exact, wd, gs, false, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         if (bf16) return launch_step_plain_bf16(h.mode, exact, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-        if (!kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
+        if (!kernel_named && prefetch_pays(t, h, compute_units))
             return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
         return launch_step_plain_f32(h.mode, wd, gs, true, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     }
     const bool wd = h.weight_decay > 0.0f;
     const bool exact = (h.flags & ERI_ADAM8_FLAG_EXACT_PARAM) != 0;
     const bool keytab = (h.flags & ERI_ADAM8_FLAG_BSEARCH) == 0;
-    if (!bf16 && !kernel_named && prefetch_pays(total_blocks, units, layout, h, compute_units))
+    if (!bf16 && !kernel_named && prefetch_pays(t, h, compute_units))
         return launch_step_pipelined_f32(h.mode, wd, gs, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     if (!bf16) return launch_step_plain_f32(h.mode, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
-    if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(total_blocks, units, layout, h, compute_units))
-        return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(units, layout, h, compute_units), rows, n_rows,
+    if (keytab && (h.flags & ERI_ADAM8_FLAG_NO_PIPELINE) == 0 && prefetch_pays(t, h, compute_units))
+        return launch_step_pipelined(h.mode, exact, wd, gs, step_fuses_ema(t, h, compute_units), rows, n_rows,
                                      total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
     return launch_step_plain_bf16(h.mode, exact, wd, gs, keytab, rows, n_rows, total_blocks, n_tails, h, lds_image, dev_scale, grid, wg, stream);
 }

@@ -300,6 +300,7 @@ struct EriAdam8Table {
         uint32_t n = 0;
         uint32_t total_blocks = 0; // full blocks only; a row's partial last block is handled per row
         uint32_t n_tails = 0;      // rows with a partial last block
+        uint32_t n_long = 0;       // rows whose partial last block is more than half a block
         char *mem = nullptr;              // device: kTableHead bytes, then what dev points to
         eri::DevTensor *dev = nullptr;    // n rows, then one uint32 row index per full block and one per partial block (BlockRowMap)
         eri::DevTensor *pinned = nullptr; // the rows only
@@ -981,6 +982,7 @@ static int table_create(const EriAdam8Tensor *rows, uint32_t n, bool grads_only,
         for (uint32_t j = 0; j < g.n; ++j) {
             full += rows[g.src[j]].numel / eri::kBlock;
             if (rows[g.src[j]].numel % eri::kBlock) ++g.n_tails;
+            if (rows[g.src[j]].numel % eri::kBlock > eri::kBlock / 2) ++g.n_long;
         }
         const size_t rows_bytes = sizeof(eri::DevTensor) * g.n;
         e = hipMalloc((void **)&g.mem, eri::kTableHead + rows_bytes + sizeof(uint32_t) * (size_t)(full + g.n_tails));
@@ -1146,10 +1148,11 @@ int eri_adam8_step_table(EriAdam8Table *t, const EriAdam8Hyper *h, void *stream)
     std::vector<EriEmaTensor> ema_rest;
     for (auto &g : t->groups) {
         if (g.n == 0 || (one_launch && (&g == &f32 || &g == &bf16))) continue;
-        shape(g.total_blocks + g.n_tails);
-        rc = eri::launch_step(g.dev, g.n, g.total_blocks, g.n_tails, g.dtype, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
+        const eri::TableShape shape_of = {g.total_blocks, g.n_tails, g.n_long, g.dtype};
+        shape(shape_of.units());
+        rc = eri::launch_step(g.dev, g.n, shape_of, hh, ctx->image, dev_scale, grid, waves_per_wg * eri::kWave, ctx->cus, stream);
         if (rc) return hip_fail((hipError_t)rc, "adam8 step launch");
-        if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(g.total_blocks + g.n_tails, g.dtype, hh, ctx->cus)) {
+        if ((hh.flags & ERI_ADAM8_FLAG_EMA) && !eri::step_fuses_ema(shape_of, hh, ctx->cus)) {
             // not the kernel that carries the EMA: this group's shadows join the plain sweep that follows the step
             for (uint32_t j = 0; j < g.n; ++j) {
                 const eri::DevTensor &d = g.pinned[j];

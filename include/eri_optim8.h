@@ -160,8 +160,8 @@ enum {
     ERI_ADAM8_FLAG_EMA = 1u << 6,         /* after the update, every row that has an ema_shadow also gets
                                              shadow = ema_decay*shadow + (1 - ema_decay)*p', the EMA update of
                                              src/trainers/ema_enhanced.rs:91-100 on the parameter as it was just
-                                             stored.  Tables of BF16 parameters (BF16 or F32 gradients) in mode
-                                             ERI beyond the small-table kernel's range do it inside the step
+                                             stored.  In mode ERI, tables of BF16 parameters above 24 blocks
+                                             per compute unit (14 with F32 gradients) do it inside the step
                                              kernel (the new parameter is still in registers: the separate
                                              sweep's read of p is saved); every other table runs one EMA sweep
                                              right after the step, in the same call.  Same results either way */

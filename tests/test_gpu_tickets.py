@@ -90,6 +90,19 @@ def test_both_sides_of_the_line_to_the_prefetching_kernel(layout, mode, over, ta
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("layout,mode", [("bf16", 0), ("bf16-f32-grads", 1), ("f32", 0)])
+@pytest.mark.parametrize("long_tails", [-1, 0, 1])
+def test_both_sides_of_the_line_for_long_partial_blocks(layout, mode, long_tails):
+    """Just as many partial blocks of more than half a block as the prefetching kernel takes, one fewer and one more."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    full = LINES[layout, mode] * UNITS + 6
+    tails = full // (3 if layout == "bf16" else 2) + long_tails
+    sizes = [2048 + 1025 + i % 9 for i in range(tails)] + [(full - tails) * 2048 + 1024]
+    for a, b in zip(whole._run(layout, mode, sizes, 0, 0.5), whole._run(layout, mode, sizes, L.FLAG_NO_PIPELINE, 0.5)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("layout,line", [("bf16", 24), ("bf16-f32-grads", 14)])
 @pytest.mark.parametrize("over", [0, 1])
 @pytest.mark.parametrize("tail", [0, 515])
@@ -147,10 +160,10 @@ def _time_of(layout, mode, sizes, kinds):
     return best
 
 
-@pytest.mark.parametrize("layout,mode,size", [("bf16", 0, 4095), ("bf16", 1, 4095), ("bf16", 2, 3549)])
+@pytest.mark.parametrize("layout,mode,size", [("bf16", 0, 4095), ("bf16", 1, 4095), ("bf16", 2, 3549), ("bf16-f32-grads", 1, 4095)])
 def test_tables_of_many_partial_blocks_take_no_longer_than_on_the_plain_kernel(layout, mode, size):
     """As many partial blocks as full ones, behind the line: 1.4 to 1.7 times as long when the prefetching kernel went
-    over the parts twice, a pass at a time."""
+    over the parts twice, a pass at a time, 1.1 to 1.2 times when it took them once."""
     from eridiffusion_amd import _lib as L
     ours, plain = _time_of(layout, mode, [size] * (140 * UNITS), [(0, False), (L.FLAG_NO_PIPELINE, False)])
-    assert ours < 1.18 * plain, (ours, plain)
+    assert ours < 1.06 * plain, (ours, plain)
