@@ -280,6 +280,21 @@ struct SweepUnit {
  *   ... fp32                                  62 | 71     89 | 96    120 | 126   287 | 277   2,606 | 2,364
  * Above it the list itself (8 bytes per block, uploaded when the rows' sizes change) is no longer small. */
 constexpr uint32_t kSmallSweepBlocksPerCu = 128;
+/* Nor is it needed there, except for partial blocks, of which the persistent kernels take one piece per wave ahead of
+ * their tickets, with eight waves per unit and nothing to hide behind.  Where these are most of a sweep the list is no
+ * longer than the rows are.  us per call, the small kernels | by ticket, 20,000 tensors (40,000 and 34,000 of the first two sizes):
+ *   elements                   301         1,501         2,148         3,075         5,597         9,693
+ *   EMA, bf16              30 |  95     53 | 133      61 |  91      69 | 106     106 | 160     181 | 236
+ *   ... fp32               36 |  66     96 | 104     112 | 113     140 | 128     218 | 221     381 | 376
+ *   32-bit step, bf16      74 | 270    204 | 311     226 | 275     287 | 319     451 | 478     768 | 776
+ *   ... with masters       82 | 273    261 | 309     292 | 326     371 | 352     588 | 577     997 | 954
+ *   ... fp32               77 | 180    249 | 257     287 | 281     361 | 304     566 | 530     975 | 903
+ * wide: fp32 tensors, or masters beside bf16 ones. */
+inline bool small_sweep(uint64_t units, uint64_t partial, bool wide, uint32_t compute_units) {
+    if (units <= (uint64_t)compute_units * kSmallSweepBlocksPerCu) return true;
+    const uint64_t full = units - partial;
+    return units < (1u << 20) && (wide ? partial > full : 2 * partial >= full);
+}
 
 /* units: the list of blocks, n_units of them, for the small kernels; null for the persistent ones, which take `grid`
  * workgroups.  scaled: every gradient is first multiplied by (grad_scale * row.scale) * (*dev_scale, 1 if null), as the

@@ -1578,9 +1578,14 @@ struct ElemCache {
                 const uint32_t n = (uint32_t)rows[gi].size();
                 g.n = 0;
                 if (n == 0) continue;
-                uint64_t units = 0;
-                for (const auto &r : rows[gi]) units += blocks_of(r.numel);
-                const bool small = units <= (uint64_t)cus * eri::kSmallSweepBlocksPerCu;
+                uint64_t units = 0, tails = 0;
+                bool wide = gi == 0;
+                for (const auto &r : rows[gi]) {
+                    units += blocks_of(r.numel);
+                    tails += r.numel % eri::kBlock != 0;
+                    wide = wide || r.e != nullptr;
+                }
+                const bool small = eri::small_sweep(units, tails, wide, cus);
                 // The list follows from the sizes alone.  Where these are what the slot had last -- gradients at new
                 // addresses every step -- it stays where it is: building and copying it (8 bytes per block) cost 13-15 us
                 // per call from 2,048 blocks on.

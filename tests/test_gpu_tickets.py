@@ -75,6 +75,72 @@ def test_sweeps_by_ticket(dtype, master, extra):
         assert torch.equal(a, b)
 
 
+def _sweep(what, dtype, sizes, parts):
+    """The sweep over tensors of these sizes, in `parts` calls; what it leaves behind, and the shortest us of a pass."""
+    import torch
+    from eridiffusion_amd import _lib as L
+    dt, tag = (torch.float32, L.DTYPE_F32) if dtype == "f32" else (torch.bfloat16, L.DTYPE_BF16)
+    stream = torch.cuda.current_stream().cuda_stream
+    at = [0]
+    for n in sizes:
+        at.append(at[-1] + (n + 15) // 16 * 16)
+    gen = torch.Generator(device="cuda").manual_seed(len(sizes))
+    p, g = [(torch.randn(at[-1], device="cuda", generator=gen) * s).to(dt) for s in (0.02, 1e-3)]
+    m, v, w = torch.randn(at[-1], device="cuda", generator=gen) * 1e-3, torch.rand(at[-1], device="cuda", generator=gen) * 1e-6, p.float()
+    calls = []
+    for k in range(parts):
+        ids = range(len(sizes) * k // parts, len(sizes) * (k + 1) // parts)
+        rows = ((L.EmaRow if what == "ema" else L.AdamW32Row) * len(ids))()
+        for r, i in zip(rows, ids):
+            r.p, r.numel, r.dtype_tag = p.data_ptr() + at[i] * p.element_size(), sizes[i], tag
+            if what == "ema":
+                r.shadow = g.data_ptr() + at[i] * g.element_size()
+            else:
+                r.g, r.m, r.v = g.data_ptr() + at[i] * g.element_size(), m.data_ptr() + 4 * at[i], v.data_ptr() + 4 * at[i]
+                r.master = w.data_ptr() + 4 * at[i] if dtype == "master" else None
+        calls.append(rows)
+    h, best = L.AdamW32Hyper(1e-3, 0.9, 0.999, 1e-8, 0.01), 1e9
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    for turn in range(4):
+        torch.cuda._sleep(20_000_000)  # the calls are queued before the first of them starts
+        ev[0].record()
+        for rows in calls:
+            if what == "ema":
+                L.check(L.lib().eri_ema_update_multi(rows, len(rows), 0.9, stream), "ema")
+            else:
+                L.check(L.lib().eri_adamw32_step_multi(rows, len(rows), C.byref(h), stream), "adamw32")
+        ev[1].record()
+        ev[1].synchronize()
+        if turn:  # the first uploads its rows
+            best = min(best, ev[0].elapsed_time(ev[1]) * 1000)
+    return (p, g, m, v, w), best
+
+
+@pytest.mark.parametrize("what,dtype,size", [("ema", "bf16", 301), ("ema", "f32", 301), ("ema", "bf16", 1501), ("adamw32", "bf16", 301),
+                                             ("adamw32", "master", 301), ("adamw32", "f32", 301)])
+def test_long_sweeps_of_partial_blocks_take_no_longer_in_one_call(what, dtype, size):
+    """40,000 tensors against twice 20,000, which take the small kernels by their number: 1.8 to 3.6 times as long on the
+    persistent ones."""
+    import torch
+    (one, t_one), (two, t_two) = (_sweep(what, dtype, [size] * 40_000, parts) for parts in (1, 2))
+    for a, b in zip(one, two):
+        assert torch.equal(a, b)
+    assert t_one < 1.4 * t_two, (t_one, t_two)
+
+
+@pytest.mark.parametrize("what,dtype,per_tail", [("ema", "bf16", 2), ("ema", "f32", 1), ("adamw32", "bf16", 2), ("adamw32", "master", 1), ("adamw32", "f32", 1)])
+@pytest.mark.parametrize("over", [-1, 0, 1])
+def test_both_sides_of_the_line_for_sweeps_of_partial_blocks(what, dtype, per_tail, over):
+    """`per_tail` full blocks to a partial one, and one block fewer and more, against the same tensors in two calls."""
+    import torch
+    sizes = [per_tail * 2048 + 1 + i * 13 % 2047 for i in range(22_000)] + [2048 * (1 + over)] * (over >= 0)
+    if over < 0:
+        sizes[0] -= 2048
+    one, two = (_sweep(what, dtype, sizes, parts)[0] for parts in (1, 3))
+    for a, b in zip(one, two):
+        assert torch.equal(a, b)
+
+
 LINES = {("bf16", 0): 48, ("bf16", 1): 96, ("bf16", 2): 128, ("bf16-f32-grads", 0): 48, ("bf16-f32-grads", 1): 48,
          ("bf16-f32-grads", 2): 56, ("f32", 0): 40, ("f32", 1): 48, ("f32", 2): 48}
 
