@@ -366,7 +366,11 @@ class Adam8bitFunctional:
     def load_state_from_tensors(self, state: Dict[str, Tuple[torch.Tensor, torch.Tensor]]) -> None:
         """The moments are read on the optimizer's stream, in its order.  Called under another stream, the moments (and
         the float32 copies made of them here) belong to that one: each is waited for before it is read, and the reading
-        before it may be freed or changed.  Otherwise device tensors that are read as they are share a launch."""
+        before it may be freed or changed.  Otherwise device tensors that are read as they are share a launch with those
+        next to them.  Names are loaded in the order of the dict; if any pair differs in size, none is."""
+        for name, (m, v) in state.items():
+            if m.numel() != v.numel():
+                raise ValueError("moments of %d and %d elements for '%s'" % (m.numel(), v.numel(), name))
         here = _stream_ptr()
         apart = here != self._stream
         together = []
@@ -374,11 +378,11 @@ class Adam8bitFunctional:
             as_is = [m, v]
             m = m.detach().to(torch.float32).contiguous().view(-1)
             v = v.detach().to(torch.float32).contiguous().view(-1)
-            if m.numel() != v.numel():
-                raise ValueError("moments of %d and %d elements for '%s'" % (m.numel(), v.numel(), name))
             if not apart and all(a.is_cuda and a.data_ptr() == b.data_ptr() for a, b in zip(as_is, (m, v))):
                 together.append((name, m, v))
                 continue
+            self._load_states(together)
+            together = []
             if apart:
                 check(lib().eri_hip_stream_sync(here), "eri_hip_stream_sync")
             check(lib().eri_adam8bit_fn_load_state_fp32(self._opt, name.encode(), m.data_ptr(), v.data_ptr(),
@@ -386,15 +390,17 @@ class Adam8bitFunctional:
             if apart:
                 check(lib().eri_hip_stream_sync(self._stream), "eri_hip_stream_sync")
             self._names[name] = None
-        k = len(together)
+        self._load_states(together)
+
+    def _load_states(self, rows) -> None:
+        k = len(rows)
         if k:
-            check(lib().eri_adam8bit_fn_load_states_fp32(self._opt, (C.c_char_p * k)(*[n.encode() for n, _, _ in together]),
-                                                         (C.c_void_p * k)(*[m.data_ptr() for _, m, _ in together]),
-                                                         (C.c_void_p * k)(*[v.data_ptr() for _, _, v in together]),
-                                                         (C.c_uint64 * k)(*[m.numel() for _, m, _ in together]), k),
+            check(lib().eri_adam8bit_fn_load_states_fp32(self._opt, (C.c_char_p * k)(*[n.encode() for n, _, _ in rows]),
+                                                         (C.c_void_p * k)(*[m.data_ptr() for _, m, _ in rows]),
+                                                         (C.c_void_p * k)(*[v.data_ptr() for _, _, v in rows]),
+                                                         (C.c_uint64 * k)(*[m.numel() for _, m, _ in rows]), k),
                   "eri_adam8bit_fn_load_states_fp32")
-            for name, _, _ in together:
-                self._names[name] = None
+            self._names.update(dict.fromkeys(n for n, _, _ in rows))
 
     def close(self) -> None:
         if self._opt:

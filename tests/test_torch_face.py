@@ -232,6 +232,38 @@ def test_moments_loaded_under_another_stream_are_waited_for(monkeypatch):
     assert [name.endswith("fp32") for name, _ in calls] == [False, True, False] * 2
 
 
+def test_moments_of_different_sizes_are_refused_before_any_is_loaded(monkeypatch):
+    from eridiffusion_amd import adam8bit
+    calls = []
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *args: calls.append(name) or 0
+    monkeypatch.setattr(adam8bit, "lib", lambda: Lib())
+    monkeypatch.setattr(adam8bit, "_stream_ptr", lambda: 11)
+    opt = adam8bit.Adam8bitFunctional()
+    del calls[:]
+    with pytest.raises(ValueError, match="8 and 9 elements for 'b'"):
+        opt.load_state_from_tensors({"a": (torch.zeros(8), torch.zeros(8)), "b": (torch.zeros(8), torch.zeros(9))})
+    assert calls == [] and not opt._names
+
+
+@pytest.mark.gpu
+def test_names_are_loaded_in_the_order_of_the_dict():
+    """Moments that are converted on the way between moments that are read as they are."""
+    from eridiffusion_amd.adam8bit import Adam8bitFunctional
+    state = {name: (torch.rand(3000, device="cuda").to(dt), torch.rand(3000, device="cuda").to(dt))
+             for name, dt in (("d", torch.float32), ("a", torch.float64), ("c", torch.float32), ("e", torch.bfloat16), ("b", torch.float32))}
+    opt = Adam8bitFunctional()
+    opt.load_state_from_tensors(state)
+    assert list(opt.get_state_as_tensors()) == list(state)
+    for name, (m, v) in state.items():
+        one = Adam8bitFunctional()
+        one.load_state_from_tensors({name: (m.float(), v.float())})
+        for a, b in zip(one.get_state_as_tensors()[name], opt.get_state_as_tensors()[name]):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("pooled", [False, True])
 def test_reload_under_another_stream(pooled):
