@@ -1556,7 +1556,9 @@ struct ElemCache {
         for (auto &c : slots)
             if (holds(c)) sl = &c;
         if (sl) {
-            if (sl->pending && hipEventQuery(sl->ev) == hipSuccess) sl->pending = false;
+            // A stream that is being captured is not asked about events of its own (that ends the capture); what it does
+            // next comes behind the upload in any case.
+            if (sl->pending && !(stream == sl->stream && is_capturing(stream)) && hipEventQuery(sl->ev) == hipSuccess) sl->pending = false;
             (void)hipGetLastError(); // hipErrorNotReady of the query is not an error
             if (sl->pending && stream != sl->stream) { // uploaded on another stream and perhaps still on its way
                 if (is_capturing(stream)) { // a capture cannot wait for an event from outside it
