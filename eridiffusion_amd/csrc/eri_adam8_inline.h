@@ -15,7 +15,7 @@
  * The grid is persistent: workgroups stage the lookup tables into LDS once, then their waves walk
  * the global block list, long lists in rounds of one block per wave that are handed out by ticket
  * (Tickets), so consecutive waves touch consecutive blocks.
- * The tensor that owns a block is found by a scalar binary search over the launch table.
+ * The step's tables name the tensor of every block (BlockRowMap); the sweeps search their rows for it.
  *
  * Arithmetic: every fp32 operation of the update is written as its own statement and the file is
  * compiled with -ffp-contract=off, because the reference runs each as a separate tensor op

@@ -246,7 +246,10 @@ int eri_adam8_table_update(EriAdam8Table *table, const EriAdam8Tensor *rows, uin
 int eri_adam8_table_destroy(EriAdam8Table *table);
 int eri_adam8_table_info(const EriAdam8Table *table, uint64_t *total_numel, uint64_t *total_blocks);
 
-/* One optimizer step over every tensor of the table: one kernel launch per dtype present. */
+/* One optimizer step over every tensor of the table: one kernel launch per dtype present.
+ * Launches of one table (steps and traffic probes, replays of graphs that hold them) must not overlap: besides the tensors
+ * themselves they share the counter that hands out the table's blocks, and after two at once a later launch may leave
+ * blocks out.  Launches on one stream, or ordered by events, do not overlap. */
 int eri_adam8_step_table(EriAdam8Table *table, const EriAdam8Hyper *hyper, void *stream);
 
 /* Global L2 norm of every gradient of the table and the clip factor it implies, both left in device
@@ -373,7 +376,9 @@ typedef struct EriAdamW32Hyper {
     float lr, beta1, beta2, eps, weight_decay; /* AdamWCfg, adamw.rs:7-8; lr is the per-call argument */
 } EriAdamW32Hyper;
 
-/* One launch per dtype over all rows; keeps a cached device copy of the rows per calling thread. */
+/* One launch per dtype over all rows; keeps a cached device copy of the rows per calling thread.  Calls of a thread over the
+ * same rows share that copy and its counter of blocks: they must not overlap, and nor may replays of graphs that hold
+ * them (see eri_adam8_step_table).  The same holds for eri_ema_update_multi. */
 int eri_adamw32_step_multi(const EriAdamW32Tensor *rows, uint32_t n, const EriAdamW32Hyper *hyper, void *stream);
 /* The same step with every gradient first multiplied by (grad_scale * row.grad_scale) * (*dev_scale), one rounded
  * fp32 product of the gradient with that factor, the factor formed in this order -- what the 8-bit step does with

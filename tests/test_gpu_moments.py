@@ -202,14 +202,14 @@ def test_loading_many_new_names_takes_time_by_their_number():
     import torch
     from eridiffusion_amd.adam8bit import Adam8bitFunctional, DevicePool
     x, times = torch.rand(64, device="cuda"), {}
-    for k in (2000, 2000, 16000):  # the first for warm-up
+    for k in (2000, 2000, 16000, 2000, 16000):  # the shorter of the two each; the first for warm-up
         opt = Adam8bitFunctional()
         opt.set_state_pool(DevicePool(32 << 20, 1), 0)
         rows = [("lora_unet_down_blocks_1_attentions_0_transformer_blocks_0_attn1_to_q.lora_down.weight.%d" % i, x, x, 64) for i in range(k)]
         torch.cuda.synchronize()
         start = time.perf_counter()
         assert _load_many(opt, rows) == 0
-        times[k] = time.perf_counter() - start
+        times[k] = min(times.get(k, 1e9), time.perf_counter() - start)
     assert times[16000] < 14 * times[2000], times  # eight times as many names; 30 with a search through those before
 
 

@@ -75,6 +75,29 @@ def test_sweeps_by_ticket(dtype, master, extra):
         assert torch.equal(a, b)
 
 
+def test_probe_step_and_step_with_ema_share_a_counter():
+    """In turn over one table, each with the rounds of its own; against the steps alone on the plain kernel, bit for bit."""
+    import torch
+    from test_gpu_graph_capture import _tensors
+    from eridiffusion_amd import _lib as L
+    sizes = [50 * UNITS * 2048 + 300, 2048, 77, 7 * 2048]
+    ours, plain = _tensors(sizes, 9), _tensors(sizes, 9)
+    stream = torch.cuda.current_stream().cuda_stream
+    for step in (1, 2, 3):
+        for flags in (L.FLAG_EMA, 0):
+            for (table, _, _, _), named in ((ours, 0), (plain, L.FLAG_NO_PIPELINE)):
+                if table is ours[0]:
+                    L.check(L.lib().eri_adam8_traffic_probe(table, stream), "traffic_probe")
+                h = L.hyper_pack(1e-3, 0.9, 0.999, 1e-8, 0.01, step, L.MODE_ERI, L.FLAG_EXACT_PARAM | flags | named)
+                h.ema_decay = 0.9
+                L.check(L.lib().eri_adam8_step_table(table, C.byref(h), stream), "step_table")
+    torch.cuda.synchronize()
+    for a, b in zip(ours[3], plain[3]):
+        assert torch.equal(a, b)
+    for tensors in (ours, plain):
+        L.lib().eri_adam8_table_destroy(tensors[0])
+
+
 def _sweep(what, dtype, sizes, parts):
     """The sweep over tensors of these sizes, in `parts` calls; what it leaves behind, and the shortest us of a pass."""
     import torch
