@@ -697,7 +697,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     // DEPTH passes, with 48 * DEPTH bytes per lane in flight (bf16; fp32 values hold twice the registers).
     static_assert(PARTIAL || !ROOMY, "a whole block has no end to stop at");
     constexpr int DEPTH = ROOMY ? 4 : ((BF16 && GBF16) ? 4 : 2) / (PARTIAL ? 2 : 1);
-    const uint32_t passes = ROOMY ? (n + 511) / 512 : 4;
+    const uint32_t passes = (n + 511) / 512;
 #pragma unroll
     for (int c0 = 0; c0 < 4; c0 += DEPTH) {
         Raw8<BF16> pr[DEPTH];
@@ -705,7 +705,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
         u32x2 mr[DEPTH], vr[DEPTH];
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
-            if ((uint32_t)(c0 + d) >= passes) continue;
+            if (ROOMY && (uint32_t)(c0 + d) >= passes) continue;
             const uint32_t o = (c0 + d) * 512 + lane * 8;
             const uint32_t count = lane_count(o, n);
             if (!PARTIAL || count == 8) {
@@ -723,7 +723,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const int c = c0 + d;
-            if ((uint32_t)c >= passes) continue;
+            if (ROOMY && (uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             float pv[8], gv[8], pn[8];
             pr[d].unpack(pv);
@@ -765,7 +765,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     if (dm.fast && dv.fast) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if ((uint32_t)c >= passes) continue;
+            if (ROOMY && (uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<true, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
@@ -775,7 +775,7 @@ __device__ __forceinline__ void full_block(const DevTensor &t, uint32_t lb, uint
     } else {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if ((uint32_t)c >= passes) continue;
+            if (ROOMY && (uint32_t)c >= passes) continue;
             const uint32_t o = c * 512 + lane * 8;
             u32x2 mw, vw;
             requant8<false, KEYTAB, MODE == ERI_ADAM8_MODE_BNB>(mf + c * 8, vf + c * 8, dm, dv, L, mw, vw);
