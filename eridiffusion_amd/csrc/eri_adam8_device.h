@@ -147,7 +147,12 @@ constexpr uint32_t kTwoDtypeBlocksPerCu = 64;
  *   fp32, mode L2        65 | 61     90 | 90                           242 | 256
  *   bf16, mode BNB       42 | 36     58 | 52     73 | 70     98 | 95   148 | 150   280 | 301   573 | 682
  *   ... fp32 gradients   45 | 39     63 | 62     81 | 84   107 | 115   166 | 180   321 | 350   655 | 781
- *   fp32, mode BNB       60 | 58     84 | 84                           220 | 241 */
+ *   fp32, mode BNB       60 | 58     84 | 84                           220 | 241
+ * Arrays side by side, as a caller's allocator places what it has for one model.  In lanes 48 GiB apart the plain kernel's
+ * fixed shares lose little, and the two are level to 3 % around the line (bf16, launches on other data each time; one
+ * table again and again is up to 2 % better for the plain kernel): 16,896 blocks 65 | 63, 21,997 with partial ones 83 | 83,
+ * 37,392 131 | 130, 74,784 257 | 262, 157,651 524 | 547.  The same run side by side: 67 | 69, 85 | 95, 135 | 147,
+ * 257 | 307, 533 | 664.  The line stands where the placement that costs more decides it. */
 inline uint32_t prefetch_blocks_per_cu(int mode, int layout) {
     if (mode == ERI_ADAM8_MODE_L2) return layout == kLayoutBF16 ? 96 : 48;
     if (mode == ERI_ADAM8_MODE_BNB) return layout == kLayoutBF16 ? 128 : layout == kLayoutBF16GradF32 ? 56 : 48;

@@ -3,10 +3,10 @@
  * dtypes of a list of tensors and their gradients, and allocating the tensors an update returns.  A step of an
  * adapter touches 60 to 1,400 tensors for 20 to 90 us of kernel, and the interpreter took about a microsecond per
  * tensor of a list and three per named tensor, so the host was what a step waited for.  Per step, before and after:
- *   1,400 LoRA tensors in a list                          1,547 -> 93 us (the kernel's time)
- *   400 ragged tensors, bf16 and fp32, in a list            445 -> 46 us (the same)
- *   256 short tensors, clipped, gradients at new addresses  349 -> 70 us
- *   60 named tensors, each with a new output                202 -> 57 us (60 allocations; 79 through the dispatcher)
+ *   1,400 LoRA tensors in a list                          1,547 -> 87 us (the kernel's time)
+ *   400 ragged tensors, bf16 and fp32, in a list            445 -> 36 us (the same)
+ *   256 short tensors, clipped, gradients at new addresses  349 -> 75 us
+ *   60 named tensors, each with a new output                202 -> 61 us (60 allocations; 79 through the dispatcher)
  *
  * Only plain cases are taken here: exact torch.Tensor / torch.nn.Parameter objects with a storage of their own, strided
  * and contiguous, no __torch_function__ mode active, a gradient that the step reads as it is.  Everything else is
